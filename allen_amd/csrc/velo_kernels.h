@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <algorithm>
 #include <cstdint>
 #include <cstddef>
 
@@ -377,8 +378,10 @@ namespace mlp {
 constexpr unsigned n_inputs = 10, n_hidden = 32;
 constexpr unsigned param_w1 = 0, param_b1 = 320, param_w2 = 352, param_b2 = 1376, param_w3 = 1408, param_b3 = 1440;
 constexpr unsigned n_params = 1441;
-constexpr unsigned rows_per_block = 64; // seeds per workgroup of the training and scoring kernels (two waves)
-inline unsigned mlp_blocks(unsigned n) { return (n + rows_per_block - 1) / rows_per_block; }
+constexpr unsigned rows_per_block = 128; // seeds per pass of a workgroup of the training and scoring kernels (four waves)
+// Workgroups of the training kernel, each with a partial gradient to be summed: one per CU at most.
+constexpr unsigned max_train_blocks = 256;
+inline unsigned mlp_blocks(unsigned n) { return n ? std::min((n - 1) / rows_per_block + 1, max_train_blocks) : 0u; }
 } // namespace mlp
 hipError_t launch_mlp_train(
   const float* features,
