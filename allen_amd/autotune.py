@@ -117,7 +117,7 @@ def tune_throughput(seqs, measure, n_events: int, candidates=THROUGHPUT_CANDIDAT
             apply(sq, knobs)
 
     # Every candidate is applied over the default, so knobs a candidate leaves out are reset.
-    base = {"search_block": 256, "search_lds_hits": 0, "search_ring_window": 0, "search_list_cap": 0}
+    base = {"search_block": 0, "search_lds_hits": 0, "search_ring_window": 0, "search_list_cap": 0}
     apply_all(base)
     default_ms = measure()
     reference = _outputs_digest(seqs[0], n_events)

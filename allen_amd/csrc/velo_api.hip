@@ -642,10 +642,10 @@ struct velo_sequence {
   size_t max_raw_bytes = 0;
   size_t sp_cap = 0, cluster_cap = 0, track_cap = 0, hits_cap = 0;
   std::map<std::string, std::pair<void*, size_t>> bufs;
-  unsigned search_block = 256;
+  unsigned search_block = 0; // 0: the launcher's choice from the number of events
   unsigned search_lds_hits = 0; // 0: the launcher's default for the kernel variant
-  unsigned search_ring_window = 0; // LDS window of the ring of tracks to follow; 0: 512
-  unsigned search_list_cap = 0;    // seeding's list of unused hits; 0: 1024
+  unsigned search_ring_window = 0; // LDS window of the ring of tracks to follow; 0: as above
+  unsigned search_list_cap = 0;    // seeding's list of unused hits; 0: as above
   bool search_largest_first = true;
   bool search_persistent = false;
   // The largest events (E / search_split of them, events by descending hit count) run on a
@@ -813,7 +813,7 @@ int velo_sequence_set_tuning(velo_sequence* s, const char* knob, unsigned value)
   const std::string k(knob);
   if (k == "search_block") {
     if (value && (value % 64 || value > 1024)) return VELO_ERR_INVALID_ARGUMENT;
-    s->search_block = value ? value : 256;
+    s->search_block = value;
     return VELO_OK;
   }
   if (k == "search_lds_hits") {

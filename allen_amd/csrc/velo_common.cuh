@@ -246,67 +246,64 @@ __device__ __forceinline__ uint64_t lanes_below_mask()
   return l == 0 ? 0ull : (~0ull >> (64 - l));
 }
 
-// Inclusive wave scan of u32.
+// The lanes below this one that are set in a ballot.
+__device__ __forceinline__ uint32_t rank_below(uint64_t ballot)
+{
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(ballot >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(ballot), 0u));
+}
+
+// Inclusive wave scan of u32 (the whole wave active): six adds with DPP operands, shifts within
+// the rows of 16 lanes and then the broadcasts of a row's last lane. No LDS round trip, where a
+// scan by shuffles takes six.
+template<int ctrl, int row_mask>
+__device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
+{
+  return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(v), ctrl, row_mask, 0xF, false));
+}
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v)
 {
-  const unsigned l = lane_id();
-#pragma unroll
-  for (unsigned d = 1; d < wave_size; d <<= 1) {
-    const uint32_t o = __shfl_up(v, d, wave_size);
-    if (l >= d) v += o;
-  }
+  v += dpp_or_zero<0x111, 0xF>(v); // row_shr:1
+  v += dpp_or_zero<0x112, 0xF>(v);
+  v += dpp_or_zero<0x114, 0xF>(v);
+  v += dpp_or_zero<0x118, 0xF>(v);
+  v += dpp_or_zero<0x142, 0xA>(v); // row_bcast:15 into rows 1 and 3
+  v += dpp_or_zero<0x143, 0xC>(v); // row_bcast:31 into rows 2 and 3
   return v;
 }
 
-// Block-wide exclusive scan of u32; `scratch` holds >= blockDim/64 + 1 u32 in LDS.
+// The waves' totals to every wave: exclusive prefix of this wave and the total of all. `scratch`
+// holds one u32 per wave (at most 64), written by each wave before; the scratch may be reused
+// when this returns. Every thread of the block must call it.
+__device__ __forceinline__ uint32_t block_wave_prefix(const uint32_t* scratch, uint32_t* total)
+{
+  const unsigned wave = threadIdx.x / wave_size;
+  const unsigned n_waves = (blockDim.x + wave_size - 1) / wave_size;
+  __syncthreads();
+  const uint32_t t = lane_id() < n_waves ? scratch[lane_id()] : 0u;
+  const uint32_t inc = wave_inclusive_scan(t);
+  *total = __builtin_amdgcn_readlane(inc, wave_size - 1);
+  const uint32_t before = __builtin_amdgcn_readlane(inc - t, __builtin_amdgcn_readfirstlane(wave));
+  __syncthreads();
+  return before;
+}
+
+// Block-wide exclusive scan of u32 over whole waves; `scratch` holds >= blockDim/64 u32 in LDS.
 // Returns the exclusive prefix of this thread and writes the block total to *total.
 // Every thread of the block must call it.
 __device__ __forceinline__ uint32_t block_exclusive_scan(uint32_t v, uint32_t* scratch, uint32_t* total)
 {
-  const unsigned wave = threadIdx.x / wave_size;
-  const unsigned n_waves = (blockDim.x + wave_size - 1) / wave_size;
   const uint32_t inc = wave_inclusive_scan(v);
-  if (lane_id() == wave_size - 1 || threadIdx.x == blockDim.x - 1) scratch[wave] = inc;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t s = 0;
-    for (unsigned w = 0; w < n_waves; ++w) {
-      const uint32_t t = scratch[w];
-      scratch[w] = s;
-      s += t;
-    }
-    scratch[n_waves] = s;
-  }
-  __syncthreads();
-  const uint32_t r = scratch[wave] + inc - v;
-  *total = scratch[n_waves];
-  __syncthreads();
-  return r;
+  if (lane_id() == wave_size - 1) scratch[threadIdx.x / wave_size] = inc;
+  return block_wave_prefix(scratch, total) + inc - v;
 }
 
 // Block-wide exclusive scan of a 0/1 flag through wave ballots.
 __device__ __forceinline__ uint32_t block_flag_scan(bool flag, uint32_t* scratch, uint32_t* total)
 {
-  const unsigned wave = threadIdx.x / wave_size;
-  const unsigned n_waves = (blockDim.x + wave_size - 1) / wave_size;
   const uint64_t b = __ballot(flag);
-  const uint32_t below = __popcll(b & lanes_below_mask());
-  if (lane_id() == 0) scratch[wave] = __popcll(b);
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint32_t s = 0;
-    for (unsigned w = 0; w < n_waves; ++w) {
-      const uint32_t t = scratch[w];
-      scratch[w] = s;
-      s += t;
-    }
-    scratch[n_waves] = s;
-  }
-  __syncthreads();
-  const uint32_t r = scratch[wave] + below;
-  *total = scratch[n_waves];
-  __syncthreads();
-  return r;
+  if (lane_id() == 0) scratch[threadIdx.x / wave_size] = __popcll(b);
+  return block_wave_prefix(scratch, total) + rank_below(b);
 }
 
 } // namespace velo

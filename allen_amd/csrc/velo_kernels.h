@@ -233,8 +233,8 @@ struct SearchLaunch {
   float phi_tolerance;
   float max_scatter;
   unsigned max_skipped_modules;
-  unsigned block_dim;          // 0 = 256
-  unsigned lds_hits;           // event hits staged in LDS (16 B each); 0 = search_default_lds_hits
+  unsigned block_dim;          // 0: the launcher's choice from the number of events (256 when scored or persistent)
+  unsigned lds_hits;           // event hits staged in LDS (16 B each); 0: as block_dim
   unsigned long long* work_stats; // optional: seeding evals, forwarding evals, extrapolations, search steps
   unsigned long long* event_clock = nullptr; // optional: per event, event_clock_words u64 of wall clock ticks
   // Optional: persistent mode, a resident grid whose workgroups take event slots from this
@@ -245,7 +245,7 @@ struct SearchLaunch {
   const float* scorer_params = nullptr;
   float scorer_threshold = 0.f;
   // LDS window of the ring of tracks to follow (a power of two, 64..512) and capacity of the
-  // seeding's list of unused hits (a multiple of 16, up to 1024); 0 = 512 and 1024.
+  // seeding's list of unused hits (a multiple of 16, up to 1024); 0: as block_dim.
   unsigned ring_window = 0;
   unsigned list_cap = 0;
 };

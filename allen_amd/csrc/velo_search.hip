@@ -18,67 +18,102 @@
 
 namespace velo {
 
-// LDS bytes per hit of the full layout: x, y, z (f32), phi (i16), flags (u8).
-constexpr unsigned search_bytes_per_hit = 15;
-// Default capacity of the list of unused hits of the previous module pair used by seeding step 1
+// LDS bytes per hit of the full layout: x, y, z (f32), then phi (i16) and flags in one word.
+constexpr unsigned search_bytes_per_hit = 16;
+// The mixed layout keeps phi (i16) and a flags byte.
+constexpr unsigned mixed_bytes_per_hit = 3;
+// Default capacity of the list of unused hits of the previous module pair used by seeding
 // (a launch parameter, at most 1024); a larger module pair takes the pendulum walk.
 constexpr unsigned unused_list_cap = 1024;
-// Default number of tracks to follow kept in LDS (a launch parameter: a power of two from 64 to
-// 512): the last ring_window positions of the ring (written through to
-// the ring in HBM, which holds all max_tracks_to_follow).
-constexpr unsigned ring_window = 512;
-constexpr unsigned ring_window_bytes = 4 + 4 + 2 + 1; // entry, last two hits, first hit, number of hits
+// Number of tracks to follow kept in LDS, the last positions of the ring (which is written through
+// to HBM and holds all max_tracks_to_follow): a launch parameter, a power of two from 64 to 512,
+// by default 1024. A forwarding step reads the ring and the tracks back from HBM when its entries
+// and those it writes exceed the window: at 512 positions that was the largest events, which set
+// the length of a launch.
+constexpr unsigned ring_window = 1024;
+constexpr unsigned max_ring_window_knob = 512;
 static_assert(max_tracks_to_follow % ring_window == 0, "window positions follow ring positions");
-static_assert(ring_window % 16 == 0, "the arrays after the window stay aligned");
 
-// Three 0/1 flags scanned at once over the block. Exclusive ranks in r[], totals in t[].
+// A window entry: the ring's entry and what forwarding reads of its track, in 8 bytes. last2: the
+// track's last two hits (low and high 16 bits). A seed (bit_seed) holds its tracklet's number in
+// 11 bits and its first hit in the 16 above; a track its number in 20 bits (an event has fewer
+// than 22 300 track slots; larger numbers stand for "beyond them") and its number of hits in the
+// 5 above. Both hold the skipped modules where the ring's entries do.
+constexpr unsigned seed_first_pos = 11, track_hits_pos = 20;
+constexpr uint32_t window_track_number = (1u << track_hits_pos) - 1;
+static_assert(max_tracks_to_follow == 1u << seed_first_pos && max_track_size < 32 && skipped_pos == 28, "window entry");
+__device__ __forceinline__ uint2 window_seed(uint32_t full, unsigned first, unsigned last2)
+{
+  return make_uint2(full | (first << seed_first_pos), last2);
+}
+__device__ __forceinline__ uint2 window_track(uint32_t skipped, uint32_t number, unsigned n_hits, unsigned last2)
+{
+  return make_uint2(skipped | min(number, window_track_number) | (n_hits << track_hits_pos), last2);
+}
+
+// The waves that work on the event: all of the workgroup's, or the first few of them (the others
+// have ended, and the hardware's barriers do not wait for them). A team of one wave needs no
+// barrier at all: its LDS accesses are performed in order.
+struct Team {
+  unsigned waves, lanes, wave; // wave: this wave's number
+  __device__ __forceinline__ void sync() const
+  {
+    if (waves > 1) {
+      __syncthreads();
+    }
+    else {
+      wave_fence();
+    }
+  }
+  static __device__ __forceinline__ void wave_fence()
+  {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
+};
+
+// Up to three 0/1 flags scanned at once over the team. Exclusive ranks in r[], totals in t[]
+// (wave-uniform, in scalar registers: they come from ballots and lane reads only).
 // One barrier: consecutive scans must alternate between two scratch buffers (a scan's reads of
 // its buffer are ordered before the next scan's barrier, hence before the reuse two scans on).
 struct Scan3 {
   uint32_t r[3];
   uint32_t t[3];
 };
-__device__ __forceinline__ Scan3 block_flag_scan3(bool f0, bool f1, bool f2, uint32_t* scratch)
+template<unsigned n>
+__device__ __forceinline__ Scan3 team_flag_scan(const Team& team, bool f0, bool f1, bool f2, uint2* scratch)
 {
-  if (blockDim.x == wave_size) {
-    // One wave: ranks straight from the ballots.
-    const uint64_t below = lanes_below_mask();
-    const uint64_t b0 = __ballot(f0), b1 = __ballot(f1), b2 = __ballot(f2);
-    Scan3 s;
-    s.r[0] = __popcll(b0 & below);
-    s.r[1] = __popcll(b1 & below);
-    s.r[2] = __popcll(b2 & below);
-    s.t[0] = __popcll(b0);
-    s.t[1] = __popcll(b1);
-    s.t[2] = __popcll(b2);
-    return s;
-  }
-  const unsigned wave = threadIdx.x / wave_size;
-  const unsigned n_waves = blockDim.x / wave_size;
-  const uint64_t below = lanes_below_mask();
-  const uint64_t b0 = __ballot(f0), b1 = __ballot(f1), b2 = __ballot(f2);
-  if (lane_id() == 0) {
-    scratch[3 * wave] = __popcll(b0);
-    scratch[3 * wave + 1] = __popcll(b1);
-    scratch[3 * wave + 2] = __popcll(b2);
-  }
-  __syncthreads();
+  const bool f[3] = {f0, f1, f2};
   Scan3 s;
-  s.r[0] = __popcll(b0 & below);
-  s.r[1] = __popcll(b1 & below);
-  s.r[2] = __popcll(b2 & below);
-  s.t[0] = s.t[1] = s.t[2] = 0;
-  for (unsigned w = 0; w < n_waves; ++w) {
-    const uint32_t c0 = scratch[3 * w], c1 = scratch[3 * w + 1], c2 = scratch[3 * w + 2];
-    if (w < wave) {
-      s.r[0] += c0;
-      s.r[1] += c1;
-      s.r[2] += c2;
-    }
-    s.t[0] += c0;
-    s.t[1] += c1;
-    s.t[2] += c2;
+#pragma unroll
+  for (unsigned k = 0; k < 3; ++k) {
+    s.r[k] = s.t[k] = 0;
+    if (k >= n) continue;
+    const uint64_t b = __ballot(f[k]);
+    s.r[k] = rank_below(b);
+    s.t[k] = __popcll(b);
   }
+  if (team.waves == 1) return s;
+  // Per wave: the first two counts as 16 bits each (at most 1024), the third in a word of its own.
+  if (lane_id() == 0) scratch[team.wave] = make_uint2(s.t[0] | (s.t[1] << 16), s.t[2]);
+  __syncthreads();
+  const uint2 c = scratch[min(lane_id(), team.waves - 1)];
+  uint32_t tot01 = 0, tot2 = 0, before01 = 0, before2 = 0;
+  for (unsigned w = 0; w < team.waves; ++w) {
+    if (w == team.wave) {
+      before01 = tot01;
+      before2 = tot2;
+    }
+    tot01 += __builtin_amdgcn_readlane(c.x, w);
+    if constexpr (n > 2) tot2 += __builtin_amdgcn_readlane(c.y, w);
+  }
+  s.r[0] += before01 & 0xFFFFu;
+  s.r[1] += before01 >> 16;
+  s.r[2] += before2;
+  s.t[0] = tot01 & 0xFFFFu;
+  s.t[1] = tot01 >> 16;
+  s.t[2] = tot2;
   return s;
 }
 
@@ -90,44 +125,47 @@ struct ModulePairData {
 };
 
 // Phi bucket tables of an event's module pairs (LDS, u8 entries, module pairs of at most 255
-// hits): entry b < phi_buckets is the first position whose phi lies in bucket b or above (bucket
-// of an int16 phi: (phi + 32768) >> 10), entry phi_buckets the number of hits.
-constexpr unsigned phi_buckets = 64;
-constexpr unsigned phi_table_stride = phi_buckets + 1;
+// hits): entry b < phi_buckets is the first position whose phi lies in bucket b or above, entry
+// phi_buckets the number of hits. 128 buckets: a window of the default tolerance then reads about
+// a third of a hit more than it holds (a module pair has some 40 hits), for 3.4 KB of LDS.
+constexpr unsigned phi_buckets = 128;
+constexpr unsigned phi_bucket_shift = 9;
+constexpr unsigned phi_table_stride = phi_buckets + 2; // even, so that two entries can be written at once
 constexpr unsigned phi_tables_bytes = (n_module_pairs * phi_table_stride + 15) & ~15u;
 constexpr unsigned no_phi_table = 0xFFFFFFFFu;
+__device__ __forceinline__ unsigned phi_bucket(int16_t phi)
+{
+  return static_cast<unsigned>(static_cast<uint16_t>(phi) ^ 0x8000u) >> phi_bucket_shift;
+}
 
-// Hits of one event, structure-of-arrays in LDS.
-// Per-hit flags byte of the LDS layouts: bit 0 = used (dev_hit_used), bit 1 = module parity of
-// the hit's sensor, ((id >> 18) & 0xFF) / 4 % 2. Marking a hit used ORs bit 0 in; lanes that mark
-// the same hit concurrently all store the same byte, so the read-modify-write cannot lose a bit.
+// Per-hit flags of the LDS layouts: bit 0 = used (dev_hit_used), bit 1 = module parity of
+// the hit's sensor, ((id >> 18) & 0xFF) / 4 % 2.
 constexpr uint8_t flag_used = 1, flag_odd = 2;
 
+struct Hit {
+  float x, y, z;
+  int16_t phi;
+  bool used, odd;
+};
+
+// Hits of one event in LDS, 16 bytes each: x, y, z, then phi in the low and the flags in the
+// high half of a word, so that one 128-bit read brings a hit (five reads of 1 to 4 bytes with an
+// address each before).
 struct LdsHits {
-  const float* xs;
-  const float* ys;
-  const float* zs;
-  const int16_t* ph;
-  uint8_t* flags;
+  uint4* h;
   const uint8_t* tables;
-  __device__ __forceinline__ float x(unsigned i) const { return xs[i]; }
-  __device__ __forceinline__ float y(unsigned i) const { return ys[i]; }
-  __device__ __forceinline__ float z(unsigned i) const { return zs[i]; }
-  __device__ __forceinline__ int16_t phi(unsigned i) const { return ph[i]; }
-  __device__ __forceinline__ const int16_t* phi_begin() const { return ph; }
-  __device__ __forceinline__ bool used(unsigned i) const { return (flags[i] & flag_used) != 0; }
-  __device__ __forceinline__ void mark_used(unsigned i) const { flags[i] |= flag_used; }
-  // Four hits at once: all four flags are read before any is written, so the four LDS round
-  // trips overlap (equal indices write equal values).
-  __device__ __forceinline__ void mark_used4(unsigned a, unsigned b, unsigned c, unsigned d) const
+  __device__ __forceinline__ Hit load(unsigned i) const
   {
-    const uint8_t fa = flags[a], fb = flags[b], fc = flags[c], fd = flags[d];
-    flags[a] = fa | flag_used;
-    flags[b] = fb | flag_used;
-    flags[c] = fc | flag_used;
-    flags[d] = fd | flag_used;
+    const uint4 v = h[i];
+    return {__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), static_cast<int16_t>(v.w & 0xFFFFu),
+            (v.w & (flag_used << 16)) != 0, (v.w & (flag_odd << 16)) != 0};
   }
-  __device__ __forceinline__ bool module_odd(unsigned i) const { return (flags[i] & flag_odd) != 0; }
+  __device__ __forceinline__ int16_t phi(unsigned i) const { return static_cast<int16_t>(h[i].w & 0xFFFFu); }
+  __device__ __forceinline__ bool used(unsigned i) const { return (h[i].w & (flag_used << 16)) != 0; }
+  __device__ __forceinline__ void mark_used(unsigned i) const
+  {
+    (void) __hip_atomic_fetch_or(&h[i].w, uint32_t(flag_used) << 16, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
 };
 
 // Module parity of a hit from its LHCbID (SearchByTriplet.cu:498-499).
@@ -140,21 +178,31 @@ struct GlobalHits {
   uint8_t* used_flags; // dev_hit_used
   const uint32_t* ids;
   const uint8_t* tables;
-  __device__ __forceinline__ float x(unsigned i) const { return xyz[3 * i]; }
-  __device__ __forceinline__ float y(unsigned i) const { return xyz[3 * i + 1]; }
-  __device__ __forceinline__ float z(unsigned i) const { return xyz[3 * i + 2]; }
+  __device__ __forceinline__ Hit load(unsigned i) const
+  {
+    return {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], ph[i], used_flags[i] != 0, module_parity(ids[i]) != 0};
+  }
   __device__ __forceinline__ int16_t phi(unsigned i) const { return ph[i]; }
-  __device__ __forceinline__ const int16_t* phi_begin() const { return ph; }
   __device__ __forceinline__ bool used(unsigned i) const { return used_flags[i] != 0; }
   __device__ __forceinline__ void mark_used(unsigned i) const { used_flags[i] = 1; }
-  __device__ __forceinline__ void mark_used4(unsigned a, unsigned b, unsigned c, unsigned d) const
+};
+
+// Hits of one event: phi and used flags in LDS, coordinates in global memory (events too large
+// for the full LDS layout). Lanes that mark the same hit concurrently all store the same byte, so
+// the read-modify-write cannot lose a bit.
+struct MixedHits {
+  const float* xyz;
+  const int16_t* ph;
+  uint8_t* flags;
+  const uint8_t* tables;
+  __device__ __forceinline__ Hit load(unsigned i) const
   {
-    used_flags[a] = 1;
-    used_flags[b] = 1;
-    used_flags[c] = 1;
-    used_flags[d] = 1;
+    const uint8_t f = flags[i];
+    return {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2], ph[i], (f & flag_used) != 0, (f & flag_odd) != 0};
   }
-  __device__ __forceinline__ bool module_odd(unsigned i) const { return module_parity(ids[i]) != 0; }
+  __device__ __forceinline__ int16_t phi(unsigned i) const { return ph[i]; }
+  __device__ __forceinline__ bool used(unsigned i) const { return (flags[i] & flag_used) != 0; }
+  __device__ __forceinline__ void mark_used(unsigned i) const { flags[i] |= flag_used; }
 };
 
 // Work counters of one thread (seeding evaluations, forwarding evaluations, extrapolations,
@@ -168,8 +216,8 @@ struct WorkCount {
 };
 
 // forwarding; h1 compaction; seeding step 1 split into the h0 search (h1 and phi reads, then
-// the search in the previous module pair), the pendulum walk, and the wait at the barrier that
-// ends the step; seeding steps 2 and 3; the rest.
+// the search in the previous module pair), the choice of the h0 candidates, and the wait at the
+// fence that ends the step; seeding steps 2 and 3; the rest.
 enum Phase {
   phase_forwarding,
   phase_compaction,
@@ -194,30 +242,30 @@ __device__ __forceinline__ void phase_mark(WorkCount& wc, Phase p)
   }
 }
 
-// First index i of the sorted array with array[i] >= value (the leftmost binary search of
-// BinarySearch.cuh, same result on every input). Eight-way: each round probes seven split
-// points at once (independent LDS reads) and keeps the eighth of the range that holds the
-// answer, so a module pair of n hits takes about log8(n) dependent round trips instead of
-// log2(n). `steps` counts the probes.
-template<bool count, typename T>
-__device__ __forceinline__ int counted_search(const T* array, unsigned size, T value, WorkCount& wc)
+// First position i of the sorted phis of hits [start, start + size) with phi >= value (the
+// leftmost binary search of BinarySearch.cuh, same result on every input). Eight-way: each round
+// probes seven split points at once (independent reads) and keeps the eighth of the range that
+// holds the answer, so n hits take about log8(n) dependent round trips instead of log2(n).
+// `steps` counts the probes.
+template<bool count, typename H>
+__device__ __forceinline__ unsigned counted_search(const H& hits, unsigned start, unsigned size, int16_t value, WorkCount& wc)
 {
-  unsigned lo = 0, hi = size; // answer in [lo, hi]; array[< lo] < value <= array[>= hi]
+  unsigned lo = 0, hi = size; // answer in [lo, hi]; phi[< lo] < value <= phi[>= hi]
   while (lo < hi) {
     const unsigned span = hi - lo;
     unsigned p[7];
     bool below[7];
-    T v[7];
+    int16_t v[7];
 #pragma unroll
     for (unsigned j = 0; j < 7; ++j) {
       p[j] = lo + ((j + 1) * span) / 8; // lo <= p[j] < hi, non-decreasing in j
-      v[j] = array[p[j]];
+      v[j] = hits.phi(start + p[j]);
     }
     // All seven reads are issued before the first compare waits for one (the scheduler would
     // otherwise interleave read, wait and compare, one LDS round trip per probe).
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (unsigned j = 0; j < 7; ++j) below[j] = v[j] < value; // true for a prefix of j (sorted array)
+    for (unsigned j = 0; j < 7; ++j) below[j] = v[j] < value; // true for a prefix of j (sorted)
     if constexpr (count) wc.steps += 7;
     unsigned nlo = lo, nhi = hi;
 #pragma unroll
@@ -229,86 +277,91 @@ __device__ __forceinline__ int counted_search(const T* array, unsigned size, T v
     lo = nlo;
     hi = nhi;
   }
-  return static_cast<int>(lo);
+  return lo;
 }
 
-// The same lower bound in a module pair's phi array through its bucket table: positions before
-// the value's bucket hold smaller phis and positions after it larger ones, so the answer is the
-// bucket's start plus the bucket's elements below the value (read directly for up to four, by
+// The same lower bound in a module pair through its bucket table: positions before the value's
+// bucket hold smaller phis and positions after it larger ones, so the answer is the bucket's
+// start plus the bucket's elements below the value (read directly for up to four, by
 // the 8-way search for more). Module pairs without a table take the 8-way search.
 template<bool count, typename H>
-__device__ __forceinline__ int mp_search(const H& hits, const ModulePairData& mp, int16_t value, WorkCount& wc)
+__device__ __forceinline__ unsigned mp_search(const H& hits, const ModulePairData& mp, int16_t value, WorkCount& wc)
 {
-  const int16_t* a = hits.phi_begin() + mp.hit_start;
-  if (mp.table == no_phi_table) return counted_search<count>(a, mp.hit_num, value, wc);
-  const unsigned b = static_cast<unsigned>(static_cast<uint16_t>(value) ^ 0x8000u) >> 10;
-  const uint8_t* t = hits.tables + mp.table;
-  const unsigned lo = t[b], hi = t[b + 1];
-  if (hi - lo > 4) return static_cast<int>(lo) + counted_search<count>(a + lo, hi - lo, value, wc);
+  if (mp.table == no_phi_table) return counted_search<count>(hits, mp.hit_start, mp.hit_num, value, wc);
+  const uint8_t* t = hits.tables + mp.table + phi_bucket(value);
+  const unsigned lo = t[0], hi = t[1];
+  if (hi - lo > 4) return lo + counted_search<count>(hits, mp.hit_start + lo, hi - lo, value, wc);
+  int16_t v[4];
+#pragma unroll
+  for (unsigned k = 0; k < 4; ++k) v[k] = hits.phi(mp.hit_start + (lo + k < hi ? lo + k : 0u));
   unsigned c = lo;
 #pragma unroll
-  for (unsigned k = 0; k < 4; ++k)
-    if (lo + k < hi && a[lo + k] < value) ++c;
-  return static_cast<int>(c);
+  for (unsigned k = 0; k < 4; ++k) c += lo + k < hi && v[k] < value ? 1u : 0u;
+  return c;
 }
 
-// Entry b of module pair mp's table: the lower bound of bucket b's first phi (b < phi_buckets),
-// or the number of hits.
-template<typename H>
-__device__ __forceinline__ uint8_t phi_table_entry(const H& hits, const ModulePairData& mp, unsigned b)
+// The phi bucket tables of all module pairs that have one, four module pairs per wave at a time:
+// a histogram of the hits' buckets in LDS (`hist`, phi_buckets 16-bit counts per module pair),
+// turned into positions by a wave scan, two buckets a lane. hist_waves: the waves that hist has
+// room for.
+constexpr unsigned hist_words = phi_buckets / 2;
+constexpr unsigned hist_bytes = 4 * hist_words * sizeof(uint32_t);
+// LDS of the ring's window, which first holds the tables' histograms.
+__host__ __device__ constexpr unsigned window_bytes(unsigned window)
 {
-  WorkCount wc;
-  return static_cast<uint8_t>(
-    b == phi_buckets ? mp.hit_num
-                     : counted_search<false>(hits.phi_begin() + mp.hit_start, mp.hit_num,
-                                             static_cast<int16_t>(static_cast<int>(b << 10) - 32768), wc));
+  return window * sizeof(uint2) > hist_bytes ? window * sizeof(uint2) : hist_bytes;
 }
-
-// Builds the tables of module pairs [m0, n_module_pairs) that have one (whole block; the
-// module-pair descriptors are in LDS and visible).
 template<typename H>
-__device__ __forceinline__ void build_phi_tables(const H& hits, const ModulePairData* mp, uint8_t* tables, unsigned m0)
+__device__ __forceinline__ void
+build_phi_tables(const H& hits, const ModulePairData* mp, uint8_t* tables, uint32_t* hist, unsigned hist_waves, const Team& team)
 {
-  for (unsigned t = m0 * phi_table_stride + threadIdx.x; t < n_module_pairs * phi_table_stride; t += blockDim.x) {
-    const unsigned m = t / phi_table_stride;
-    if (mp[m].table != no_phi_table) tables[t] = phi_table_entry(hits, mp[m], t % phi_table_stride);
+  static_assert(hist_words == wave_size, "two buckets per lane");
+  const unsigned builders = min(team.waves, hist_waves);
+  if (team.wave >= builders) return;
+  const unsigned l = lane_id();
+  uint32_t* h = hist + 4 * hist_words * team.wave;
+  const auto count = [&](unsigned u, int16_t phi) {
+    const unsigned b = phi_bucket(phi);
+    atomicAdd(&h[u * hist_words + b / 2], b & 1u ? 0x10000u : 1u);
+  };
+  for (unsigned m0 = 4 * team.wave; m0 < n_module_pairs; m0 += 4 * builders) {
+    unsigned start[4], n[4];
+    int16_t p[4];
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+      const unsigned m = min(m0 + u, n_module_pairs - 1);
+      const bool has = m0 + u < n_module_pairs && mp[m].table != no_phi_table;
+      start[u] = mp[m].hit_start;
+      n[u] = has ? mp[m].hit_num : 0u;
+      h[u * hist_words + l] = 0;
+    }
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) p[u] = l < n[u] ? hits.phi(start[u] + l) : int16_t(0);
+    Team::wave_fence();
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+      if (l < n[u]) count(u, p[u]);
+      for (unsigned i = l + wave_size; i < n[u]; i += wave_size) count(u, hits.phi(start[u] + i));
+    }
+    Team::wave_fence();
+#pragma unroll
+    for (unsigned u = 0; u < 4; ++u) {
+      const uint32_t c = h[u * hist_words + l];
+      const uint32_t both = (c & 0xFFFFu) + (c >> 16);
+      const uint32_t before = wave_inclusive_scan(both) - both;
+      if (m0 + u < n_module_pairs) {
+        uint16_t* t = reinterpret_cast<uint16_t*>(tables + (m0 + u) * phi_table_stride);
+        t[l] = static_cast<uint16_t>(before | (before + (c & 0xFFFFu)) << 8);
+        if (l == 0) t[phi_buckets / 2] = static_cast<uint16_t>(n[u]);
+      }
+    }
+    Team::wave_fence();
   }
 }
-
-// Module pairs whose tables are built at the start of an event; every other table is built
-// during an earlier seeding (see track_seeding's `build`), before its first use.
-constexpr unsigned phi_tables_at_start = 4;
-
-// Hits of one event: phi and used flags in LDS, coordinates in global memory (events too large
-// for the full LDS layout).
-struct MixedHits {
-  const float* xyz;
-  const int16_t* ph;
-  uint8_t* flags;
-  const uint8_t* tables;
-  __device__ __forceinline__ float x(unsigned i) const { return xyz[3 * i]; }
-  __device__ __forceinline__ float y(unsigned i) const { return xyz[3 * i + 1]; }
-  __device__ __forceinline__ float z(unsigned i) const { return xyz[3 * i + 2]; }
-  __device__ __forceinline__ int16_t phi(unsigned i) const { return ph[i]; }
-  __device__ __forceinline__ const int16_t* phi_begin() const { return ph; }
-  __device__ __forceinline__ bool used(unsigned i) const { return (flags[i] & flag_used) != 0; }
-  __device__ __forceinline__ void mark_used(unsigned i) const { flags[i] |= flag_used; }
-  // Four hits at once: all four flags are read before any is written, so the four LDS round
-  // trips overlap (equal indices write equal values).
-  __device__ __forceinline__ void mark_used4(unsigned a, unsigned b, unsigned c, unsigned d) const
-  {
-    const uint8_t fa = flags[a], fb = flags[b], fc = flags[c], fd = flags[d];
-    flags[a] = fa | flag_used;
-    flags[b] = fb | flag_used;
-    flags[c] = fc | flag_used;
-    flags[d] = fd | flag_used;
-  }
-  __device__ __forceinline__ bool module_odd(unsigned i) const { return (flags[i] & flag_odd) != 0; }
-};
 
 struct SearchShared {
   ModulePairData mp[n_module_pairs]; // hit range (event-relative) and module z of every module pair
-  uint32_t scan[2][3 * 16 + 4];      // block_flag_scan3 scratch, used alternately
+  uint2 scan[2][16];                 // team_flag_scan scratch, used alternately
 };
 
 // The event's counters, identical in every lane of the workgroup (updated from block-wide
@@ -322,25 +375,37 @@ struct Counters {
   unsigned scan_buffer = 0;
 };
 
-__device__ __forceinline__ Scan3 scan3(SearchShared& sh, Counters& c, bool f0, bool f1, bool f2)
+template<unsigned n>
+__device__ __forceinline__ Scan3 scan(const Team& team, SearchShared& sh, Counters& c, bool f0, bool f1 = false, bool f2 = false)
 {
-  const Scan3 s = block_flag_scan3(f0, f1, f2, sh.scan[c.scan_buffer]);
+  const Scan3 s = team_flag_scan<n>(team, f0, f1, f2, sh.scan[c.scan_buffer]);
   c.scan_buffer ^= 1u;
   return s;
 }
 
-// Seeding scratch for one chunk of h1 hits, blockDim entries each, in dynamic LDS.
-// Seeding scratch of a chunk of blockDim h1 hits: per h1, its h0 candidates (up to
-// max_h0_candidates), their number and the chosen seed (h0 | h2 << 16, or no_seed).
-static_assert(max_h0_candidates >= initial_seeding_h0_candidates, "room for every h0 candidate");
+// A module pair's descriptor in scalar registers (the index is the same in every lane).
+__device__ __forceinline__ ModulePairData module_pair_data(const SearchShared& sh, unsigned i)
+{
+  const ModulePairData m = sh.mp[i];
+  ModulePairData r;
+  r.hit_start = __builtin_amdgcn_readfirstlane(m.hit_start);
+  r.hit_num = __builtin_amdgcn_readfirstlane(m.hit_num);
+  r.z[0] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m.z[0])));
+  r.z[1] = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(m.z[1])));
+  r.table = __builtin_amdgcn_readfirstlane(m.table);
+  return r;
+}
+
+// Seeding scratch in dynamic LDS, blockDim entries of each: the unused hits of the current module
+// pair (one compaction chunk), the h0 candidate of every (h1, h0) pair, and in scored mode the
+// chosen seed of every h1 (h0 | h2 << 16, or no_seed).
 static_assert(initial_seeding_h0_candidates == 8 && seeding_h0_candidates == 4, "track_seeding splits lanes by K = 4 or 8");
 constexpr uint32_t no_seed = 0xFFFFFFFFu;
-constexpr unsigned seed_scratch_bytes_per_lane = 2 * max_h0_candidates + 4 + 2 + 1;
+constexpr unsigned seed_scratch_bytes_per_lane = 4 + 2 + 2;
 struct SeedScratch {
-  uint16_t* h0;
   uint32_t* seed;
-  uint16_t* h1_chunk; // unused hits of the current module pair, one compaction chunk
-  uint8_t* n_h0;
+  uint16_t* h0;
+  uint16_t* h1_chunk;
   uint16_t* unused;   // unused hits of the previous module pair (relative indices, ascending)
   uint16_t* before;   // per position of the previous module pair: the unused hits before it
   unsigned list_cap;  // entries of `unused` and `before`
@@ -353,12 +418,7 @@ struct EventOutputs {
   TrackletHits* three_hit_tracks;
   TrackletHits* tracklets;
   uint32_t* ttf;        // the ring of tracks to follow in HBM (max_tracks_to_follow entries)
-  uint32_t* ttf_window; // its last `window` positions, in LDS (position p at p & window_mask)
-  // Beside each window entry, what forwarding reads of its track: the last two hits (low and
-  // high 16 bits), the first hit (read for a three-hit seed) and the number of hits.
-  uint32_t* ttf_last2;
-  uint16_t* ttf_first;
-  uint8_t* ttf_n;
+  uint2* window_entries; // its last `window` positions in LDS (position p at p & window_mask)
   uint16_t* h1_indices;
   unsigned track_capacity;
   unsigned event_number;
@@ -369,59 +429,123 @@ struct EventOutputs {
   unsigned window_mask; // window - 1
 };
 
-// Four consecutive positions of an h2 window, read at once: position j of the window is hit
-// (c + j) % n of the module pair (SearchByTriplet.cu:393-395, 520-522); positions past the
-// module pair read the window's first hit and are not used.
-struct Window4 {
-  unsigned index[4];
-  int16_t phi[4];
-  bool used[4];
-  float x[4], y[4], z[4];
-  template<typename H>
-  __device__ __forceinline__ void
-  load(const H& hits, unsigned start, unsigned n, unsigned c, unsigned j0, bool with_used)
-  {
-    // c <= n (a lower bound) and j < n, so c + j < 2 n and one conditional subtraction wraps it.
-#pragma unroll
-    for (unsigned k = 0; k < 4; ++k) {
-      const unsigned j = j0 + k < n ? j0 + k : j0;
-      const unsigned w = c + j;
-      index[k] = start + (w >= n ? w - n : w);
-    }
-#pragma unroll
-    for (unsigned k = 0; k < 4; ++k) {
-      phi[k] = hits.phi(index[k]);
-      used[k] = with_used ? hits.used(index[k]) : false;
-      x[k] = hits.x(index[k]);
-      y[k] = hits.y(index[k]);
-      z[k] = hits.z(index[k]);
+// A line to be continued into a module pair: its start, slopes and phi at the module pair.
+struct Line {
+  float x0, y0, z0, tx, ty;
+  int16_t phi;
+};
+__device__ __forceinline__ float scatter_at(const Line& l, const Hit& h)
+{
+  const float dz = h.z - l.z0;
+  const float predx = l.x0 + l.tx * dz;
+  const float predy = l.y0 + l.ty * dz;
+  const float dx = predx - h.x;
+  const float dy = predy - h.y;
+  return dx * dx + dy * dy;
+}
+
+// The closest hit as the reference walks to it: from the leftmost hit at or above
+// phi - phi_tolerance, wrapping around, until one lies further than phi_tolerance from phi
+// (SearchByTriplet.cu:384-433, 520-560); unused_only: used hits are passed over (seeding).
+template<bool count, bool unused_only, typename H>
+__device__ __forceinline__ bool closest_hit_walk(
+  WorkCount& wc, const H& hits, const ModulePairData& mp, const Line& l, int16_t phi_tolerance, float& best, uint32_t& best_index)
+{
+  bool any = false;
+  unsigned p = counted_search<count>(hits, mp.hit_start, mp.hit_num, static_cast<int16_t>(l.phi - phi_tolerance), wc);
+  for (unsigned j = 0; j < mp.hit_num; ++j, ++p) {
+    if (p >= mp.hit_num) p -= mp.hit_num;
+    const Hit h = hits.load(mp.hit_start + p);
+    const int16_t phi_diff = h.phi - l.phi;
+    const int16_t abs_phi_diff = phi_diff < 0 ? -phi_diff : phi_diff;
+    if (abs_phi_diff > phi_tolerance) break;
+    if (unused_only && h.used) continue;
+    if constexpr (count) ++(unused_only ? wc.seed_eval : wc.fwd_eval);
+    const float scatter = scatter_at(l, h);
+    if (scatter < best) {
+      best = scatter;
+      best_index = mp.hit_start + p;
+      any = true;
     }
   }
-};
+  return any;
+}
 
-// SearchByTriplet.cu:272-292
-template<bool count, typename H>
-__device__ __forceinline__ void find_forward_candidate(
-  WorkCount& wc,
-  const H& hits,
-  const ModulePairData& mp,
-  float h0x,
-  float h0y,
-  float tx,
-  float ty,
-  float dz,
-  int16_t phi_tolerance,
-  int16_t& candidate,
-  int16_t& extrapolated_phi)
+// Tolerances up to this one (an eighth of a turn) make every walk one run of the sorted hits.
+constexpr int16_t max_run_tolerance = 8192;
+
+// The hit of a module pair closest to a line: the first strict minimum of the scatter below
+// `best`, in the order of closest_hit_walk and with the same result. Returns whether there is one.
+// The hits within the tolerance are one run of the module pair's circle of hits, and the phi
+// buckets of its two ends bound it from both sides with two table reads, so no search for its
+// start and no hit read to find its end: the run and the few hits of the end buckets outside
+// it are read four at a time and evaluated without branches, which lets their arithmetic overlap
+// (one dependent operation takes 8 cycles here, an independent one 5; an LDS read 64). Nearly
+// always one pass of four serves the whole wave. Where the walk differs from the run: its
+// |difference| of 16 bits takes a hit exactly opposite for one within any tolerance, which it can
+// reach only as its first hit, with none in the run; those lanes, and tolerances
+// beyond max_run_tolerance, take the walk itself.
+template<bool count, bool unused_only, typename H>
+__device__ __forceinline__ bool closest_hit(
+  WorkCount& wc, const H& hits, const ModulePairData& mp, const Line& l, int16_t phi_tolerance, float& best, uint32_t& best_index)
+{
+  const unsigned n = mp.hit_num;
+  if (n == 0) return false;
+  if (phi_tolerance < 0 || phi_tolerance > max_run_tolerance)
+    return closest_hit_walk<count, unused_only>(wc, hits, mp, l, phi_tolerance, best, best_index);
+  const int16_t from = static_cast<int16_t>(l.phi - phi_tolerance), to = static_cast<int16_t>(l.phi + phi_tolerance);
+  unsigned lo, hi;
+  if (mp.table == no_phi_table) {
+    lo = counted_search<count>(hits, mp.hit_start, n, from, wc);
+    hi = to == 32767 ? n : counted_search<count>(hits, mp.hit_start, n, static_cast<int16_t>(to + 1), wc);
+  }
+  else {
+    const uint8_t* t = hits.tables + mp.table;
+    lo = t[phi_bucket(from)];
+    hi = t[phi_bucket(to) + 1];
+  }
+  const unsigned length = to < from ? n - lo + hi : hi - lo;
+  const unsigned width = 2u * static_cast<unsigned>(phi_tolerance);
+  // Position lo + j of the circle; positions beyond the run only stay in range.
+  const auto position = [&](unsigned j) { return mp.hit_start + min(min(lo + j, lo + j - n), n - 1); };
+  const int16_t after = hits.phi(position(length));
+  bool any = false, none_in_run = true;
+  for (unsigned j0 = 0; j0 < length; j0 += 4) {
+    unsigned index[4];
+    Hit h[4];
+#pragma unroll
+    for (unsigned k = 0; k < 4; ++k) index[k] = position(j0 + k);
+#pragma unroll
+    for (unsigned k = 0; k < 4; ++k) h[k] = hits.load(index[k]);
+    __builtin_amdgcn_sched_barrier(0); // all four reads are in flight before the first is waited for
+#pragma unroll
+    for (unsigned k = 0; k < 4; ++k) {
+      const float scatter = scatter_at(l, h[k]);
+      const bool in_run = j0 + k < length && static_cast<uint16_t>(h[k].phi - from) <= width;
+      none_in_run = none_in_run && !in_run;
+      const bool visited = in_run && !(unused_only && h[k].used);
+      if constexpr (count) (unused_only ? wc.seed_eval : wc.fwd_eval) += visited;
+      const bool closer = visited && scatter < best;
+      best = closer ? scatter : best;
+      best_index = closer ? index[k] : best_index;
+      any = any || closer;
+    }
+  }
+  if (none_in_run && static_cast<uint16_t>(after - l.phi) == 0x8000u)
+    return closest_hit_walk<count, unused_only>(wc, hits, mp, l, phi_tolerance, best, best_index);
+  return any;
+}
+
+// SearchByTriplet.cu:272-292: the phi at dz along the line from h0.
+template<bool count>
+__device__ __forceinline__ int16_t extrapolated_phi(WorkCount& wc, float h0x, float h0y, float tx, float ty, float dz)
 {
   const float predx = tx * dz;
   const float predy = ty * dz;
   const float xp = h0x + predx;
   const float yp = h0y + predy;
-  const int16_t phi = hit_phi_16(xp, yp);
   if constexpr (count) ++wc.extrap;
-  candidate = static_cast<int16_t>(mp_search<count>(hits, mp, static_cast<int16_t>(phi - phi_tolerance), wc));
-  extrapolated_phi = phi;
+  return hit_phi_16(xp, yp);
 }
 
 // The learned scorer's weights in LDS (scored mode): W1 (K padded to 16) and W2 as bf16, the
@@ -542,9 +666,10 @@ template<typename H>
 __device__ __forceinline__ void
 seed_features(const H& hits, unsigned h0, unsigned h1, unsigned h2, unsigned module_pair, float* f)
 {
-  const float x0 = hits.x(h0), y0 = hits.y(h0), z0 = hits.z(h0);
-  const float x1 = hits.x(h1), y1 = hits.y(h1), z1 = hits.z(h1);
-  const float x2 = hits.x(h2), y2 = hits.y(h2), z2 = hits.z(h2);
+  const Hit a = hits.load(h0), b = hits.load(h1), c = hits.load(h2);
+  const float x0 = a.x, y0 = a.y, z0 = a.z;
+  const float x1 = b.x, y1 = b.y, z1 = b.z;
+  const float x2 = c.x, y2 = c.y, z2 = c.z;
   const float td = 1.0f / (z1 - z0);
   const float tx = (x1 - x0) * td;
   const float ty = (y1 - y0) * td;
@@ -555,8 +680,8 @@ seed_features(const H& hits, unsigned h0, unsigned h1, unsigned h2, unsigned mod
   const float dz1 = z1 - z0;
   const float dx1 = (x0 + ((x2 - x0) * td02) * dz1) - x1;
   const float dy1 = (y0 + ((y2 - y0) * td02) * dz1) - y1;
-  const int16_t dphi01 = static_cast<int16_t>(hits.phi(h1) - hits.phi(h0));
-  const int16_t dphi12 = static_cast<int16_t>(hits.phi(h2) - hits.phi(h1));
+  const int16_t dphi01 = static_cast<int16_t>(b.phi - a.phi);
+  const int16_t dphi12 = static_cast<int16_t>(c.phi - b.phi);
   f[0] = dx2 * 4.0f;
   f[1] = dy2 * 4.0f;
   f[2] = dx1 * 4.0f;
@@ -569,90 +694,100 @@ seed_features(const H& hits, unsigned h0, unsigned h1, unsigned h2, unsigned mod
   f[9] = static_cast<float>(module_pair) * (1.0f / 32.0f);
 }
 
-// The first K unused hits of the previous module pair in the pendulum order of track_seeding
-// (SearchByTriplet.cu:348-370), from the ascending list `unused` (u entries) of the module
-// pair's unused hits (relative indices) instead of a walk over every position.
-// The pendulum visits position start + off, off = 0, +1, -1, +2, -2, ..., each wrapped once
-// into [0, n): position x gets rank 2d - 1 if d = (x - start) mod n lies in [1, n/2] (right of
-// start), else 2 ((start - x) mod n) (left, start itself included); ranks are a permutation of
-// 0..n-1, and the walk keeps the unused positions of the K smallest ranks, in rank order. Those
-// are among the K nearest unused entries on either side of start in the circular list, so the
-// 2K entries around its lower bound (all u if u <= 2K) are ranked, sorted by a fixed Batcher
-// odd-even merge network on (rank, position) keys, and the first K taken. Writes hit_start +
-// position to out[0..) and returns how many (<= K).
-template<unsigned K>
-__device__ __forceinline__ unsigned h0_candidates_from_list(
-  const uint16_t* unused,
-  const uint16_t* before,
-  unsigned u,
-  unsigned n,
-  unsigned hit_start,
-  int start,
-  uint16_t* out)
+// For the wave's seeding lanes: values of the other lanes of a group of K = 4 or 8, and the least
+// key of the group, by DPP moves (quad permutations, and the mirror of half a row for K = 8).
+template<int ctrl>
+__device__ __forceinline__ uint32_t dpp(uint32_t v)
 {
-  if (u == 0) return 0;
-  const unsigned s0 = static_cast<unsigned>(start) >= n ? static_cast<unsigned>(start) - n : static_cast<unsigned>(start);
-  // The lower bound of s0 in the list: the number of unused positions below s0.
-  const unsigned p = before[s0];
-  // key = rank << 16 | position (n <= 1024 on this path: rank < 2048, position < 1024).
-  constexpr unsigned M = 2 * K;
-  constexpr unsigned none = 0xFFFFFFFFu;
-  const bool all = u <= M;
-  unsigned key[M];
-#pragma unroll
-  for (unsigned j = 0; j < M; ++j) {
-    unsigned ix;
-    if (all) {
-      ix = j < u ? j : 0u;
-    }
-    else {
-      const int q = static_cast<int>(p) + static_cast<int>(j) - static_cast<int>(K);
-      ix = static_cast<unsigned>(q < 0 ? q + static_cast<int>(u) : (q >= static_cast<int>(u) ? q - static_cast<int>(u) : q));
-    }
-    const unsigned x = unused[ix];
-    const unsigned d = x >= s0 ? x - s0 : x + n - s0;
-    const unsigned r = d == 0 ? 0u : (d <= n / 2 ? 2 * d - 1 : 2 * (n - d));
-    key[j] = (!all || j < u) ? (r << 16 | x) : none;
+  return static_cast<uint32_t>(__builtin_amdgcn_mov_dpp(static_cast<int>(v), ctrl, 0xF, 0xF, true));
+}
+constexpr int dpp_xor1 = 0xB1, dpp_xor2 = 0x4E, dpp_xor3 = 0x1B, dpp_half_mirror = 0x141;
+
+// How many of a group's 2 K keys (two per lane) lie below `mine`, of which a and b are this
+// lane's own pair.
+__device__ __forceinline__ uint32_t below4(uint32_t a, uint32_t b, uint32_t mine)
+{
+  uint32_t c = 0;
+  c += dpp<dpp_xor1>(a) < mine ? 1u : 0u;
+  c += dpp<dpp_xor2>(a) < mine ? 1u : 0u;
+  c += dpp<dpp_xor3>(a) < mine ? 1u : 0u;
+  c += dpp<dpp_xor1>(b) < mine ? 1u : 0u;
+  c += dpp<dpp_xor2>(b) < mine ? 1u : 0u;
+  c += dpp<dpp_xor3>(b) < mine ? 1u : 0u;
+  return c;
+}
+
+template<int ctrl>
+__device__ __forceinline__ void least(uint32_t& hi, uint32_t& lo)
+{
+  const uint32_t oh = dpp<ctrl>(hi), ol = dpp<ctrl>(lo);
+  const bool less = oh < hi || (oh == hi && ol < lo);
+  hi = less ? oh : hi;
+  lo = less ? ol : lo;
+}
+
+// The seeds of the lanes with `found`, appended to the tracklets and the tracks to follow in lane order.
+__device__ __forceinline__ void append_seeds(
+  const Team& team, SearchShared& sh, Counters& cn, const EventOutputs& o, bool found, unsigned h0, unsigned h1, unsigned h2)
+{
+  const Scan3 s = scan<1>(team, sh, cn, found);
+  if (found) {
+    const unsigned tn = (cn.ttf + s.r[0]) % max_tracks_to_follow;
+    TrackletHits tl;
+    tl.hits[0] = static_cast<uint16_t>(h0);
+    tl.hits[1] = static_cast<uint16_t>(h1);
+    tl.hits[2] = static_cast<uint16_t>(h2);
+    o.tracklets[tn] = tl;
+    o.ttf[tn] = bit_seed | tn;
+    o.window_entries[tn & o.window_mask] = window_seed(bit_seed | tn, h0, h1 | (h2 << 16));
   }
-  // Batcher's odd-even merge sort of the M keys (compile-time indices: a fixed network of
-  // min/max pairs on registers).
+  cn.ttf += s.t[0];
+}
+
+// One record of the seed log; features and logit as the scorer had them, or computed here.
+template<typename H>
+__device__ __forceinline__ void log_seed(
+  const H& hits, const EventOutputs& o, unsigned module_pair, unsigned h0, unsigned h1, unsigned h2, const float* features,
+  const float* logit)
+{
+  const unsigned slot = atomicAdd(o.seed_log.counter, 1u);
+  if (slot >= o.seed_log.capacity) return;
+  uint32_t* rec = o.seed_log.records + 5 * (size_t) slot;
+  rec[0] = o.event_number;
+  rec[1] = module_pair;
+  rec[2] = h0;
+  rec[3] = h1;
+  rec[4] = h2;
+  float f[n_seed_features];
+  if (!features) seed_features(hits, h0, h1, h2, module_pair, f);
+  float* fo = o.seed_log.features + n_seed_features * (size_t) slot;
 #pragma unroll
-  for (unsigned pp = 1; pp < M; pp <<= 1) {
-#pragma unroll
-    for (unsigned k = pp; k >= 1; k >>= 1) {
-#pragma unroll
-      for (unsigned j = k % pp; j + k < M; j += 2 * k) {
-#pragma unroll
-        for (unsigned i = 0; i < k && i + j + k < M; ++i) {
-          if ((i + j) / (2 * pp) == (i + j + k) / (2 * pp)) {
-            const unsigned a = key[i + j], b = key[i + j + k];
-            key[i + j] = min(a, b);
-            key[i + j + k] = max(a, b);
-          }
-        }
-      }
-    }
-  }
-  unsigned found = 0;
-#pragma unroll
-  for (unsigned k = 0; k < K; ++k) {
-    if (key[k] != none) {
-      out[k] = static_cast<uint16_t>(hit_start + (key[k] & 0xFFFFu));
-      found = k + 1;
-    }
-  }
-  return found;
+  for (unsigned k = 0; k < n_seed_features; ++k) fo[k] = features ? features[k] : f[k];
+  if (logit && o.seed_log.logits) o.seed_log.logits[slot] = *logit;
 }
 
 // SearchByTriplet.cu:298-446, ordered, with the (h1, h0) pairs spread over lanes.
 //
 // The reference walks, per h1, its h0 candidates in pendulum order and, per h0, the h2 window
-// in phi order, keeping the first strictly smaller scatter. Here a chunk of blockDim unused h1
-// hits is processed at once (K = h0 candidates considered): every lane collects the h0
-// candidates of one h1, then in rounds of C = blockDim / K h1 hits every lane scores one
-// (h1, h0) pair over its h2 window (first strict minimum) and the K lanes of an h1 keep the
-// first strict minimum over its h0 candidates in pendulum order by cross-lane exchanges: the
-// same pair the sequential double loop selects. The chunk's seeds are then appended in h1 order.
+// in phi order, keeping the first strictly smaller scatter. Here rounds of C = lanes / K unused h1
+// hits (K = h0 candidates considered) give every (h1, h0) pair a lane: the K lanes of an h1 choose
+// its h0 candidates together, each scores its own over the h2 window (first strict minimum), and
+// they keep the first strict minimum over the candidates in pendulum order: the same pair the
+// sequential double loop selects. The round's seeds are appended in h1 order. Nothing between the
+// choice of the candidates and the append crosses a wave, so a round has one barrier (in the
+// append's scan) where it had three, and the choice takes two keys per lane where one lane ranked
+// and sorted eight or sixteen.
+//
+// Choice of the h0 candidates, the first K unused hits of the previous module pair in the pendulum
+// order (SearchByTriplet.cu:348-370), from the ascending list `unused` (u entries) of the module
+// pair's unused hits (relative indices) instead of a walk over every position: the pendulum
+// visits position start + off, off = 0, +1, -1, +2, -2, ..., each wrapped once into [0, n), so
+// position x gets rank 2d - 1 if d = (x - start) mod n lies in [1, n/2] (right of start), else
+// 2 ((start - x) mod n) (left, start itself included); ranks are a permutation of 0..n-1, and the
+// walk keeps the unused positions of the K smallest ranks, in rank order. Those are among the K
+// nearest unused entries on either side of start in the circular list, so of the 2 K entries
+// around its lower bound (all u if u <= 2 K) every lane takes two, and an entry with c < K
+// smaller ranks is candidate number c.
 template<bool count, int seed_mode, typename H>
 __device__ __forceinline__ void track_seeding(
   WorkCount& wc,
@@ -661,272 +796,199 @@ __device__ __forceinline__ void track_seeding(
   SearchShared& sh,
   Counters& cn,
   const EventOutputs& o,
+  const Team& team,
   const ModulePairData prev,
   const ModulePairData cur,
   const ModulePairData next,
   unsigned module_pair,
   float max_scatter,
   int16_t phi_tolerance,
-  unsigned h0_candidates_to_consider,
-  const ModulePairData* build,
-  uint8_t* tables)
+  unsigned K)
 {
-  const unsigned K = h0_candidates_to_consider;
   const unsigned log2K = K == 8 ? 3u : 2u; // K is 4 or 8
-  const unsigned C = blockDim.x >> log2K;
+  const unsigned C = team.lanes >> log2K;
   const float dz_next = next.z[0] - prev.z[0];
+  const unsigned tid = threadIdx.x;
 
-  // The list of unused hits of the previous module pair for step 1 (its writes are ordered
-  // before step 1 by the barrier of the compaction scan below).
-  // The first blockDim hits of both lists are compacted by one scan (seeding marks no hit used,
+  // The list of unused hits of the previous module pair (its writes are ordered
+  // before the rounds by the barrier before them).
+  // The first team.lanes hits of both lists are compacted by one scan (seeding marks no hit used,
   // so both read the flags the last forwarding left).
   const bool use_list = prev.hit_num <= ss.list_cap;
-  const bool free0 = use_list && threadIdx.x < prev.hit_num && !hits.used(prev.hit_start + threadIdx.x);
-  const bool act0 = threadIdx.x < cur.hit_num && !hits.used(cur.hit_start + threadIdx.x);
-  const Scan3 first = scan3(sh, cn, free0, act0, false);
-  if (free0) ss.unused[first.r[0]] = static_cast<uint16_t>(threadIdx.x);
-  if (use_list && threadIdx.x < prev.hit_num) ss.before[threadIdx.x] = static_cast<uint16_t>(first.r[0]);
+  const bool free0 = use_list && tid < prev.hit_num && !hits.used(prev.hit_start + tid);
+  const bool act0 = tid < cur.hit_num && !hits.used(cur.hit_start + tid);
+  const Scan3 first = scan<2>(team, sh, cn, free0, act0);
+  if (free0) ss.unused[first.r[0]] = static_cast<uint16_t>(tid);
+  if (use_list && tid < prev.hit_num) ss.before[tid] = static_cast<uint16_t>(first.r[0]);
   unsigned n_unused = first.t[0];
   if (use_list) {
-    for (unsigned c0 = blockDim.x; c0 < prev.hit_num; c0 += blockDim.x) {
-      const unsigned r = c0 + threadIdx.x;
+    for (unsigned c0 = team.lanes; c0 < prev.hit_num; c0 += team.lanes) {
+      const unsigned r = c0 + tid;
       const bool free_hit = r < prev.hit_num && !hits.used(prev.hit_start + r);
-      const Scan3 sc = scan3(sh, cn, free_hit, false, false);
+      const Scan3 sc = scan<1>(team, sh, cn, free_hit);
       if (free_hit) ss.unused[n_unused + sc.r[0]] = static_cast<uint16_t>(r);
       if (r < prev.hit_num) ss.before[r] = static_cast<uint16_t>(n_unused + sc.r[0]);
       n_unused += sc.t[0];
     }
   }
 
-  // The phi table of module pair `build` (first searched in the forwarding after the next
-  // seeding, so any later barrier orders it), by the block's last wave: during step 1 of the
-  // first chunk, where that wave is idle when the chunk has no more h1 hits than the other waves
-  // have lanes, or here when the module pair has no hit to seed from.
-  const auto build_table = [&]() {
-    if (!build || build->table == no_phi_table) return;
-    const unsigned builders = blockDim.x > wave_size ? blockDim.x - wave_size : 0u;
-    if (threadIdx.x >= builders) {
-      const unsigned b = threadIdx.x - builders;
-      tables[build->table + b] = phi_table_entry(hits, *build, b);
-      if (b == 0) tables[build->table + phi_buckets] = static_cast<uint8_t>(build->hit_num);
-    }
-  };
-  if (cur.hit_num == 0) build_table();
-
-  // Unused hits of the current module pair, compacted in index order one chunk of blockDim
+  // Unused hits of the current module pair, compacted in index order one chunk of team.lanes
   // hits at a time (dev_rel_indices in global memory, the chunk's list in LDS); the seeds of a
   // chunk are made before the next chunk, which keeps the h1 order of the reference.
   uint32_t base = 0;
-  for (unsigned c0 = 0; c0 < cur.hit_num; c0 += blockDim.x) {
-    const unsigned r = c0 + threadIdx.x;
+  for (unsigned c0 = 0; c0 < cur.hit_num; c0 += team.lanes) {
+    const unsigned r = c0 + tid;
     bool act = act0;
-    Scan3 sc;
-    if (c0 == 0) {
-      sc.r[0] = first.r[1];
-      sc.t[0] = first.t[1];
-    }
-    else {
+    unsigned rank = first.r[1], n_h1 = first.t[1];
+    if (c0 != 0) {
       act = r < cur.hit_num && !hits.used(cur.hit_start + r);
-      sc = scan3(sh, cn, act, false, false);
+      const Scan3 sc = scan<1>(team, sh, cn, act);
+      rank = sc.r[0];
+      n_h1 = sc.t[0];
     }
     if (act) {
-      o.h1_indices[base + sc.r[0]] = cur.hit_start + r;
-      ss.h1_chunk[sc.r[0]] = cur.hit_start + r;
+      o.h1_indices[base + rank] = cur.hit_start + r;
+      ss.h1_chunk[rank] = cur.hit_start + r;
     }
-    base += sc.t[0];
-    const unsigned n_h1 = sc.t[0];
-    __syncthreads();
+    base += n_h1;
+    if (n_h1 == 0) continue;
+    team.sync();
     phase_mark<count>(wc, phase_compaction);
 
-    if (c0 == 0) build_table();
-    // 1. h0 candidates of every h1 of the chunk (lane t: the chunk's h1 number t), pendulum order.
-    {
-      const unsigned rel = threadIdx.x;
-      unsigned n_found = 0;
-      if (rel < n_h1) {
-        const unsigned h1_index = ss.h1_chunk[rel];
-        const int16_t h1_phi = hits.phi(h1_index);
-        const int start = mp_search<count>(hits, prev, h1_phi, wc);
-        phase_mark<count>(wc, phase_seed1_search);
-        uint16_t* h0_out = ss.h0 + rel * max_h0_candidates;
-        if (use_list) {
-          n_found = K == initial_seeding_h0_candidates
-                      ? h0_candidates_from_list<initial_seeding_h0_candidates>(
-                          ss.unused, ss.before, n_unused, prev.hit_num, prev.hit_start, start, h0_out)
-                      : h0_candidates_from_list<seeding_h0_candidates>(
-                          ss.unused, ss.before, n_unused, prev.hit_num, prev.hit_start, start, h0_out);
+    for (unsigned r0 = 0; r0 < n_h1; r0 += C) {
+      Team::wave_fence(); // the last round's candidates have been read
+      // 1. The K lanes of h1 number q choose its h0 candidates.
+      const unsigned k = tid & (K - 1);
+      const unsigned q = r0 + (tid >> log2K);
+      const bool active = q < n_h1;
+      const unsigned h1_index = ss.h1_chunk[active ? q : 0u];
+      const Hit h1 = hits.load(h1_index);
+      uint16_t* const choice = ss.h0 + (tid & ~(K - 1));
+      unsigned n_h0;
+      if (use_list) {
+        n_h0 = min(n_unused, K);
+        if (n_unused) {
+          const unsigned n = prev.hit_num, u = n_unused;
+          const unsigned start = mp_search<count>(hits, prev, h1.phi, wc);
+          phase_mark<count>(wc, phase_seed1_search);
+          const unsigned s0 = start >= n ? start - n : start;
+          // The lower bound of s0 in the list: the number of unused positions below s0.
+          const unsigned p = ss.before[s0];
+          // key = rank << 16 | position (n <= 1024 on this path: rank < 2048, position < 1024).
+          constexpr uint32_t none = 0xFFFFFFFFu;
+          const bool all = u <= 2 * K;
+          uint32_t key[2], x[2];
+          bool has[2];
+#pragma unroll
+          for (unsigned e = 0; e < 2; ++e) {
+            const unsigned j = 2 * k + e;
+            const int around = static_cast<int>(p + j) - static_cast<int>(K);
+            const unsigned ring = static_cast<unsigned>(
+              around < 0 ? around + static_cast<int>(u) : (around >= static_cast<int>(u) ? around - static_cast<int>(u) : around));
+            has[e] = !all || j < u;
+            x[e] = ss.unused[all ? (j < u ? j : 0u) : ring];
+          }
+#pragma unroll
+          for (unsigned e = 0; e < 2; ++e) {
+            const unsigned d = x[e] >= s0 ? x[e] - s0 : x[e] + n - s0;
+            const unsigned rk = d == 0 ? 0u : (d <= n / 2 ? 2 * d - 1 : 2 * (n - d));
+            key[e] = has[e] ? (rk << 16 | x[e]) : none;
+          }
+          uint32_t below[2] = {below4(key[0], key[1], key[0]) + (key[1] < key[0] ? 1u : 0u),
+                               below4(key[0], key[1], key[1]) + (key[0] < key[1] ? 1u : 0u)};
+          if (K == 8) {
+            const uint32_t m0 = dpp<dpp_half_mirror>(key[0]), m1 = dpp<dpp_half_mirror>(key[1]);
+#pragma unroll
+            for (unsigned e = 0; e < 2; ++e)
+              below[e] += below4(m0, m1, key[e]) + (m0 < key[e] ? 1u : 0u) + (m1 < key[e] ? 1u : 0u);
+          }
+#pragma unroll
+          for (unsigned e = 0; e < 2; ++e)
+            if (active && has[e] && below[e] < K) choice[below[e]] = static_cast<uint16_t>(prev.hit_start + x[e]);
         }
-        else {
-          // Module pairs beyond the list's capacity: the pendulum walk itself, start, +1, -1,
-          // +2, -2, ... (each wrapped once into the module pair).
+      }
+      else {
+        // Module pairs beyond the list's capacity: the pendulum walk itself, start, +1, -1,
+        // +2, -2, ... (each wrapped once into the module pair), by the h1's first lane.
+        unsigned n_found = 0;
+        if (active && k == 0) {
           const int n = static_cast<int>(prev.hit_num);
-          int phi_index = start;
+          int phi_index = static_cast<int>(mp_search<count>(hits, prev, h1.phi, wc));
           for (unsigned i = 0; i < prev.hit_num && n_found < K; ++i) {
             phi_index += (i & 1u) ? static_cast<int>(i) : -static_cast<int>(i);
             const int in_bounds = phi_index < 0 ? phi_index + n : (phi_index >= n ? phi_index - n : phi_index);
             const unsigned h0_index = prev.hit_start + static_cast<unsigned>(in_bounds);
-            if (!hits.used(h0_index)) h0_out[n_found++] = h0_index;
+            if (!hits.used(h0_index)) choice[n_found++] = static_cast<uint16_t>(h0_index);
           }
         }
-        phase_mark<count>(wc, phase_seed1_pendulum);
+        n_h0 = __shfl(n_found, lane_id() & ~(K - 1), wave_size);
       }
-      ss.n_h0[rel] = n_found;
-    }
-    __syncthreads();
-    phase_mark<count>(wc, phase_seed1_wait);
+      Team::wave_fence();
+      phase_mark<count>(wc, phase_seed1_pendulum);
 
-    // 2. Rounds of C h1 hits: lane t K + k scores the pair (h1 number r C + t, its h0 number k)
-    // over the h2 window (first strict minimum), and the K lanes of an h1 (consecutive lanes of
-    // one wave) keep the least (scatter, k) by exchanging keys: the first strict minimum over
-    // the h0 candidates in pendulum order, the pair the sequential double loop selects. A
-    // scatter below max_scatter is a non-negative float, ordered as its bit pattern.
-    for (unsigned r0 = 0; r0 < n_h1; r0 += C) {
-      const unsigned t = threadIdx.x >> log2K;
-      const unsigned k = threadIdx.x & (K - 1);
-      const unsigned q = r0 + t;
+      // 2. Lane k of h1 scores the pair (h1, h0 number k) over the h2 window (first strict
+      // minimum), and the K lanes keep the least (scatter, k): the first strict minimum over
+      // the h0 candidates in pendulum order. A scatter below max_scatter is a non-negative float,
+      // ordered as its bit pattern.
       float best = max_scatter;
-      uint16_t best_h2 = 0;
-      // The pair's h1 and h0 are read together with the candidate count (all within the
-      // chunk's scratch for q < n_h1), one LDS round trip instead of two.
-      const bool in_chunk = t < C && q < n_h1;
-      const unsigned qq = in_chunk ? q : 0u;
-      const unsigned n_h0_q = ss.n_h0[qq];
-      const unsigned h1_index = ss.h1_chunk[qq];
-      const unsigned h0_index = ss.h0[qq * max_h0_candidates + k];
-      if (in_chunk && k < n_h0_q) {
-        const float h1x = hits.x(h1_index), h1y = hits.y(h1_index), h1z = hits.z(h1_index);
-        const float h0x = hits.x(h0_index), h0y = hits.y(h0_index), h0z = hits.z(h0_index);
-        const float td = 1.0f / (h1z - h0z);
-        const float txn = h1x - h0x;
-        const float tyn = h1y - h0y;
+      uint32_t best_h2 = 0;
+      if (active && k < n_h0) {
+        const Hit h0 = hits.load(choice[k]);
+        const float td = 1.0f / (h1.z - h0.z);
+        const float txn = h1.x - h0.x;
+        const float tyn = h1.y - h0.y;
         const float tx = txn * td;
         const float ty = tyn * td;
-        int16_t cand, ephi;
-        find_forward_candidate<count>(wc, hits, next, h0x, h0y, tx, ty, dz_next, phi_tolerance, cand, ephi);
-        // The h2 window in phi order from the candidate, four positions read per round.
-        const unsigned n2 = next.hit_num;
-        const unsigned c2 = static_cast<unsigned>(static_cast<int>(cand));
-        for (unsigned j0 = 0; j0 < n2; j0 += 4) {
-          Window4 w;
-          w.load(hits, next.hit_start, n2, c2, j0, true);
-          bool stop = false;
-#pragma unroll
-          for (unsigned kk = 0; kk < 4; ++kk) {
-            if (stop || j0 + kk >= n2) continue;
-            const int16_t phi_diff = w.phi[kk] - ephi;
-            const int16_t abs_phi_diff = phi_diff < 0 ? -phi_diff : phi_diff;
-            if (abs_phi_diff > phi_tolerance) {
-              stop = true;
-              continue;
-            }
-            if (!w.used[kk]) {
-              if constexpr (count) ++wc.seed_eval;
-              const float dz = w.z[kk] - h0z;
-              const float predx = h0x + tx * dz;
-              const float predy = h0y + ty * dz;
-              const float dx = predx - w.x[kk];
-              const float dy = predy - w.y[kk];
-              const float scatter = dx * dx + dy * dy;
-              if (scatter < best) {
-                best = scatter;
-                best_h2 = w.index[kk];
-              }
-            }
-          }
-          if (stop) break;
+        const Line line {h0.x, h0.y, h0.z, tx, ty, extrapolated_phi<count>(wc, h0.x, h0.y, tx, ty, dz_next)};
+        closest_hit<count, true>(wc, hits, next, line, phi_tolerance, best, best_h2);
+      }
+      uint32_t key_hi = __float_as_uint(best), key_lo = (k << 16) | best_h2;
+      least<dpp_xor1>(key_hi, key_lo);
+      least<dpp_xor2>(key_hi, key_lo);
+      if (K == 8) least<dpp_half_mirror>(key_hi, key_lo); // quads agree: any lane of the other one
+      const bool found = active && k == 0 && __uint_as_float(key_hi) < max_scatter;
+      const unsigned best_h0 = choice[found ? key_lo >> 16 : 0u];
+      phase_mark<count>(wc, phase_seed2);
+      if constexpr (seed_mode == seed_mode_scored) {
+        // Decided below, a group at a time.
+        if (active && k == 0) ss.seed[q] = found ? best_h0 | key_lo << 16 : no_seed;
+      }
+      else {
+        const uint16_t h2_index = static_cast<uint16_t>(key_lo & 0xFFFFu);
+        if constexpr (seed_mode == seed_mode_log) {
+          if (found) log_seed(hits, o, module_pair, best_h0, h1_index, h2_index, nullptr, nullptr);
         }
+        // 3. The round's seeds in h1 order.
+        append_seeds(team, sh, cn, o, found, best_h0, h1_index, h2_index);
       }
-      // key = scatter bits, k, h2; the whole wave takes part in the exchange.
-      unsigned long long key = (static_cast<unsigned long long>(__float_as_uint(best)) << 32) | (k << 16) | best_h2;
-      for (unsigned d = K / 2; d > 0; d >>= 1) {
-        const unsigned long long other = __shfl_xor(key, d, wave_size);
-        key = other < key ? other : key;
-      }
-      if (k == 0 && t < C && q < n_h1) {
-        const bool found = __uint_as_float(static_cast<uint32_t>(key >> 32)) < max_scatter;
-        const unsigned kb = static_cast<unsigned>(key >> 16) & 0xFFu;
-        ss.seed[q] = found ? (static_cast<uint32_t>(ss.h0[q * max_h0_candidates + kb]) |
-                              (static_cast<uint32_t>(key & 0xFFFFu) << 16))
-                           : no_seed;
-      }
-    }
-    __syncthreads();
-    phase_mark<count>(wc, phase_seed2);
-
-    // 3. The chunk's seeds in h1 order (lane t: h1 number t).
-    uint32_t seed = no_seed;
-    uint16_t h1_index = 0;
-    if (threadIdx.x < n_h1) {
-      seed = ss.seed[threadIdx.x];
-      h1_index = ss.h1_chunk[threadIdx.x];
-    }
-    bool found = seed != no_seed;
-    const uint16_t best_h0 = static_cast<uint16_t>(seed & 0xFFFFu);
-    const uint16_t best_h2 = static_cast<uint16_t>(seed >> 16);
-    if constexpr (seed_mode == seed_mode_log) {
-      if (found) {
-        float f[n_seed_features];
-        seed_features(hits, best_h0, h1_index, best_h2, module_pair, f);
-        const unsigned slot = atomicAdd(o.seed_log.counter, 1u);
-        if (slot < o.seed_log.capacity) {
-          uint32_t* rec = o.seed_log.records + 5 * (size_t) slot;
-          rec[0] = o.event_number;
-          rec[1] = module_pair;
-          rec[2] = best_h0;
-          rec[3] = h1_index;
-          rec[4] = best_h2;
-          float* fo = o.seed_log.features + n_seed_features * (size_t) slot;
-#pragma unroll
-          for (unsigned kk = 0; kk < n_seed_features; ++kk) fo[kk] = f[kk];
-        }
-      }
+      phase_mark<count>(wc, phase_seed3);
     }
     if constexpr (seed_mode == seed_mode_scored) {
       // Seeds are decided in groups of C consecutive h1 hits (a wave, or half of one when
-      // C = 32). A seed is kept when its logit reaches the threshold; a group whose seeds would
-      // all go keeps them (plain search as fallback).
+      // C = 32), lane t: the chunk's h1 number t. A seed is kept when its logit reaches the
+      // threshold; a group whose seeds would all go keeps them (plain search as fallback).
+      team.sync();
+      uint32_t seed = no_seed;
+      unsigned h1_index = 0;
+      if (tid < n_h1) {
+        seed = ss.seed[tid];
+        h1_index = ss.h1_chunk[tid];
+      }
+      bool found = seed != no_seed;
+      const unsigned best_h0 = seed & 0xFFFFu, h2_index = seed >> 16;
       float fp[n_seed_features];
 #pragma unroll
       for (unsigned kk = 0; kk < n_seed_features; ++kk) fp[kk] = 0.f;
-      if (found) seed_features(hits, best_h0, h1_index, best_h2, module_pair, fp);
+      if (found) seed_features(hits, best_h0, h1_index, h2_index, module_pair, fp);
       const uint64_t live = __ballot(found);
       const float logit = live ? scorer_logit(fp, live, *o.scorer) : 0.f;
       const bool keep = found && logit >= o.scorer_threshold;
-      if (found && o.seed_log.counter) {
-        const unsigned slot = atomicAdd(o.seed_log.counter, 1u);
-        if (slot < o.seed_log.capacity) {
-          uint32_t* rec = o.seed_log.records + 5 * (size_t) slot;
-          rec[0] = o.event_number;
-          rec[1] = module_pair;
-          rec[2] = best_h0;
-          rec[3] = h1_index;
-          rec[4] = best_h2;
-          float* fo = o.seed_log.features + n_seed_features * (size_t) slot;
-#pragma unroll
-          for (unsigned kk = 0; kk < n_seed_features; ++kk) fo[kk] = fp[kk];
-          if (o.seed_log.logits) o.seed_log.logits[slot] = logit;
-        }
-      }
+      if (found && o.seed_log.counter) log_seed(hits, o, module_pair, best_h0, h1_index, h2_index, fp, &logit);
       const uint64_t group = C >= wave_size ? ~0ull : (((1ull << C) - 1) << (lane_id() / C * C));
       if (__ballot(keep) & group) found = keep;
+      append_seeds(team, sh, cn, o, found, best_h0, h1_index, h2_index);
+      phase_mark<count>(wc, phase_seed3);
     }
-    const Scan3 s = scan3(sh, cn, found, false, false);
-    if (found) {
-      const unsigned tn = (cn.ttf + s.r[0]) % max_tracks_to_follow;
-      TrackletHits tl;
-      tl.hits[0] = best_h0;
-      tl.hits[1] = h1_index;
-      tl.hits[2] = best_h2;
-      o.tracklets[tn] = tl;
-      o.ttf[tn] = bit_seed | tn;
-      const unsigned wslot = tn & o.window_mask;
-      o.ttf_window[wslot] = bit_seed | tn;
-      o.ttf_last2[wslot] = static_cast<uint32_t>(h1_index) | (static_cast<uint32_t>(best_h2) << 16);
-      o.ttf_first[wslot] = best_h0;
-      o.ttf_n[wslot] = 3;
-    }
-    cn.ttf += s.t[0];
-    phase_mark<count>(wc, phase_seed3);
   }
   cn.local_hits = base;
 }
@@ -939,6 +1001,7 @@ __device__ __forceinline__ void track_forwarding(
   SearchShared& sh,
   Counters& cn,
   const EventOutputs& o,
+  const Team& team,
   const ModulePairData next,
   unsigned prev_ttf,
   unsigned diff_ttf,
@@ -947,13 +1010,15 @@ __device__ __forceinline__ void track_forwarding(
   float max_scatter,
   unsigned max_skipped_modules)
 {
-  for (unsigned c = 0; c < diff_ttf; c += blockDim.x) {
+  for (unsigned c = 0; c < diff_ttf; c += team.lanes) {
     const unsigned e = c + threadIdx.x;
     bool promote = false, reinsert = false, three = false;
-    uint32_t full = 0;
+    bool is_seed = false;
+    unsigned skipped = 0; // the entry's bit_skipped field, in place
     unsigned number_of_hits = 0;
-    int best_h2 = -1;
-    uint16_t th[3] = {0, 0, 0};
+    bool found = false;
+    uint32_t best_h2 = 0;
+    unsigned first_hit = 0;
     unsigned track_number = 0;
     bool valid = false;
     unsigned h0_num = 0, h1_num = 0;
@@ -961,25 +1026,23 @@ __device__ __forceinline__ void track_forwarding(
       const unsigned q = (prev_ttf + e) % max_tracks_to_follow;
       if (window) {
         // The entry and its track's last hits from LDS (written with the entry).
-        const unsigned wslot = q & o.window_mask;
-        full = o.ttf_window[wslot];
-        const uint32_t last2 = o.ttf_last2[wslot];
-        h0_num = last2 & 0xFFFFu;
-        h1_num = last2 >> 16;
-        number_of_hits = o.ttf_n[wslot];
-        th[0] = o.ttf_first[wslot];
-        th[1] = static_cast<uint16_t>(h0_num);
-        th[2] = static_cast<uint16_t>(h1_num);
-        track_number = full & bit_track_number;
-        if ((full & bit_seed) == bit_seed) valid = track_number < max_tracks_to_follow;
+        const uint2 w = o.window_entries[q & o.window_mask];
+        is_seed = (w.x & bit_seed) != 0;
+        skipped = w.x & bit_skipped;
+        h0_num = w.y & 0xFFFFu;
+        h1_num = w.y >> 16;
+        first_hit = (w.x >> seed_first_pos) & 0xFFFFu;
+        number_of_hits = is_seed ? 3u : (w.x >> track_hits_pos) & 31u;
+        track_number = w.x & (is_seed ? max_tracks_to_follow - 1 : window_track_number);
         // Guards that only matter once the slots of an event have overflowed (status raised).
-        else valid = track_number < o.track_capacity && number_of_hits >= 3 && number_of_hits < max_track_size;
+        valid = is_seed || (track_number < o.track_capacity && number_of_hits >= 3 && number_of_hits < max_track_size);
       }
       else {
-        full = o.ttf[q];
+        uint32_t full = o.ttf[q];
         track_number = full & bit_track_number;
+        is_seed = (full & bit_seed) != 0;
         const uint16_t* t_hits = nullptr;
-        if ((full & bit_seed) == bit_seed) {
+        if (is_seed) {
           valid = track_number < max_tracks_to_follow;
           if (valid) t_hits = o.tracklets[track_number].hits;
           number_of_hits = 3;
@@ -993,111 +1056,80 @@ __device__ __forceinline__ void track_forwarding(
         if (valid) {
           h0_num = t_hits[number_of_hits - 2];
           h1_num = t_hits[number_of_hits - 1];
-          th[0] = t_hits[0];
-          th[1] = t_hits[1];
-          th[2] = t_hits[2];
+          first_hit = t_hits[0];
         }
+        // These reads are waited for here. Left pending, they would make the code after the
+        // branch wait for all memory traffic, which on the usual path (the window) is the wave's
+        // stores: a round trip to memory several times per module pair.
+        asm volatile("" : "+v"(full), "+v"(h0_num), "+v"(h1_num), "+v"(first_hit), "+v"(number_of_hits));
+        skipped = full & bit_skipped;
       }
     }
     if (valid) {
-      const unsigned skipped = (full & bit_skipped) >> skipped_pos;
-      const float h0x = hits.x(h0_num), h0y = hits.y(h0_num), h0z = hits.z(h0_num);
-      const float h1x = hits.x(h1_num), h1y = hits.y(h1_num), h1z = hits.z(h1_num);
-      const float td = 1.0f / (h1z - h0z);
-      const float txn = h1x - h0x;
-      const float tyn = h1y - h0y;
+      const Hit h0 = hits.load(h0_num), h1 = hits.load(h1_num);
+      const float td = 1.0f / (h1.z - h0.z);
+      const float txn = h1.x - h0.x;
+      const float tyn = h1.y - h0.y;
       const float tx = txn * td;
       const float ty = tyn * td;
       float best_fit = max_scatter;
-      int16_t cand, ephi;
-      find_forward_candidate<count>(
-        wc, hits, next, h0x, h0y, tx, ty, (hits.module_odd(h0_num) ? next.z[1] : next.z[0]) - h0z, phi_tolerance, cand, ephi);
-      const unsigned n2 = next.hit_num;
-      const unsigned c2 = static_cast<unsigned>(static_cast<int>(cand));
-      for (unsigned j0 = 0; j0 < n2; j0 += 4) {
-        Window4 w;
-        w.load(hits, next.hit_start, n2, c2, j0, false);
-        bool stop = false;
-#pragma unroll
-        for (unsigned k = 0; k < 4; ++k) {
-          if (stop || j0 + k >= n2) continue;
-          const int16_t phi_diff = w.phi[k] - ephi;
-          const int16_t abs_phi_diff = phi_diff < 0 ? -phi_diff : phi_diff;
-          if (abs_phi_diff > phi_tolerance) {
-            stop = true;
-            continue;
-          }
-          if constexpr (count) ++wc.fwd_eval;
-          const float dz = w.z[k] - h0z;
-          const float predx = h0x + tx * dz;
-          const float predy = h0y + ty * dz;
-          const float dx = predx - w.x[k];
-          const float dy = predy - w.y[k];
-          const float scatter = dx * dx + dy * dy;
-          if (scatter < best_fit) {
-            best_fit = scatter;
-            best_h2 = w.index[k];
-          }
-        }
-        if (stop) break;
-      }
-      if (best_h2 != -1) {
+      const Line line {h0.x, h0.y, h0.z, tx, ty,
+                       extrapolated_phi<count>(wc, h0.x, h0.y, tx, ty, (h0.odd ? next.z[1] : next.z[0]) - h0.z)};
+      found = closest_hit<count, false>(wc, hits, next, line, phi_tolerance, best_fit, best_h2);
+      if (found) {
         promote = number_of_hits == 3;
         reinsert = number_of_hits + 1 < max_track_size;
       }
-      else if (skipped < max_skipped_modules) {
+      else if ((skipped >> skipped_pos) < max_skipped_modules) {
         reinsert = true;
-        track_number = ((skipped + 1) << skipped_pos) | (full & (bit_seed | bit_track_number));
       }
       else if (number_of_hits == 3) {
         three = true;
       }
     }
-    const Scan3 s = scan3(sh, cn, promote, reinsert, three);
+    const Scan3 s = scan<3>(team, sh, cn, promote, reinsert, three);
     if (valid) {
-      if (best_h2 != -1) {
+      if (found) {
+        hits.mark_used(best_h2);
         if (promote) {
-          hits.mark_used4(best_h2, th[0], th[1], th[2]);
+          hits.mark_used(first_hit);
+          hits.mark_used(h0_num);
+          hits.mark_used(h1_num);
           track_number = cn.n_tracks + s.r[0];
           if (track_number < o.track_capacity) {
             TrackHits& t = o.tracks[track_number];
-            t.hits[0] = th[0];
-            t.hits[1] = th[1];
-            t.hits[2] = th[2];
-            t.hits[3] = best_h2;
+            t.hits[0] = static_cast<uint16_t>(first_hit);
+            t.hits[1] = static_cast<uint16_t>(h0_num);
+            t.hits[2] = static_cast<uint16_t>(h1_num);
+            t.hits[3] = static_cast<uint16_t>(best_h2);
             t.hitsNum = 4;
           }
         }
         else {
-          hits.mark_used(best_h2);
           TrackHits& t = o.tracks[track_number];
-          t.hits[number_of_hits] = best_h2;
+          t.hits[number_of_hits] = static_cast<uint16_t>(best_h2);
           t.hitsNum = number_of_hits + 1;
         }
       }
       if (reinsert) {
-        const unsigned p = (cn.ttf + s.r[1]) % max_tracks_to_follow;
+        // Found: the track with the new hit. Not found: the same entry, one module more skipped.
         // A promoted track beyond the slots of its event is skipped when read back.
-        o.ttf[p] = track_number;
-        const unsigned wslot = p & o.window_mask;
-        o.ttf_window[wslot] = track_number;
-        if (best_h2 != -1) {
-          o.ttf_last2[wslot] = h1_num | (static_cast<uint32_t>(best_h2) << 16);
-          o.ttf_n[wslot] = static_cast<uint8_t>(number_of_hits + 1);
-        }
-        else {
-          o.ttf_last2[wslot] = h0_num | (h1_num << 16);
-          o.ttf_n[wslot] = static_cast<uint8_t>(number_of_hits);
-        }
-        o.ttf_first[wslot] = th[0];
+        const unsigned p = (cn.ttf + s.r[1]) % max_tracks_to_follow;
+        const unsigned last2 = found ? h1_num | (best_h2 << 16) : h0_num | (h1_num << 16);
+        const uint32_t skips = found ? 0u : skipped + (1u << skipped_pos);
+        const bool seed = is_seed && !found;
+        const uint32_t full = skips | (seed ? bit_seed : 0u) | track_number;
+        o.ttf[p] = full;
+        o.window_entries[p & o.window_mask] =
+          seed ? window_seed(full, first_hit, last2) : window_track(skips, track_number, number_of_hits + (found ? 1u : 0u), last2);
       }
       if (three) {
         const unsigned p = cn.three + s.r[2];
         if (p < o.track_capacity) {
           TrackletHits t;
-          t.hits[0] = th[0];
-          t.hits[1] = th[1];
-          t.hits[2] = th[2];
+          t.hits[0] = static_cast<uint16_t>(first_hit);
+          t.hits[1] = static_cast<uint16_t>(h0_num);
+          t.hits[2] = static_cast<uint16_t>(h1_num);
           o.three_hit_tracks[p] = t;
         }
       }
@@ -1121,10 +1153,10 @@ __device__ __forceinline__ void search_event(
   SearchShared& sh,
   Counters& cn,
   const EventOutputs& o,
+  const Team& team,
   float phi_tolerance_f,
   float max_scatter,
-  unsigned max_skipped_modules,
-  uint8_t* tables)
+  unsigned max_skipped_modules)
 {
   // Module pairs are visited from the last one upstream: seeding on (first, first - 1,
   // first - 2), forwarding into first - 2 (SearchByTriplet.cu:160-236).
@@ -1132,18 +1164,18 @@ __device__ __forceinline__ void search_event(
   const int16_t phi_tolerance = f32_to_i16(phi_tolerance_f * convert_factor_i16);
   unsigned first_module_pair = n_module_pairs - 1;
   unsigned last_ttf = 0;
-  // Seeding with first = F searches the tables of F and F - 2, the forwarding after it that of
-  // F - 3; seeding F builds the table of F - 4, so the first four are built at the event's start.
-  static_assert(phi_tables_at_start == 4 && phi_buckets == wave_size, "table schedule");
-  const auto seed = [&](unsigned h0_candidates) {
+  ModulePairData prev = module_pair_data(sh, first_module_pair), cur = module_pair_data(sh, first_module_pair - 1),
+                 next = module_pair_data(sh, first_module_pair - 2);
+  for (;;) {
+    // One inlined copy of track_seeding for both numbers of h0 candidates keeps the code small.
     track_seeding<count, seed_mode>(
-      wc, hits, ss, sh, cn, o, sh.mp[first_module_pair], sh.mp[first_module_pair - 1], sh.mp[first_module_pair - 2],
-      first_module_pair - 1, max_scatter, phi_tolerance, h0_candidates,
-      first_module_pair >= phi_tables_at_start ? &sh.mp[first_module_pair - phi_tables_at_start] : nullptr,
-      tables);
+      wc, hits, ss, sh, cn, o, team, prev, cur, next, first_module_pair - 1, max_scatter, phi_tolerance,
+      first_module_pair == n_module_pairs - 1 ? initial_seeding_h0_candidates : seeding_h0_candidates);
     --first_module_pair;
-  };
-  const auto forward = [&]() {
+    if (first_module_pair <= 1) break;
+    prev = cur;
+    cur = next;
+    next = module_pair_data(sh, first_module_pair - 2);
     const unsigned prev_ttf = last_ttf;
     last_ttf = cn.ttf;
     const unsigned diff_ttf = last_ttf - prev_ttf;
@@ -1154,106 +1186,92 @@ __device__ __forceinline__ void search_event(
     // read back from HBM, after a fence that makes this workgroup's ring writes visible to it.
     const bool window = 2 * diff_ttf <= o.window;
     if (!window) __threadfence_block();
-    // Orders the ring slots and tracklets written by the last seeding chunk before they are
-    // read (seeding chunks end right after their writes, without a barrier).
-    __syncthreads();
+    // Orders the ring slots and tracklets written by the last seeding round before they are
+    // read (seeding rounds end right after their writes, without a barrier).
+    team.sync();
     track_forwarding<count>(
-      wc, hits, sh, cn, o, sh.mp[first_module_pair - 2], prev_ttf, diff_ttf, window, phi_tolerance, max_scatter,
-      max_skipped_modules);
-    __syncthreads();
+      wc, hits, sh, cn, o, team, next, prev_ttf, diff_ttf, window, phi_tolerance, max_scatter, max_skipped_modules);
+    team.sync();
     phase_mark<count>(wc, phase_forwarding);
-  };
-  if constexpr (seed_mode == seed_mode_scored) {
-    // One inlined copy of track_seeding (the largest body, here with the scorer) keeps the
-    // kernel's code small.
-    for (;;) {
-      seed(first_module_pair == n_module_pairs - 1 ? initial_seeding_h0_candidates : seeding_h0_candidates);
-      if (first_module_pair <= 1) break;
-      forward();
-    }
   }
-  else {
-    // The first call peeled: both copies see a constant h0 window.
-    seed(initial_seeding_h0_candidates);
-    while (first_module_pair > 1) {
-      forward();
-      seed(seeding_h0_candidates);
-    }
-  }
-  __syncthreads();
+  team.sync();
   const unsigned prev_ttf = last_ttf;
   last_ttf = cn.ttf;
   const unsigned diff_ttf = last_ttf - prev_ttf;
   if (diff_ttf >= max_tracks_to_follow) cn.status |= status_ttf_ring_overflow;
+  // Both the entries (where they have left the window) and the tracklets are read back from HBM.
   const bool window = diff_ttf <= o.window; // nothing is written while these are read
-  if (!window) {
-    __threadfence_block();
-    __syncthreads();
-  }
-  for (unsigned c = 0; c < diff_ttf; c += blockDim.x) {
+  __threadfence_block();
+  team.sync();
+  for (unsigned c = 0; c < diff_ttf; c += team.lanes) {
     const unsigned e = c + threadIdx.x;
     bool seed = false;
     uint32_t full = 0;
     if (e < diff_ttf) {
       const unsigned q = (prev_ttf + e) % max_tracks_to_follow;
-      full = window ? o.ttf_window[q & o.window_mask] : o.ttf[q];
-      seed = (full & bit_seed) == bit_seed;
+      full = window ? o.window_entries[q & o.window_mask].x : o.ttf[q];
+      seed = (full & bit_seed) != 0;
     }
-    const Scan3 s = scan3(sh, cn, seed, false, false);
+    const Scan3 s = scan<1>(team, sh, cn, seed);
     if (seed) {
       const unsigned p = cn.three + s.r[0];
-      if (p < o.track_capacity) o.three_hit_tracks[p] = o.tracklets[full & bit_track_number];
+      if (p < o.track_capacity) o.three_hit_tracks[p] = o.tracklets[full & (max_tracks_to_follow - 1)];
     }
     cn.three += s.t[0];
     if (cn.three > o.track_capacity) cn.status |= status_three_hit_slots_overflow;
   }
 }
 
+struct SearchArgs {
+  const uint32_t* event_list;
+  const uint32_t* number_of_events;
+  const char* sorted_container;
+  const uint32_t* offsets_estimated_input_size;
+  const uint32_t* module_cluster_num;
+  const Geometry* geometry;
+  TrackHits* tracks;
+  TrackletHits* tracklets;
+  uint32_t* tracks_to_follow;
+  TrackletHits* three_hit_tracks;
+  uint8_t* hit_used;
+  uint32_t* atomics_velo;
+  uint16_t* rel_indices;
+  uint32_t* number_of_velo_tracks;
+  uint32_t* status;
+  float phi_tolerance;
+  float max_scatter;
+  unsigned max_skipped_modules;
+  unsigned lds_hits;
+  unsigned hits_per_wave; // waves of a workgroup that work on an event: one more for every so many hits; 0: all
+  unsigned long long* work_stats;
+  unsigned long long* event_clock;
+  unsigned n_list;
+  uint32_t* work_counter;
+  SeedLog seed_log;
+  const float* scorer_params;
+  float scorer_threshold;
+  unsigned window;
+  unsigned list_cap;
+};
+
 // One workgroup per event, or (persistent, launched with a work counter) a resident grid whose
 // workgroups take the next event slot from the counter until the slots run out; the persistent
-// grid is an instantiation of its own, so the one-event kernel keeps no loop state live. Dynamic LDS: the seeding scratch
-// (seed_scratch_bytes_per_lane per lane), the LDS window of the ring of tracks to follow
-// (ring_window entries; the ring itself, 2048 x u32, is written through to HBM), the list of
+// grid is an instantiation of its own, so the one-event kernel keeps no loop state live. Dynamic
+// LDS: the seeding scratch (seed_scratch_bytes_per_lane per lane), the LDS window of the ring of
+// tracks to follow (the ring itself, 2048 x u32, is written through to HBM), the list of
 // unused hits of the previous module pair and, per position, the number of unused hits before
-// it (list_cap x u16 each), the module pairs' phi bucket tables, then `lds_hits` hits as x[],
-// y[], z[] (f32), phi[] (i16)
-// and a flags byte (used, module parity). Events with up to 5 x lds_hits hits keep phi and the
+// it (list_cap x u16 each), the module pairs' phi bucket tables, then `lds_hits` hits of 16 bytes.
+// Events with up to 16/3 x lds_hits hits keep phi and the
 // flags in LDS and read coordinates from global memory; larger events run on global memory.
+// Bound by the latency of an event's chain of 25 dependent seeding and forwarding steps and, with
+// many events in flight, by VALU issue.
 // The `count` instantiation also accumulates the work counters into work_stats[4] (one
 // atomic per wave). With event_clock, each workgroup stores at event_clock[10 * event_number]
 // its event's start and end time (wall clock ticks) and, in the counting instantiation, the
 // ticks spent in each Phase.
 template<bool count, int seed_mode, bool persistent>
 __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, seed_mode == seed_mode_scored ? 3 : 1)
-  k_search_by_triplet(
-  const uint32_t* event_list,
-  const uint32_t* number_of_events,
-  const char* sorted_container,
-  const uint32_t* offsets_estimated_input_size,
-  const uint32_t* module_cluster_num,
-  const Geometry* geometry,
-  TrackHits* tracks_all,
-  TrackletHits* tracklets_all,
-  uint32_t* ttf_all,
-  TrackletHits* three_hit_all,
-  uint8_t* hit_used_all,
-  uint32_t* atomics_all,
-  uint16_t* rel_indices_all,
-  uint32_t* number_of_velo_tracks,
-  uint32_t* status,
-  float phi_tolerance,
-  float max_scatter,
-  unsigned max_skipped_modules,
-  unsigned lds_hits,
-  unsigned long long* work_stats,
-  unsigned long long* event_clock,
-  unsigned n_list,
-  uint32_t* work_counter,
-  SeedLog seed_log,
-  const float* scorer_params,
-  float scorer_threshold,
-  unsigned window,
-  unsigned list_cap)
+  k_search_by_triplet(const SearchArgs a)
 {
   extern __shared__ __align__(16) char dyn_all[];
   __shared__ SearchShared sh;
@@ -1262,58 +1280,57 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
   SeedScratch ss;
   ss.seed = reinterpret_cast<uint32_t*>(dyn_all);
   ss.h0 = reinterpret_cast<uint16_t*>(ss.seed + blockDim.x);
-  ss.h1_chunk = ss.h0 + max_h0_candidates * blockDim.x;
-  ss.n_h0 = reinterpret_cast<uint8_t*>(ss.h1_chunk + blockDim.x);
-  uint32_t* ring = reinterpret_cast<uint32_t*>(dyn_all + ((seed_scratch_bytes_per_lane * blockDim.x + 15) & ~15u));
-  uint32_t* ring_last2 = ring + window;
-  uint16_t* ring_first = reinterpret_cast<uint16_t*>(ring_last2 + window);
-  uint8_t* ring_n = reinterpret_cast<uint8_t*>(ring_first + window);
-  ss.unused = reinterpret_cast<uint16_t*>(ring_n + window);
-  ss.before = ss.unused + list_cap;
-  ss.list_cap = list_cap;
-  uint8_t* phi_tables = reinterpret_cast<uint8_t*>(ss.before + list_cap);
+  ss.h1_chunk = ss.h0 + blockDim.x;
+  uint2* window_entries = reinterpret_cast<uint2*>(ss.h1_chunk + blockDim.x);
+  ss.unused = reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(window_entries) + window_bytes(a.window));
+  ss.before = ss.unused + a.list_cap;
+  ss.list_cap = a.list_cap;
+  uint8_t* phi_tables = reinterpret_cast<uint8_t*>(ss.before + a.list_cap);
   char* dyn = reinterpret_cast<char*>(phi_tables + phi_tables_bytes);
   ScorerLds* scorer = nullptr;
   if constexpr (seed_mode == seed_mode_scored) {
-    scorer = reinterpret_cast<ScorerLds*>(dyn + (((size_t) lds_hits * search_bytes_per_hit + 15) & ~size_t(15)));
-    load_scorer(scorer_params, *scorer);
+    scorer = reinterpret_cast<ScorerLds*>(dyn + (size_t) a.lds_hits * search_bytes_per_hit);
+    load_scorer(a.scorer_params, *scorer);
     __syncthreads();
   }
-  // One event per workgroup (work_counter == NULL), or a resident grid whose workgroups take
-  // event slots from the counter until they run out (the counter starts at 0).
+  const unsigned total = a.offsets_estimated_input_size[n_module_pairs * a.number_of_events[0]];
   // One event: slot `slot` of the event list (the whole workgroup, uniform).
   const auto process_event = [&](unsigned slot) {
-    const unsigned long long t_start = event_clock ? wall_clock64() : 0ull;
+    const unsigned long long t_start = a.event_clock ? wall_clock64() : 0ull;
     wc.last = t_start;
-    const unsigned event_number = event_list ? event_list[slot] : slot;
-    const unsigned n_events = number_of_events[0];
-    const unsigned total = offsets_estimated_input_size[n_module_pairs * n_events];
-    const uint32_t* mhs = offsets_estimated_input_size + event_number * n_module_pairs;
-    const uint32_t* mhn = module_cluster_num + event_number * n_module_pairs;
+    const unsigned event_number = a.event_list ? a.event_list[slot] : slot;
+    const unsigned n_events = a.number_of_events[0];
+    const uint32_t* mhs = a.offsets_estimated_input_size + event_number * n_module_pairs;
+    const uint32_t* mhn = a.module_cluster_num + event_number * n_module_pairs;
     const unsigned hit_offset = mhs[0];
     const unsigned n_hits = mhs[n_module_pairs] - hit_offset;
-    const Clusters cc {const_cast<char*>(sorted_container), total};
+    Team team;
+    team.wave = __builtin_amdgcn_readfirstlane(threadIdx.x / wave_size);
+    team.waves = blockDim.x / wave_size;
+    if constexpr (!persistent && seed_mode != seed_mode_scored) {
+      if (a.hits_per_wave) team.waves = min(team.waves, n_hits / a.hits_per_wave + 1);
+      if (team.wave >= team.waves) return;
+    }
+    team.lanes = team.waves * wave_size;
+    const Clusters cc {const_cast<char*>(a.sorted_container), total};
 
-    const unsigned toff = track_offset(offsets_estimated_input_size, event_number);
+    const unsigned toff = track_offset(a.offsets_estimated_input_size, event_number);
     const unsigned container = track_container_size(total, n_events);
     const unsigned next_off =
-      event_number + 1 < n_events ? track_offset(offsets_estimated_input_size, event_number + 1) : container;
+      event_number + 1 < n_events ? track_offset(a.offsets_estimated_input_size, event_number + 1) : container;
     EventOutputs o;
-    o.tracks = tracks_all + toff;
-    o.three_hit_tracks = three_hit_all + toff;
-    o.tracklets = tracklets_all + (size_t) event_number * max_tracks_to_follow;
-    o.ttf = ttf_all + (size_t) event_number * max_tracks_to_follow;
-    o.ttf_window = ring;
-    o.ttf_last2 = ring_last2;
-    o.ttf_first = ring_first;
-    o.ttf_n = ring_n;
-    o.h1_indices = rel_indices_all + hit_offset;
+    o.tracks = a.tracks + toff;
+    o.three_hit_tracks = a.three_hit_tracks + toff;
+    o.tracklets = a.tracklets + (size_t) event_number * max_tracks_to_follow;
+    o.ttf = a.tracks_to_follow + (size_t) event_number * max_tracks_to_follow;
+    o.window_entries = window_entries;
+    o.h1_indices = a.rel_indices + hit_offset;
     o.event_number = event_number;
-    o.seed_log = seed_log;
+    o.seed_log = a.seed_log;
     o.scorer = scorer;
-    o.scorer_threshold = scorer_threshold;
-    o.window = window;
-    o.window_mask = window - 1;
+    o.scorer_threshold = a.scorer_threshold;
+    o.window = a.window;
+    o.window_mask = a.window - 1;
     // Slots of this event; the reference lets a busy event run into its neighbour's slots, here
     // nothing is written past the container and the overflow is reported.
     o.track_capacity = min(next_off > toff ? next_off - toff : 0u, container - min(toff, container));
@@ -1324,53 +1341,47 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
       const unsigned m = threadIdx.x;
       sh.mp[m].hit_start = mhs[m] - hit_offset;
       sh.mp[m].hit_num = mhn[m];
-      sh.mp[m].z[0] = geometry->module_zs[2 * m];
-      sh.mp[m].z[1] = geometry->module_zs[2 * m + 1];
+      sh.mp[m].z[0] = a.geometry->module_zs[2 * m];
+      sh.mp[m].z[1] = a.geometry->module_zs[2 * m + 1];
       sh.mp[m].table = mhn[m] <= 255u ? m * phi_table_stride : no_phi_table;
     }
     const uint32_t* gids = cc.ids() + hit_offset;
     const int16_t* gph = cc.phis() + hit_offset;
     const float* gxyz = cc.xyz() + 3 * (size_t) hit_offset;
-    uint8_t* gused = hit_used_all + hit_offset;
-    if (n_hits <= lds_hits) {
-      float* xs = reinterpret_cast<float*>(dyn);
-      float* ys = xs + lds_hits;
-      float* zs = ys + lds_hits;
-      int16_t* ph = reinterpret_cast<int16_t*>(zs + lds_hits);
-      uint8_t* flags = reinterpret_cast<uint8_t*>(ph + lds_hits);
+    uint8_t* gused = a.hit_used + hit_offset;
+    // The ring window holds nothing yet: it is the tables' histograms.
+    uint32_t* const hist = reinterpret_cast<uint32_t*>(window_entries);
+    const unsigned hist_waves = window_bytes(a.window) / hist_bytes;
+    if (n_hits <= a.lds_hits) {
+      uint4* hit = reinterpret_cast<uint4*>(dyn);
       // Two hits per lane and round, every load issued before the first store waits (the
       // scheduler would otherwise wait out one memory round trip per field).
-      for (unsigned i0 = threadIdx.x; i0 < n_hits; i0 += 2 * blockDim.x) {
-        const unsigned i1 = i0 + blockDim.x < n_hits ? i0 + blockDim.x : i0;
+      for (unsigned i0 = threadIdx.x; i0 < n_hits; i0 += 2 * team.lanes) {
+        const unsigned i1 = i0 + team.lanes < n_hits ? i0 + team.lanes : i0;
         const float x0 = gxyz[3 * i0], y0 = gxyz[3 * i0 + 1], z0 = gxyz[3 * i0 + 2];
         const float x1 = gxyz[3 * i1], y1 = gxyz[3 * i1 + 1], z1 = gxyz[3 * i1 + 2];
         const int16_t p0 = gph[i0], p1 = gph[i1];
         const uint32_t id0 = gids[i0], id1 = gids[i1];
         __builtin_amdgcn_sched_barrier(0);
-        xs[i0] = x0;
-        ys[i0] = y0;
-        zs[i0] = z0;
-        ph[i0] = p0;
-        flags[i0] = module_parity(id0) ? flag_odd : 0;
-        xs[i1] = x1;
-        ys[i1] = y1;
-        zs[i1] = z1;
-        ph[i1] = p1;
-        flags[i1] = module_parity(id1) ? flag_odd : 0;
+        const auto word = [](int16_t p, uint32_t id) {
+          return static_cast<uint16_t>(p) | (module_parity(id) ? uint32_t(flag_odd) << 16 : 0u);
+        };
+        hit[i0] = make_uint4(__float_as_uint(x0), __float_as_uint(y0), __float_as_uint(z0), word(p0, id0));
+        hit[i1] = make_uint4(__float_as_uint(x1), __float_as_uint(y1), __float_as_uint(z1), word(p1, id1));
       }
-      __syncthreads();
-      const LdsHits hits {xs, ys, zs, ph, flags, phi_tables};
-      build_phi_tables(hits, sh.mp, phi_tables, n_module_pairs - phi_tables_at_start);
-      __syncthreads();
-      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, phi_tolerance, max_scatter, max_skipped_modules, phi_tables);
-      __syncthreads();
-      for (unsigned i = threadIdx.x; i < n_hits; i += blockDim.x) gused[i] = flags[i] & flag_used;
+      team.sync();
+      const LdsHits hits {hit, phi_tables};
+      build_phi_tables(hits, sh.mp, phi_tables, hist, hist_waves, team);
+      team.sync();
+      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
+      team.sync();
+      for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = hits.used(i) ? 1 : 0;
     }
-    else if (3 * n_hits <= search_bytes_per_hit * lds_hits) {
+    else if (mixed_bytes_per_hit * n_hits <= search_bytes_per_hit * a.lds_hits) {
       int16_t* ph = reinterpret_cast<int16_t*>(dyn);
       uint8_t* flags = reinterpret_cast<uint8_t*>(ph + n_hits);
-      for (unsigned i0 = threadIdx.x; i0 < n_hits; i0 += 2 * blockDim.x) {
-        const unsigned i1 = i0 + blockDim.x < n_hits ? i0 + blockDim.x : i0;
+      for (unsigned i0 = threadIdx.x; i0 < n_hits; i0 += 2 * team.lanes) {
+        const unsigned i1 = i0 + team.lanes < n_hits ? i0 + team.lanes : i0;
         const int16_t p0 = gph[i0], p1 = gph[i1];
         const uint32_t id0 = gids[i0], id1 = gids[i1];
         __builtin_amdgcn_sched_barrier(0);
@@ -1380,24 +1391,24 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
         flags[i1] = module_parity(id1) ? flag_odd : 0;
       }
       cn.status |= status_lds_fallback;
-      __syncthreads();
+      team.sync();
       const MixedHits hits {gxyz, ph, flags, phi_tables};
-      build_phi_tables(hits, sh.mp, phi_tables, n_module_pairs - phi_tables_at_start);
-      __syncthreads();
-      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, phi_tolerance, max_scatter, max_skipped_modules, phi_tables);
-      __syncthreads();
-      for (unsigned i = threadIdx.x; i < n_hits; i += blockDim.x) gused[i] = flags[i] & flag_used;
+      build_phi_tables(hits, sh.mp, phi_tables, hist, hist_waves, team);
+      team.sync();
+      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
+      team.sync();
+      for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = flags[i] & flag_used;
     }
     else {
-      for (unsigned i = threadIdx.x; i < n_hits; i += blockDim.x) gused[i] = 0;
+      for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = 0;
       cn.status |= status_lds_fallback;
       __threadfence_block();
-      __syncthreads();
+      team.sync();
       const GlobalHits hits {gxyz, gph, gused, gids, phi_tables};
-      build_phi_tables(hits, sh.mp, phi_tables, n_module_pairs - phi_tables_at_start);
-      __syncthreads();
-      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, phi_tolerance, max_scatter, max_skipped_modules, phi_tables);
-      __syncthreads();
+      build_phi_tables(hits, sh.mp, phi_tables, hist, hist_waves, team);
+      team.sync();
+      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
+      team.sync();
     }
     if constexpr (count) {
       // Wave reduction, then one atomic per wave.
@@ -1406,20 +1417,19 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
       for (int k = 0; k < 4; ++k) {
 #pragma unroll
         for (unsigned d = 32; d > 0; d >>= 1) v[k] += __shfl_xor(v[k], d, wave_size);
-        if (lane_id() == 0 && v[k]) atomicAdd(work_stats + k, v[k]);
+        if (lane_id() == 0 && v[k]) atomicAdd(a.work_stats + k, v[k]);
       }
       wc.seed_eval = wc.fwd_eval = wc.extrap = wc.steps = 0;
     }
-    __syncthreads();
     if (threadIdx.x == 0) {
-      uint32_t* at = atomics_all + event_number * num_atomics;
+      uint32_t* at = a.atomics_velo + event_number * num_atomics;
       at[atomic_three_hit] = cn.three;
       at[atomic_ttf] = cn.ttf;
       at[atomic_local_hits] = cn.local_hits;
-      number_of_velo_tracks[event_number] = min(cn.n_tracks, o.track_capacity);
-      if (cn.status && status) atomicOr(status, cn.status);
-      if (event_clock) {
-        unsigned long long* ec = event_clock + event_clock_words * event_number;
+      a.number_of_velo_tracks[event_number] = min(cn.n_tracks, o.track_capacity);
+      if (cn.status && a.status) atomicOr(a.status, cn.status);
+      if (a.event_clock) {
+        unsigned long long* ec = a.event_clock + event_clock_words * event_number;
         const unsigned long long t_end = wall_clock64();
         ec[0] = t_start;
         ec[1] = t_end;
@@ -1433,20 +1443,20 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
         }
       }
     }
-    __syncthreads(); // the next event reuses the LDS
+    if constexpr (persistent) __syncthreads(); // the next event reuses the LDS
   };
   if constexpr (persistent) {
     for (;;) {
-      if (threadIdx.x == 0) s_slot = atomicAdd(work_counter, 1u);
+      if (threadIdx.x == 0) s_slot = atomicAdd(a.work_counter, 1u);
       __syncthreads();
       const unsigned slot = s_slot;
       __syncthreads();
-      if (slot >= n_list) break;
+      if (slot >= a.n_list) break;
       process_event(slot);
     }
   }
   else {
-    if (blockIdx.x < n_list) process_event(blockIdx.x);
+    if (blockIdx.x < a.n_list) process_event(blockIdx.x);
   }
 }
 
@@ -1561,7 +1571,7 @@ __global__ void k_three_hit_filter(
   uint32_t* number_of_output,
   float max_chi2)
 {
-  __shared__ uint32_t scan[3 * 16 + 4];
+  __shared__ uint32_t scan[16];
   const unsigned event_number = event_list ? event_list[blockIdx.x] : blockIdx.x;
   const unsigned n_events = number_of_events[0];
   const unsigned total = offsets_estimated_input_size[n_module_pairs * n_events];
@@ -1588,9 +1598,10 @@ __global__ void k_three_hit_filter(
       const float chi2 = means_square_fit_chi2(cc, hit_offset, t);
       keep = !any_used && chi2 < max_chi2;
     }
-    const Scan3 s = block_flag_scan3(keep, false, false, scan);
-    if (keep) out[base + s.r[0]] = t;
-    base += s.t[0];
+    uint32_t kept;
+    const uint32_t r = block_flag_scan(keep, scan, &kept);
+    if (keep) out[base + r] = t;
+    base += kept;
   }
   if (threadIdx.x == 0) number_of_output[event_number] = base;
 }
@@ -1598,28 +1609,51 @@ __global__ void k_three_hit_filter(
 // Launch geometry: the seeding scratch, the ring window, the unused-hit list, then the hits.
 size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
 {
-  return ((seed_scratch_bytes_per_lane * (size_t) block + 15) & ~size_t(15)) + ring_window_bytes * (size_t) window +
-         2 * 2 * (size_t) list_cap + phi_tables_bytes + (size_t) lds_hits * search_bytes_per_hit;
+  return seed_scratch_bytes_per_lane * (size_t) block + window_bytes(window) + 2 * 2 * (size_t) list_cap +
+         phi_tables_bytes + (size_t) lds_hits * search_bytes_per_hit;
+}
+
+// Shape of a launch whose workgroup size is left to it: lanes, hits in LDS, ring window,
+// unused-hit list, and the hits of an event per working wave.
+struct SearchShape {
+  unsigned block, lds_hits, window, list_cap, hits_per_wave;
+};
+// Few events: every event has its LDS to itself (two workgroups fit a CU), and the launch lasts as
+// long as its largest event: four waves for events from 2100 hits on, all hits in LDS (200 events
+// of up to 1700 hits: 123 us against 142 us with 1500 hits in LDS and coordinates from memory).
+// Up to a few thousand: all of them have to be in flight at once, so the LDS is what four
+// workgroups a CU leave (1000 pile-up events: 210 us; with 1760 hits 220 us, with 128-lane
+// workgroups 310 us, with 512 lanes 213 us). Beyond, the workgroups stream through the chip and the
+// most resident waves win: two waves per event and little LDS (20 000 events: 1.62 ms; 1.93 ms
+// with 256 lanes, 2.46 ms with 1500 hits in LDS, 4.32 ms with 256 lanes and 1760 hits before).
+static SearchShape search_shape(unsigned n_events)
+{
+  if (n_events <= 512) return {256, 3072, 1024, 512, 700};
+  if (n_events <= 4096) return {256, 1500, 1024, 512, 700};
+  return {128, 384, 512, 512, 0};
 }
 
 hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
 {
   if (!a.n_list) return hipSuccess;
-  const unsigned block = a.block_dim ? a.block_dim : 256;
-  // Dynamic LDS stays within the device's per-workgroup limit (less the static part).
-  const int max_lds = device_max_lds_per_block();
-  if (!max_lds) return hipErrorInvalidDevice;
   // Scored mode: seeds are decided in groups of block / K unused h1 hits of each chunk of block
   // positions (the pruning rule with seed_block = block), and a group's seeds must lie in one
   // wave for the in-wave scorer and decision: workgroups of 64, 128 or 256 lanes. The scorer's
   // weights take LDS from the hits (same residency).
   const bool scored = a.scorer_params != nullptr;
+  const bool shaped = !a.block_dim && !scored && !a.work_counter;
+  const SearchShape shape = shaped ? search_shape(a.n_list) : SearchShape {256, search_default_lds_hits, ring_window, unused_list_cap, 0};
+  const unsigned block = a.block_dim ? a.block_dim : shape.block;
+  const unsigned hits_per_wave = shape.hits_per_wave;
+  // Dynamic LDS stays within the device's per-workgroup limit (less the static part).
+  const int max_lds = device_max_lds_per_block();
+  if (!max_lds) return hipErrorInvalidDevice;
   if (scored && block != 64 && block != 128 && block != 256) return hipErrorInvalidConfiguration;
   // The LDS window of the ring: a power of two from 64 to 512 (it divides the ring); the list
   // of unused hits: a multiple of 16 up to 1024 (relative positions fit 16 bits either way).
-  const unsigned window = a.ring_window ? a.ring_window : ring_window;
-  const unsigned list_cap = a.list_cap ? a.list_cap : unused_list_cap;
-  if (window < 64 || window > ring_window || (window & (window - 1)) || list_cap % 16 || list_cap > unused_list_cap)
+  const unsigned window = a.ring_window ? a.ring_window : shape.window;
+  const unsigned list_cap = a.list_cap ? a.list_cap : shape.list_cap;
+  if (window < 64 || a.ring_window > max_ring_window_knob || (window & (window - 1)) || list_cap % 16 || list_cap > unused_list_cap)
     return hipErrorInvalidValue;
   const size_t extra = scored ? scorer_lds_bytes + 16 : 0;
   const size_t fixed = search_dynamic_lds(block, 0, window, list_cap) + extra + 1024;
@@ -1627,7 +1661,7 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   const unsigned max_hits = static_cast<unsigned>(((size_t) max_lds - fixed) / search_bytes_per_hit);
   const unsigned default_hits =
     scored ? search_default_lds_hits - static_cast<unsigned>((extra + search_bytes_per_hit - 1) / search_bytes_per_hit)
-           : search_default_lds_hits;
+           : shape.lds_hits;
   const unsigned lds_hits = min(a.lds_hits ? a.lds_hits : default_hits, max_hits);
   const size_t dyn = search_dynamic_lds(block, lds_hits, window, list_cap) + extra;
   // Persistent mode: as many workgroups as stay resident (they take events from the counter).
@@ -1642,16 +1676,37 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
     const unsigned resident = device_resident_blocks(kernel, block, dyn);
     if (resident) grid = min(grid, resident);
   }
-#define VELO_LAUNCH_SEARCH_P(C, L, P)                                                                               \
-  hipLaunchKernelGGL(                                                                                               \
-    (k_search_by_triplet<C, L, P>), dim3(grid), dim3(block), dyn, s, a.event_list, a.number_of_events,              \
-    a.sorted_container, a.offsets_estimated_input_size, a.module_cluster_num,                                       \
-    reinterpret_cast<const Geometry*>(a.geometry), reinterpret_cast<TrackHits*>(a.tracks),                          \
-    reinterpret_cast<TrackletHits*>(a.tracklets), a.tracks_to_follow,                                               \
-    reinterpret_cast<TrackletHits*>(a.three_hit_tracks), a.hit_used, a.atomics_velo, a.rel_indices,                \
-    a.number_of_velo_tracks, a.status, a.phi_tolerance, a.max_scatter, a.max_skipped_modules, lds_hits,             \
-    a.work_stats, a.event_clock, a.n_list, a.work_counter, a.seed_log, a.scorer_params, a.scorer_threshold, window,   \
-    list_cap)
+  SearchArgs k;
+  k.event_list = a.event_list;
+  k.number_of_events = a.number_of_events;
+  k.sorted_container = a.sorted_container;
+  k.offsets_estimated_input_size = a.offsets_estimated_input_size;
+  k.module_cluster_num = a.module_cluster_num;
+  k.geometry = reinterpret_cast<const Geometry*>(a.geometry);
+  k.tracks = reinterpret_cast<TrackHits*>(a.tracks);
+  k.tracklets = reinterpret_cast<TrackletHits*>(a.tracklets);
+  k.tracks_to_follow = a.tracks_to_follow;
+  k.three_hit_tracks = reinterpret_cast<TrackletHits*>(a.three_hit_tracks);
+  k.hit_used = a.hit_used;
+  k.atomics_velo = a.atomics_velo;
+  k.rel_indices = a.rel_indices;
+  k.number_of_velo_tracks = a.number_of_velo_tracks;
+  k.status = a.status;
+  k.phi_tolerance = a.phi_tolerance;
+  k.max_scatter = a.max_scatter;
+  k.max_skipped_modules = a.max_skipped_modules;
+  k.lds_hits = lds_hits;
+  k.hits_per_wave = hits_per_wave;
+  k.work_stats = a.work_stats;
+  k.event_clock = a.event_clock;
+  k.n_list = a.n_list;
+  k.work_counter = a.work_counter;
+  k.seed_log = a.seed_log;
+  k.scorer_params = a.scorer_params;
+  k.scorer_threshold = a.scorer_threshold;
+  k.window = window;
+  k.list_cap = list_cap;
+#define VELO_LAUNCH_SEARCH_P(C, L, P) hipLaunchKernelGGL((k_search_by_triplet<C, L, P>), dim3(grid), dim3(block), dyn, s, k)
 #define VELO_LAUNCH_SEARCH(C, L)                                                                                    \
   do {                                                                                                              \
     if (a.work_counter) VELO_LAUNCH_SEARCH_P(C, L, true);                                                           \

@@ -317,7 +317,7 @@ typedef struct {
   float phi_tolerance;              /* 0.045 */
   float max_scatter;                /* 0.08 */
   unsigned max_skipped_modules;     /* 1 */
-  unsigned block_dim_x;             /* 0 = library default (256) */
+  unsigned block_dim_x;             /* 0: chosen from the number of events */
 } velo_search_by_triplet_params;
 int velo_search_by_triplet(const velo_search_by_triplet_params* p, hipStream_t stream);
 /* track_container_size of SearchByTriplet.cu:18-28 */
@@ -470,9 +470,12 @@ int velo_sequence_buffer(velo_sequence* s, const char* name, void** dev_ptr, siz
 /* Waits for the stream and returns the OR of the VELO_STATUS_* bits of the last run. */
 int velo_sequence_status(velo_sequence* s, hipStream_t stream, unsigned* status);
 /* Knobs applied to subsequent runs:
- *   "search_block"      workgroup size of search_by_triplet (multiple of 64, <= 1024; 0 = 256)
+ *   "search_block"      workgroup size of search_by_triplet (multiple of 64, <= 1024; 0,
+ *                       the default: this and the shape's other knobs left at 0 are chosen from
+ *                       the number of events; 256 with the scorer or "search_persistent")
  *   "search_lds_hits"   hits of an event staged in LDS by search_by_triplet (<= 8192, within the
- *                       device's LDS per workgroup; 0 = 1760); up to 5x that many hits keep phi
+ *                       device's LDS per workgroup; 0: as "search_block", 1760 for a workgroup
+ *                       size that is set); up to 16/3 of that many hits keep phi
  *                       and flags in LDS and coordinates in global memory, larger events run on
  *                       global memory
  *   "search_largest_first"  1 (default): search_by_triplet takes the events in descending order

@@ -266,3 +266,28 @@ def test_pruned_search_physics_on_20k_events(geometry, beamline):
     assert pruned["ghost_rate"] <= plain["ghost_rate"]
     seq.close()
     constants.close()
+
+
+@pytest.mark.parametrize("n", [1, 31, 33, 128, 129, 32769, 131105])
+def test_mlp_kernels_at_wave_and_grid_edges(n):
+    """Row counts around a wave's 32 seeds, a workgroup's 128, the training grid's cap (32 768 seeds
+    in one pass) and the scoring grid's (131 072): logits, loss and gradient, against the
+    restatement. Features start at an address that is a multiple of 4 bytes only. Bounds: the
+    logits' sums of 32 products round to about 1e-6 of their terms, and a hidden activation that
+    rounds to the other bf16 neighbour moves a logit by up to 2^-9 of one of its 32 terms; the
+    gradient's bf16 operands do the same to its terms (as in the tests above)."""
+    import torch
+    from allen_amd import scorer
+    x, y = _data(n, 100 + n)
+    p = scorer.init_params(13)
+    p[320:352] = 0.1
+    p[1376:1408] = -0.05
+    buf = torch.zeros(10 * n + 1, dtype=torch.float32, device="cuda")
+    buf[1:].copy_(torch.from_numpy(x.ravel()))
+    xd = buf[1:].view(n, 10)
+    net = scorer.MLP(p)
+    np.testing.assert_allclose(net.score(xd).cpu().numpy(), ref.forward(x, p)["z3"], rtol=1e-4, atol=2e-3)
+    loss, g = net.train_step(xd, torch.from_numpy(y).cuda(), 0.0, want_grad=True)
+    want = ref.gradient(x, y.astype(np.float64), p)
+    np.testing.assert_allclose(g, want, rtol=2e-3, atol=2e-3 * np.abs(want).max())
+    np.testing.assert_allclose(loss, ref.loss(x, y, p) / n, rtol=1e-4)
