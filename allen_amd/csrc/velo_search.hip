@@ -133,6 +133,11 @@ constexpr unsigned phi_bucket_shift = 9;
 constexpr unsigned phi_table_stride = phi_buckets + 2; // even, so that two entries can be written at once
 constexpr unsigned phi_tables_bytes = (n_module_pairs * phi_table_stride + 15) & ~15u;
 constexpr unsigned no_phi_table = 0xFFFFFFFFu;
+// A module pair whose phis are not in order: retina words of one pixel that differ only in their
+// fractions share a sorting key and so a slot, and the slot left over among the module pair's hits
+// holds whatever was there (one module pair in a few thousand events). Tables and runs need
+// order, so such a module pair is searched as irregular_search states.
+constexpr unsigned irregular_phis = 0xFFFFFFFEu;
 __device__ __forceinline__ unsigned phi_bucket(int16_t phi)
 {
   return static_cast<unsigned>(static_cast<uint16_t>(phi) ^ 0x8000u) >> phi_bucket_shift;
@@ -280,6 +285,27 @@ __device__ __forceinline__ unsigned counted_search(const H& hits, unsigned start
   return lo;
 }
 
+// The search in a module pair whose phis are out of order, where the answer depends on the way: the
+// 8-way search for the bounds of the value's bucket of 1024, then that bucket's elements, counted
+// directly for up to four (module pairs of more than 255 hits: the 8-way search over all hits).
+template<bool count, typename H>
+__device__ __forceinline__ unsigned irregular_search(const H& hits, const ModulePairData& mp, int16_t value, WorkCount& wc)
+{
+  unsigned lo = 0, hi = mp.hit_num;
+  if (mp.hit_num <= 255u) {
+    const int first = value & ~1023;
+    lo = counted_search<count>(hits, mp.hit_start, mp.hit_num, static_cast<int16_t>(first), wc);
+    if (first + 1024 <= 32767) hi = counted_search<count>(hits, mp.hit_start, mp.hit_num, static_cast<int16_t>(first + 1024), wc);
+    if (hi <= lo) return lo;
+    if (hi - lo <= 4) {
+      unsigned c = lo;
+      for (unsigned k = lo; k < hi; ++k) c += hits.phi(mp.hit_start + k) < value ? 1u : 0u;
+      return c;
+    }
+  }
+  return lo + counted_search<count>(hits, mp.hit_start + lo, hi - lo, value, wc);
+}
+
 // The same lower bound in a module pair through its bucket table: positions before the value's
 // bucket hold smaller phis and positions after it larger ones, so the answer is the bucket's
 // start plus the bucket's elements below the value (read directly for up to four, by
@@ -287,6 +313,7 @@ __device__ __forceinline__ unsigned counted_search(const H& hits, unsigned start
 template<bool count, typename H>
 __device__ __forceinline__ unsigned mp_search(const H& hits, const ModulePairData& mp, int16_t value, WorkCount& wc)
 {
+  if (mp.table == irregular_phis) return irregular_search<count>(hits, mp, value, wc);
   if (mp.table == no_phi_table) return counted_search<count>(hits, mp.hit_start, mp.hit_num, value, wc);
   const uint8_t* t = hits.tables + mp.table + phi_bucket(value);
   const unsigned lo = t[0], hi = t[1];
@@ -303,7 +330,7 @@ __device__ __forceinline__ unsigned mp_search(const H& hits, const ModulePairDat
 // The phi bucket tables of all module pairs that have one, four module pairs per wave at a time:
 // a histogram of the hits' buckets in LDS (`hist`, phi_buckets 16-bit counts per module pair),
 // turned into positions by a wave scan, two buckets a lane. hist_waves: the waves that hist has
-// room for.
+// room for. Module pairs whose phis are out of order are marked here.
 constexpr unsigned hist_words = phi_buckets / 2;
 constexpr unsigned hist_bytes = 4 * hist_words * sizeof(uint32_t);
 // LDS of the ring's window, which first holds the tables' histograms.
@@ -313,7 +340,7 @@ __host__ __device__ constexpr unsigned window_bytes(unsigned window)
 }
 template<typename H>
 __device__ __forceinline__ void
-build_phi_tables(const H& hits, const ModulePairData* mp, uint8_t* tables, uint32_t* hist, unsigned hist_waves, const Team& team)
+build_phi_tables(const H& hits, ModulePairData* mp, uint8_t* tables, uint32_t* hist, unsigned hist_waves, const Team& team)
 {
   static_assert(hist_words == wave_size, "two buckets per lane");
   const unsigned builders = min(team.waves, hist_waves);
@@ -326,22 +353,32 @@ build_phi_tables(const H& hits, const ModulePairData* mp, uint8_t* tables, uint3
   };
   for (unsigned m0 = 4 * team.wave; m0 < n_module_pairs; m0 += 4 * builders) {
     unsigned start[4], n[4];
-    int16_t p[4];
+    int16_t p[4], q[4];
+    bool table[4];
 #pragma unroll
     for (unsigned u = 0; u < 4; ++u) {
       const unsigned m = min(m0 + u, n_module_pairs - 1);
-      const bool has = m0 + u < n_module_pairs && mp[m].table != no_phi_table;
       start[u] = mp[m].hit_start;
-      n[u] = has ? mp[m].hit_num : 0u;
+      n[u] = m0 + u < n_module_pairs ? mp[m].hit_num : 0u;
+      table[u] = mp[m].table != no_phi_table;
       h[u * hist_words + l] = 0;
     }
 #pragma unroll
-    for (unsigned u = 0; u < 4; ++u) p[u] = l < n[u] ? hits.phi(start[u] + l) : int16_t(0);
+    for (unsigned u = 0; u < 4; ++u) {
+      p[u] = l < n[u] ? hits.phi(start[u] + l) : int16_t(0);
+      q[u] = l > 0 && l < n[u] ? hits.phi(start[u] + l - 1) : p[u]; // the hit before
+    }
     Team::wave_fence();
 #pragma unroll
     for (unsigned u = 0; u < 4; ++u) {
-      if (l < n[u]) count(u, p[u]);
-      for (unsigned i = l + wave_size; i < n[u]; i += wave_size) count(u, hits.phi(start[u] + i));
+      if (table[u] && l < n[u]) count(u, p[u]);
+      bool ordered = q[u] <= p[u];
+      for (unsigned i = l + wave_size; i < n[u]; i += wave_size) {
+        const int16_t phi = hits.phi(start[u] + i);
+        ordered = ordered && hits.phi(start[u] + i - 1) <= phi;
+        if (table[u]) count(u, phi);
+      }
+      if (__ballot(!ordered) && l == 0) mp[m0 + u].table = irregular_phis;
     }
     Team::wave_fence();
 #pragma unroll
@@ -349,7 +386,7 @@ build_phi_tables(const H& hits, const ModulePairData* mp, uint8_t* tables, uint3
       const uint32_t c = h[u * hist_words + l];
       const uint32_t both = (c & 0xFFFFu) + (c >> 16);
       const uint32_t before = wave_inclusive_scan(both) - both;
-      if (m0 + u < n_module_pairs) {
+      if (table[u] && m0 + u < n_module_pairs) {
         uint16_t* t = reinterpret_cast<uint16_t*>(tables + (m0 + u) * phi_table_stride);
         t[l] = static_cast<uint16_t>(before | (before + (c & 0xFFFFu)) << 8);
         if (l == 0) t[phi_buckets / 2] = static_cast<uint16_t>(n[u]);
@@ -452,7 +489,7 @@ __device__ __forceinline__ bool closest_hit_walk(
   WorkCount& wc, const H& hits, const ModulePairData& mp, const Line& l, int16_t phi_tolerance, float& best, uint32_t& best_index)
 {
   bool any = false;
-  unsigned p = counted_search<count>(hits, mp.hit_start, mp.hit_num, static_cast<int16_t>(l.phi - phi_tolerance), wc);
+  unsigned p = mp_search<count>(hits, mp, static_cast<int16_t>(l.phi - phi_tolerance), wc);
   for (unsigned j = 0; j < mp.hit_num; ++j, ++p) {
     if (p >= mp.hit_num) p -= mp.hit_num;
     const Hit h = hits.load(mp.hit_start + p);
@@ -483,15 +520,15 @@ constexpr int16_t max_run_tolerance = 8192;
 // (one dependent operation takes 8 cycles here, an independent one 5; an LDS read 64). Nearly
 // always one pass of four serves the whole wave. Where the walk differs from the run: its
 // |difference| of 16 bits takes a hit exactly opposite for one within any tolerance, which it can
-// reach only as its first hit, with none in the run; those lanes, and tolerances
-// beyond max_run_tolerance, take the walk itself.
+// reach only as its first hit, with none in the run; those lanes, tolerances
+// beyond max_run_tolerance and module pairs out of order take the walk itself.
 template<bool count, bool unused_only, typename H>
 __device__ __forceinline__ bool closest_hit(
   WorkCount& wc, const H& hits, const ModulePairData& mp, const Line& l, int16_t phi_tolerance, float& best, uint32_t& best_index)
 {
   const unsigned n = mp.hit_num;
   if (n == 0) return false;
-  if (phi_tolerance < 0 || phi_tolerance > max_run_tolerance)
+  if (phi_tolerance < 0 || phi_tolerance > max_run_tolerance || mp.table == irregular_phis)
     return closest_hit_walk<count, unused_only>(wc, hits, mp, l, phi_tolerance, best, best_index);
   const int16_t from = static_cast<int16_t>(l.phi - phi_tolerance), to = static_cast<int16_t>(l.phi + phi_tolerance);
   unsigned lo, hi;

@@ -104,3 +104,36 @@ def test_retina_drop_in_entry_points(geometry, beamline, constants):
     r = parity.cluster_views(ref["sorted_velo_cluster_container"], total)
     for a, b in zip(g, r):
         np.testing.assert_array_equal(a[slots_f].view(np.uint8), b[slots_f].view(np.uint8))
+
+
+def test_module_pair_out_of_order_is_searched_alike_in_every_layout(geometry, beamline):
+    """Retina words of one pixel with different fractions share a sorting key, and the slot left over
+    holds whatever was there: the module pair's phis are out of order. Every layout of the hits
+    (LDS, mixed, global) and workgroup size gives the same tracks."""
+    from allen_amd import synth, velo
+    ev = synth.generate(n_events=2180, pileup=0, mean_tracks=120.0, retina=1, seed=101 * 64 + 1, keep_truth=False)
+    constants = velo.VeloConstants(geometry, beamline)
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    dev = velo.DeviceEvents(ev)
+    got = {}
+    for name, knobs in {"default": {}, "one_wave": {"search_block": 64}, "mixed": {"search_block": 256, "search_lds_hits": 400},
+                        "global": {"search_block": 128, "search_lds_hits": 64}}.items():
+        for k in ("search_block", "search_lds_hits"):
+            seq.set_tuning(k, knobs.get(k, 0))
+        seq.run(dev)
+        assert seq.status() & velo.STATUS_OVERFLOW_MASK == 0
+        n = int(seq.fetch("offsets_all_velo_tracks", np.uint32, ev.n_events + 1)[-1])
+        hits = int(seq.fetch("offsets_velo_track_hit_number", np.uint32, n + 1)[-1])
+        got[name] = (seq.fetch("offsets_all_velo_tracks", np.uint32, ev.n_events + 1),
+                     seq.fetch("velo_track_hits", np.uint8, 16 * hits))
+    est = seq.fetch("offsets_estimated_input_size", np.uint32, 26 * ev.n_events + 1).astype(np.int64)
+    key = seq.fetch("hit_sorting_key", np.int64, int(est[-1]))
+    mp = np.repeat(np.arange(est.size - 1), np.diff(est))
+    order = np.lexsort((key, mp))
+    same = (np.diff(mp[order]) == 0) & (np.diff(key[order]) == 0) & (key[order][1:] != 0x7FFFFFFFFFFFFFFF)
+    assert same.any(), "no two words of a module pair share a key: the events no longer hold the case"
+    for name, (offsets, track_hits) in got.items():
+        np.testing.assert_array_equal(offsets, got["default"][0], err_msg=name)
+        np.testing.assert_array_equal(track_hits, got["default"][1], err_msg=name)
+    seq.close()
+    constants.close()
