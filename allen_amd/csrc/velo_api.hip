@@ -662,7 +662,7 @@ struct velo_sequence {
   bool scorer_on = false;         // buffer "scorer_params" holds the scorer's parameters
   float scorer_threshold = 0.f;
   unsigned kalman_fp64_fallback = 0;
-  bool consolidate_lds_map = true; // 0: consolidation takes the binary-search path for every event
+  bool consolidate_lds_map = true; // 0: consolidation and fit read every event's hits from memory
   unsigned pv_finder = 0;         // 1: PV finder after the fit; 2: also the z histograms ("zhisto")
   bool fused_clustering = true;
   bool count_work = false;
@@ -705,10 +705,7 @@ int velo_sequence_create(const velo_constants* c, unsigned max_events, size_t ma
   const unsigned T = static_cast<unsigned>(std::min<size_t>(s->cluster_cap, 0xFFFFFFF0u));
   s->track_cap = velo::track_container_size(T, max_events) + 1;
   s->hits_cap = s->track_cap * (velo::max_track_size + 3);
-  const size_t scan_words =
-    std::max({velo::prefix_sum_scratch_words(26 * max_events), velo::prefix_sum_scratch_words(velo::n_sensors * max_events),
-              velo::prefix_sum_scratch_words(2 * s->track_cap)}) +
-    1;
+  const size_t scan_words = velo::prefix_sum_scratch_words(velo::n_module_pairs * max_events) + 1;
   const std::vector<std::pair<const char*, size_t>> layout = {
     {"number_of_events", 4},
     {"status", 4},
@@ -748,6 +745,9 @@ int velo_sequence_create(const velo_constants* c, unsigned max_events, size_t ma
     {"search_event_clock", velo::event_clock_words * sizeof(unsigned long long) * E},
     {"search_order", 4 * E},
     {"search_counter", 4},
+    {"event_totals", 4 * E},
+    {"event_track_hits", 4 * E},
+    {"event_track_hit_offsets", 4 * (E + 1)},
     {"sp_flags", s->sp_cap},
     {"bank_directory", 16 * 8 * 26 * E},
     {"bank_directory_count", 4 * 26 * E},
@@ -974,8 +974,9 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     if (rcm_ != VELO_OK) return rcm_;                                                                               \
   } while (0)
   VELO_MARK(mark_begin(VELO_STAGE_ALL));
-  VELO_TRY(velo::launch_fill_u32(n_events_dev, 1, E, stream));
-  VELO_TRY(velo::launch_fill_u32(status, 1, 0, stream));
+  auto* event_totals = s->get<uint32_t>("event_totals");
+  // The events in descending order of their hits, for the search.
+  uint32_t* order = s->search_largest_first ? s->get<uint32_t>("search_order") : nullptr;
 
   auto* est_off = s->get<uint32_t>("offsets_estimated_input_size");
   auto* mcn = s->get<uint32_t>("module_cluster_num");
@@ -997,12 +998,21 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     r1.each_sensor_pair_size = s->get<uint32_t>("each_sensor_pair_size");
     r1.retina_bank_index = s->get<uint32_t>("retina_bank_index");
     VELO_MARK(mark_begin(VELO_STAGE_CANDIDATES));
-    VELO_TRY(velo::launch_fill_u32(r1.retina_bank_index, slots, 0xFFFFFFFFu, stream));
+    r1.event_totals = event_totals;
+    r1.number_of_events = n_events_dev;
+    r1.status = status;
     VELO_TRY(velo::launch_retina_sensor_sizes(r1, stream));
     VELO_MARK(mark_end(VELO_STAGE_CANDIDATES));
     auto* sp_off = s->get<uint32_t>("offsets_each_sensor_pair_size");
     VELO_MARK(mark_begin(VELO_STAGE_ESTIMATE));
-    VELO_TRY(velo::launch_prefix_sum(r1.each_sensor_pair_size, slots * E, sp_off, scratch, stream));
+    velo::EventScanLaunch scan;
+    scan.counts = r1.each_sensor_pair_size;
+    scan.per_event = slots;
+    scan.totals = event_totals;
+    scan.n_events = E;
+    scan.offsets = sp_off;
+    scan.order = order;
+    VELO_TRY(velo::launch_scan_events(scan, stream));
     VELO_MARK(mark_end(VELO_STAGE_ESTIMATE));
     velo::RetinaDecodeLaunch r2;
     r2.version = in->bank_version;
@@ -1045,11 +1055,19 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     if (s->fused_clustering) {
       k1.directory = s->get<void>("bank_directory");
       k1.directory_count = s->get<uint32_t>("bank_directory_count");
+      k1.number_of_events = n_events_dev;
+      k1.status = status;
+      k1.event_totals = event_totals;
+    }
+    else {
+      VELO_TRY(velo::launch_fill_u32(n_events_dev, 1, E, stream));
+      VELO_TRY(velo::launch_fill_u32(status, 1, 0, stream));
     }
     VELO_MARK(mark_begin(VELO_STAGE_CANDIDATES));
     VELO_TRY(velo::launch_number_of_candidates(k1, stream));
     VELO_MARK(mark_end(VELO_STAGE_CANDIDATES));
-    VELO_TRY(velo::launch_prefix_sum(k1.number_of_candidates, E, s->get<uint32_t>("candidates_offsets"), scratch, stream));
+    if (!s->fused_clustering)
+      VELO_TRY(velo::launch_prefix_sum(k1.number_of_candidates, E, s->get<uint32_t>("candidates_offsets"), scratch, stream));
 
     velo::EstimateLaunch k2;
     k2.version = in->bank_version;
@@ -1075,6 +1093,7 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
       e.directory_count = k1.directory_count;
       e.n_events = E;
       e.estimated_input_size = k2.estimated_input_size;
+      e.event_totals = event_totals;
       e.sp_flags = sp_flags;
       e.resident_grid = s->clustering_resident_grid;
       VELO_TRY(velo::launch_estimate_mp(e, stream));
@@ -1084,7 +1103,22 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
       VELO_TRY(velo::launch_estimate_input_size(k2, stream));
     }
     VELO_MARK(mark_end(VELO_STAGE_ESTIMATE));
-    VELO_TRY(velo::launch_prefix_sum(k2.estimated_input_size, 26 * E, est_off, scratch, stream));
+    if (s->fused_clustering) {
+      velo::EventScanLaunch scan;
+      scan.counts = k2.estimated_input_size;
+      scan.per_event = velo::n_module_pairs;
+      scan.totals = event_totals;
+      scan.n_events = E;
+      scan.offsets = est_off;
+      scan.candidates = k1.number_of_candidates;
+      scan.candidates_offsets = s->get<uint32_t>("candidates_offsets");
+      scan.order = order;
+      VELO_TRY(velo::launch_scan_events(scan, stream));
+    }
+    else {
+      VELO_TRY(velo::launch_prefix_sum(k2.estimated_input_size, 26 * E, est_off, scratch, stream));
+      if (order) VELO_TRY(velo::launch_order_events_by_hits(est_off, n_events_dev, order, stream));
+    }
 
     VELO_MARK(mark_begin(VELO_STAGE_CLUSTERING));
     if (s->fused_clustering) {
@@ -1164,6 +1198,10 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
   k5.phi_tolerance = in->phi_tolerance;
   k5.max_scatter = in->max_scatter;
   k5.max_skipped_modules = in->max_skipped_modules;
+  k5.three_hit_tracks_output = s->get<void>("three_hit_tracks_output");
+  k5.number_of_three_hit_tracks_output = s->get<uint32_t>("number_of_three_hit_tracks_output");
+  k5.event_track_hits = s->get<uint32_t>("event_track_hits");
+  k5.max_chi2 = in->max_chi2;
   k5.block_dim = s->search_block;
   k5.lds_hits = s->search_lds_hits;
   k5.ring_window = s->search_ring_window;
@@ -1188,10 +1226,7 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     k5.work_counter = s->get<uint32_t>("search_counter");
     VELO_TRY(velo::launch_fill_u32(k5.work_counter, 1, 0, stream));
   }
-  if (s->search_largest_first) {
-    k5.event_list = s->get<uint32_t>("search_order");
-    VELO_TRY(velo::launch_order_events_by_hits(est_off, n_events_dev, const_cast<uint32_t*>(k5.event_list), stream));
-  }
+  k5.event_list = order;
   // The largest events on the sequence's second stream (fork and join through events, so the
   // run stays one stream to the caller and capturable); the persistent grid takes every event.
   const unsigned n_big = s->search_largest_first && !s->search_persistent && s->search_split ? E / s->search_split : 0u;
@@ -1203,72 +1238,43 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     VELO_TRY(velo::launch_search_by_triplet(k5, stream));
   }
   VELO_MARK(mark_end(VELO_STAGE_SEARCH));
-  auto* off_tracks = s->get<uint32_t>("offsets_velo_tracks");
-  VELO_TRY(velo::launch_prefix_sum(k5.number_of_velo_tracks, E, off_tracks, scratch, stream));
-
-  velo::ThreeHitFilterLaunch k6;
-  k6.event_list = nullptr;
-  k6.n_list = E;
-  k6.number_of_events = n_events_dev;
-  k6.sorted_container = sorted;
-  k6.offsets_estimated_input_size = est_off;
-  k6.three_hit_tracks_input = k5.three_hit_tracks;
-  k6.atomics_velo = k5.atomics_velo;
-  k6.hit_used = k5.hit_used;
-  k6.three_hit_tracks_output = s->get<void>("three_hit_tracks_output");
-  k6.number_of_three_hit_tracks_output = s->get<uint32_t>("number_of_three_hit_tracks_output");
-  k6.max_chi2 = in->max_chi2;
+  // The three-hit filter ran at the end of each event's search; the consolidation's launch holds
+  // the fit. Their stages' brackets are empty.
   VELO_MARK(mark_begin(VELO_STAGE_THREE_HIT_FILTER));
-  VELO_TRY(velo::launch_three_hit_tracks_filter(k6, stream));
   VELO_MARK(mark_end(VELO_STAGE_THREE_HIT_FILTER));
-  auto* off_three = s->get<uint32_t>("offsets_three_hit_tracks_filtered");
-  VELO_TRY(velo::launch_prefix_sum(k6.number_of_three_hit_tracks_output, E, off_three, scratch, stream));
-
-  velo::CopyHitNumberLaunch k7;
+  velo::TrackOffsetsLaunch k7;
   k7.n_events = E;
-  k7.tracks = k5.tracks;
-  k7.offsets_velo_tracks = off_tracks;
-  k7.offsets_estimated_input_size = est_off;
-  k7.offsets_three_hit = off_three;
-  k7.velo_track_hit_number = s->get<uint32_t>("velo_track_hit_number");
+  k7.number_of_velo_tracks = k5.number_of_velo_tracks;
+  k7.number_of_three_hit_tracks = k5.number_of_three_hit_tracks_output;
+  k7.event_track_hits = k5.event_track_hits;
+  k7.offsets_velo_tracks = s->get<uint32_t>("offsets_velo_tracks");
+  k7.offsets_three_hit = s->get<uint32_t>("offsets_three_hit_tracks_filtered");
   k7.offsets_all_velo_tracks = s->get<uint32_t>("offsets_all_velo_tracks");
-  VELO_TRY(velo::launch_copy_track_hit_number(k7, stream));
-  auto* off_hits = s->get<uint32_t>("offsets_velo_track_hit_number");
-  VELO_TRY(velo::launch_prefix_sum_dyn(
-    k7.velo_track_hit_number, k7.offsets_all_velo_tracks + E, 2 * s->track_cap, off_hits, scratch, stream));
-
-  velo::ConsolidateLaunch k8;
-  k8.lds_map = s->consolidate_lds_map;
-  k8.event_list = nullptr;
-  k8.n_list = E;
-  k8.number_of_events = n_events_dev;
-  k8.offsets_all_velo_tracks = k7.offsets_all_velo_tracks;
-  k8.tracks = k5.tracks;
-  k8.offsets_velo_track_hit_number = off_hits;
-  k8.sorted_container = sorted;
+  k7.event_hit_offsets = s->get<uint32_t>("event_track_hit_offsets");
+  velo::TrackFitLaunch k8;
+  k8.n_events = E;
   k8.offsets_estimated_input_size = est_off;
-  k8.three_hit_tracks_output = k6.three_hit_tracks_output;
-  k8.offsets_three_hit = off_three;
+  k8.offsets_all_velo_tracks = k7.offsets_all_velo_tracks;
+  k8.offsets_three_hit = k7.offsets_three_hit;
+  k8.event_hit_offsets = k7.event_hit_offsets;
+  k8.sorted_container = sorted;
+  k8.tracks = k5.tracks;
+  k8.three_hit_tracks_output = k5.three_hit_tracks_output;
+  k8.beamline = s->constants->dev_beamline;
+  k8.lds_hits = s->consolidate_lds_map;
+  k8.fp64_fallback = s->kalman_fp64_fallback;
+  k8.velo_track_hit_number = s->get<uint32_t>("velo_track_hit_number");
+  k8.offsets_velo_track_hit_number = s->get<uint32_t>("offsets_velo_track_hit_number");
   k8.velo_track_hits = s->get<char>("velo_track_hits");
   k8.accepted_velo_tracks = s->get<uint8_t>("accepted_velo_tracks");
+  k8.is_backward = s->get<uint8_t>("is_backward");
+  k8.beamline_states = s->get<char>("velo_kalman_beamline_states");
+  k8.endvelo_states = s->get<char>("velo_kalman_endvelo_states");
   VELO_MARK(mark_begin(VELO_STAGE_CONSOLIDATE));
-  VELO_TRY(velo::launch_consolidate_tracks(k8, stream));
+  VELO_TRY(velo::launch_track_offsets(k7, stream));
+  VELO_TRY(velo::launch_consolidate_and_fit(k8, stream));
   VELO_MARK(mark_end(VELO_STAGE_CONSOLIDATE));
-
-  velo::KalmanLaunch k9;
-  k9.event_list = nullptr;
-  k9.n_list = E;
-  k9.number_of_events = n_events_dev;
-  k9.offsets_all_velo_tracks = k7.offsets_all_velo_tracks;
-  k9.offsets_velo_track_hit_number = off_hits;
-  k9.velo_track_hits = k8.velo_track_hits;
-  k9.beamline = s->constants->dev_beamline;
-  k9.is_backward = s->get<uint8_t>("is_backward");
-  k9.beamline_states = s->get<char>("velo_kalman_beamline_states");
-  k9.fp64_fallback = s->kalman_fp64_fallback;
-  k9.endvelo_states = s->get<char>("velo_kalman_endvelo_states");
   VELO_MARK(mark_begin(VELO_STAGE_KALMAN));
-  VELO_TRY(velo::launch_kalman_filter(k9, stream));
   VELO_MARK(mark_end(VELO_STAGE_KALMAN));
   if (s->pv_finder) {
     velo::PVLaunch pv;

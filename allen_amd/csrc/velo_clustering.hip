@@ -345,10 +345,89 @@ __global__ void k_number_of_candidates(
   if (lane_id() == 0) number_of_candidates[event_number] = 2 * n;
 }
 
+// dev_velo_bank_index as the CPU target leaves it: events of CPU block 0 (ev_idx = 0, G, 2G, ...)
+// write in order and the last write of each entry wins. Walk those events backwards and keep the
+// first value seen per entry; stop once every sensor has one.
+struct BankIndexShared {
+  int best[n_sensors];
+  uint8_t written[n_sensors];
+  unsigned n_written;
+};
+template<int version>
+__device__ __forceinline__ void bank_index_block(
+  const char* raw,
+  const uint32_t* offsets,
+  const uint32_t* sizes,
+  const uint32_t* types,
+  unsigned mep,
+  const uint32_t* event_list,
+  unsigned n_list,
+  unsigned event_start,
+  unsigned cpu_grid,
+  uint32_t* bank_index,
+  BankIndexShared& sh)
+{
+  int(&best)[n_sensors] = sh.best;
+  uint8_t(&written)[n_sensors] = sh.written;
+  unsigned& n_written = sh.n_written;
+  for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) written[i] = 0;
+  if (threadIdx.x == 0) n_written = 0;
+  __syncthreads();
+  if (n_list == 0) return;
+  const unsigned last = ((n_list - 1) / cpu_grid) * cpu_grid;
+  for (int ev_idx = last; ev_idx >= 0; ev_idx -= cpu_grid) {
+    for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) best[i] = -1;
+    __syncthreads();
+    const unsigned event_number = event_list ? event_list[ev_idx] : ev_idx;
+    const RawEvent ev(raw, offsets, sizes, types, mep, event_number + event_start);
+    for (unsigned b = threadIdx.x; b < ev.n_banks; b += blockDim.x) {
+      const RawBank bank = raw_bank<version>(ev, b);
+      const uint32_t pair = bank.sourceID & 0x1FFu;
+      // Entries beyond the 208 sensors would be written out of bounds by the reference;
+      // they are skipped here.
+      if constexpr (version > 3) {
+        if ((pair << 1) < n_sensors) atomicMax(&best[pair << 1], (int) b);
+        if (((pair << 1) | 1u) < n_sensors) atomicMax(&best[(pair << 1) | 1u], (int) b);
+      }
+      else {
+        if (pair < n_sensors) atomicMax(&best[pair], (int) b);
+      }
+    }
+    __syncthreads();
+    for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) {
+      if (best[i] >= 0 && !written[i]) {
+        bank_index[i] = best[i];
+        written[i] = 1;
+        atomicAdd(&n_written, 1u);
+      }
+    }
+    __syncthreads();
+    if (n_written >= n_sensors) break;
+  }
+}
+
+template<int version>
+__global__ void k_bank_index(
+  const char* raw,
+  const uint32_t* offsets,
+  const uint32_t* sizes,
+  const uint32_t* types,
+  unsigned mep,
+  const uint32_t* event_list,
+  unsigned n_list,
+  unsigned event_start,
+  unsigned cpu_grid,
+  uint32_t* bank_index)
+{
+  __shared__ BankIndexShared sh;
+  bank_index_block<version>(raw, offsets, sizes, types, mep, event_list, n_list, event_start, cpu_grid, bank_index, sh);
+}
+
 // Bank directory of the whole-sequence path: one wave per event reads the bank headers once
 // and writes, per (event, module pair), the module pair's banks in bank order (at most 8) as
 // {first SP word (index into the raw buffer in 32-bit words), SP words, sourceID}, plus their
-// number. Also writes dev_number_of_candidates (2 x SP words of the VELO banks).
+// number. Also writes dev_number_of_candidates (2 x SP words of the VELO banks), what later
+// launches of the run start from, and (the last workgroup) dev_velo_bank_index.
 template<int version>
 __global__ void k_bank_directory(
   const char* raw,
@@ -359,8 +438,22 @@ __global__ void k_bank_directory(
   unsigned n_events,
   uint32_t* number_of_candidates,
   BankEntry* directory,
-  uint32_t* directory_count)
+  uint32_t* directory_count,
+  uint32_t* event_totals,
+  uint32_t* number_of_events,
+  uint32_t* status,
+  unsigned cpu_grid,
+  uint32_t* bank_index)
 {
+  if (blockIdx.x + 1 == gridDim.x) {
+    __shared__ BankIndexShared sh;
+    if (threadIdx.x == 0) {
+      number_of_events[0] = n_events;
+      status[0] = 0;
+    }
+    bank_index_block<version>(raw, offsets, sizes, types, mep, nullptr, n_events, 0, cpu_grid, bank_index, sh);
+    return;
+  }
   constexpr bool v23 = (version == 2 || version == 3);
   const unsigned waves = blockDim.x / wave_size;
   const unsigned e = blockIdx.x * waves + threadIdx.x / wave_size;
@@ -404,61 +497,9 @@ __global__ void k_bank_directory(
 #pragma unroll
   for (unsigned d = 32; d > 0; d >>= 1) total += __shfl_xor(total, d, wave_size);
   if (lane_id() < n_module_pairs) directory_count[e * n_module_pairs + lane_id()] = min(my_count, max_banks_per_mp);
-  if (lane_id() == 0) number_of_candidates[e] = 2 * total;
-}
-
-// dev_velo_bank_index as the CPU target leaves it: events of CPU block 0 (ev_idx = 0, G, 2G, ...)
-// write in order and the last write of each entry wins. Walk those events backwards and keep the
-// first value seen per entry; stop once every sensor has one.
-template<int version>
-__global__ void k_bank_index(
-  const char* raw,
-  const uint32_t* offsets,
-  const uint32_t* sizes,
-  const uint32_t* types,
-  unsigned mep,
-  const uint32_t* event_list,
-  unsigned n_list,
-  unsigned event_start,
-  unsigned cpu_grid,
-  uint32_t* bank_index)
-{
-  __shared__ int best[n_sensors];
-  __shared__ uint8_t written[n_sensors];
-  __shared__ unsigned n_written;
-  for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) written[i] = 0;
-  if (threadIdx.x == 0) n_written = 0;
-  __syncthreads();
-  if (n_list == 0) return;
-  const unsigned last = ((n_list - 1) / cpu_grid) * cpu_grid;
-  for (int ev_idx = last; ev_idx >= 0; ev_idx -= cpu_grid) {
-    for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) best[i] = -1;
-    __syncthreads();
-    const unsigned event_number = event_list ? event_list[ev_idx] : ev_idx;
-    const RawEvent ev(raw, offsets, sizes, types, mep, event_number + event_start);
-    for (unsigned b = threadIdx.x; b < ev.n_banks; b += blockDim.x) {
-      const RawBank bank = raw_bank<version>(ev, b);
-      const uint32_t pair = bank.sourceID & 0x1FFu;
-      // Entries beyond the 208 sensors would be written out of bounds by the reference;
-      // they are skipped here.
-      if constexpr (version > 3) {
-        if ((pair << 1) < n_sensors) atomicMax(&best[pair << 1], (int) b);
-        if (((pair << 1) | 1u) < n_sensors) atomicMax(&best[(pair << 1) | 1u], (int) b);
-      }
-      else {
-        if (pair < n_sensors) atomicMax(&best[pair], (int) b);
-      }
-    }
-    __syncthreads();
-    for (unsigned i = threadIdx.x; i < n_sensors; i += blockDim.x) {
-      if (best[i] >= 0 && !written[i]) {
-        bank_index[i] = best[i];
-        written[i] = 1;
-        atomicAdd(&n_written, 1u);
-      }
-    }
-    __syncthreads();
-    if (n_written >= n_sensors) break;
+  if (lane_id() == 0) {
+    number_of_candidates[e] = 2 * total;
+    event_totals[e] = 0;
   }
 }
 
@@ -659,199 +700,28 @@ __global__ void k_sort_by_phi(
 }
 
 // ---------------------------------------------------------------------------------------
-// Fused K2+K3+K4 per (module pair, event), used by the whole-sequence path after the
-// estimate scan. The module pair's SP words are staged in LDS; clusters are built into LDS,
-// ranked by (phi, id) and written to their sorted slot. A module pair that does not fit
-// the LDS budget is processed the same way out of global memory.
-constexpr unsigned fused_word_cap = 1024;
-constexpr unsigned fused_cluster_cap = 1024;
-
-template<int version>
-__global__ void __launch_bounds__(256) k_cluster_sorted(
-  const char* raw,
-  const uint32_t* offsets,
-  const uint32_t* sizes,
-  const uint32_t* types,
-  unsigned mep,
-  unsigned n_events,
-  const uint32_t* offsets_estimated_input_size,
-  const Geometry* geometry,
-  const uint8_t* sp_patterns,
-  const float* sp_fx,
-  const float* sp_fy,
-  uint32_t* module_cluster_num,
-  char* sorted_container,
-  char* unsorted_scratch,
-  uint32_t* status)
-{
-  __shared__ uint32_t s_words[fused_word_cap];
-  __shared__ int16_t s_phi[fused_cluster_cap];
-  __shared__ uint32_t s_id[fused_cluster_cap];
-  __shared__ float s_xyz[3 * fused_cluster_cap];
-  __shared__ uint32_t s_bank_start[max_banks_per_mp + 1];
-  __shared__ uint32_t s_bank_num[max_banks_per_mp];
-  __shared__ uint32_t s_bank_src[max_banks_per_mp];
-  __shared__ unsigned s_nbanks, s_count;
-
-  constexpr bool v23 = (version == 2 || version == 3);
-  const unsigned mp = blockIdx.x;
-  const unsigned event_number = blockIdx.y;
-  const unsigned total = offsets_estimated_input_size[n_module_pairs * n_events];
-  const unsigned start = offsets_estimated_input_size[event_number * n_module_pairs + mp];
-  const unsigned estimate = offsets_estimated_input_size[event_number * n_module_pairs + mp + 1] - start;
-  const Geometry& g = *geometry;
-  const RawEvent ev(raw, offsets, sizes, types, mep, event_number);
-
-  // Banks of this module pair, in bank order.
-  if (threadIdx.x == 0) s_nbanks = 0;
-  __syncthreads();
-  for (unsigned b = threadIdx.x; b < ev.n_banks; b += blockDim.x) {
-    const RawBank bank = raw_bank<version>(ev, b);
-    if (!is_velo_bank(bank.type)) continue;
-    const uint32_t pair = bank.sourceID & 0x1FFu;
-    const unsigned bmp = v23 ? pair / 8 : (pair << 1) / 8;
-    if (bmp == mp) {
-      const unsigned k = atomicAdd(&s_nbanks, 1u);
-      if (k < max_banks_per_mp) s_bank_num[k] = b;
-    }
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    const unsigned nb = min(s_nbanks, max_banks_per_mp);
-    // insertion sort: a handful of banks
-    for (unsigned i = 1; i < nb; ++i) {
-      const uint32_t v = s_bank_num[i];
-      int j = i - 1;
-      while (j >= 0 && s_bank_num[j] > v) {
-        s_bank_num[j + 1] = s_bank_num[j];
-        --j;
-      }
-      s_bank_num[j + 1] = v;
-    }
-    uint32_t acc = 0;
-    for (unsigned i = 0; i < nb; ++i) {
-      const RawBank bank = raw_bank<version>(ev, s_bank_num[i]);
-      s_bank_start[i] = acc;
-      s_bank_src[i] = bank.sourceID;
-      acc += bank_n_sp<version>(bank);
-    }
-    s_bank_start[nb] = acc;
-    s_nbanks = nb;
-    s_count = 0;
-  }
-  __syncthreads();
-  const unsigned nb = s_nbanks;
-  const unsigned n_words = s_bank_start[nb];
-  const bool words_in_lds = n_words <= fused_word_cap;
-  const bool clusters_in_lds = estimate <= fused_cluster_cap;
-  if (!words_in_lds || !clusters_in_lds) {
-    if (threadIdx.x == 0) atomicOr(status, (uint32_t) status_lds_fallback);
-  }
-  if (words_in_lds) {
-    for (unsigned bi = 0; bi < nb; ++bi) {
-      const RawBank bank = raw_bank<version>(ev, s_bank_num[bi]);
-      const unsigned n = s_bank_start[bi + 1] - s_bank_start[bi];
-      for (unsigned s = threadIdx.x; s < n; s += blockDim.x) s_words[s_bank_start[bi] + s] = bank.word[s];
-    }
-  }
-  __syncthreads();
-
-  // Clusters go to LDS, or to the unsorted scratch container (same gapped layout) if too many.
-  const Clusters scratch {unsorted_scratch, total};
-  auto emit = [&](const ClusterOut& c) {
-    const unsigned slot = atomicAdd(&s_count, 1u);
-    if (slot >= estimate) return; // cannot happen for well-formed banks: estimate bounds the count
-    if (clusters_in_lds) {
-      s_phi[slot] = c.phi;
-      s_id[slot] = c.id;
-      s_xyz[3 * slot] = c.x;
-      s_xyz[3 * slot + 1] = c.y;
-      s_xyz[3 * slot + 2] = c.z;
-    }
-    else {
-      store_cluster(scratch, start + slot, c);
-    }
-  };
-
-  for (unsigned w = threadIdx.x; w < n_words; w += blockDim.x) {
-    unsigned bi = 0;
-    while (bi + 1 < nb && s_bank_start[bi + 1] <= w) ++bi;
-    const unsigned s = w - s_bank_start[bi];
-    RawBank bank;
-    bank.sourceID = s_bank_src[bi];
-    const unsigned n_sp = s_bank_start[bi + 1] - s_bank_start[bi];
-    const uint32_t* words;
-    if (words_in_lds) words = s_words + s_bank_start[bi];
-    else words = raw_bank<version>(ev, s_bank_num[bi]).word;
-    const uint32_t sp_word = words[s];
-    if (sp_word & 0x80000000u) {
-      ClusterOut c0, c1;
-      const unsigned n = isolated_sp_clusters<version>(g, sp_patterns, sp_fx, sp_fy, bank, sp_word, c0, c1);
-      emit(c0);
-      if (n > 1) emit(c1);
-    }
-    else {
-      unsigned p0 = 0, p1 = 0;
-      const unsigned m = sp_candidates(sp_word, words, n_sp, &p0, &p1);
-      const uint32_t pair = bank.sourceID & 0x1FFu;
-      const uint32_t sensor_number = v23 ? pair : ((pair << 1) | ((sp_word >> 23) & 0x1u));
-      ClusterOut c;
-      if ((m & 1) && masked_cluster<version>(g, words, n_sp, s, sensor_number, p0, &c)) emit(c);
-      if ((m & 2) && masked_cluster<version>(g, words, n_sp, s, sensor_number, p1, &c)) emit(c);
-    }
-  }
-  __threadfence_block();
-  __syncthreads();
-  const unsigned n = min(s_count, estimate);
-  if (threadIdx.x == 0) module_cluster_num[event_number * n_module_pairs + mp] = n;
-  const Clusters out {sorted_container, total};
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
-    unsigned r;
-    ClusterOut c;
-    if (clusters_in_lds) {
-      r = phi_rank(s_phi, s_id, n, i);
-      c.id = s_id[i];
-      c.phi = s_phi[i];
-      c.x = s_xyz[3 * i];
-      c.y = s_xyz[3 * i + 1];
-      c.z = s_xyz[3 * i + 2];
-    }
-    else {
-      r = phi_rank(scratch.phis() + start, scratch.ids() + start, n, i);
-      c.id = scratch.ids()[start + i];
-      c.phi = scratch.phis()[start + i];
-      c.x = scratch.xyz()[3 * (size_t)(start + i)];
-      c.y = scratch.xyz()[3 * (size_t)(start + i) + 1];
-      c.z = scratch.xyz()[3 * (size_t)(start + i) + 2];
-    }
-    store_cluster(out, start + r, c);
-  }
-}
-
-// ---------------------------------------------------------------------------------------
 // Host launchers.
 template<int version>
 static hipError_t launch_candidates_v(const CandidatesLaunch& a, hipStream_t s)
 {
   const unsigned waves = 4;
   const unsigned grid = (a.n_list + waves - 1) / waves;
-  if (grid && a.directory) {
-    if (a.event_list || a.event_start) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(
-      k_bank_directory<version>, dim3(grid), dim3(waves * wave_size), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),
-      a.n_list, a.number_of_candidates, static_cast<BankEntry*>(a.directory), a.directory_count);
-  }
-  else if (grid) {
-    hipLaunchKernelGGL(
-      k_number_of_candidates<version>, dim3(grid), dim3(waves * wave_size), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),
-      a.event_list, a.n_list, a.event_start, a.number_of_candidates);
-  }
   const unsigned cpu_grid = (a.n_list + a.block_dim_x - 1) / a.block_dim_x;
-  if (a.n_list) {
+  if (!grid) return hipSuccess;
+  if (a.directory) {
+    if (a.event_list || a.event_start || !a.event_totals || !a.number_of_events || !a.status) return hipErrorInvalidValue;
     hipLaunchKernelGGL(
-      k_bank_index<version>, dim3(1), dim3(256), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list, a.n_list,
-      a.event_start, cpu_grid, a.bank_index);
+      k_bank_directory<version>, dim3(grid + 1), dim3(waves * wave_size), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),
+      a.n_list, a.number_of_candidates, static_cast<BankEntry*>(a.directory), a.directory_count, a.event_totals,
+      a.number_of_events, a.status, cpu_grid, a.bank_index);
+    return hipGetLastError();
   }
+  hipLaunchKernelGGL(
+    k_number_of_candidates<version>, dim3(grid), dim3(waves * wave_size), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),
+    a.event_list, a.n_list, a.event_start, a.number_of_candidates);
+  hipLaunchKernelGGL(
+    k_bank_index<version>, dim3(1), dim3(256), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list, a.n_list,
+    a.event_start, cpu_grid, a.bank_index);
   return hipGetLastError();
 }
 
@@ -906,24 +776,6 @@ hipError_t launch_sort_by_phi(const SortLaunch& a, hipStream_t s)
     a.offsets_estimated_input_size, a.module_cluster_num, a.cluster_container, a.sorted_container, a.hit_permutation);
   return hipGetLastError();
 }
-
-hipError_t launch_cluster_sorted(const FusedClusterLaunch& a, hipStream_t s)
-{
-  if (!a.n_events) return hipSuccess;
-#define VELO_LAUNCH_FUSED(V)                                                                                        \
-  hipLaunchKernelGGL(                                                                                               \
-    k_cluster_sorted<V>, dim3(n_module_pairs, a.n_events), dim3(256), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),     \
-    a.n_events, a.offsets_estimated_input_size, reinterpret_cast<const Geometry*>(a.geometry), a.sp_patterns,        \
-    a.sp_fx, a.sp_fy, a.module_cluster_num, a.sorted_container, a.unsorted_scratch, a.status)
-  switch (a.version) {
-  case 2: VELO_LAUNCH_FUSED(2); break;
-  case 3: VELO_LAUNCH_FUSED(3); break;
-  default: VELO_LAUNCH_FUSED(4); break;
-  }
-#undef VELO_LAUNCH_FUSED
-  return hipGetLastError();
-}
-
 
 // ---------------------------------------------------------------------------------------
 // Whole-sequence clustering, one wave per (event, module pair), no block barriers.
@@ -1099,6 +951,7 @@ __device__ __forceinline__ void estimate_item(
   uint32_t* lw,
   uint32_t* table_slots,
   uint32_t* estimated_input_size,
+  uint32_t* event_totals,
   uint8_t* sp_flags)
 {
   mp::load_banks(raw, dir, B);
@@ -1195,7 +1048,10 @@ __device__ __forceinline__ void estimate_item(
   }
 #pragma unroll
   for (unsigned d = 32; d > 0; d >>= 1) count += __shfl_xor(count, d, wave_size);
-  if (lane_id() == 0) estimated_input_size[idx] = count;
+  if (lane_id() == 0) {
+    estimated_input_size[idx] = count;
+    atomicAdd(event_totals + idx / n_module_pairs, count);
+  }
 }
 
 // Resident grid: each wave takes items idx, idx + stride, ... and fetches the next item's
@@ -1207,6 +1063,7 @@ __global__ void __launch_bounds__(mp::waves_per_block* wave_size) k_estimate_mp(
   const uint32_t* directory_count,
   unsigned n_events,
   uint32_t* estimated_input_size,
+  uint32_t* event_totals,
   uint8_t* sp_flags)
 {
   __shared__ uint32_t s_words[mp::waves_per_block][mp::word_cap];
@@ -1222,7 +1079,7 @@ __global__ void __launch_bounds__(mp::waves_per_block* wave_size) k_estimate_mp(
     mp::DirFetch next = cur;
     if (idx + stride < n_items) next = mp::fetch_dir(directory, directory_count, idx + stride);
     estimate_item(raw, cur, idx, s_banks[wave], s_words[wave], s_table[wave], estimated_input_size,
-                  sp_flags);
+                  event_totals, sp_flags);
     cur = next;
   }
 }
@@ -1638,7 +1495,8 @@ hipError_t launch_estimate_mp(const EstimateMpLaunch& a, hipStream_t s)
 #define VELO_LAUNCH_EMP(V)                                                                                          \
   hipLaunchKernelGGL(                                                                                               \
     k_estimate_mp<V>, dim3(grid), dim3(mp::waves_per_block * wave_size), 0, s, a.raw,                               \
-    static_cast<const BankEntry*>(a.directory), a.directory_count, a.n_events, a.estimated_input_size, a.sp_flags)
+    static_cast<const BankEntry*>(a.directory), a.directory_count, a.n_events, a.estimated_input_size,            \
+    a.event_totals, a.sp_flags)
   switch (a.version) {
   case 2: VELO_LAUNCH_EMP(2); break;
   case 3: VELO_LAUNCH_EMP(3); break;

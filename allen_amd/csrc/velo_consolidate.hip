@@ -5,6 +5,8 @@
 //   k_kalman_filter           VeloKalmanFilter.cu:335-418, VeloKalmanFilter.cuh:25-158 (one thread per track)
 //   k_create_velo_views       VeloConsolidateTracks.cu:11-46 (Allen's view objects, byte for byte)
 //   k_clusters_views          MaskedVeloClustering.cu:519-522, DecodeRetinaClusters.cu:331-346
+//   k_consolidate_and_fit     the three above in one launch (whole sequence; one workgroup per event)
+//   k_scan_events, k_track_offsets  the whole sequence's offsets from per-event totals
 //   k_scan_*                  replaces host_prefix_sum_t (HostPrefixSum.cpp:76-107) by a device scan
 #include "velo_amd.h"
 #include "velo_common.cuh"
@@ -24,24 +26,17 @@ namespace velo {
 constexpr unsigned scan_block = 1024;
 constexpr unsigned scan_items = 4;
 constexpr unsigned scan_tile = scan_block * scan_items;
-constexpr unsigned one_pass_items = 32;
-constexpr unsigned one_pass_max = scan_block * one_pass_items;
+constexpr unsigned one_pass_max = 32 * scan_block;
 
 __device__ __forceinline__ uint32_t block_scan_1024(uint32_t v, uint32_t* scratch, uint32_t* total)
 {
   return block_exclusive_scan(v, scratch, total);
 }
 
-__device__ __forceinline__ unsigned scan_length(const uint32_t* n_dev, unsigned n_cap)
-{
-  return n_dev ? min(n_dev[0], n_cap) : n_cap;
-}
-
 __global__ void __launch_bounds__(scan_block)
-  k_scan_tile_sums(const uint32_t* in, const uint32_t* n_dev, unsigned n_cap, uint32_t* tile_sums)
+  k_scan_tile_sums(const uint32_t* in, unsigned n, uint32_t* tile_sums)
 {
   __shared__ uint32_t scratch[scan_block / wave_size + 1];
-  const unsigned n = scan_length(n_dev, n_cap);
   const size_t base = (size_t) blockIdx.x * scan_tile;
   uint32_t s = 0;
 #pragma unroll
@@ -69,19 +64,17 @@ __global__ void __launch_bounds__(scan_block) k_scan_small_inplace(uint32_t* v, 
   }
 }
 
-// Per-tile scan: thread t owns items [t*items, (t+1)*items) of its tile (contiguous, so the
+// Per-tile scan: thread t owns items [t*scan_items, (t+1)*scan_items) of its tile (contiguous, so the
 // prefix within a thread is a short serial sum).
-template<unsigned items>
 __global__ void __launch_bounds__(scan_block)
-  k_scan_tiles(const uint32_t* in, const uint32_t* n_dev, unsigned n_cap, uint32_t* out, const uint32_t* tile_offsets)
+  k_scan_tiles(const uint32_t* in, unsigned n, uint32_t* out, const uint32_t* tile_offsets)
 {
   __shared__ uint32_t scratch[scan_block / wave_size + 1];
-  const unsigned n = scan_length(n_dev, n_cap);
-  const size_t base = (size_t) blockIdx.x * scan_block * items + (size_t) threadIdx.x * items;
-  uint32_t v[items];
+  const size_t base = (size_t) blockIdx.x * scan_block * scan_items + (size_t) threadIdx.x * scan_items;
+  uint32_t v[scan_items];
   uint32_t s = 0;
 #pragma unroll
-  for (unsigned k = 0; k < items; ++k) {
+  for (unsigned k = 0; k < scan_items; ++k) {
     const size_t i = base + k;
     v[k] = i < n ? in[i] : 0u;
     s += v[k];
@@ -90,42 +83,104 @@ __global__ void __launch_bounds__(scan_block)
   uint32_t run = block_scan_1024(s, scratch, &total) + (tile_offsets ? tile_offsets[blockIdx.x] : 0u);
   if (blockIdx.x == 0 && threadIdx.x == 0) out[0] = 0;
 #pragma unroll
-  for (unsigned k = 0; k < items; ++k) {
+  for (unsigned k = 0; k < scan_items; ++k) {
     const size_t i = base + k;
     run += v[k];
     if (i < n) out[i + 1] = run;
   }
 }
 
-size_t prefix_sum_scratch_words(unsigned n) { return (n + scan_tile - 1) / scan_tile; }
-
-hipError_t launch_prefix_sum_dyn(
-  const uint32_t* in,
-  const uint32_t* n_dev,
-  unsigned n_cap,
-  uint32_t* out,
-  uint32_t* scratch,
-  hipStream_t s)
+// Prefix over n arrays of equal length (per event, say) by one workgroup of 1024: wave w takes a
+// contiguous range, sums it, and scans it again from the sum of the waves before. emit(i, k,
+// inclusive prefix) is called for every item and array. Every read is a whole wave's line.
+template<unsigned n, typename F>
+__device__ __forceinline__ void
+scan_by_waves(const uint32_t* const (&in)[n], unsigned n_events, uint32_t (&scratch)[n][scan_block / wave_size], F&& emit)
 {
-  const unsigned tiles = (n_cap + scan_tile - 1) / scan_tile;
-  if (tiles <= 1) {
-    hipLaunchKernelGGL(k_scan_tiles<scan_items>, dim3(1), dim3(scan_block), 0, s, in, n_dev, n_cap, out, nullptr);
-    return hipGetLastError();
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / wave_size), l = lane_id();
+  const unsigned range = (n_events + scan_block - 1) / scan_block * wave_size;
+  const unsigned begin = min(wave * range, n_events), end = min(begin + range, n_events);
+  uint32_t sum[n];
+#pragma unroll
+  for (unsigned k = 0; k < n; ++k) sum[k] = 0;
+  for (unsigned i = begin + l; i < end; i += wave_size)
+#pragma unroll
+    for (unsigned k = 0; k < n; ++k) sum[k] += in[k][i];
+#pragma unroll
+  for (unsigned k = 0; k < n; ++k) {
+    const uint32_t inc = wave_inclusive_scan(sum[k]);
+    if (l == wave_size - 1) scratch[k][wave] = inc;
   }
-  if (n_cap <= one_pass_max) {
-    hipLaunchKernelGGL(k_scan_tiles<one_pass_items>, dim3(1), dim3(scan_block), 0, s, in, n_dev, n_cap, out, nullptr);
-    return hipGetLastError();
+  __syncthreads();
+  uint32_t carry[n];
+#pragma unroll
+  for (unsigned k = 0; k < n; ++k) {
+    const uint32_t t = l < scan_block / wave_size ? scratch[k][l] : 0u;
+    carry[k] = __builtin_amdgcn_readlane(wave_inclusive_scan(t) - t, wave);
   }
-  if (!scratch) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_scan_tile_sums, dim3(tiles), dim3(scan_block), 0, s, in, n_dev, n_cap, scratch);
-  hipLaunchKernelGGL(k_scan_small_inplace, dim3(1), dim3(scan_block), 0, s, scratch, tiles);
-  hipLaunchKernelGGL(k_scan_tiles<scan_items>, dim3(tiles), dim3(scan_block), 0, s, in, n_dev, n_cap, out, scratch);
-  return hipGetLastError();
+  for (unsigned i0 = begin; i0 < end; i0 += wave_size) {
+    const unsigned i = i0 + l;
+#pragma unroll
+    for (unsigned k = 0; k < n; ++k) {
+      const uint32_t inc = wave_inclusive_scan(i < end ? in[k][i] : 0u);
+      if (i < end) emit(i, k, carry[k] + inc);
+      carry[k] += __builtin_amdgcn_readlane(inc, wave_size - 1);
+    }
+  }
 }
+
+// A prefix sum of up to one_pass_max items by one workgroup: wave w takes a contiguous range, a line
+// per read, all of them in flight at once and before any write (in and out may overlap). 13 000
+// items: 5.9 us; with 32 consecutive items per thread, whose reads went over the L1's lines
+// eight times, 15.5 us, and 27 us for 26 000.
+constexpr unsigned one_pass_items = one_pass_max / scan_block;
+__global__ void __launch_bounds__(scan_block) k_scan_one(const uint32_t* in, unsigned n, uint32_t* out)
+{
+  __shared__ uint32_t scratch[scan_block / wave_size];
+  const unsigned wave = __builtin_amdgcn_readfirstlane(threadIdx.x / wave_size), l = lane_id();
+  const unsigned lines = (n + scan_block - 1) / scan_block; // per wave
+  const unsigned begin = wave * lines * wave_size;
+  uint32_t v[one_pass_items], sum = 0;
+#pragma unroll
+  for (unsigned k = 0; k < one_pass_items; ++k) {
+    const unsigned i = begin + k * wave_size + l;
+    v[k] = k < lines && i < n ? in[i] : 0u;
+  }
+#pragma unroll
+  for (unsigned k = 0; k < one_pass_items; ++k) sum += v[k];
+  const uint32_t inc = wave_inclusive_scan(sum);
+  if (l == wave_size - 1) scratch[wave] = inc;
+  uint32_t total;
+  uint32_t carry = block_wave_prefix(scratch, &total);
+  if (threadIdx.x == 0) out[0] = 0;
+#pragma unroll
+  for (unsigned k = 0; k < one_pass_items; ++k) {
+    const unsigned i = begin + k * wave_size + l;
+    if (k >= lines) continue;
+    const uint32_t run = wave_inclusive_scan(v[k]);
+    if (i < n) out[i + 1] = carry + run;
+    carry += __builtin_amdgcn_readlane(run, wave_size - 1);
+  }
+}
+
+size_t prefix_sum_scratch_words(unsigned n) { return (n + scan_tile - 1) / scan_tile; }
 
 hipError_t launch_prefix_sum(const uint32_t* in, unsigned n, uint32_t* out, uint32_t* scratch, hipStream_t s)
 {
-  return launch_prefix_sum_dyn(in, nullptr, n, out, scratch, s);
+  const unsigned tiles = (n + scan_tile - 1) / scan_tile;
+  if (tiles <= 1) {
+    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(scan_block), 0, s, in, n, out, nullptr);
+    return hipGetLastError();
+  }
+  if (n <= one_pass_max) {
+    hipLaunchKernelGGL(k_scan_one, dim3(1), dim3(scan_block), 0, s, in, n, out);
+    return hipGetLastError();
+  }
+  if (!scratch) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_scan_tile_sums, dim3(tiles), dim3(scan_block), 0, s, in, n, scratch);
+  hipLaunchKernelGGL(k_scan_small_inplace, dim3(1), dim3(scan_block), 0, s, scratch, tiles);
+  hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(scan_block), 0, s, in, n, out, scratch);
+  return hipGetLastError();
 }
 
 // Tile sums of the allocation-free prefix sum: one u32 per scan tile, room for
@@ -175,7 +230,7 @@ hipError_t launch_prefix_sum_static(const uint32_t* in, unsigned n, uint32_t* ou
   uint32_t* p = nullptr;
   const hipError_t e = static_scratch(&p);
   if (e != hipSuccess) return e;
-  return launch_prefix_sum_dyn(in, nullptr, n, out, p, s);
+  return launch_prefix_sum(in, n, out, p, s);
 }
 
 __global__ void k_fill_u32(uint32_t* p, size_t n, uint32_t value)
@@ -242,6 +297,153 @@ unsigned device_resident_blocks(const void* kernel, unsigned block, size_t dyn_l
 }
 
 // ---------------------------------------------------------------------------------------
+// Whole-sequence scans: every count belongs to an event, so the offsets follow from the events'
+// totals, which the kernels that make the counts add up on the way.
+
+// Events in descending order of their hit count (buckets of 32 hits, order within a bucket
+// unspecified), for launching search_by_triplet largest events first: with every event in
+// flight at once, the largest event sets the duration of the launch. Results do not depend on
+// the order. One workgroup of 1024 threads.
+constexpr unsigned order_buckets = 1024;
+template<typename F>
+__device__ __forceinline__ void
+order_events(unsigned n, F&& hits_of, uint32_t (&bucket)[order_buckets], uint32_t* scratch, uint32_t* order)
+{
+  static_assert(order_buckets == scan_block, "a bucket per thread");
+  bucket[threadIdx.x] = 0;
+  __syncthreads();
+  const auto key = [&](unsigned e) { return order_buckets - 1 - min(hits_of(e) >> 5, order_buckets - 1); }; // descending
+  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) atomicAdd(&bucket[key(e)], 1u);
+  __syncthreads();
+  uint32_t total;
+  const uint32_t ex = block_exclusive_scan(bucket[threadIdx.x], scratch, &total);
+  bucket[threadIdx.x] = ex;
+  __syncthreads();
+  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) order[atomicAdd(&bucket[key(e)], 1u)] = e;
+}
+
+__global__ void __launch_bounds__(scan_block) k_order_events_by_hits(
+  const uint32_t* offsets_estimated_input_size,
+  const uint32_t* number_of_events,
+  uint32_t* order)
+{
+  __shared__ uint32_t bucket[order_buckets];
+  __shared__ uint32_t scratch[scan_block / wave_size];
+  order_events(
+    number_of_events[0],
+    [&](unsigned e) {
+      return offsets_estimated_input_size[(e + 1) * n_module_pairs] - offsets_estimated_input_size[e * n_module_pairs];
+    },
+    bucket, scratch, order);
+}
+
+hipError_t launch_order_events_by_hits(
+  const uint32_t* offsets_estimated_input_size,
+  const uint32_t* number_of_events,
+  uint32_t* order,
+  hipStream_t s)
+{
+  hipLaunchKernelGGL(
+    k_order_events_by_hits, dim3(1), dim3(scan_block), 0, s, offsets_estimated_input_size, number_of_events, order);
+  return hipGetLastError();
+}
+
+// The offsets of a.per_event counts per event (26 module pairs, or a retina slot each), about
+// scan_tile of them per workgroup: a workgroup starts from the sum of the totals of the events
+// before its own, so one launch does what a scan in three launches did, or one workgroup with 32
+// strided items per thread (27 us for the 26 000 counts of 1000 events). Two more workgroups,
+// where asked for, scan the candidates and order the events meanwhile.
+__global__ void __launch_bounds__(scan_block) k_scan_events(const EventScanLaunch a, unsigned events_per_block, unsigned scan_blocks)
+{
+  __shared__ uint32_t scratch[1][scan_block / wave_size];
+  __shared__ uint32_t bucket[order_buckets];
+  unsigned b = blockIdx.x;
+  if (b >= scan_blocks) {
+    if (a.candidates && b == scan_blocks) {
+      const uint32_t* const in[1] = {a.candidates};
+      if (threadIdx.x == 0) a.candidates_offsets[0] = 0;
+      scan_by_waves<1>(in, a.n_events, scratch, [&](unsigned e, unsigned, uint32_t v) { a.candidates_offsets[e + 1] = v; });
+    }
+    else {
+      order_events(a.n_events, [&](unsigned e) { return a.totals[e]; }, bucket, scratch[0], a.order);
+    }
+    return;
+  }
+  const unsigned first = b * events_per_block;
+  const unsigned last = min(first + events_per_block, a.n_events);
+  uint32_t before = 0;
+  for (unsigned e = threadIdx.x; e < first; e += scan_block) before += a.totals[e];
+  uint32_t base;
+  block_exclusive_scan(before, scratch[0], &base);
+  const size_t begin = (size_t) first * a.per_event, end = (size_t) last * a.per_event;
+  if (b == 0 && threadIdx.x == 0) a.offsets[0] = 0;
+  for (size_t c = begin; c < end; c += scan_tile) {
+    // Thread t owns scan_items consecutive counts.
+    const size_t i = c + (size_t) threadIdx.x * scan_items;
+    uint32_t v[scan_items] = {};
+    if (i + scan_items <= end) {
+      __builtin_memcpy(v, a.counts + i, sizeof(v));
+    }
+    else {
+      for (unsigned k = 0; k < scan_items; ++k)
+        if (i + k < end) v[k] = a.counts[i + k];
+    }
+    uint32_t s = 0;
+#pragma unroll
+    for (unsigned k = 0; k < scan_items; ++k) s += v[k];
+    uint32_t total;
+    uint32_t run = base + block_exclusive_scan(s, scratch[0], &total);
+#pragma unroll
+    for (unsigned k = 0; k < scan_items; ++k) {
+      run += v[k];
+      if (i + k < end) a.offsets[i + k + 1] = run;
+    }
+    base += total;
+  }
+}
+
+hipError_t launch_scan_events(const EventScanLaunch& a, hipStream_t s)
+{
+  if (!a.n_events) return hipSuccess;
+  const unsigned events_per_block = std::max(scan_tile / a.per_event, 1u);
+  const unsigned blocks = (a.n_events + events_per_block - 1) / events_per_block;
+  hipLaunchKernelGGL(
+    k_scan_events, dim3(blocks + (a.candidates ? 1 : 0) + (a.order ? 1 : 0)), dim3(scan_block), 0, s, a, events_per_block,
+    blocks);
+  return hipGetLastError();
+}
+
+// Offsets of the events' tracks, kept three-hit tracks, all tracks and track hits, by one workgroup.
+__global__ void __launch_bounds__(scan_block) k_track_offsets(const TrackOffsetsLaunch a)
+{
+  __shared__ uint32_t scratch[3][scan_block / wave_size];
+  const uint32_t* const in[3] = {a.number_of_velo_tracks, a.number_of_three_hit_tracks, a.event_track_hits};
+  if (threadIdx.x == 0)
+    a.offsets_velo_tracks[0] = a.offsets_three_hit[0] = a.offsets_all_velo_tracks[0] = a.event_hit_offsets[0] = 0;
+  uint32_t tracks = 0;
+  scan_by_waves<3>(in, a.n_events, scratch, [&](unsigned e, unsigned k, uint32_t v) {
+    if (k == 0) {
+      a.offsets_velo_tracks[e + 1] = v;
+      tracks = v;
+    }
+    else if (k == 1) {
+      a.offsets_three_hit[e + 1] = v;
+      a.offsets_all_velo_tracks[e + 1] = tracks + v;
+    }
+    else {
+      a.event_hit_offsets[e + 1] = v;
+    }
+  });
+}
+
+hipError_t launch_track_offsets(const TrackOffsetsLaunch& a, hipStream_t s)
+{
+  if (!a.n_events) return hipSuccess;
+  hipLaunchKernelGGL(k_track_offsets, dim3(1), dim3(scan_block), 0, s, a);
+  return hipGetLastError();
+}
+
+// ---------------------------------------------------------------------------------------
 // K7 (grid = number of events).
 __global__ void k_copy_track_hit_number(
   const TrackHits* tracks_all,
@@ -279,8 +481,7 @@ __global__ void k_consolidate_tracks(
   const TrackletHits* three_hit_output_all,
   const uint32_t* offsets_three_hit,
   char* velo_track_hits,
-  uint8_t* accepted,
-  bool lds_map)
+  uint8_t* accepted)
 {
   const unsigned e = event_list ? event_list[blockIdx.x] : blockIdx.x;
   const unsigned n_events = number_of_events[0];
@@ -305,7 +506,7 @@ __global__ void k_consolidate_tracks(
   __shared__ uint32_t s_off[consolidate_lds_tracks + 1];
   __shared__ uint16_t s_map[consolidate_lds_hits];
   const bool in_lds = n_total <= consolidate_lds_tracks;
-  const bool mapped = lds_map && in_lds && h_end - h_begin <= consolidate_lds_hits;
+  const bool mapped = in_lds && h_end - h_begin <= consolidate_lds_hits;
   if (in_lds)
     for (unsigned i = threadIdx.x; i <= n_total; i += blockDim.x) s_off[i] = offsets_velo_track_hit_number[t0 + i];
   __syncthreads();
@@ -405,9 +606,28 @@ struct TrackEnds {
   float f[3], f1[3], l1[3], l[3];
 };
 
-template<bool upstream, bool fp64_fallback>
+// A hit's coordinates, and how a fit reads the hits of its track: consecutive coordinates in memory,
+// or by the track's hit indices from the event's hits (both may be in LDS).
+struct Xyz {
+  float c[3];
+};
+struct PackedHits {
+  const float* xyz;
+  __device__ __forceinline__ Xyz operator()(unsigned i) const { return {xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2]}; }
+};
+struct GatheredHits {
+  const uint16_t* index;
+  const float* xyz;
+  __device__ __forceinline__ Xyz operator()(unsigned i) const
+  {
+    const unsigned h = 3u * index[i];
+    return {xyz[h], xyz[h + 1], xyz[h + 2]};
+  }
+};
+
+template<bool upstream, bool fp64_fallback, typename H>
 __device__ __forceinline__ KState
-simplified_fit(const float* xyz, unsigned nh, const TrackEnds& te, float at_tx, float at_ty, const float* beamline, bool backward)
+simplified_fit(const H& hits, unsigned nh, const TrackEnds& te, float at_tx, float at_ty, const float* beamline, bool backward)
 {
   const int direction = (backward ? 1 : -1) * (upstream ? 1 : -1);
   const float layer_noise = 1e-8f + 7e-6f * (at_tx * at_tx + at_ty * at_ty);
@@ -439,9 +659,10 @@ simplified_fit(const float* xyz, unsigned nh, const TrackEnds& te, float at_tx, 
   for (int i = first + step; i != last + step; i += step) {
     const float hx = nx, hy = ny, hz = nz;
     if (i + step != last + step) {
-      nx = xyz[3 * (i + step)];
-      ny = xyz[3 * (i + step) + 1];
-      nz = xyz[3 * (i + step) + 2];
+      const Xyz next = hits(static_cast<unsigned>(i + step));
+      nx = next.c[0];
+      ny = next.c[1];
+      nz = next.c[2];
     }
     s.c22 += layer_noise;
     s.c33 += layer_noise;
@@ -487,9 +708,10 @@ __device__ __forceinline__ void store_state(float* base, unsigned total_tracks, 
 }
 
 // One track: linear_fit, the upstream fit to the beamline and the downstream fit to the end of
-// the VELO (VeloKalmanFilter.cu:384-399); xyz holds its nh hits' x, y, z.
+// the VELO (VeloKalmanFilter.cu:384-399).
+template<typename H>
 __device__ __forceinline__ void fit_track(
-  const float* xyz,
+  const H& hits,
   unsigned nh,
   unsigned t,
   unsigned total_tracks,
@@ -500,12 +722,15 @@ __device__ __forceinline__ void fit_track(
   unsigned fp64_fallback)
 {
   TrackEnds te;
+  {
+    const Xyz f = hits(0), f1 = hits(1), l1 = hits(nh - 2), l = hits(nh - 1);
 #pragma unroll
-  for (unsigned c = 0; c < 3; ++c) {
-    te.f[c] = xyz[c];
-    te.f1[c] = xyz[3 + c];
-    te.l1[c] = xyz[3 * (nh - 2) + c];
-    te.l[c] = xyz[3 * (nh - 1) + c];
+    for (unsigned c = 0; c < 3; ++c) {
+      te.f[c] = f.c[c];
+      te.f1[c] = f1.c[c];
+      te.l1[c] = l1.c[c];
+      te.l[c] = l.c[c];
+    }
   }
   __builtin_amdgcn_sched_barrier(0); // the four hits' loads are in flight together
   // linear_fit (VeloKalmanFilter.cu:335-355)
@@ -518,14 +743,14 @@ __device__ __forceinline__ void fit_track(
   const bool backward = lin_z > fz;
   is_backward[t] = backward;
   if (fp64_fallback) {
-    const KState b = simplified_fit<true, true>(xyz, nh, te, ltx, lty, bl, backward);
-    const KState v = simplified_fit<false, true>(xyz, nh, te, b.tx, b.ty, bl, backward);
+    const KState b = simplified_fit<true, true>(hits, nh, te, ltx, lty, bl, backward);
+    const KState v = simplified_fit<false, true>(hits, nh, te, b.tx, b.ty, bl, backward);
     store_state(beamline_states, total_tracks, t, b);
     store_state(endvelo_states, total_tracks, t, v);
   }
   else {
-    const KState b = simplified_fit<true, false>(xyz, nh, te, ltx, lty, bl, backward);
-    const KState v = simplified_fit<false, false>(xyz, nh, te, b.tx, b.ty, bl, backward);
+    const KState b = simplified_fit<true, false>(hits, nh, te, ltx, lty, bl, backward);
+    const KState v = simplified_fit<false, false>(hits, nh, te, b.tx, b.ty, bl, backward);
     store_state(beamline_states, total_tracks, t, b);
     store_state(endvelo_states, total_tracks, t, v);
   }
@@ -582,7 +807,7 @@ __global__ void k_kalman_filter(
       if (tr.number_of_hits < 2) continue;
       const float* xyz = reinterpret_cast<const float*>(h.base_pointer) + h.total_number_of_hits +
                          3 * (size_t) (h.offset + tr.offset);
-      fit_track(xyz, tr.number_of_hits, tv.offset + i, total_tracks, bl, is_backward, beamline_states,
+      fit_track(PackedHits {xyz}, tr.number_of_hits, tv.offset + i, total_tracks, bl, is_backward, beamline_states,
                 endvelo_states, fp64_fallback);
     }
   }
@@ -594,10 +819,157 @@ __global__ void k_kalman_filter(
       const unsigned h0 = offsets_velo_track_hit_number[t];
       const unsigned nh = offsets_velo_track_hit_number[t + 1] - h0;
       if (nh < 2) continue; // every VELO track has >= 3 hits
-      fit_track(xyz_all + 3 * (size_t) h0, nh, t, total_tracks, bl, is_backward, beamline_states, endvelo_states,
+      fit_track(PackedHits {xyz_all + 3 * (size_t) h0}, nh, t, total_tracks, bl, is_backward, beamline_states, endvelo_states,
                 fp64_fallback);
     }
   }
+}
+
+// Copies `words` 32-bit words (from any 2-byte boundary) to 16-byte aligned LDS by the workgroup, 16
+// bytes a lane, four of those in flight (one at a time, every pass waits out a memory round trip).
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_unaligned __attribute__((aligned(2)));
+typedef uint32_t u32_unaligned __attribute__((aligned(2)));
+__device__ __forceinline__ void copy_to_lds(uint32_t* to, const void* from, unsigned words)
+{
+  const auto* src = static_cast<const u32x4_unaligned*>(from);
+  const unsigned quads = words / 4;
+  for (unsigned q0 = threadIdx.x; q0 < quads; q0 += 4 * blockDim.x) {
+    u32x4 v[4];
+#pragma unroll
+    for (unsigned k = 0; k < 4; ++k) v[k] = src[min(q0 + k * blockDim.x, quads - 1)];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (unsigned k = 0; k < 4; ++k)
+      if (q0 + k * blockDim.x < quads) reinterpret_cast<u32x4*>(to)[q0 + k * blockDim.x] = v[k];
+  }
+  const unsigned w = 4 * quads + threadIdx.x;
+  if (w < words) to[w] = static_cast<const u32_unaligned*>(from)[w];
+}
+
+// K7, K8 and K9 of one event by one workgroup (whole-sequence path): the tracks' hit numbers and
+// offsets from the event's hit offset, the consolidated hits, and both fits of every track. The
+// event's coordinates (nearly all of its hits end in tracks) and its tracks, 256 at a time, are
+// copied to LDS in whole lines, so the fits wait for no memory: a load in their chain of steps
+// would also wait for every store issued before it. Sixteen lanes copy a track's hits, so that
+// neighbouring lanes write neighbouring slots, four tracks read before the first is written. Bound by the divisions of the fits' chains, and
+// with many events in flight by the bytes (about 50 KB an event). Events with more hits than the
+// LDS holds read the coordinates from the container.
+constexpr unsigned fit_block = 256;
+constexpr unsigned fit_copy_lanes = 16;
+constexpr unsigned fit_lds_hits = 1920; // with the tracks 37 KB: four workgroups a CU, so 1000 events are in flight at once
+struct FitChunk {
+  const TrackHits* tracks; // in LDS
+  const uint32_t* first;   // in LDS
+  unsigned n;
+  unsigned t0;             // number of the first track
+  unsigned total_tracks;
+};
+template<bool fp64_fallback>
+__device__ __forceinline__ void copy_and_fit(
+  const TrackFitLaunch& a, const FitChunk& f, const uint32_t* ids, const float* xyz, const Clusters& out, const float* bl)
+{
+  const unsigned tid = threadIdx.x;
+  constexpr unsigned groups = fit_block / fit_copy_lanes, batch = 4;
+  for (unsigned j = tid % fit_copy_lanes; j < max_track_size; j += fit_copy_lanes) {
+    for (unsigned g0 = tid / fit_copy_lanes; g0 < f.n; g0 += batch * groups) {
+      uint32_t id[batch];
+      Xyz p[batch];
+      bool has[batch];
+#pragma unroll
+      for (unsigned k = 0; k < batch; ++k) {
+        const unsigned g = min(g0 + k * groups, f.n - 1);
+        has[k] = g0 + k * groups < f.n && j < f.tracks[g].hitsNum;
+        const unsigned h = f.tracks[g].hits[has[k] ? j : 0u];
+        id[k] = ids[h];
+        p[k] = {xyz[3 * h], xyz[3 * h + 1], xyz[3 * h + 2]};
+      }
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (unsigned k = 0; k < batch; ++k) {
+        if (!has[k]) continue;
+        const size_t at = (size_t) f.first[g0 + k * groups] + j;
+        out.ids()[at] = id[k];
+        out.xyz()[3 * at] = p[k].c[0];
+        out.xyz()[3 * at + 1] = p[k].c[1];
+        out.xyz()[3 * at + 2] = p[k].c[2];
+      }
+    }
+  }
+  if (tid < f.n && f.tracks[tid].hitsNum >= 2) // every VELO track has >= 3 hits
+    fit_track(GatheredHits {f.tracks[tid].hits, xyz}, f.tracks[tid].hitsNum, f.t0 + tid, f.total_tracks, bl, a.is_backward,
+              reinterpret_cast<float*>(a.beamline_states), reinterpret_cast<float*>(a.endvelo_states), fp64_fallback);
+}
+
+template<bool fp64_fallback>
+__global__ void __launch_bounds__(fit_block) k_consolidate_and_fit(const TrackFitLaunch a)
+{
+  __shared__ __align__(16) float s_xyz[3 * fit_lds_hits];
+  __shared__ __align__(16) TrackHits s_tracks[fit_block]; // a chunk of tracks
+  __shared__ uint32_t s_first[fit_block];   // their first hits' slots
+  __shared__ uint32_t s_scan[fit_block / wave_size];
+  const unsigned e = blockIdx.x, tid = threadIdx.x;
+  const uint32_t* est = a.offsets_estimated_input_size;
+  const unsigned total_clusters = est[n_module_pairs * a.n_events];
+  const unsigned hit_offset = est[e * n_module_pairs];
+  const unsigned n_hits = est[(e + 1) * n_module_pairs] - hit_offset;
+  const unsigned toff = track_offset(est, e);
+  const unsigned t0 = a.offsets_all_velo_tracks[e];
+  const unsigned n_total = a.offsets_all_velo_tracks[e + 1] - t0;
+  const unsigned n_main = n_total - (a.offsets_three_hit[e + 1] - a.offsets_three_hit[e]);
+  const unsigned total_tracks = a.offsets_all_velo_tracks[a.n_events];
+  const unsigned total_hits = a.event_hit_offsets[a.n_events];
+  const float bl[2] = {a.beamline[0], a.beamline[1]};
+  const Clusters in {const_cast<char*>(a.sorted_container), total_clusters};
+  const Clusters out {a.velo_track_hits, total_hits};
+  const uint32_t* ids = in.ids() + hit_offset;
+  const float* xyz = in.xyz() + 3 * (size_t) hit_offset;
+  const TrackHits* tracks = static_cast<const TrackHits*>(a.tracks) + toff;
+  const TrackletHits* three = static_cast<const TrackletHits*>(a.three_hit_tracks_output) + toff;
+  const bool staged = a.lds_hits && n_hits <= fit_lds_hits;
+  if (staged) copy_to_lds(reinterpret_cast<uint32_t*>(s_xyz), xyz, 3 * n_hits);
+  unsigned slot = a.event_hit_offsets[e];
+  for (unsigned c = 0; c < n_total; c += fit_block) {
+    const unsigned i = c + tid;
+    // The chunk's tracks in words, from a 2-byte boundary (an odd number of tracks leaves half a word,
+    // the last one's number of hits), kept three-hit tracks after them.
+    const unsigned n_copy = min(fit_block, n_main - min(n_main, c));
+    copy_to_lds(reinterpret_cast<uint32_t*>(s_tracks), tracks + c, sizeof(TrackHits) * n_copy / 4);
+    if (tid == 0 && n_copy % 2) s_tracks[n_copy - 1].hitsNum = tracks[c + n_copy - 1].hitsNum;
+    if (i >= n_main && i < n_total) {
+      const TrackletHits t = three[i - n_main];
+      s_tracks[tid].hits[0] = t.hits[0];
+      s_tracks[tid].hits[1] = t.hits[1];
+      s_tracks[tid].hits[2] = t.hits[2];
+      s_tracks[tid].hitsNum = 3;
+    }
+    __syncthreads();
+    const unsigned nh = i < n_total ? s_tracks[tid].hitsNum : 0u;
+    uint32_t chunk_hits;
+    const unsigned first = slot + block_exclusive_scan(nh, s_scan, &chunk_hits);
+    slot += chunk_hits;
+    s_first[tid] = first;
+    if (i < n_total) {
+      a.velo_track_hit_number[t0 + i] = nh;
+      a.offsets_velo_track_hit_number[t0 + i] = first;
+      a.accepted_velo_tracks[t0 + i] = 1;
+    }
+    __syncthreads();
+    // Two copies of the code: a read that may go to LDS or to memory would be a generic (flat) one.
+    const FitChunk f {s_tracks, s_first, min(fit_block, n_total - c), t0 + c, total_tracks};
+    if (staged) copy_and_fit<fp64_fallback>(a, f, ids, s_xyz, out, bl);
+    else copy_and_fit<fp64_fallback>(a, f, ids, xyz, out, bl);
+    __syncthreads(); // the chunk's tracks have been read
+  }
+  if (e + 1 == a.n_events && tid == 0) a.offsets_velo_track_hit_number[total_tracks] = total_hits;
+}
+
+hipError_t launch_consolidate_and_fit(const TrackFitLaunch& a, hipStream_t s)
+{
+  if (!a.n_events) return hipSuccess;
+  if (a.fp64_fallback) hipLaunchKernelGGL(k_consolidate_and_fit<true>, dim3(a.n_events), dim3(fit_block), 0, s, a);
+  else hipLaunchKernelGGL(k_consolidate_and_fit<false>, dim3(a.n_events), dim3(fit_block), 0, s, a);
+  return hipGetLastError();
 }
 
 // create_velo_views (VeloConsolidateTracks.cu:11-46): event e's Hits and Tracks views and one
@@ -705,7 +1077,7 @@ hipError_t launch_consolidate_tracks(const ConsolidateLaunch& a, hipStream_t s)
     k_consolidate_tracks, dim3(a.n_list), dim3(256), 0, s, a.event_list, a.number_of_events, a.offsets_all_velo_tracks,
     reinterpret_cast<const TrackHits*>(a.tracks), a.offsets_velo_track_hit_number, a.sorted_container,
     a.offsets_estimated_input_size, reinterpret_cast<const TrackletHits*>(a.three_hit_tracks_output),
-    a.offsets_three_hit, a.velo_track_hits, a.accepted_velo_tracks, a.lds_map);
+    a.offsets_three_hit, a.velo_track_hits, a.accepted_velo_tracks);
   return hipGetLastError();
 }
 

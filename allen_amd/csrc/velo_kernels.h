@@ -25,6 +25,11 @@ struct CandidatesLaunch {
   // (event, module pair) up to 8 BankEntry records in bank order and their number.
   void* directory = nullptr;
   uint32_t* directory_count = nullptr;
+  // Beside the directory: what later launches of the run start from, the number of events, a
+  // cleared status word and a zero estimate total for every event.
+  uint32_t* number_of_events = nullptr;
+  uint32_t* status = nullptr;
+  uint32_t* event_totals = nullptr;
 };
 
 // Retina-cluster decoding (velo_retina.hip).
@@ -40,6 +45,11 @@ struct RetinaSizesLaunch {
   unsigned event_start;
   uint32_t* each_sensor_pair_size; // slots per event: 208 (v2/v3) or 104 (v4)
   uint32_t* retina_bank_index;     // slots
+  // Whole-sequence path (optional, together): every event's total, the number of events, a cleared
+  // status word, and all ones for the slots of the bank index that the first event leaves out.
+  uint32_t* event_totals = nullptr;
+  uint32_t* number_of_events = nullptr;
+  uint32_t* status = nullptr;
 };
 struct RetinaDecodeLaunch {
   int version;
@@ -150,25 +160,6 @@ struct SortLaunch {
   uint32_t* hit_permutation;
 };
 
-struct FusedClusterLaunch {
-  int version;
-  const char* raw;
-  const uint32_t* offsets;
-  const uint32_t* sizes;
-  const uint32_t* types;
-  bool mep = false; // MEP layout (MEPTools.h:59-200)
-  unsigned n_events;
-  const uint32_t* offsets_estimated_input_size;
-  const void* geometry;
-  const uint8_t* sp_patterns;
-  const float* sp_fx;
-  const float* sp_fy;
-  uint32_t* module_cluster_num;
-  char* sorted_container;
-  char* unsorted_scratch;
-  uint32_t* status;
-};
-
 struct EstimateMpLaunch {
   int version;
   bool resident_grid = false; // one wave per item (default) or a resident grid looping over items
@@ -178,6 +169,7 @@ struct EstimateMpLaunch {
   unsigned n_events;
   uint32_t* estimated_input_size;
   uint8_t* sp_flags; // one byte per 32-bit word of the raw buffer
+  uint32_t* event_totals; // per event, zero before the launch: the estimates of its module pairs are added
 };
 
 struct ClusterMpLaunch {
@@ -248,6 +240,12 @@ struct SearchLaunch {
   // seeding's list of unused hits (a multiple of 16, up to 1024); 0: as block_dim.
   unsigned ring_window = 0;
   unsigned list_cap = 0;
+  // Optional: run the three-hit filter at the end of each event (its outputs as in
+  // ThreeHitFilterLaunch) and write the number of hits of each event's tracks.
+  void* three_hit_tracks_output = nullptr;
+  uint32_t* number_of_three_hit_tracks_output = nullptr;
+  uint32_t* event_track_hits = nullptr;
+  float max_chi2 = 0.f;
 };
 
 struct ThreeHitFilterLaunch {
@@ -287,7 +285,6 @@ struct ConsolidateLaunch {
   const uint32_t* offsets_three_hit;
   char* velo_track_hits;
   uint8_t* accepted_velo_tracks; // optional
-  bool lds_map = true;           // hits find their track through an LDS map (else a binary search)
 };
 
 struct KalmanLaunch {
@@ -307,6 +304,53 @@ struct KalmanLaunch {
   const void* tracks_view = nullptr;
   void* beamline_states_view = nullptr;
   void* endvelo_states_view = nullptr;
+};
+
+// Offsets of `per_event` counts per event from the events' totals; optionally also the offsets of
+// the candidates and the events by descending total.
+struct EventScanLaunch {
+  const uint32_t* counts;
+  unsigned per_event;
+  const uint32_t* totals;
+  unsigned n_events;
+  uint32_t* offsets;
+  const uint32_t* candidates = nullptr;
+  uint32_t* candidates_offsets = nullptr;
+  uint32_t* order = nullptr;
+};
+
+// Per-event offsets after the search: tracks, kept three-hit tracks, both, and their hits.
+struct TrackOffsetsLaunch {
+  unsigned n_events;
+  const uint32_t* number_of_velo_tracks;
+  const uint32_t* number_of_three_hit_tracks;
+  const uint32_t* event_track_hits;
+  uint32_t* offsets_velo_tracks;
+  uint32_t* offsets_three_hit;
+  uint32_t* offsets_all_velo_tracks;
+  uint32_t* event_hit_offsets;
+};
+
+// K7, K8 and K9 of the whole sequence in one launch.
+struct TrackFitLaunch {
+  unsigned n_events;
+  const uint32_t* offsets_estimated_input_size;
+  const uint32_t* offsets_all_velo_tracks;
+  const uint32_t* offsets_three_hit;
+  const uint32_t* event_hit_offsets;
+  const char* sorted_container;
+  const void* tracks;
+  const void* three_hit_tracks_output;
+  const float* beamline;
+  bool lds_hits; // stage an event's hits in LDS where they fit
+  unsigned fp64_fallback;
+  uint32_t* velo_track_hit_number;
+  uint32_t* offsets_velo_track_hit_number;
+  char* velo_track_hits;
+  uint8_t* accepted_velo_tracks;
+  uint8_t* is_backward;
+  char* beamline_states;
+  char* endvelo_states;
 };
 
 // create_velo_views (VeloConsolidateTracks.cu:11-46): one workgroup per event of the batch.
@@ -342,7 +386,6 @@ hipError_t launch_number_of_candidates(const CandidatesLaunch& a, hipStream_t s)
 hipError_t launch_estimate_input_size(const EstimateLaunch& a, hipStream_t s);
 hipError_t launch_masked_clustering(const MaskedClusteringLaunch& a, hipStream_t s);
 hipError_t launch_sort_by_phi(const SortLaunch& a, hipStream_t s);
-hipError_t launch_cluster_sorted(const FusedClusterLaunch& a, hipStream_t s);
 hipError_t launch_estimate_mp(const EstimateMpLaunch& a, hipStream_t s);
 hipError_t launch_cluster_mp(const ClusterMpLaunch& a, hipStream_t s);
 hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s);
@@ -371,6 +414,9 @@ hipError_t launch_three_hit_tracks_filter(const ThreeHitFilterLaunch& a, hipStre
 hipError_t launch_copy_track_hit_number(const CopyHitNumberLaunch& a, hipStream_t s);
 hipError_t launch_consolidate_tracks(const ConsolidateLaunch& a, hipStream_t s);
 hipError_t launch_kalman_filter(const KalmanLaunch& a, hipStream_t s);
+hipError_t launch_scan_events(const EventScanLaunch& a, hipStream_t s);
+hipError_t launch_track_offsets(const TrackOffsetsLaunch& a, hipStream_t s);
+hipError_t launch_consolidate_and_fit(const TrackFitLaunch& a, hipStream_t s);
 
 // Learned seed scorer (10 -> 32 -> 32 -> 1 MLP). Parameter layout (FP32): W1 [10][32], b1 [32],
 // W2 [32][32], b2 [32], w3 [32], b3.
@@ -409,14 +455,6 @@ hipError_t launch_mlp_score(const float* features, unsigned n, const float* para
 // Device exclusive scan with a leading zero: out[0] = 0, out[i+1] = sum(in[0..i]).
 size_t prefix_sum_scratch_words(unsigned n);
 hipError_t launch_prefix_sum(const uint32_t* in, unsigned n, uint32_t* out, uint32_t* scratch, hipStream_t s);
-// Same, with the length read on the device: min(*n_dev, n_cap).
-hipError_t launch_prefix_sum_dyn(
-  const uint32_t* in,
-  const uint32_t* n_dev,
-  unsigned n_cap,
-  uint32_t* out,
-  uint32_t* scratch,
-  hipStream_t s);
 // Same, with the tile sums in a static device array of the library (no allocation): at most
 // prefix_sum_static_max_items items. prefix_sum_static_init() looks the current device's copy up.
 constexpr unsigned prefix_sum_static_max_items = 1u << 28;

@@ -108,7 +108,10 @@ __global__ void __launch_bounds__(wave_size) k_retina_sensor_sizes(
   const uint32_t* event_list,
   unsigned event_start,
   uint32_t* each_sensor_pair_size,
-  uint32_t* retina_bank_index)
+  uint32_t* retina_bank_index,
+  uint32_t* event_totals,
+  uint32_t* number_of_events,
+  uint32_t* status)
 {
   constexpr unsigned S = slots<version>();
   __shared__ int s_retina[S];
@@ -130,10 +133,21 @@ __global__ void __launch_bounds__(wave_size) k_retina_sensor_sizes(
   }
   wave_sync_lds();
   uint32_t* out = each_sensor_pair_size + static_cast<size_t>(event_number) * S;
+  uint32_t words = 0;
   for (unsigned i = l; i < S; i += wave_size) {
     const int bi = s_retina[i];
-    out[i] = bi >= 0 ? bank_n_sp<version>(raw_bank<version>(ev, static_cast<unsigned>(bi))) : 0u;
-    if (blockIdx.x == 0 && s_any[i] >= 0) retina_bank_index[i] = static_cast<uint32_t>(s_any[i]);
+    const uint32_t n = bi >= 0 ? bank_n_sp<version>(raw_bank<version>(ev, static_cast<unsigned>(bi))) : 0u;
+    out[i] = n;
+    words += n;
+    if (blockIdx.x == 0 && (s_any[i] >= 0 || event_totals)) retina_bank_index[i] = static_cast<uint32_t>(s_any[i]);
+  }
+  if (event_totals) {
+    const uint32_t total = wave_inclusive_scan(words);
+    if (l == wave_size - 1) event_totals[event_number] = total;
+    if (blockIdx.x == 0 && l == 0) {
+      number_of_events[0] = gridDim.x;
+      status[0] = 0;
+    }
   }
 }
 
@@ -273,7 +287,8 @@ hipError_t launch_retina_sensor_sizes(const RetinaSizesLaunch& a, hipStream_t s)
 #define VELO_LAUNCH_RSS(V)                                                                                          \
   hipLaunchKernelGGL(                                                                                               \
     k_retina_sensor_sizes<V>, dim3(a.n_list), dim3(wave_size), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep),            \
-    a.event_list, a.event_start, a.each_sensor_pair_size, a.retina_bank_index)
+    a.event_list, a.event_start, a.each_sensor_pair_size, a.retina_bank_index, a.event_totals, a.number_of_events,   \
+    a.status)
   switch (a.version) {
   case 2: VELO_LAUNCH_RSS(2); break;
   case 3: VELO_LAUNCH_RSS(3); break;

@@ -397,6 +397,7 @@ build_phi_tables(const H& hits, ModulePairData* mp, uint8_t* tables, uint32_t* h
 }
 
 struct SearchShared {
+  uint32_t extended;                 // hits added to tracks of four or more hits, all waves
   ModulePairData mp[n_module_pairs]; // hit range (event-relative) and module z of every module pair
   uint2 scan[2][16];                 // team_flag_scan scratch, used alternately
 };
@@ -409,6 +410,7 @@ struct Counters {
   uint32_t local_hits = 0; // atomics::local_number_of_hits
   uint32_t n_tracks = 0;   // dev_number_of_velo_tracks[event]
   uint32_t status = 0;
+  uint32_t extended = 0;   // this wave's part of SearchShared::extended
   unsigned scan_buffer = 0;
 };
 
@@ -1125,6 +1127,7 @@ __device__ __forceinline__ void track_forwarding(
       }
     }
     const Scan3 s = scan<3>(team, sh, cn, promote, reinsert, three);
+    cn.extended += __popcll(__ballot(found && !promote));
     if (valid) {
       if (found) {
         hits.mark_used(best_h2);
@@ -1289,7 +1292,93 @@ struct SearchArgs {
   float scorer_threshold;
   unsigned window;
   unsigned list_cap;
+  // Optional: the three-hit filter at the end of each event, with its outputs and the event's track hits.
+  TrackletHits* three_hit_tracks_output;
+  uint32_t* number_of_three_hit_tracks_output;
+  uint32_t* event_track_hits;
+  float max_chi2;
 };
+
+// ThreeHitTracksFilter.cu:48-107
+__device__ __forceinline__ float means_square_fit_chi2(const Hit& a, const Hit& b, const Hit& c)
+{
+  float s0, sx, sz, sxz, sz2, u0, uy, uz, uyz, uz2;
+  s0 = sx = sz = sxz = sz2 = 0.0f;
+  u0 = uy = uz = uyz = uz2 = 0.0f;
+  const float xs[3] = {a.x, b.x, c.x}, ys[3] = {a.y, b.y, c.y}, zs[3] = {a.z, b.z, c.z};
+#pragma unroll
+  for (unsigned h = 0; h < 3; ++h) {
+    const float x = xs[h], y = ys[h], z = zs[h];
+    const float wx = param_w;
+    const float wx_t_x = wx * x;
+    const float wx_t_z = wx * z;
+    s0 += wx;
+    sx += wx_t_x;
+    sz += wx_t_z;
+    sxz += wx_t_x * z;
+    sz2 += wx_t_z * z;
+    const float wy = param_w;
+    const float wy_t_y = wy * y;
+    const float wy_t_z = wy * z;
+    u0 += wy;
+    uy += wy_t_y;
+    uz += wy_t_z;
+    uyz += wy_t_y * z;
+    uz2 += wy_t_z * z;
+  }
+  const float dens = 1.0f / (sz2 * s0 - sz * sz);
+  const float state_tx = (sxz * s0 - sx * sz) * dens;
+  const float state_x = (sx * sz2 - sxz * sz) * dens;
+  const float denu = 1.0f / (uz2 * u0 - uz * uz);
+  const float state_ty = (uyz * u0 - uy * uz) * denu;
+  const float state_y = (uy * uz2 - uyz * uz) * denu;
+  float chi2 = 0.0f;
+#pragma unroll
+  for (unsigned h = 0; h < 3; ++h) {
+    const float z = zs[h];
+    const float x = state_x + state_tx * z;
+    const float y = state_y + state_ty * z;
+    const float dx = x - xs[h];
+    const float dy = y - ys[h];
+    chi2 += dx * dx * param_w + dy * dy * param_w;
+  }
+  return chi2 * 0.5f;
+}
+
+// The three-hit filter (ThreeHitTracksFilter.cu:109-169, ordered output) on the event's own
+// three-hit tracks, with the hits and their flags where the search has them, and the number of
+// hits of the event's tracks (four for each track, one for each extension, three for each kept
+// three-hit track): what the filter, the track-hit count and two scans over the tracks took a
+// launch each for.
+template<typename H>
+__device__ __forceinline__ void finish_event(
+  const H& hits, const Team& team, SearchShared& sh, Counters& cn, const EventOutputs& o, const SearchArgs& a, unsigned toff)
+{
+  if (!a.three_hit_tracks_output) return;
+  if (lane_id() == 0 && cn.extended) atomicAdd(&sh.extended, cn.extended);
+  __threadfence_block(); // other lanes wrote the three-hit tracks
+  team.sync();
+  const unsigned n_in = min(cn.three, o.track_capacity);
+  TrackletHits* out = a.three_hit_tracks_output + toff;
+  unsigned kept = 0;
+  for (unsigned c = 0; c < n_in; c += team.lanes) {
+    const unsigned i = c + threadIdx.x;
+    bool keep = false;
+    TrackletHits t;
+    if (i < n_in) {
+      t = o.three_hit_tracks[i];
+      const Hit h0 = hits.load(t.hits[0]), h1 = hits.load(t.hits[1]), h2 = hits.load(t.hits[2]);
+      keep = !(h0.used || h1.used || h2.used) && means_square_fit_chi2(h0, h1, h2) < a.max_chi2;
+    }
+    const Scan3 s = scan<1>(team, sh, cn, keep);
+    if (keep) out[kept + s.r[0]] = t;
+    kept += s.t[0];
+  }
+  if (threadIdx.x == 0) {
+    a.number_of_three_hit_tracks_output[o.event_number] = kept;
+    a.event_track_hits[o.event_number] = 4 * min(cn.n_tracks, o.track_capacity) + sh.extended + 3 * kept;
+  }
+}
 
 // One workgroup per event, or (persistent, launched with a work counter) a resident grid whose
 // workgroups take the next event slot from the counter until the slots run out; the persistent
@@ -1373,6 +1462,7 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
     o.track_capacity = min(next_off > toff ? next_off - toff : 0u, container - min(toff, container));
 
     Counters cn;
+    if (threadIdx.x == 0) sh.extended = 0;
     cn.status = n_hits > 65536u ? status_hit_index_overflow : 0u;
     if (threadIdx.x < n_module_pairs) {
       const unsigned m = threadIdx.x;
@@ -1413,6 +1503,7 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
       search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
       team.sync();
       for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = hits.used(i) ? 1 : 0;
+      finish_event(hits, team, sh, cn, o, a, toff);
     }
     else if (mixed_bytes_per_hit * n_hits <= search_bytes_per_hit * a.lds_hits) {
       int16_t* ph = reinterpret_cast<int16_t*>(dyn);
@@ -1435,6 +1526,7 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
       search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
       team.sync();
       for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = flags[i] & flag_used;
+      finish_event(hits, team, sh, cn, o, a, toff);
     }
     else {
       for (unsigned i = threadIdx.x; i < n_hits; i += team.lanes) gused[i] = 0;
@@ -1445,7 +1537,9 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
       build_phi_tables(hits, sh.mp, phi_tables, hist, hist_waves, team);
       team.sync();
       search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
+      __threadfence_block(); // the used flags are read back from global memory
       team.sync();
+      finish_event(hits, team, sh, cn, o, a, toff);
     }
     if constexpr (count) {
       // Wave reduction, then one atomic per wave.
@@ -1497,104 +1591,6 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, se
   }
 }
 
-// Events in descending order of their hit count (buckets of 32 hits, order within a bucket
-// unspecified), for launching search_by_triplet largest events first: with every event in
-// flight at once, the largest event sets the duration of the launch. Results do not depend on
-// the order. One workgroup of 1024 threads.
-constexpr unsigned order_buckets = 1024;
-__global__ void __launch_bounds__(1024) k_order_events_by_hits(
-  const uint32_t* offsets_estimated_input_size,
-  const uint32_t* number_of_events,
-  uint32_t* order)
-{
-  __shared__ uint32_t bucket[order_buckets];
-  __shared__ uint32_t scan_scratch[1024 / wave_size + 1];
-  const unsigned n = number_of_events[0];
-  for (unsigned b = threadIdx.x; b < order_buckets; b += blockDim.x) bucket[b] = 0;
-  __syncthreads();
-  auto key = [&](unsigned e) {
-    const unsigned hits =
-      offsets_estimated_input_size[(e + 1) * n_module_pairs] - offsets_estimated_input_size[e * n_module_pairs];
-    return order_buckets - 1 - min(hits >> 5, order_buckets - 1); // descending
-  };
-  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) atomicAdd(&bucket[key(e)], 1u);
-  __syncthreads();
-  for (unsigned b0 = 0, carry = 0; b0 < order_buckets; b0 += blockDim.x) {
-    const unsigned b = b0 + threadIdx.x;
-    const uint32_t v = b < order_buckets ? bucket[b] : 0u;
-    uint32_t tot = 0;
-    const uint32_t ex = block_exclusive_scan(v, scan_scratch, &tot);
-    if (b < order_buckets) bucket[b] = carry + ex;
-    carry += tot;
-    __syncthreads();
-  }
-  for (unsigned e = threadIdx.x; e < n; e += blockDim.x) order[atomicAdd(&bucket[key(e)], 1u)] = e;
-}
-
-hipError_t launch_order_events_by_hits(
-  const uint32_t* offsets_estimated_input_size,
-  const uint32_t* number_of_events,
-  uint32_t* order,
-  hipStream_t s)
-{
-  hipLaunchKernelGGL(
-    k_order_events_by_hits, dim3(1), dim3(1024), 0, s, offsets_estimated_input_size, number_of_events, order);
-  return hipGetLastError();
-}
-
-// ThreeHitTracksFilter.cu:48-107
-__device__ __forceinline__ float means_square_fit_chi2(const Clusters& cc, unsigned hit_offset, const TrackletHits& t)
-{
-  float s0, sx, sz, sxz, sz2, u0, uy, uz, uyz, uz2;
-  s0 = sx = sz = sxz = sz2 = 0.0f;
-  u0 = uy = uz = uyz = uz2 = 0.0f;
-  float xs[3], ys[3], zs[3];
-#pragma unroll
-  for (unsigned h = 0; h < 3; ++h) {
-    const size_t i = (size_t) hit_offset + t.hits[h];
-    xs[h] = cc.xyz()[3 * i];
-    ys[h] = cc.xyz()[3 * i + 1];
-    zs[h] = cc.xyz()[3 * i + 2];
-  }
-#pragma unroll
-  for (unsigned h = 0; h < 3; ++h) {
-    const float x = xs[h], y = ys[h], z = zs[h];
-    const float wx = param_w;
-    const float wx_t_x = wx * x;
-    const float wx_t_z = wx * z;
-    s0 += wx;
-    sx += wx_t_x;
-    sz += wx_t_z;
-    sxz += wx_t_x * z;
-    sz2 += wx_t_z * z;
-    const float wy = param_w;
-    const float wy_t_y = wy * y;
-    const float wy_t_z = wy * z;
-    u0 += wy;
-    uy += wy_t_y;
-    uz += wy_t_z;
-    uyz += wy_t_y * z;
-    uz2 += wy_t_z * z;
-  }
-  const float dens = 1.0f / (sz2 * s0 - sz * sz);
-  const float state_tx = (sxz * s0 - sx * sz) * dens;
-  const float state_x = (sx * sz2 - sxz * sz) * dens;
-  const float denu = 1.0f / (uz2 * u0 - uz * uz);
-  const float state_ty = (uyz * u0 - uy * uz) * denu;
-  const float state_y = (uy * uz2 - uyz * uz) * denu;
-  float chi2 = 0.0f;
-#pragma unroll
-  for (unsigned h = 0; h < 3; ++h) {
-    const float z = zs[h];
-    const float x = state_x + state_tx * z;
-    const float y = state_y + state_ty * z;
-    const float dx = x - xs[h];
-    const float dy = y - ys[h];
-    chi2 += dx * dx * param_w + dy * dy * param_w;
-  }
-  return chi2 * 0.5f;
-}
-
 // ThreeHitTracksFilter.cu:109-169, ordered output.
 __global__ void k_three_hit_filter(
   const uint32_t* event_list,
@@ -1613,7 +1609,6 @@ __global__ void k_three_hit_filter(
   const unsigned n_events = number_of_events[0];
   const unsigned total = offsets_estimated_input_size[n_module_pairs * n_events];
   const unsigned hit_offset = offsets_estimated_input_size[event_number * n_module_pairs];
-  const uint8_t* used = hit_used_all + hit_offset;
   const Clusters cc {const_cast<char*>(sorted_container), total};
   const unsigned toff = track_offset(offsets_estimated_input_size, event_number);
   const TrackletHits* in = input_all + toff;
@@ -1631,9 +1626,10 @@ __global__ void k_three_hit_filter(
     TrackletHits t;
     if (i < n_in) {
       t = in[i];
-      const bool any_used = used[t.hits[0]] || used[t.hits[1]] || used[t.hits[2]];
-      const float chi2 = means_square_fit_chi2(cc, hit_offset, t);
-      keep = !any_used && chi2 < max_chi2;
+      const GlobalHits hits {cc.xyz() + 3 * (size_t) hit_offset, cc.phis() + hit_offset,
+                             const_cast<uint8_t*>(hit_used_all) + hit_offset, cc.ids() + hit_offset, nullptr};
+      const Hit h0 = hits.load(t.hits[0]), h1 = hits.load(t.hits[1]), h2 = hits.load(t.hits[2]);
+      keep = !(h0.used || h1.used || h2.used) && means_square_fit_chi2(h0, h1, h2) < max_chi2;
     }
     uint32_t kept;
     const uint32_t r = block_flag_scan(keep, scan, &kept);
@@ -1743,6 +1739,10 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   k.scorer_threshold = a.scorer_threshold;
   k.window = window;
   k.list_cap = list_cap;
+  k.three_hit_tracks_output = reinterpret_cast<TrackletHits*>(a.three_hit_tracks_output);
+  k.number_of_three_hit_tracks_output = a.number_of_three_hit_tracks_output;
+  k.event_track_hits = a.event_track_hits;
+  k.max_chi2 = a.max_chi2;
 #define VELO_LAUNCH_SEARCH_P(C, L, P) hipLaunchKernelGGL((k_search_by_triplet<C, L, P>), dim3(grid), dim3(block), dyn, s, k)
 #define VELO_LAUNCH_SEARCH(C, L)                                                                                    \
   do {                                                                                                              \

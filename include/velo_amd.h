@@ -494,10 +494,9 @@ int velo_sequence_status(velo_sequence* s, hipStream_t stream, unsigned* status)
  *                       reference algorithms one after the other
  *   "timed_stage"       VELO_STAGE_* to bracket with HIP events on the run's stream (0 = none)
  *   "kalman_fp64_fallback"  1: velo_kalman_filter's covariance_fp64_fallback (default 0)
- *   "consolidate_lds_map"   1 (default): consolidation maps an event's track hits to their
- *                       tracks in LDS (events up to 2047 tracks and 4096 track hits); 0: every
- *                       hit finds its track by a binary search over the hit-number offsets, as
- *                       larger events always do. Outputs do not depend on it
+ *   "consolidate_lds_map"   1 (default): consolidation and fit stage an event's hits in LDS
+ *                       (events up to 1920 hits); 0: they read them from the sorted container,
+ *                       as larger events always do. Outputs do not depend on it
  *   "count_work"        1: search_by_triplet also counts its work into the buffer "search_work"
  *                       (u64 x 4: seeding evaluations, forwarding evaluations, extrapolations,
  *                       phi-search probes) and, per event, the start and end wall-clock
@@ -511,9 +510,9 @@ enum {
   VELO_STAGE_ESTIMATE = 3,         /* velo_estimate_input_size */
   VELO_STAGE_CLUSTERING = 4,       /* masked clustering + sort by phi */
   VELO_STAGE_SEARCH = 5,           /* velo_search_by_triplet */
-  VELO_STAGE_THREE_HIT_FILTER = 6, /* velo_three_hit_tracks_filter */
-  VELO_STAGE_CONSOLIDATE = 7,      /* velo_consolidate_tracks */
-  VELO_STAGE_KALMAN = 8,           /* velo_kalman_filter */
+  VELO_STAGE_THREE_HIT_FILTER = 6, /* nothing: the filter is part of the search's launch */
+  VELO_STAGE_CONSOLIDATE = 7,      /* track offsets, consolidation and the Kalman fit, one launch */
+  VELO_STAGE_KALMAN = 8,           /* nothing: see VELO_STAGE_CONSOLIDATE */
   VELO_STAGE_PV = 9,               /* the beamline PV finder (knob "pv_finder") */
   VELO_STAGE_COUNT = 9
 };
