@@ -178,16 +178,6 @@ __device__ __forceinline__ unsigned candidates_final(uint32_t pixels, unsigned* 
   return m;
 }
 
-__device__ __forceinline__ unsigned
-sp_candidates(uint32_t sp_word, const uint32_t* words, unsigned n_sp, unsigned* p0, unsigned* p1)
-{
-  const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
-  const uint32_t sp_row = sp_addr & 0x3Fu, sp_col = sp_addr >> 6;
-  uint32_t pixels = neighbourhood_init(sp_word);
-  for (unsigned k = 0; k < n_sp; ++k) neighbour_acc(sp_row, sp_col, words[k], pixels);
-  return candidates_final(pixels, p0, p1);
-}
-
 __device__ __forceinline__ unsigned isolated_cluster_count(uint32_t sp)
 {
   const bool pattern_0 = (sp & 0x88) && !(sp & 0x44) && (sp & 0x33);
@@ -503,9 +493,71 @@ __global__ void k_bank_directory(
   }
 }
 
-// K2: one workgroup per event; wave w takes banks w, w+W, ...; lanes take SP words.
+// Banks of an event as one wave sees them: lane l holds the header of its l-th bank, so the
+// dependent reads of the headers (offset, source, count) take one round trip each for up to 64
+// banks, not for every bank.
+struct BankHeader {
+  uint32_t pair, n_sp;
+  const uint32_t* word;
+  bool velo;
+};
 template<int version>
-__global__ void k_estimate_input_size(
+__device__ __forceinline__ BankHeader bank_header(const RawEvent& ev, unsigned b)
+{
+  BankHeader h {0, 0, nullptr, false};
+  if (b < ev.n_banks) {
+    const RawBank bank = raw_bank<version>(ev, b);
+    h.velo = is_velo_bank(bank.type);
+    h.pair = bank.sourceID & 0x1FFu;
+    h.n_sp = bank_n_sp<version>(bank);
+    h.word = bank.word;
+  }
+  return h;
+}
+__device__ __forceinline__ BankHeader lane_header(const BankHeader& h, unsigned lane)
+{
+  const uint64_t p = reinterpret_cast<uint64_t>(h.word);
+  BankHeader r;
+  r.pair = __builtin_amdgcn_readlane(h.pair, lane);
+  r.n_sp = __builtin_amdgcn_readlane(h.n_sp, lane);
+  r.word = reinterpret_cast<const uint32_t*>(
+    static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(p), lane))) |
+    static_cast<uint64_t>(static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<uint32_t>(p >> 32), lane))) << 32);
+  r.velo = __builtin_amdgcn_readlane(h.velo, lane) != 0;
+  return r;
+}
+
+// Pixels that the words held by the wave's lanes (n of them, lane k the k-th) add to each lane's
+// neighbourhood: what neighbour_acc does with every word, from a difference of SP addresses
+// (column << 6 | row). The word is the same in all lanes, so taking it apart is scalar work and
+// costs the lanes 16 instructions a word. The pixels of the row above or below a lane at the edge
+// of its column, which the difference takes from the next column, are masked out at the end.
+__device__ __forceinline__ uint32_t neighbours_of_lanes(uint32_t words, unsigned n, uint32_t sp_addr)
+{
+  uint32_t pixels = 0;
+  for (unsigned k = 0; k < n; ++k) {
+    const uint32_t other = __builtin_amdgcn_readlane(words, k);
+    const uint32_t osp = other & 0xFFu;
+    const uint32_t d = ((other & 0x007FFF00u) >> 8) - sp_addr;
+    pixels |= d == 1u ? (osp & 0x01) << 4 | (osp & 0x10) << 6 : 0u;
+    pixels |= d == 65u ? (osp & 0x01) << 16 : 0u;
+    pixels |= d == 64u ? (osp & 0x0F) << 12 : 0u;
+    pixels |= d == 63u ? (osp & 0x08) << 8 : 0u;
+    pixels |= d == 0xFFFFFFFFu ? (osp & 0x80) >> 2 : 0u;
+  }
+  const uint32_t row = sp_addr & 0x3Fu;
+  if (row == 63u) pixels &= ~((1u << 4) | (1u << 10) | (1u << 16));
+  if (row == 0u) pixels &= ~((1u << 11) | (1u << 5));
+  return pixels;
+}
+
+// K2: one workgroup per event; wave w takes banks w, w+W, ...; lanes take SP words. Bound by the
+// latency of a bank (its words, then the scan over them): 16 waves share an event's 104 or 208
+// banks, and the words a lane is compared with come from the other lanes' registers instead of
+// memory. 500 pile-up events: 118 us, 410 us before.
+constexpr unsigned estimate_block = 1024;
+template<int version>
+__global__ void __launch_bounds__(estimate_block) k_estimate_input_size(
   const char* raw,
   const uint32_t* offsets,
   const uint32_t* sizes,
@@ -526,31 +578,46 @@ __global__ void k_estimate_input_size(
   __syncthreads();
   uint32_t* cands = cluster_candidates + candidates_offsets[event_number];
   const RawEvent ev(raw, offsets, sizes, types, mep, event_number + event_start);
-  const unsigned waves = blockDim.x / wave_size;
-  for (unsigned b = threadIdx.x / wave_size; b < ev.n_banks; b += waves) {
-    const RawBank bank = raw_bank<version>(ev, b);
-    if (!is_velo_bank(bank.type)) continue;
-    const unsigned n_sp = bank_n_sp<version>(bank);
-    const uint32_t pair = bank.sourceID & 0x1FFu;
-    const unsigned mp = (version == 2 || version == 3) ? pair / 8 : (pair << 1) / 8;
-    if (mp >= n_module_pairs) continue; // sourceID outside the 208 sensors
-    uint32_t count = 0;
-    for (unsigned s = lane_id(); s < n_sp; s += wave_size) {
-      const uint32_t w = bank.word[s];
-      if (w & 0x80000000u) {
-        count += isolated_cluster_count(w & 0xFFu);
+  const unsigned waves = blockDim.x / wave_size, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / wave_size);
+  const unsigned l = lane_id();
+  for (unsigned b0 = wave; b0 < ev.n_banks; b0 += waves * wave_size) {
+    const BankHeader headers = bank_header<version>(ev, b0 + waves * l);
+    const unsigned n_mine = min(wave_size, (ev.n_banks - b0 + waves - 1) / waves);
+    for (unsigned i = 0; i < n_mine; ++i) {
+      const BankHeader bank = lane_header(headers, i);
+      const unsigned mp = (version == 2 || version == 3) ? bank.pair / 8 : (bank.pair << 1) / 8;
+      if (!bank.velo || mp >= n_module_pairs) continue; // mp: a sourceID outside the 208 sensors
+      uint32_t count = 0;
+      for (unsigned s0 = 0; s0 < bank.n_sp; s0 += wave_size) {
+        const unsigned s = s0 + l;
+        const uint32_t w = s < bank.n_sp ? bank.word[s] : 0x80000000u;
+        const bool isolated = w & 0x80000000u;
+        const uint32_t sp_addr = (w & 0x007FFF00u) >> 8;
+        unsigned m = 0, p0 = 0, p1 = 0;
+        if (__ballot(!isolated)) {
+          uint32_t pixels = neighbourhood_init(w);
+          for (unsigned t0 = 0; t0 < bank.n_sp; t0 += wave_size) {
+            const uint32_t others = t0 == s0 ? w : t0 + l < bank.n_sp ? bank.word[t0 + l] : 0u;
+            pixels |= neighbours_of_lanes(others, min(wave_size, bank.n_sp - t0), sp_addr);
+          }
+          if (!isolated) m = candidates_final(pixels, &p0, &p1);
+        }
+        const uint64_t b0s = __ballot(m & 1), b1s = __ballot(m & 2);
+        const unsigned n_new = __popcll(b0s) + __popcll(b1s);
+        if (n_new) {
+          uint32_t slot = 0;
+          if (l == 0) slot = atomicAdd(&n_cand, n_new);
+          slot = __builtin_amdgcn_readfirstlane(slot) + rank_below(b0s) + rank_below(b1s);
+          const uint32_t sensor_number =
+            (version == 2 || version == 3) ? bank.pair : ((bank.pair << 1) | ((w >> 23) & 0x1u));
+          if (m & 1) cands[slot++] = (s << 11) | (sensor_number << 3) | p0;
+          if (m & 2) cands[slot] = (s << 11) | (sensor_number << 3) | p1;
+        }
+        const bool one = isolated && s < bank.n_sp;
+        count += n_new + __popcll(__ballot(one)) + __popcll(__ballot(one && isolated_cluster_count(w & 0xFFu) == 2));
       }
-      else {
-        unsigned p0 = 0, p1 = 0;
-        const unsigned m = sp_candidates(w, bank.word, n_sp, &p0, &p1);
-        const uint32_t sensor_number =
-          (version == 2 || version == 3) ? pair : ((pair << 1) | ((w >> 23) & 0x1u));
-        if (m & 1) cands[atomicAdd(&n_cand, 1u)] = (s << 11) | (sensor_number << 3) | p0;
-        if (m & 2) cands[atomicAdd(&n_cand, 1u)] = (s << 11) | (sensor_number << 3) | p1;
-        count += __popc(m);
-      }
+      if (l == 0 && count) atomicAdd(&est[mp], count);
     }
-    if (count) atomicAdd(&est[mp], count);
   }
   __syncthreads();
   for (unsigned i = threadIdx.x; i < n_module_pairs; i += blockDim.x)
@@ -559,8 +626,9 @@ __global__ void k_estimate_input_size(
 }
 
 // K3: one workgroup per event. Phase 1 takes isolated SPs of all banks, phase 2 the candidates.
+constexpr unsigned masked_block = 1024;
 template<int version>
-__global__ void k_masked_clustering(
+__global__ void __launch_bounds__(masked_block) k_masked_clustering(
   const char* raw,
   const uint32_t* offsets,
   const uint32_t* sizes,
@@ -739,7 +807,7 @@ hipError_t launch_estimate_input_size(const EstimateLaunch& a, hipStream_t s)
   if (!a.n_list) return hipSuccess;
 #define VELO_LAUNCH_EST(V)                                                                                          \
   hipLaunchKernelGGL(                                                                                               \
-    k_estimate_input_size<V>, dim3(a.n_list), dim3(256), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,    \
+    k_estimate_input_size<V>, dim3(a.n_list), dim3(estimate_block), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,    \
     a.event_start, a.candidates_offsets, a.estimated_input_size, a.module_candidate_num, a.cluster_candidates)
   switch (a.version) {
   case 2: VELO_LAUNCH_EST(2); break;
@@ -755,7 +823,7 @@ hipError_t launch_masked_clustering(const MaskedClusteringLaunch& a, hipStream_t
   if (!a.n_list) return hipSuccess;
 #define VELO_LAUNCH_MC(V)                                                                                           \
   hipLaunchKernelGGL(                                                                                               \
-    k_masked_clustering<V>, dim3(a.n_list), dim3(256), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,      \
+    k_masked_clustering<V>, dim3(a.n_list), dim3(masked_block), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,      \
     a.event_start, a.number_of_events, a.offsets_estimated_input_size, a.module_candidate_num, a.cluster_candidates, \
     a.candidates_offsets, a.bank_index, reinterpret_cast<const Geometry*>(a.geometry), a.sp_patterns, a.sp_fx,       \
     a.sp_fy, a.module_cluster_num, a.cluster_container)
