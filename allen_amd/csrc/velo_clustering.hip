@@ -269,10 +269,13 @@ __device__ __forceinline__ bool masked_cluster_final(
     keep = !(ext.pixels & 0x8000800080008000ull) && !(ext.pixels & 0xFFFFull);
   }
   if (!keep) return false;
-  const unsigned cx = x / n;
-  const unsigned cy = y / n;
-  const float fx = x / static_cast<float>(n) - cx;
-  const float fy = y / static_cast<float>(n) - cy;
+  // Their integer parts are the quotients of the integers: n is at most 128 pixels and a quotient below
+  // 2^10, so one that is no integer lies at least 2^-7 from one, and rounding moves it by 2^-14 at most.
+  const float qx = x / static_cast<float>(n), qy = y / static_cast<float>(n);
+  const unsigned cx = static_cast<unsigned>(qx);
+  const unsigned cy = static_cast<unsigned>(qy);
+  const float fx = qx - cx;
+  const float fy = qy - cy;
   *out = place_cluster(g, ltg, lhcb_id_of(sensor_number, cx >> 8, cx & 0xFFu, cy), cx, cy, fx, fy);
   return true;
 }
@@ -1100,22 +1103,22 @@ __device__ __forceinline__ void estimate_item(
       mp::for_words(B, n_words, resident, lw, active && !isolated, B.start[bi], B.start[bi + 1],
                     [&](uint32_t other) { neighbour_acc(sp_row, sp_col, other, pixels); });
     }
+    unsigned clusters = 0;
     if (active) {
       if (isolated) {
-        count += isolated_cluster_count(sp_word & 0xFFu);
+        clusters = isolated_cluster_count(sp_word & 0xFFu);
       }
       else {
         unsigned p0 = 0, p1 = 0;
         const unsigned mk = candidates_final(pixels, &p0, &p1);
-        count += __popc(mk);
+        clusters = __popc(mk);
         const uint32_t* wp = B.word(bi) + (w - B.start[bi]);
         sp_flags[static_cast<size_t>(reinterpret_cast<const char*>(wp) - raw) / 4] =
           static_cast<uint8_t>(mk | (p0 << 2) | (p1 << 5));
       }
     }
+    count += __popcll(__ballot(clusters > 0)) + __popcll(__ballot(clusters > 1)); // one or two a word
   }
-#pragma unroll
-  for (unsigned d = 32; d > 0; d >>= 1) count += __shfl_xor(count, d, wave_size);
   if (lane_id() == 0) {
     estimated_input_size[idx] = count;
     atomicAdd(event_totals + idx / n_module_pairs, count);
@@ -1212,15 +1215,14 @@ __device__ __forceinline__ void cluster_item(
   const bool resident = n_words <= mp::word_cap;
   const bool clusters_in_lds = estimate <= mp::cluster_cap;
   uint32_t* lw = sl.lw;
-  if (resident) mp::load_words(B, 0, n_words, lw);
   const Clusters scratch {unsorted_scratch, total};
   uint64_t* lkey = sl.lkey;
   float* lxyz = sl.lxyz;
   unsigned n = 0; // clusters so far (wave-uniform)
-  // Appends up to two clusters per lane in lane order (wave scan of the per-lane counts).
+  // Appends up to two clusters per lane in lane order (ranks from ballots).
   auto emit = [&](unsigned k, const ClusterOut& c0, const ClusterOut& c1) {
-    const unsigned inc = wave_inclusive_scan(k);
-    const unsigned slot0 = n + inc - k;
+    const uint64_t one = __ballot(k > 0), two = __ballot(k > 1);
+    const unsigned slot0 = n + rank_below(one) + rank_below(two);
     for (unsigned j = 0; j < k; ++j) {
       const unsigned slot = slot0 + j;
       const ClusterOut& c = j == 0 ? c0 : c1;
@@ -1236,7 +1238,7 @@ __device__ __forceinline__ void cluster_item(
         }
       }
     }
-    n += __shfl(inc, wave_size - 1, wave_size);
+    n += __popcll(one) + __popcll(two);
   };
   // The order in which clusters are appended does not reach the output: the module pair's
   // clusters are ranked by their distinct (phi, id) keys below.
@@ -1253,15 +1255,22 @@ __device__ __forceinline__ void cluster_item(
     static_assert(3 * mp::cluster_cap >= mp::word_cap && 2 * mp::cluster_cap >= mp::word_cap, "sort scratch");
     uint32_t* keys = reinterpret_cast<uint32_t*>(lxyz);
     uint32_t* sorted = reinterpret_cast<uint32_t*>(lkey);
-    // Distinct for distinct positions k; isolated words above the non-isolated ones.
-    auto sort_key = [](uint32_t word, unsigned k) { return (word & 0x80000000u) | (((word >> 8) & field) << 9) | k; };
+    // A word's key: isolated bit, bank (the same for all words it is compared with), then sensor,
+    // column and row, then its position, distinct for distinct words. The words and their candidate
+    // bytes are read together, so the sort waits for memory once.
+    static_assert(mp::word_cap <= 512 && max_banks_per_mp == 8, "sort key fields");
+    mp::wave_sync_lds();
     uint32_t bank_nonisolated = 0; // lane k counts bank k's non-isolated words
     for (unsigned base = 0; base < n_words; base += wave_size) {
       const unsigned w = base + lane_id();
       uint32_t word = 0x80000000u;
       if (w < n_words) {
-        word = lw[w];
-        keys[w] = sort_key(word, w);
+        const unsigned bi = mp::bank_of(B, w);
+        const unsigned at = B.word_offset[bi] + (w - B.start[bi]);
+        word = B.base[at];
+        const uint32_t f = sp_flags[at]; // written for non-isolated words
+        keys[w] = (word & 0x80000000u) | (bi << 26) | (((word >> 8) & field) << 9) | w;
+        lw[w] = (word & (v23 ? 0x007FFFFFu : 0x00FFFFFFu)) | (word & 0x80000000u ? 0u : f << 24);
       }
       const uint64_t m = __ballot(!(word & 0x80000000u));
       const unsigned l = lane_id();
@@ -1287,7 +1296,7 @@ __device__ __forceinline__ void cluster_item(
       const unsigned w = base + lane_id();
       if (w < n_words) {
         const uint32_t key = keys[w];
-        const unsigned bi = mp::bank_of(B, w);
+        const unsigned bi = (key >> 26) & (max_banks_per_mp - 1);
         const unsigned a = B.start[bi], b = B.start[bi + 1];
         unsigned rank = 0, k = a;
         for (; k + 4 <= b; k += 4) {
@@ -1298,13 +1307,7 @@ __device__ __forceinline__ void cluster_item(
           for (unsigned u = 0; u < 4; ++u) rank += v[u] < key ? 1u : 0u;
         }
         for (; k < b; ++k) rank += keys[k] < key ? 1u : 0u;
-        const uint32_t word = lw[w];
-        uint32_t f = 0;
-        if (!(word & 0x80000000u)) {
-          const uint32_t* wp = B.word(bi) + (w - a);
-          f = sp_flags[static_cast<size_t>(reinterpret_cast<const char*>(wp) - raw) / 4];
-        }
-        sorted[a + rank] = (f << 24) | (word & (v23 ? 0x007FFFFFu : 0x00FFFFFFu));
+        sorted[a + rank] = lw[w];
       }
     }
     mp::wave_sync_lds(); // every entry written
@@ -1352,10 +1355,9 @@ __device__ __forceinline__ void cluster_item(
   // from the SP's lane, and the kept clusters are appended in list order. A round has at most 128
   // candidates.
   auto candidates_round = [&](uint32_t sp_word, uint32_t sensor_number, uint32_t f, const Window& win) {
-    const unsigned nc = __popc(f & 3u);
-    const unsigned nc_inc = wave_inclusive_scan(nc);
-    const unsigned n_cand = __shfl(nc_inc, wave_size - 1, wave_size);
-    const unsigned first = nc_inc - nc;
+    const uint64_t firsts = __ballot(f & 1u), seconds = __ballot(f & 2u);
+    const unsigned n_cand = __popcll(firsts) + __popcll(seconds);
+    const unsigned first = rank_below(firsts) + rank_below(seconds);
     mp::wave_sync_lds(); // the previous round's list has been read
     if (f & 1u) sl.lcand[first] = static_cast<uint8_t>(lane_id());
     if (f & 2u) sl.lcand[first + (f & 1u)] = static_cast<uint8_t>(lane_id() | 0x80u);
