@@ -67,9 +67,24 @@ struct ClusterOut {
   int16_t phi;
 };
 
-__device__ __forceinline__ ClusterOut
-place_cluster(const Geometry& g, const float* ltg, uint32_t lhcb_id, unsigned cx, unsigned cy, float fx, float fy)
+// A cluster before it is placed: its id holds sensor (bits 18-27), column and row of its pixel
+// (cx = bits 8-17, cy = bits 0-7), fx and fy the fractions.
+struct ClusterSeed {
+  uint32_t id;
+  float fx, fy;
+};
+
+// The index of a seed's sensor in the geometry.
+template<int version>
+__device__ __forceinline__ uint32_t seed_sensor(const ClusterSeed& s)
 {
+  return (s.id >> 18) & (version == 2 || version == 3 ? 0x1FFu : 0x3FFu);
+}
+
+__device__ __forceinline__ ClusterOut place_cluster(const Geometry& g, uint32_t sensor, const ClusterSeed& s)
+{
+  const float* ltg = g.ltg + 12 * sensor;
+  const unsigned cx = (s.id >> 8) & 0x3FFu, cy = s.id & 0xFFu;
   // Every geometry load is issued before the first is used (the scheduler would otherwise wait
   // out several memory round trips one after another).
   float m[12];
@@ -77,10 +92,10 @@ place_cluster(const Geometry& g, const float* ltg, uint32_t lhcb_id, unsigned cx
   for (unsigned k = 0; k < 12; ++k) m[k] = ltg[k];
   const float lx = g.local_x[cx], pitch = g.x_pitch[cx];
   __builtin_amdgcn_sched_barrier(0);
-  const float local_x = lx + fx * pitch;
-  const float local_y = (cy + 0.5f + fy) * pixel_size;
+  const float local_x = lx + s.fx * pitch;
+  const float local_y = (cy + 0.5f + s.fy) * pixel_size;
   ClusterOut c;
-  c.id = lhcb_id;
+  c.id = s.id;
   c.x = m[0] * local_x + m[1] * local_y + m[9];
   c.y = m[3] * local_x + m[4] * local_y + m[10];
   c.z = m[6] * local_x + m[7] * local_y + m[11];
@@ -89,49 +104,39 @@ place_cluster(const Geometry& g, const float* ltg, uint32_t lhcb_id, unsigned cx
 }
 
 // One or two clusters of an isolated SP from the pattern table (MaskedVeloClustering.cu:165-286).
-// Returns the number written into out[].
+// Returns the number written into s0, s1.
 template<int version>
 __device__ __forceinline__ unsigned isolated_sp_clusters(
-  const Geometry& g,
   const uint8_t* sp_patterns,
   const float* sp_fx,
   const float* sp_fy,
-  const RawBank& bank,
+  uint32_t source,
   uint32_t sp_word,
-  ClusterOut& out0,
-  ClusterOut& out1)
+  ClusterSeed& s0,
+  ClusterSeed& s1)
 {
   constexpr bool v23 = (version == 2 || version == 3);
+  const uint32_t sensor_bit = (sp_word >> 23) & 1u;
+  const uint32_t sensor_index = v23 ? source : (((source & 0x1FFu) << 1) | sensor_bit);
   const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
-  const bool sensor_bit = (sp_word & 0x800000u) != 0;
-  const uint32_t pair = bank.sourceID & 0x1FFu;
-  const uint32_t sensor_index = v23 ? bank.sourceID : ((pair << 1) | (sensor_bit ? 1u : 0u));
-  const float* ltg = g.ltg + 12 * (v23 ? pair : ((pair << 1) | (sensor_bit ? 1u : 0u)));
   const uint32_t sp_row = sp_addr & 0x3Fu;
   const uint32_t sp_col = sp_addr >> 6;
   const uint32_t sp = sp_word & 0xFFu;
   const uint32_t idx = sp_patterns[sp];
-  const uint32_t chip = sp_col >> 7;
-  unsigned n = 0;
-#pragma unroll
-  for (unsigned k = 0; k < 2; ++k) {
-    if (k == 1 && !(idx & 8)) break;
-    const uint32_t row = k == 0 ? (idx & 0x03u) : ((idx >> 4) & 3u);
-    const uint32_t col = k == 0 ? ((idx >> 2) & 1u) : ((idx >> 6) & 1u);
+  auto seed = [&](uint32_t row, uint32_t col, unsigned k) {
     const uint32_t cx = sp_col * 2 + col;
     const uint32_t cy = sp_row * 4 + row;
-    const ClusterOut c =
-      place_cluster(g, ltg, lhcb_id_of(sensor_index, chip, cx & 0xFFu, cy), cx, cy, sp_fx[sp * 2 + k], sp_fy[sp * 2 + k]);
-    if (k == 0) out0 = c;
-    else out1 = c;
-    ++n;
-  }
-  return n;
+    return ClusterSeed {lhcb_id_of(sensor_index, sp_col >> 7, cx & 0xFFu, cy), sp_fx[sp * 2 + k], sp_fy[sp * 2 + k]};
+  };
+  s0 = seed(idx & 0x03u, (idx >> 2) & 1u, 0);
+  if (!(idx & 8)) return 1;
+  s1 = seed((idx >> 4) & 3u, (idx >> 6) & 1u, 1);
+  return 2;
 }
 
 // Candidate pixels of a non-isolated SP (EstimateInputSize.cu:104-204), in two steps:
-// neighbour_acc() ORs into the 18-bit neighbourhood `pixels` what one other SP word of the bank
-// contributes, candidates_final() applies the candidate mask. The neighbour scan keeps the
+// Neighbours collects in the 18-bit neighbourhood what the other SP words of the bank
+// contribute, candidates_final() applies the candidate mask. The neighbour scan keeps the
 // reference's behaviour: every word of the bank, of either sensor and isolated or not,
 // contributes (EstimateInputSize.cu:111-141).
 __device__ __forceinline__ uint32_t neighbourhood_init(uint32_t sp_word)
@@ -140,20 +145,38 @@ __device__ __forceinline__ uint32_t neighbourhood_init(uint32_t sp_word)
   return (sp & 0x0F) | ((sp & 0xF0) << 2);
 }
 
-__device__ __forceinline__ void neighbour_acc(uint32_t sp_row, uint32_t sp_col, uint32_t other, uint32_t& pixels)
-{
-  const uint32_t oaddr = (other & 0x007FFF00u) >> 8;
-  const uint32_t orow = oaddr & 0x3Fu;
-  const uint32_t ocol = oaddr >> 6;
-  const uint32_t osp = other & 0xFFu;
-  const bool top = orow == sp_row + 1, mid = orow == sp_row, bot = orow == sp_row - 1;
-  const bool same_col = ocol == sp_col, right_col = ocol == sp_col + 1;
-  if (top && same_col) pixels |= ((osp & 0x01) | ((osp & 0x10) << 2)) << 4;
-  if (top && right_col) pixels |= (osp & 0x01) << 16;
-  if (mid && right_col) pixels |= (osp & 0x0F) << 12;
-  if (bot && right_col) pixels |= (osp & 0x08) << 8;
-  if (bot && same_col) pixels |= (osp & 0x80) >> 2;
-}
+// The pixels that other words of the bank add to an SP's neighbourhood: the OR of the words at the five
+// addresses that matter, in three masks whose bits don't collide. Fourteen instructions a word.
+struct Neighbours {
+  uint32_t top, top_right, right, bot_right, bot; // addresses; all ones: outside the SP grid
+  uint32_t column = 0, side = 0, corner = 0;
+  __device__ __forceinline__ Neighbours(uint32_t sp_addr)
+  {
+    constexpr uint32_t outside = 0xFFFFFFFFu;
+    const uint32_t row = sp_addr & 0x3Fu;
+    const bool up = row < 63u, down = row > 0u, east = sp_addr < (511u << 6);
+    top = up ? sp_addr + 1u : outside;
+    bot = down ? sp_addr - 1u : outside;
+    right = east ? sp_addr + 64u : outside;
+    top_right = up && east ? sp_addr + 65u : outside;
+    bot_right = down && east ? sp_addr + 63u : outside;
+  }
+  __device__ __forceinline__ void add(uint32_t other)
+  {
+    const uint32_t address = (other >> 8) & 0x7FFFu;
+    uint32_t mask = address == top ? 0x11u : 0u;
+    mask = address == bot ? 0x80u : mask;
+    mask = address == bot_right ? 0x08u : mask;
+    column |= other & mask;
+    side |= other & (address == right ? 0x0Fu : 0u);
+    corner |= other & (address == top_right ? 0x01u : 0u);
+  }
+  __device__ __forceinline__ uint32_t pixels() const
+  {
+    return ((column & 0x01u) << 4) | ((column & 0x10u) << 6) | (corner << 16) | (side << 12) | ((column & 0x08u) << 8) |
+           ((column & 0x80u) >> 2);
+  }
+};
 
 // Returns a 2-bit mask: bit0 = first candidate (pixels 0,1,4,5), bit1 = second; the pixel
 // numbers are returned in *p0, *p1.
@@ -188,8 +211,7 @@ __device__ __forceinline__ unsigned isolated_cluster_count(uint32_t sp)
 // rest_of_clusters (MaskedVeloClustering.cu:290-496) for one candidate pixel, in two steps:
 // window_acc() ORs one other SP word of the bank into the 5-column x 4-row SP window around the
 // candidate's SP (pa[c]: one SP column, rows bottom to top, 16 bits per pixel column), and
-// masked_cluster_final() grows the cluster, applies the precedence and window-edge rules and
-// places it.
+// masked_cluster_final() grows the cluster and applies the precedence and window-edge rules.
 struct Window {
   uint32_t pa0, pa1, pa2, pa3, pa4;
 };
@@ -216,34 +238,13 @@ window_acc(int32_t sp_row_lower, int32_t sp_col_lower, uint32_t sensor_number, u
   }
 }
 
-// window_acc() for a word already known to be non-isolated and on the candidate's sensor (the
-// sorted lists of k_cluster_mp hold only such words in a candidate's range). Bits 24-31 of
-// `other` are not read.
-__device__ __forceinline__ void window_acc_same_sensor(int32_t sp_row_lower, int32_t sp_col_lower, uint32_t other, Window& w)
-{
-  const uint32_t oaddr = (other & 0x007FFF00u) >> 8;
-  const int32_t rr = static_cast<int32_t>(oaddr & 0x3Fu) - sp_row_lower;
-  const int32_t rc = static_cast<int32_t>(oaddr >> 6) - sp_col_lower;
-  if (rr >= 0 && rr <= 3 && rc >= 0 && rc <= 4) {
-    const uint32_t osp = other & 0xFFu;
-    const uint32_t bits = ((osp & 0x0Fu) << (4 * rr)) | ((osp & 0xF0u) << (12 + 4 * rr));
-    w.pa0 |= rc == 0 ? bits : 0u;
-    w.pa1 |= rc == 1 ? bits : 0u;
-    w.pa2 |= rc == 2 ? bits : 0u;
-    w.pa3 |= rc == 3 ? bits : 0u;
-    w.pa4 |= rc == 4 ? bits : 0u;
-  }
-}
-
 __device__ __forceinline__ bool masked_cluster_final(
-  const Geometry& g,
   uint32_t sp_word,
   uint32_t sensor_number,
   uint32_t starting_pixel_location,
   const Window& pa,
-  ClusterOut* out)
+  ClusterSeed* out)
 {
-  const float* ltg = g.ltg + 12 * sensor_number;
   const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
   const int32_t sp_row = sp_addr & 0x3Fu;
   const int32_t sp_col = sp_addr >> 6;
@@ -276,20 +277,19 @@ __device__ __forceinline__ bool masked_cluster_final(
   const unsigned cy = static_cast<unsigned>(qy);
   const float fx = qx - cx;
   const float fy = qy - cy;
-  *out = place_cluster(g, ltg, lhcb_id_of(sensor_number, cx >> 8, cx & 0xFFu, cy), cx, cy, fx, fy);
+  *out = ClusterSeed {lhcb_id_of(sensor_number, cx >> 8, cx & 0xFFu, cy), fx, fy};
   return true;
 }
 
 // The whole of rest_of_clusters for the SP at `sp_index` of a bank whose words are `words`.
 template<int version>
 __device__ __forceinline__ bool masked_cluster(
-  const Geometry& g,
   const uint32_t* words,
   unsigned n_sp,
   unsigned sp_index,
   uint32_t sensor_number,
   uint32_t starting_pixel_location,
-  ClusterOut* out)
+  ClusterSeed* out)
 {
   const uint32_t sp_word = words[sp_index];
   const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
@@ -297,7 +297,7 @@ __device__ __forceinline__ bool masked_cluster(
   const int32_t sp_col_lower = static_cast<int32_t>(sp_addr >> 6) - 3;
   Window w {0, 0, 0, 0, 0};
   for (unsigned k = 0; k < n_sp; ++k) window_acc<version>(sp_row_lower, sp_col_lower, sensor_number, words[k], w);
-  return masked_cluster_final(g, sp_word, sensor_number, starting_pixel_location, w, out);
+  return masked_cluster_final(sp_word, sensor_number, starting_pixel_location, w, out);
 }
 
 __device__ __forceinline__ void store_cluster(const Clusters& c, unsigned i, const ClusterOut& o)
@@ -531,7 +531,7 @@ __device__ __forceinline__ BankHeader lane_header(const BankHeader& h, unsigned 
 }
 
 // Pixels that the words held by the wave's lanes (n of them, lane k the k-th) add to each lane's
-// neighbourhood: what neighbour_acc does with every word, from a difference of SP addresses
+// neighbourhood: what Neighbours does with every word, from a difference of SP addresses
 // (column << 6 | row). The word is the same in all lanes, so taking it apart is scalar work and
 // costs the lanes 16 instructions a word. The pixels of the row above or below a lane at the edge
 // of its column, which the difference takes from the next column, are masked out at the end.
@@ -672,12 +672,13 @@ __global__ void __launch_bounds__(masked_block) k_masked_clustering(
     for (unsigned s = lane_id(); s < n_sp; s += wave_size) {
       const uint32_t w = bank.word[s];
       if (!(w & 0x80000000u)) continue;
-      ClusterOut c0, c1;
-      const unsigned n = isolated_sp_clusters<version>(g, sp_patterns, sp_fx, sp_fy, bank, w, c0, c1);
+      ClusterSeed s0, s1;
+      const unsigned n = isolated_sp_clusters<version>(sp_patterns, sp_fx, sp_fy, bank.sourceID, w, s0, s1);
       const unsigned slot = atomicAdd(&count[mp], n);
       const unsigned cap = mp_start[mp + 1] - mp_start[mp];
-      if (slot < cap) store_cluster(clusters, mp_start[mp] + slot, c0);
-      if (n > 1 && slot + 1 < cap) store_cluster(clusters, mp_start[mp] + slot + 1, c1);
+      if (slot < cap) store_cluster(clusters, mp_start[mp] + slot, place_cluster(g, seed_sensor<version>(s0), s0));
+      if (n > 1 && slot + 1 < cap)
+        store_cluster(clusters, mp_start[mp] + slot + 1, place_cluster(g, seed_sensor<version>(s1), s1));
     }
   }
   __syncthreads();
@@ -688,11 +689,12 @@ __global__ void __launch_bounds__(masked_block) k_masked_clustering(
     const uint32_t sensor_number = (cand >> 3) & 0xFFu;
     if (sensor_number >= n_sensors) continue;
     const RawBank bank = raw_bank<version>(ev, bank_index[sensor_number]);
-    ClusterOut c;
-    if (masked_cluster<version>(g, bank.word, bank_n_sp<version>(bank), cand >> 11, sensor_number, cand & 7u, &c)) {
+    ClusterSeed c;
+    if (masked_cluster<version>(bank.word, bank_n_sp<version>(bank), cand >> 11, sensor_number, cand & 7u, &c)) {
       const unsigned mp = sensor_number / 8;
       const unsigned slot = atomicAdd(&count[mp], 1u);
-      if (mp < n_module_pairs && slot < mp_start[mp + 1] - mp_start[mp]) store_cluster(clusters, mp_start[mp] + slot, c);
+      if (mp < n_module_pairs && slot < mp_start[mp + 1] - mp_start[mp]) 
+        store_cluster(clusters, mp_start[mp] + slot, place_cluster(g, sensor_number, c));
     }
   }
   __syncthreads();
@@ -860,25 +862,21 @@ hipError_t launch_sort_by_phi(const SortLaunch& a, hipStream_t s)
 //                   run of them), clusters appended with wave ballots, then ranked by (phi, id)
 //                   and written sorted
 //
-// Each wave stages the SP words of its module pair's banks in its own LDS slice; a module pair
-// larger than the slice runs the same code on global memory.
+// Each wave works in its own LDS slice; a module pair larger than the slice runs tile by tile.
+// Two waves to a workgroup: a finished wave keeps its LDS until its workgroup ends, and module pairs
+// differ (20 000 one-vertex events: 665 + 940 us with two, 692 + 978 with four, 660 + 941 with one).
 namespace mp {
-constexpr unsigned waves_per_block = 4;
-constexpr unsigned word_cap = 384;
-// Clusters of a module pair kept in LDS (more go through global memory): 192 keeps k_cluster_mp's
-// workgroup at 22 880 B of LDS, so seven fit a CU; about 0.1 % of pileup_1000's module pairs and
-// 1.4 % of batched_20k's have a larger estimate.
-constexpr unsigned cluster_cap = 192;
-constexpr unsigned hash_bits = 10;  // estimate: (bank, SP address) table of a resident module pair,
+constexpr unsigned waves_per_block = 2;
+constexpr unsigned hash_bits = 10;  // estimate: (bank, SP address) table of a module pair,
 constexpr unsigned hash_slots = 1u << hash_bits; // more slots than words, so an empty slot ends every probe
+constexpr unsigned table_words = 704; // most words that enter it
 constexpr uint32_t hash_empty = 0xFFFFFFFFu; // an empty slot; keys have 18 bits, so no slot of a key is all ones
 constexpr uint32_t hash_no_key = 0x01000000u; // a lookup key that matches no slot (nor an empty one)
-constexpr unsigned hash_min_bank = 16; // largest bank (words) above which the table beats the scan (measured)
-static_assert(hash_slots > word_cap, "hash table load");
+constexpr unsigned hash_min_bank = 12; // largest bank (words) above which the table beats the scan (measured)
+static_assert(hash_slots > table_words, "hash table load");
 
-// Banks of one module pair (at most 8), kept in the wave's LDS slice. Bank k's words start at
-// base + word_offset[k] (32-bit offsets in place of pointers: 112 B per wave, so that seven
-// workgroups of k_estimate_mp fit a CU's LDS).
+// Banks of one module pair (at most 8), kept in the wave's LDS slice while it is worked on in tiles.
+// Bank k's words start at base + word_offset[k].
 struct Banks {
   const uint32_t* base;
   unsigned n;
@@ -886,13 +884,6 @@ struct Banks {
   uint32_t source[max_banks_per_mp];
   uint32_t word_offset[max_banks_per_mp];
   __device__ __forceinline__ const uint32_t* word(unsigned k) const { return base + word_offset[k]; }
-};
-
-// k_cluster_mp's sorted banks: each bank's non-isolated words first, then its isolated ones.
-struct SortedBanks {
-  uint32_t sorted[max_banks_per_mp + 1];          // non-isolated words of the banks before each
-  uint32_t first_isolated[max_banks_per_mp];      // a bank's first isolated position
-  uint32_t isolated_before[max_banks_per_mp + 1]; // isolated words of the banks before each
 };
 
 __device__ __forceinline__ void wave_sync_lds()
@@ -969,157 +960,183 @@ __device__ __forceinline__ void load_words(const Banks& B, unsigned t0, unsigned
   wave_sync_lds();
 }
 
-// Calls f(word) for every word of the flattened range [lo, hi): straight from the resident
-// slice, or tile by tile through it (wave-uniform tile loop, per-lane ranges).
+// Calls f(word) for every word of the flattened range [lo, hi), tile by tile through the slice
+// (wave-uniform tile loop, per-lane ranges; eight LDS reads in flight at a time).
 template<typename F>
 __device__ __forceinline__ void
-for_words(const Banks& B, unsigned n_words, bool resident, uint32_t* lw, bool active, unsigned lo, unsigned hi, F&& f)
+for_words(const Banks& B, unsigned n_words, uint32_t* lw, unsigned tile, bool active, unsigned lo, unsigned hi, F&& f)
 {
-  // Words [a, b) of the slice in order, eight LDS reads in flight at a time.
-  auto scan = [&](const uint32_t* w, unsigned a, unsigned b) {
-    unsigned k = a;
-    for (; k + 8 <= b; k += 8) {
+  for (unsigned t0 = 0; t0 < n_words; t0 += tile) {
+    const unsigned tn = min(tile, n_words - t0);
+    load_words(B, t0, tn, lw);
+    if (!active) continue;
+    unsigned k = max(lo, t0) - t0;
+    const unsigned end = min(hi, t0 + tn) - t0;
+    if (hi <= t0) continue;
+    for (; k + 8 <= end; k += 8) {
       uint32_t v[8];
 #pragma unroll
-      for (unsigned u = 0; u < 8; ++u) v[u] = w[k + u];
+      for (unsigned u = 0; u < 8; ++u) v[u] = lw[k + u];
 #pragma unroll
       for (unsigned u = 0; u < 8; ++u) f(v[u]);
     }
-    for (; k < b; ++k) f(w[k]);
-  };
-  if (resident) {
-    if (active) scan(lw, lo, hi);
-    return;
-  }
-  for (unsigned t0 = 0; t0 < n_words; t0 += word_cap) {
-    const unsigned tn = min(word_cap, n_words - t0);
-    load_words(B, t0, tn, lw);
-    if (active) {
-      const unsigned a = max(lo, t0), b = min(hi, t0 + tn);
-      if (a < b) scan(lw, a - t0, b - t0);
-    }
+    for (; k < end; ++k) f(lw[k]);
   }
 }
-} // namespace mp
 
-namespace mp {
 // Slot of a (bank, SP address) key in a table of 2^bits slots: multiplicative hashing.
 __device__ __forceinline__ unsigned hash_slot(uint32_t key, unsigned bits) { return (key * 2654435761u) >> (32 - bits); }
 } // namespace mp
 
+// What one wave of k_estimate_mp holds in LDS: 5.5 KB, so that 28 waves fit a CU.
+namespace mp {
+struct alignas(16) EstimateLds {
+  static constexpr unsigned word_cap = 336;
+  uint32_t table[hash_slots];
+  uint4 bank[max_banks_per_mp]; // word offset less the words before the bank, first word, end
+  uint32_t words[word_cap];
+  // A module pair that is worked on in tiles has its banks where the table would be.
+  __device__ __forceinline__ Banks& banks() { return *reinterpret_cast<Banks*>(table); }
+};
+static_assert(max_banks_per_mp * hash_min_bank <= EstimateLds::word_cap, "words of small banks");
+} // namespace mp
+
 // K2 of one module pair (idx = event * 26 + module pair) by one wave. The neighbourhood of a
 // non-isolated SP is what the reference collects by scanning every word of its bank: the SP
-// bytes of the words at five neighbouring addresses, OR-ed (EstimateInputSize.cu:111-141). For a
-// module pair resident in LDS the words are first entered in a hash table keyed by (bank, SP
-// address) whose value is the OR of their SP bytes (one word per slot: key << 8 | value), and
-// each SP looks its five neighbours up; OR-ing is order-free, so the result is the scan's.
-// Larger module pairs, and those whose banks are all small, scan.
+// bytes of the words at five neighbouring addresses, OR-ed (EstimateInputSize.cu:111-141). OR-ing is
+// order-free and a word at another address adds nothing, so three ways give the same:
+//  - banks that are all small: the scan, from LDS;
+//  - larger ones: the words are first entered in a hash table keyed by (bank, SP address) whose
+//    value is the OR of their SP bytes (one word per slot: key << 8 | value), and each SP looks its
+//    five neighbours up. A scan costs a wave 17 instructions for each word of its largest bank, the
+//    table about 200;
+//  - more words than the table takes: the scan, tile by tile.
+// Bound by VALU issue. 20 000 one-vertex events: 482 us (692 with 27 instructions for each word that is
+// compared and module pairs of more than 384 words in tiles), 2000 stress events: 104 us (200).
+// Scans of banks of up to 10, 16 and 24 words: 480, 486 and 520 us.
 __device__ __forceinline__ void estimate_item(
   const char* raw,
-  const mp::DirFetch& dir,
+  const mp::DirFetch& f,
   unsigned idx,
-  mp::Banks& B,
-  uint32_t* lw,
-  uint32_t* table_slots,
+  mp::EstimateLds& L,
   uint32_t* estimated_input_size,
   uint32_t* event_totals,
   uint8_t* sp_flags)
 {
-  mp::load_banks(raw, dir, B);
-  const unsigned n_words = B.start[B.n];
-  const bool resident = n_words <= mp::word_cap;
-  // A scan costs a wave about as many steps as its largest bank has words; the table, a fixed
-  // number of LDS round trips. The table serves resident module pairs whose largest bank has
-  // more than hash_min_bank words.
+  const unsigned l = lane_id();
+  const unsigned n_sp = l < f.nb ? f.en.n_sp : 0u;
+  const unsigned inc = wave_inclusive_scan(n_sp), first = inc - n_sp; // words before this lane's bank
+  const unsigned n_words = __builtin_amdgcn_readlane(inc, max_banks_per_mp - 1);
   unsigned largest_bank = 0;
-  for (unsigned k = 0; k < B.n; ++k) largest_bank = max(largest_bank, B.start[k + 1] - B.start[k]);
-  const bool table = resident && largest_bank > mp::hash_min_bank;
-  // Table of four times as many slots as words, 64 to 1024 (load at most 3/8: the wave waits for
-  // its longest probe, so the probes must stay short everywhere).
-  const unsigned bits = min(mp::hash_bits, max(6u, 32u - __clz(4 * n_words - 1)));
+  for (unsigned k = 0; k < f.nb; ++k) largest_bank = max(largest_bank, static_cast<unsigned>(__builtin_amdgcn_readlane(n_sp, k)));
+  const bool scan = largest_bank <= mp::hash_min_bank;
+  const bool table = !scan && n_words <= mp::table_words;
+  // Table of eight times as many slots as words, 256 to 1024: the wave waits for its longest probe,
+  // so the probes must stay short everywhere.
+  const unsigned bits = min(mp::hash_bits, max(8u, 32u - __clz(8 * n_words - 1)));
   const unsigned hmask = (1u << bits) - 1;
-  if (resident) mp::load_words(B, 0, n_words, lw);
-  if (table) {
-    for (unsigned h = lane_id(); h <= hmask; h += wave_size) table_slots[h] = mp::hash_empty;
-    mp::wave_sync_lds();
-    for (unsigned w = lane_id(); w < n_words; w += wave_size) {
-      const uint32_t word = lw[w];
-      const uint32_t key = (mp::bank_of(B, w) << 15) | ((word & 0x007FFF00u) >> 8);
+  const uint32_t* raw_words = reinterpret_cast<const uint32_t*>(raw);
+  // The number of the bank holding word w: the banks after the first that start at or before it.
+  auto bank_of = [&](unsigned w) {
+    unsigned bi = 0;
+    for (unsigned j = 1; j < f.nb; ++j) bi += w >= static_cast<unsigned>(__builtin_amdgcn_readlane(first, j));
+    return bi;
+  };
+  mp::wave_sync_lds();
+  if (l < f.nb) L.bank[l] = make_uint4(f.en.word_offset - first, first, inc, 0);
+  if (table)
+    for (unsigned h = 4 * l; h <= hmask; h += 4 * wave_size)
+      *reinterpret_cast<uint4*>(L.table + h) = make_uint4(mp::hash_empty, mp::hash_empty, mp::hash_empty, mp::hash_empty);
+  mp::wave_sync_lds();
+  if (scan || table) {
+    for (unsigned w = l; w < n_words; w += wave_size) {
+      const unsigned bi = bank_of(w);
+      const uint32_t word = raw_words[L.bank[bi].x + w];
+      if (w < mp::EstimateLds::word_cap) L.words[w] = word;
+      if (scan) continue;
+      const uint32_t key = (bi << 15) | ((word & 0x007FFF00u) >> 8);
       for (unsigned h = mp::hash_slot(key, bits);; h = (h + 1) & hmask) {
-        const uint32_t old = atomicCAS(&table_slots[h], mp::hash_empty, (key << 8) | (word & 0xFFu));
+        const uint32_t old = atomicCAS(&L.table[h], mp::hash_empty, (key << 8) | (word & 0xFFu));
         if (old == mp::hash_empty) break;
         if ((old >> 8) == key) {
-          atomicOr(&table_slots[h], word & 0xFFu);
+          atomicOr(&L.table[h], word & 0xFFu);
           break;
         }
       }
     }
-    mp::wave_sync_lds();
   }
+  else mp::load_banks(raw, f, L.banks());
+  mp::wave_sync_lds();
   uint32_t count = 0;
   for (unsigned base = 0; base < n_words; base += wave_size) {
-    const unsigned w = base + lane_id();
+    const unsigned w = base + l;
     const bool active = w < n_words;
-    const unsigned bi = active ? mp::bank_of(B, w) : 0;
-    const uint32_t sp_word = active ? (resident ? lw[w] : B.word(bi)[w - B.start[bi]]) : 0u;
-    const bool isolated = (sp_word & 0x80000000u) != 0;
-    const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
-    const uint32_t sp_row = sp_addr & 0x3Fu, sp_col = sp_addr >> 6;
+    const unsigned bi = bank_of(w);
+    const uint4 bank = L.bank[bi];
+    uint32_t sp_word = 0;
+    if (active) {
+      if ((scan || table) && w < mp::EstimateLds::word_cap) sp_word = L.words[w];
+      else sp_word = raw_words[bank.x + w];
+    }
+    const bool isolated = (sp_word & 0x80000000u) != 0, non = active && !isolated;
+    const uint32_t sp_addr = (sp_word >> 8) & 0x7FFFu;
+    Neighbours around(sp_addr);
     uint32_t pixels = neighbourhood_init(sp_word);
     if (table) {
-      if (active && !isolated) {
-        // neighbour_acc's five cases, each from the OR of the words at that address (rows and
-        // columns outside the SP grid match no word).
+      if (non) {
         // The five first probes are issued together, then the rare longer probes.
         const uint32_t kb = bi << 15;
-        const uint32_t cols[5] = {sp_col, sp_col + 1, sp_col + 1, sp_col + 1, sp_col};
-        const uint32_t rows[5] = {sp_row + 1, sp_row + 1, sp_row, sp_row - 1, sp_row - 1};
+        const uint32_t address[5] = {around.top, around.top_right, around.right, around.bot_right, around.bot};
         uint32_t key[5], got[5], v[5];
         unsigned h[5];
 #pragma unroll
         for (unsigned k = 0; k < 5; ++k) {
-          const bool valid = rows[k] < 64u && cols[k] < 512u;
-          key[k] = valid ? (kb | (cols[k] << 6) | rows[k]) : mp::hash_no_key;
+          const bool valid = address[k] != 0xFFFFFFFFu;
+          key[k] = valid ? (kb | address[k]) : mp::hash_no_key;
           h[k] = mp::hash_slot(key[k], bits);
-          got[k] = valid ? table_slots[h[k]] : mp::hash_empty;
+          got[k] = valid ? L.table[h[k]] : mp::hash_empty;
         }
 #pragma unroll
         for (unsigned k = 0; k < 5; ++k)
           while ((got[k] >> 8) != key[k] && got[k] != mp::hash_empty) {
             h[k] = (h[k] + 1) & hmask;
-            got[k] = table_slots[h[k]];
+            got[k] = L.table[h[k]];
           }
 #pragma unroll
-        for (unsigned k = 0; k < 5; ++k) v[k] = (got[k] >> 8) == key[k] ? (got[k] & 0xFFu) : 0u;
-        const uint32_t top = v[0], top_right = v[1], right = v[2], bot_right = v[3], bot = v[4];
-        pixels |= ((top & 0x01) | ((top & 0x10) << 2)) << 4;
-        pixels |= (top_right & 0x01) << 16;
-        pixels |= (right & 0x0F) << 12;
-        pixels |= (bot_right & 0x08) << 8;
-        pixels |= (bot & 0x80) >> 2;
+        for (unsigned k = 0; k < 5; ++k) v[k] = (got[k] >> 8) == key[k] ? got[k] : 0u;
+        around.column = (v[0] & 0x11u) | (v[3] & 0x08u) | (v[4] & 0x80u);
+        around.corner = v[1] & 0x01u;
+        around.side = v[2] & 0x0Fu;
       }
+    }
+    else if (scan) {
+      if (non) // four words at a time; the last is taken again where fewer are left
+        for (unsigned k = bank.y; k < bank.z; k += 4) {
+          uint32_t v[4];
+#pragma unroll
+          for (unsigned u = 0; u < 4; ++u) v[u] = L.words[min(k + u, bank.z - 1)];
+#pragma unroll
+          for (unsigned u = 0; u < 4; ++u) around.add(v[u]);
+        }
     }
     else {
-      mp::for_words(B, n_words, resident, lw, active && !isolated, B.start[bi], B.start[bi + 1],
-                    [&](uint32_t other) { neighbour_acc(sp_row, sp_col, other, pixels); });
+      mp::for_words(L.banks(), n_words, L.words, mp::EstimateLds::word_cap, non, bank.y, bank.z,
+                    [&](uint32_t other) { around.add(other); });
     }
+    pixels |= around.pixels();
     unsigned clusters = 0;
-    if (active) {
-      if (isolated) {
-        clusters = isolated_cluster_count(sp_word & 0xFFu);
-      }
-      else {
-        unsigned p0 = 0, p1 = 0;
-        const unsigned mk = candidates_final(pixels, &p0, &p1);
-        clusters = __popc(mk);
-        const uint32_t* wp = B.word(bi) + (w - B.start[bi]);
-        sp_flags[static_cast<size_t>(reinterpret_cast<const char*>(wp) - raw) / 4] =
-          static_cast<uint8_t>(mk | (p0 << 2) | (p1 << 5));
-      }
+    if (isolated) {
+      clusters = isolated_cluster_count(sp_word & 0xFFu);
+    }
+    else if (active) {
+      unsigned p0 = 0, p1 = 0;
+      const unsigned mk = candidates_final(pixels, &p0, &p1);
+      clusters = __popc(mk);
+      sp_flags[bank.x + w] = static_cast<uint8_t>(mk | (p0 << 2) | (p1 << 5));
     }
     count += __popcll(__ballot(clusters > 0)) + __popcll(__ballot(clusters > 1)); // one or two a word
   }
-  if (lane_id() == 0) {
+  if (l == 0) {
     estimated_input_size[idx] = count;
     atomicAdd(event_totals + idx / n_module_pairs, count);
   }
@@ -1137,9 +1154,7 @@ __global__ void __launch_bounds__(mp::waves_per_block* wave_size) k_estimate_mp(
   uint32_t* event_totals,
   uint8_t* sp_flags)
 {
-  __shared__ uint32_t s_words[mp::waves_per_block][mp::word_cap];
-  __shared__ uint32_t s_table[mp::waves_per_block][mp::hash_slots];
-  __shared__ mp::Banks s_banks[mp::waves_per_block];
+  __shared__ mp::EstimateLds s_lds[mp::waves_per_block];
   const unsigned wave = threadIdx.x / wave_size;
   const unsigned n_items = n_events * n_module_pairs;
   const unsigned stride = gridDim.x * mp::waves_per_block;
@@ -1149,19 +1164,41 @@ __global__ void __launch_bounds__(mp::waves_per_block* wave_size) k_estimate_mp(
   for (; idx < n_items; idx += stride) {
     mp::DirFetch next = cur;
     if (idx + stride < n_items) next = mp::fetch_dir(directory, directory_count, idx + stride);
-    estimate_item(raw, cur, idx, s_banks[wave], s_words[wave], s_table[wave], estimated_input_size,
-                  event_totals, sp_flags);
+    estimate_item(raw, cur, idx, s_lds[wave], estimated_input_size, event_totals, sp_flags);
     cur = next;
   }
 }
 
-// The wave-private LDS slices of k_cluster_mp.
-struct ClusterSlices {
-  uint32_t* lw;
-  uint64_t* lkey;
-  float* lxyz;
-  uint8_t* lcand; // 2 x wave_size: the candidate pixels of one word round, (lane | pixel << 7)
+// What one wave of k_cluster_mp holds in LDS: 5.8 KB, so that seven workgroups fit a CU.
+namespace mp {
+constexpr unsigned non_isolated_cap = 256; // non-isolated SP words of a module pair
+constexpr unsigned cluster_cap = 192;      // its clusters; more of them go through global memory
+// The ranking's memory for `cap` clusters: each phi bucket's newest cluster and their number, the keys,
+// each cluster's successor in its bucket.
+constexpr unsigned rank_bytes(unsigned cap) { return 2 * 4 * wave_size + 10 * cap; }
+struct ClusterLds {
+  // The non-isolated words (then the list of candidates), the sorted ones, and the sort's keys (then
+  // the candidates' windows). Once the seeds are found, the ranking keys take this memory.
+  static constexpr unsigned window_words = 5 * wave_size;
+  uint64_t work[(2 * non_isolated_cap + window_words) / 2];
+  float xyz[3 * cluster_cap];           // a seed's fx, fy and id, then the placed cluster's x, y, z
+  uint2 bank[max_banks_per_mp];         // word offset less the words before the bank, source
+  uint32_t non_start[max_banks_per_mp + 1]; // non-isolated words before each bank
+  __device__ __forceinline__ uint32_t* words() { return reinterpret_cast<uint32_t*>(work); }
+  __device__ __forceinline__ uint32_t* sorted() { return words() + non_isolated_cap; }
+  __device__ __forceinline__ uint32_t* keys() { return words() + 2 * non_isolated_cap; }
+  // A module pair that is worked on in tiles has its banks where the sort's keys would be.
+  static constexpr unsigned tile = 2 * non_isolated_cap;
+  __device__ __forceinline__ Banks& banks() { return *reinterpret_cast<Banks*>(keys()); }
+  // Most clusters that are ranked with nothing else in the slice, and in tiles of keys alone.
+  static constexpr unsigned rank_cap = (4 * (2 * non_isolated_cap + window_words + 3 * cluster_cap) - rank_bytes(0)) / 10;
+  static constexpr unsigned key_tile = (2 * non_isolated_cap + window_words + 3 * cluster_cap) / 2;
 };
+static_assert(non_isolated_cap <= ClusterLds::window_words && non_isolated_cap <= 256, "sort keys");
+static_assert(sizeof(ClusterLds::work) >= rank_bytes(cluster_cap) && cluster_cap % 2 == 0, "ranking");
+static_assert(sizeof(Banks) <= 4 * ClusterLds::window_words && non_isolated_cap % 2 == 0, "banks");
+static_assert(offsetof(ClusterLds, xyz) == sizeof(ClusterLds::work), "the ranking reaches into xyz");
+} // namespace mp
 
 // (phi, id) as one unsigned 64-bit key: phi (signed) in the high word, offset to unsigned. Key
 // order is the sort's (phi, id) order (SortByPhi.cu:90-125), and distinct clusters of a module
@@ -1171,8 +1208,7 @@ __device__ __forceinline__ uint64_t phi_id_key(int16_t phi, uint32_t id)
   return (static_cast<uint64_t>(static_cast<uint16_t>(phi) ^ 0x8000u) << 32) | id;
 }
 
-// The number of keys[0 .. n) below `key` (n is wave-uniform: every lane reads the same key,
-// eight reads in flight at a time).
+// The number of keys[0 .. n) below `key` (eight reads in flight at a time).
 __device__ __forceinline__ unsigned keys_below(const uint64_t* keys, unsigned n, uint64_t key)
 {
   unsigned below = 0, j = 0;
@@ -1187,251 +1223,231 @@ __device__ __forceinline__ unsigned keys_below(const uint64_t* keys, unsigned n,
   return below;
 }
 
+struct ClusterArgs {
+  const char* raw;
+  const BankEntry* directory;
+  const uint32_t* directory_count;
+  const uint32_t* offsets_estimated_input_size;
+  const uint8_t* sp_flags;
+  const Geometry* geometry;
+  const uint8_t* sp_patterns;
+  const float* sp_fx;
+  const float* sp_fy;
+  uint32_t* module_cluster_num;
+  char* sorted_container;
+  char* unsorted_scratch;
+};
+
 // K3 + K4 of one module pair (idx = event * 26 + module pair) by one wave.
+//
+// Every word is read once. An isolated word becomes one or two seeds through the pattern table; the
+// non-isolated ones are kept, and sorted within their bank by (sensor, SP column, SP row) (v2/v3: the
+// bank is the sensor, bit 23 cleared), each with its candidate byte in bits 24-31. A candidate's
+// window then takes only the words of its bank and sensor in SP columns col - 3 .. col + 1, a run
+// found by binary search, instead of every word of the bank; OR-ing the window is order-free, so the
+// windows are the scan's. The candidates form one list and each lane grows one of them. The seeds of
+// all words are placed together, so that the transform and phi run with full lanes, and ranked by
+// (phi, id).
+//
+// Bound by VALU issue, and by the largest module pair where there are few events. 20 000 one-vertex
+// events: 806 us (1155 with a sort of all words, windows in registers, each cluster placed where it was
+// found and ranked against all others); 1000 pile-up events: 48 us (82); 8 of them: 14 us (27). Two
+// module pairs to a wave, which fills the lanes better, needs more LDS and lost more by the fewer
+// waves that then fit a CU: 1066 against 980 us.
 template<int version>
-__device__ __forceinline__ void cluster_item(
-  const char* raw,
-  const mp::DirFetch& dir,
-  unsigned idx,
-  unsigned total,
-  const uint32_t* offsets_estimated_input_size,
-  const uint8_t* sp_flags,
-  const Geometry& g,
-  const uint8_t* sp_patterns,
-  const float* sp_fx,
-  const float* sp_fy,
-  uint32_t* module_cluster_num,
-  char* sorted_container,
-  char* unsorted_scratch,
-  mp::Banks& B,
-  mp::SortedBanks& S,
-  const ClusterSlices& sl)
-{
-  constexpr bool v23 = (version == 2 || version == 3);
-  const unsigned start = offsets_estimated_input_size[idx];
-  const unsigned estimate = offsets_estimated_input_size[idx + 1] - start;
-  mp::load_banks(raw, dir, B);
-  const unsigned n_words = B.start[B.n];
-  const bool resident = n_words <= mp::word_cap;
-  const bool clusters_in_lds = estimate <= mp::cluster_cap;
-  uint32_t* lw = sl.lw;
-  const Clusters scratch {unsorted_scratch, total};
-  uint64_t* lkey = sl.lkey;
-  float* lxyz = sl.lxyz;
-  unsigned n = 0; // clusters so far (wave-uniform)
-  // Appends up to two clusters per lane in lane order (ranks from ballots).
-  auto emit = [&](unsigned k, const ClusterOut& c0, const ClusterOut& c1) {
+struct ClusterItem {
+  static constexpr bool v23 = (version == 2 || version == 3);
+  const ClusterArgs& a;
+  mp::ClusterLds& L;
+  const unsigned total, idx, start, estimate;
+  const bool in_lds;
+  unsigned n = 0; // clusters so far
+  static constexpr uint32_t none = 0xFFFFu; // ends a bucket's list
+
+  __device__ __forceinline__ ClusterItem(const ClusterArgs& args, mp::ClusterLds& lds, unsigned total_clusters, unsigned item) :
+    a(args), L(lds), total(total_clusters), idx(item), start(a.offsets_estimated_input_size[item]),
+    estimate(a.offsets_estimated_input_size[item + 1] - start), in_lds(estimate <= mp::cluster_cap)
+  {}
+
+  __device__ __forceinline__ void keep_seed(unsigned slot, const ClusterSeed& s)
+  {
+    if (slot >= estimate) return;
+    if (in_lds) {
+      float* at = L.xyz + 3 * slot;
+      at[0] = s.fx;
+      at[1] = s.fy;
+      at[2] = __uint_as_float(s.id);
+    }
+    else {
+      const Clusters scratch {a.unsorted_scratch, total};
+      const size_t at = start + slot;
+      scratch.ids()[at] = s.id;
+      scratch.xyz()[3 * at] = s.fx;
+      scratch.xyz()[3 * at + 1] = s.fy;
+    }
+  }
+
+  // Appends k (0, 1 or 2) seeds of each lane. The order in which they are appended does not reach the
+  // output: the clusters are ranked by their distinct (phi, id) keys.
+  __device__ __forceinline__ void emit(unsigned k, const ClusterSeed& s0, const ClusterSeed& s1)
+  {
     const uint64_t one = __ballot(k > 0), two = __ballot(k > 1);
-    const unsigned slot0 = n + rank_below(one) + rank_below(two);
-    for (unsigned j = 0; j < k; ++j) {
-      const unsigned slot = slot0 + j;
-      const ClusterOut& c = j == 0 ? c0 : c1;
-      if (slot < estimate) {
-        if (clusters_in_lds) {
-          lkey[slot] = phi_id_key(c.phi, c.id);
-          lxyz[3 * slot] = c.x;
-          lxyz[3 * slot + 1] = c.y;
-          lxyz[3 * slot + 2] = c.z;
-        }
-        else {
-          store_cluster(scratch, start + slot, c);
-        }
-      }
-    }
+    const unsigned slot = n + rank_below(one) + rank_below(two);
+    if (k > 0) keep_seed(slot, s0);
+    if (k > 1) keep_seed(slot + 1, s1);
     n += __popcll(one) + __popcll(two);
-  };
-  // The order in which clusters are appended does not reach the output: the module pair's
-  // clusters are ranked by their distinct (phi, id) keys below.
-  constexpr uint32_t field = v23 ? 0x7FFFu : 0xFFFFu;
-  if (resident) {
-    // Every bank's words sorted in the slice by (isolated, sensor, SP column, SP row, position)
-    // (v2/v3: the bank is the sensor, bit 23 cleared), each with its candidate byte in bits 24-31:
-    // a bank's non-isolated words first, then its isolated ones. A candidate's window then takes
-    // only the words of its bank and sensor in SP columns col - 3 .. col + 1, a contiguous run
-    // found by binary search, instead of every word of the bank; OR-ing the window is order-free,
-    // so the windows are the scan's. The cluster slices are still empty here and serve as the
-    // sort's scratch: keys in the xyz slice, sorted entries in the key slice, copied back over
-    // the words at the end.
-    static_assert(3 * mp::cluster_cap >= mp::word_cap && 2 * mp::cluster_cap >= mp::word_cap, "sort scratch");
-    uint32_t* keys = reinterpret_cast<uint32_t*>(lxyz);
-    uint32_t* sorted = reinterpret_cast<uint32_t*>(lkey);
-    // A word's key: isolated bit, bank (the same for all words it is compared with), then sensor,
-    // column and row, then its position, distinct for distinct words. The words and their candidate
-    // bytes are read together, so the sort waits for memory once.
-    static_assert(mp::word_cap <= 512 && max_banks_per_mp == 8, "sort key fields");
+  }
+
+  // The module pair's seeds with its non-isolated words in the slice. False, with nothing written but
+  // scratch, if they don't fit.
+  __device__ __forceinline__ bool seeds(const mp::DirFetch& f)
+  {
+    constexpr uint32_t field = v23 ? 0x7FFFu : 0xFFFFu;
+    const unsigned l = lane_id();
+    const unsigned inc = wave_inclusive_scan(l < f.nb ? f.en.n_sp : 0u);
+    const unsigned first = l < f.nb ? inc - f.en.n_sp : inc; // words before this lane's bank
+    const unsigned n_words = __builtin_amdgcn_readlane(inc, max_banks_per_mp - 1);
+    if (l < f.nb) L.bank[l] = make_uint2(f.en.word_offset - first, f.en.source);
     mp::wave_sync_lds();
-    uint32_t bank_nonisolated = 0; // lane k counts bank k's non-isolated words
+    const uint32_t* raw_words = reinterpret_cast<const uint32_t*>(a.raw);
+    uint32_t* words = L.words();
+    uint32_t* sorted = L.sorted();
+    uint32_t* keys = L.keys();
+    unsigned n_non = 0, non_before = 0; // non_before: those before this lane's bank
     for (unsigned base = 0; base < n_words; base += wave_size) {
-      const unsigned w = base + lane_id();
-      uint32_t word = 0x80000000u;
-      if (w < n_words) {
-        const unsigned bi = mp::bank_of(B, w);
-        const unsigned at = B.word_offset[bi] + (w - B.start[bi]);
-        word = B.base[at];
-        const uint32_t f = sp_flags[at]; // written for non-isolated words
-        keys[w] = (word & 0x80000000u) | (bi << 26) | (((word >> 8) & field) << 9) | w;
-        lw[w] = (word & (v23 ? 0x007FFFFFu : 0x00FFFFFFu)) | (word & 0x80000000u ? 0u : f << 24);
+      const unsigned w = base + l;
+      // The number of the bank holding word w: the banks after the first that start at or before it.
+      unsigned bi = 0;
+      for (unsigned j = 1; j < f.nb; ++j) bi += w >= static_cast<unsigned>(__builtin_amdgcn_readlane(first, j));
+      const uint2 bank = L.bank[bi];
+      const bool active = w < n_words;
+      uint32_t word = 0, flags = 0;
+      if (active) {
+        word = raw_words[bank.x + w];
+        flags = a.sp_flags[bank.x + w]; // written for non-isolated words
       }
-      const uint64_t m = __ballot(!(word & 0x80000000u));
-      const unsigned l = lane_id();
-      if (l < B.n) {
-        auto below = [](unsigned x) { return x >= wave_size ? ~0ull : ((1ull << x) - 1); };
-        const unsigned lo = B.start[l] <= base ? 0u : min(B.start[l] - base, wave_size);
-        const unsigned hi = B.start[l + 1] <= base ? 0u : min(B.start[l + 1] - base, wave_size);
-        bank_nonisolated += __popcll(m & below(hi)) - __popcll(m & below(lo));
+      const bool isolated = active && (word & 0x80000000u), non = active && !isolated;
+      ClusterSeed s0, s1;
+      unsigned n_seeds = 0;
+      if (isolated) n_seeds = isolated_sp_clusters<version>(a.sp_patterns, a.sp_fx, a.sp_fy, bank.y, word, s0, s1);
+      emit(n_seeds, s0, s1);
+      const uint64_t nons = __ballot(non);
+      const unsigned slot = n_non + rank_below(nons);
+      const unsigned to_bank = first > base ? min(first - base, wave_size) : 0u;
+      non_before += __popcll(nons & (to_bank >= wave_size ? ~0ull : (1ull << to_bank) - 1));
+      n_non += __popcll(nons);
+      if (n_non > mp::non_isolated_cap) return false;
+      if (non) {
+        // Distinct for distinct words: bank, sensor, column and row, then the slot.
+        keys[slot] = (bi << 24) | (((word >> 8) & field) << 8) | slot;
+        words[slot] = (word & (v23 ? 0x007FFFFFu : 0x00FFFFFFu)) | (flags << 24);
       }
     }
-    {
-      const unsigned l = lane_id();
-      const uint32_t cnt = l < B.n ? bank_nonisolated : 0u;
-      const uint32_t inc = wave_inclusive_scan(cnt);
-      if (l <= B.n) {
-        S.sorted[l] = inc - cnt;
-        S.isolated_before[l] = B.start[l] - (inc - cnt);
-      }
-      if (l < B.n) S.first_isolated[l] = B.start[l] + cnt;
-    }
-    mp::wave_sync_lds(); // keys and counts written
-    for (unsigned base = 0; base < n_words; base += wave_size) {
-      const unsigned w = base + lane_id();
-      if (w < n_words) {
-        const uint32_t key = keys[w];
-        const unsigned bi = (key >> 26) & (max_banks_per_mp - 1);
-        const unsigned a = B.start[bi], b = B.start[bi + 1];
-        unsigned rank = 0, k = a;
-        for (; k + 4 <= b; k += 4) {
+    if (l < f.nb) L.non_start[l] = non_before;
+    if (l == f.nb) L.non_start[l] = n_non;
+    mp::wave_sync_lds(); // keys and words written
+    // Ranks within the bank; the candidates of the sorted words, as (word, bank, which). The list
+    // takes the place of the words: 64 (r + 1) of these have been read after round r, and the list
+    // holds at most 128 (r + 1) entries of half a word.
+    uint16_t* candidates = reinterpret_cast<uint16_t*>(words);
+    unsigned n_cand = 0;
+    for (unsigned base = 0; base < n_non; base += wave_size) {
+      const unsigned slot = base + l;
+      unsigned at = 0;
+      uint32_t word = 0;
+      if (slot < n_non) {
+        const uint32_t key = keys[slot];
+        word = words[slot];
+        const unsigned bi = key >> 24;
+        const unsigned from = L.non_start[bi], to = L.non_start[bi + 1];
+        unsigned rank = 0, j = from;
+        for (; j + 4 <= to; j += 4) {
           uint32_t v[4];
 #pragma unroll
-          for (unsigned u = 0; u < 4; ++u) v[u] = keys[k + u];
+          for (unsigned u = 0; u < 4; ++u) v[u] = keys[j + u];
 #pragma unroll
           for (unsigned u = 0; u < 4; ++u) rank += v[u] < key ? 1u : 0u;
         }
-        for (; k < b; ++k) rank += keys[k] < key ? 1u : 0u;
-        sorted[a + rank] = lw[w];
+        for (; j < to; ++j) rank += keys[j] < key ? 1u : 0u;
+        at = (from + rank) | (bi << 8);
+        sorted[from + rank] = word;
       }
+      const uint64_t firsts = __ballot(word & (1u << 24)), seconds = __ballot(word & (2u << 24));
+      unsigned c = n_cand + rank_below(firsts) + rank_below(seconds);
+      n_cand += __popcll(firsts) + __popcll(seconds);
+      mp::wave_sync_lds(); // this round's words have been read
+      if (word & (1u << 24)) candidates[c++] = static_cast<uint16_t>(at);
+      if (word & (2u << 24)) candidates[c] = static_cast<uint16_t>(at | 0x1000u);
     }
-    mp::wave_sync_lds(); // every entry written
-    for (unsigned w = lane_id(); w < n_words; w += wave_size) lw[w] = sorted[w];
-    mp::wave_sync_lds(); // the cluster slices are free again
-  }
-  // Isolated SPs. Resident: the isolated tails of the sorted banks, one after another, so every
-  // lane of a round takes an isolated word (positions in the same order as a walk over all words
-  // would visit them). Otherwise every word, in place, by its isolated bit.
-  if (resident) {
-    const unsigned n_isolated = S.isolated_before[B.n];
-    for (unsigned base = 0; base < n_isolated; base += wave_size) {
-      const unsigned t = base + lane_id();
-      ClusterOut c0, c1;
-      unsigned k = 0;
-      if (t < n_isolated) {
-        const unsigned bi = mp::bank_at(S.isolated_before, B.n, t);
-        const uint32_t sp_word = lw[S.first_isolated[bi] + (t - S.isolated_before[bi])];
-        RawBank bank;
-        bank.sourceID = B.source[bi];
-        k = isolated_sp_clusters<version>(g, sp_patterns, sp_fx, sp_fy, bank, sp_word, c0, c1);
-      }
-      emit(k, c0, c1);
-    }
-  }
-  else {
-    for (unsigned base = 0; base < n_words; base += wave_size) {
-      const unsigned w = base + lane_id();
-      ClusterOut c0, c1;
-      unsigned k = 0;
-      if (w < n_words) {
-        const unsigned bi = mp::bank_of(B, w);
-        const uint32_t sp_word = B.word(bi)[w - B.start[bi]];
-        if (sp_word & 0x80000000u) {
-          RawBank bank;
-          bank.sourceID = B.source[bi];
-          k = isolated_sp_clusters<version>(g, sp_patterns, sp_fx, sp_fy, bank, sp_word, c0, c1);
-        }
-      }
-      emit(k, c0, c1);
-    }
-  }
-  // The candidates of one round of (at most 64) SPs: their pixels as one list, an SP's first
-  // pixel before its second; each lane grows one of them with its SP's window and word fetched
-  // from the SP's lane, and the kept clusters are appended in list order. A round has at most 128
-  // candidates.
-  auto candidates_round = [&](uint32_t sp_word, uint32_t sensor_number, uint32_t f, const Window& win) {
-    const uint64_t firsts = __ballot(f & 1u), seconds = __ballot(f & 2u);
-    const unsigned n_cand = __popcll(firsts) + __popcll(seconds);
-    const unsigned first = rank_below(firsts) + rank_below(seconds);
-    mp::wave_sync_lds(); // the previous round's list has been read
-    if (f & 1u) sl.lcand[first] = static_cast<uint8_t>(lane_id());
-    if (f & 2u) sl.lcand[first + (f & 1u)] = static_cast<uint8_t>(lane_id() | 0x80u);
-    mp::wave_sync_lds();
-    for (unsigned c0 = 0; c0 < n_cand; c0 += wave_size) {
-      const unsigned j = c0 + lane_id();
-      const unsigned e = j < n_cand ? sl.lcand[j] : 0u;
-      const int src = static_cast<int>(e & 0x3Fu);
-      Window ws;
-      ws.pa0 = __shfl(win.pa0, src, wave_size);
-      ws.pa1 = __shfl(win.pa1, src, wave_size);
-      ws.pa2 = __shfl(win.pa2, src, wave_size);
-      ws.pa3 = __shfl(win.pa3, src, wave_size);
-      ws.pa4 = __shfl(win.pa4, src, wave_size);
-      const uint32_t word_s = __shfl(sp_word, src, wave_size);
-      const uint32_t sensor_s = __shfl(sensor_number, src, wave_size);
-      const uint32_t f_s = __shfl(f, src, wave_size);
-      const uint32_t location = (e & 0x80u) ? (f_s >> 5) & 7u : (f_s >> 2) & 7u;
-      ClusterOut c, unused;
-      const bool keep = j < n_cand && masked_cluster_final(g, word_s, sensor_s, location, ws, &c);
-      emit(keep ? 1u : 0u, c, unused);
-    }
-  };
-  if (resident) {
-    // The non-isolated words, bank after bank: word t of the list is position
-    // start[bank] + t - sorted[bank] of the slice.
-    const unsigned n_sorted = S.sorted[B.n];
-    for (unsigned base = 0; base < n_sorted; base += wave_size) {
-      const unsigned t = base + lane_id();
-      const bool active = t < n_sorted;
-      const unsigned bi = active ? mp::bank_at(S.sorted, B.n, t) : 0u;
-      const unsigned j = B.start[bi] + (t - S.sorted[bi]);
-      const uint32_t e = active ? lw[j] : 0u;
-      const uint32_t f = e >> 24;
-      const uint32_t sp_word = e & 0x00FFFFFFu;
-      const uint32_t pair = B.source[bi] & 0x1FFu;
-      const uint32_t sensor_number = v23 ? pair : ((pair << 1) | ((sp_word >> 23) & 0x1u));
-      Window win {0, 0, 0, 0, 0};
-      if (f & 3u) {
-        const uint32_t key = (e >> 8) & 0xFFFFu;
+    mp::wave_sync_lds(); // the list and the sorted words written; the keys are free
+    uint32_t* window = keys + l; // SP column c of this lane's window at [64 c]
+    for (unsigned base = 0; base < n_cand; base += wave_size) {
+      bool keep = false;
+      ClusterSeed s, unused;
+      if (base + l < n_cand) {
+        const unsigned e = candidates[base + l];
+        const unsigned bi = (e >> 8) & 7u, at = e & 255u;
+        const uint32_t word = sorted[at];
+        const unsigned end = L.non_start[bi + 1];
+        unsigned lo = L.non_start[bi], hi = at;
+        const uint32_t pair = L.bank[bi].y & 0x1FFu;
+#pragma unroll
+        for (unsigned c = 0; c < 5; ++c) window[wave_size * c] = 0;
+        const uint32_t key = (word >> 8) & 0xFFFFu;
         const uint32_t sensor = key & 0x8000u;
         const uint32_t col = (key >> 6) & 0x1FFu;
         const uint32_t lower = sensor | ((max(col, 3u) - 3u) << 6);
         const uint32_t upper = sensor + min((col + 2u) << 6, 0x8000u);
-        unsigned lo = B.start[bi], hi = S.first_isolated[bi];
-        const unsigned end = hi;
-        while (lo < hi) {
+        while (lo < hi) { // the first word at or above `lower`; the candidate's own is
           const unsigned mid = (lo + hi) >> 1;
-          if (((lw[mid] >> 8) & 0xFFFFu) < lower) lo = mid + 1;
+          if (((sorted[mid] >> 8) & 0xFFFFu) < lower) lo = mid + 1;
           else hi = mid;
         }
-        const int32_t row_lower = static_cast<int32_t>(key & 0x3Fu) - 2;
-        const int32_t col_lower = static_cast<int32_t>(col) - 3;
-        for (unsigned k = lo; k < end; ++k) {
-          const uint32_t o = lw[k];
-          if (((o >> 8) & 0xFFFFu) >= upper) break;
-          window_acc_same_sensor(row_lower, col_lower, o, win);
+        const uint32_t row_lower = (key & 0x3Fu) - 2u, col_lower = (key >> 6) - 3u;
+        for (unsigned j = lo; j < end; ++j) {
+          const uint32_t o = sorted[j];
+          const uint32_t address = (o >> 8) & 0xFFFFu;
+          if (address >= upper) break;
+          const uint32_t row = (address & 0x3Fu) - row_lower;
+          // Four rows of two pixel columns, 16 bits apart, into the word's SP column: an LDS OR each
+          // costs the VALU half of what selecting one of five registers does.
+          if (row < 4u)
+            atomicOr(window + wave_size * ((address >> 6) - col_lower),
+                     ((o & 0x0Fu) | ((o & 0xF0u) << 12)) << (4 * row));
         }
+        const Window win {window[0], window[wave_size], window[2 * wave_size], window[3 * wave_size], window[4 * wave_size]};
+        keep = masked_cluster_final(word & 0x00FFFFFFu, v23 ? pair : ((pair << 1) | (sensor >> 15)),
+                                    (e & 0x1000u) ? word >> 29 : (word >> 26) & 7u, win, &s);
       }
-      candidates_round(sp_word, sensor_number, f, win);
+      emit(keep ? 1u : 0u, s, unused);
     }
+    return true;
   }
-  else {
-    // Larger module pairs: every candidate scans its bank, tile by tile through the slice.
+
+  // The seeds of a module pair with too many words for the slice: every word in place by its
+  // isolated bit, and every SP with candidates scans its bank, tile by tile through the slice.
+  __device__ __forceinline__ void seeds_in_tiles(const mp::DirFetch& f)
+  {
+    n = 0;
+    mp::Banks& B = L.banks();
+    mp::wave_sync_lds();
+    mp::load_banks(a.raw, f, B);
+    const unsigned n_words = B.start[B.n];
     for (unsigned base = 0; base < n_words; base += wave_size) {
       const unsigned w = base + lane_id();
       const bool active = w < n_words;
       const unsigned bi = active ? mp::bank_of(B, w) : 0;
-      const uint32_t sp_word = active ? B.word(bi)[w - B.start[bi]] : 0x80000000u;
-      uint32_t f = 0;
-      if (active && !(sp_word & 0x80000000u)) {
-        const uint32_t* wp = B.word(bi) + (w - B.start[bi]);
-        f = sp_flags[static_cast<size_t>(reinterpret_cast<const char*>(wp) - raw) / 4];
+      const size_t at = active ? B.word_offset[bi] + (w - B.start[bi]) : 0;
+      const uint32_t sp_word = active ? B.base[at] : 0x80000000u;
+      uint32_t flags = 0;
+      ClusterSeed s0, s1;
+      unsigned k = 0;
+      if (active) {
+        if (sp_word & 0x80000000u)
+          k = isolated_sp_clusters<version>(a.sp_patterns, a.sp_fx, a.sp_fy, B.source[bi], sp_word, s0, s1);
+        else flags = a.sp_flags[at];
       }
+      emit(k, s0, s1);
       const uint32_t pair = B.source[bi] & 0x1FFu;
       const uint32_t sensor_number = v23 ? pair : ((pair << 1) | ((sp_word >> 23) & 0x1u));
       const uint32_t sp_addr = (sp_word & 0x007FFF00u) >> 8;
@@ -1439,106 +1455,162 @@ __device__ __forceinline__ void cluster_item(
       const int32_t sp_col_lower = static_cast<int32_t>(sp_addr >> 6) - 3;
       Window win {0, 0, 0, 0, 0};
       // Both candidates of an SP share its window.
-      mp::for_words(B, n_words, resident, lw, (f & 3) != 0, B.start[bi], B.start[bi + 1], [&](uint32_t other) {
-        window_acc<version>(sp_row_lower, sp_col_lower, sensor_number, other, win);
-      });
-      candidates_round(sp_word, sensor_number, f, win);
-    }
-  }
-  n = min(n, estimate);
-  mp::wave_sync_lds();
-  if (lane_id() == 0) module_cluster_num[idx] = n;
-  const Clusters out {sorted_container, total};
-  if (clusters_in_lds) {
-    for (unsigned i = lane_id(); i < n; i += wave_size) {
-      const uint64_t key = lkey[i];
-      ClusterOut c;
-      c.id = static_cast<uint32_t>(key);
-      c.phi = static_cast<int16_t>(static_cast<uint16_t>(key >> 32) ^ 0x8000u);
-      c.x = lxyz[3 * i];
-      c.y = lxyz[3 * i + 1];
-      c.z = lxyz[3 * i + 2];
-      const unsigned rank = keys_below(lkey, n, key);
-      store_cluster(out, start + rank, c);
-    }
-    return;
-  }
-  // Too many clusters for the slice: they sit in the scratch container; rank them against
-  // tiles of (phi, id) staged through the slice.
-  __threadfence_block();
-  for (unsigned i0 = 0; i0 < n; i0 += wave_size) {
-    const unsigned i = i0 + lane_id();
-    const bool mine = i < n;
-    ClusterOut c;
-    if (mine) {
-      c.id = scratch.ids()[start + i];
-      c.phi = scratch.phis()[start + i];
-      c.x = scratch.xyz()[3 * (size_t)(start + i)];
-      c.y = scratch.xyz()[3 * (size_t)(start + i) + 1];
-      c.z = scratch.xyz()[3 * (size_t)(start + i) + 2];
-    }
-    unsigned rank = 0;
-    for (unsigned t0 = 0; t0 < n; t0 += mp::cluster_cap) {
-      const unsigned tn = min(mp::cluster_cap, n - t0);
-      mp::wave_sync_lds();
-      for (unsigned j = lane_id(); j < tn; j += wave_size)
-        lkey[j] = phi_id_key(scratch.phis()[start + t0 + j], scratch.ids()[start + t0 + j]);
-      mp::wave_sync_lds();
-      if (mine) {
-        const uint64_t key = phi_id_key(c.phi, c.id);
-        rank += keys_below(lkey, tn, key);
+      mp::for_words(B, n_words, L.words(), mp::ClusterLds::tile, (flags & 3) != 0, B.start[bi], B.start[bi + 1],
+                    [&](uint32_t other) { window_acc<version>(sp_row_lower, sp_col_lower, sensor_number, other, win); });
+#pragma nounroll
+      for (unsigned which = 0; which < 2; ++which) {
+        const bool candidate = (flags >> which) & 1u;
+        const bool keep = candidate && masked_cluster_final(
+                                         sp_word & 0x00FFFFFFu, sensor_number, (flags >> (2 + 3 * which)) & 7u, win, &s0);
+        emit(keep ? 1u : 0u, s0, s1);
       }
     }
-    if (mine) store_cluster(out, start + rank, c);
   }
+
+  // Places the seeds and writes them in the order of their keys.
+  __device__ __forceinline__ void finish()
+  {
+    const Clusters out {a.sorted_container, total};
+    n = min(n, estimate);
+    if (lane_id() == 0) a.module_cluster_num[idx] = n;
+    mp::wave_sync_lds(); // seeds written, windows read
+    if (n <= mp::ClusterLds::rank_cap) {
+      // 64 buckets of phi: a cluster's rank is the number of clusters in the buckets before its own and
+      // of those in its own with a smaller key, which it finds by their list. Against every key it
+      // would be n comparisons of 64 bits: 228 clusters took 13 us, four rounds over all keys.
+      const unsigned l = lane_id();
+      const unsigned cap = in_lds ? mp::cluster_cap : mp::ClusterLds::rank_cap;
+      uint32_t* newest = L.words();
+      uint32_t* counts = newest + wave_size;
+      uint64_t* keys = L.work + wave_size;
+      uint16_t* next = reinterpret_cast<uint16_t*>(keys + cap);
+      const Clusters scratch {a.unsorted_scratch, total};
+      newest[l] = none;
+      counts[l] = 0;
+      if (!in_lds) __threadfence_block();
+      mp::wave_sync_lds();
+      for (unsigned i = l; i < n; i += wave_size) {
+        float* at = in_lds ? L.xyz + 3 * i : nullptr;
+        ClusterSeed s;
+        if (in_lds) s = ClusterSeed {__float_as_uint(at[2]), at[0], at[1]};
+        else s = ClusterSeed {scratch.ids()[start + i], scratch.xyz()[3 * (size_t)(start + i)], scratch.xyz()[3 * (size_t)(start + i) + 1]};
+        const ClusterOut c = place_cluster(*a.geometry, seed_sensor<version>(s), s);
+        const uint64_t key = phi_id_key(c.phi, c.id);
+        const unsigned bucket = static_cast<unsigned>(key >> 42);
+        keys[i] = key;
+        atomicAdd(counts + bucket, 1u);
+        next[i] = static_cast<uint16_t>(atomicExch(newest + bucket, i));
+        if (in_lds) {
+          at[0] = c.x;
+          at[1] = c.y;
+          at[2] = c.z;
+        }
+        else store_cluster(scratch, start + i, c);
+      }
+      if (!in_lds) __threadfence_block();
+      mp::wave_sync_lds();
+      const unsigned count = counts[l], before = wave_inclusive_scan(count) - count;
+      mp::wave_sync_lds();
+      counts[l] = before;
+      mp::wave_sync_lds();
+      for (unsigned i = l; i < n; i += wave_size) {
+        const uint64_t key = keys[i];
+        const unsigned bucket = static_cast<unsigned>(key >> 42);
+        unsigned rank = counts[bucket];
+        for (unsigned j = newest[bucket]; j != none;) {
+          const uint64_t other = keys[j];
+          j = next[j];
+          rank += other < key;
+        }
+        ClusterOut c;
+        c.id = static_cast<uint32_t>(key);
+        c.phi = static_cast<int16_t>(static_cast<uint16_t>(key >> 32) ^ 0x8000u);
+        if (in_lds) {
+          c.x = L.xyz[3 * i];
+          c.y = L.xyz[3 * i + 1];
+          c.z = L.xyz[3 * i + 2];
+        }
+        else {
+          const float* at = scratch.xyz() + 3 * (size_t)(start + i);
+          c.x = at[0];
+          c.y = at[1];
+          c.z = at[2];
+        }
+        store_cluster(out, start + rank, c);
+      }
+      return;
+    }
+    // Too many clusters for that: they sit in the scratch container; rank them against
+    // tiles of (phi, id) staged through the slice.
+    uint64_t* keys = L.work;
+    const Clusters scratch {a.unsorted_scratch, total};
+    __threadfence_block();
+    for (unsigned i = lane_id(); i < n; i += wave_size) {
+      const size_t at = start + i;
+      const ClusterSeed s {scratch.ids()[at], scratch.xyz()[3 * at], scratch.xyz()[3 * at + 1]};
+      store_cluster(scratch, start + i, place_cluster(*a.geometry, seed_sensor<version>(s), s));
+    }
+    __threadfence_block();
+    unsigned tile = ~0u; // the one whose keys are in the slice
+    for (unsigned i0 = 0; i0 < n; i0 += wave_size) {
+      const unsigned i = i0 + lane_id();
+      const bool mine = i < n;
+      ClusterOut c;
+      if (mine) {
+        c.id = scratch.ids()[start + i];
+        c.phi = scratch.phis()[start + i];
+        c.x = scratch.xyz()[3 * (size_t)(start + i)];
+        c.y = scratch.xyz()[3 * (size_t)(start + i) + 1];
+        c.z = scratch.xyz()[3 * (size_t)(start + i) + 2];
+      }
+      unsigned rank = 0;
+      for (unsigned t0 = 0; t0 < n; t0 += mp::ClusterLds::key_tile) {
+        const unsigned tn = min(mp::ClusterLds::key_tile, n - t0);
+        if (t0 != tile) {
+          mp::wave_sync_lds();
+          for (unsigned j = lane_id(); j < tn; j += wave_size)
+            keys[j] = phi_id_key(scratch.phis()[start + t0 + j], scratch.ids()[start + t0 + j]);
+          mp::wave_sync_lds();
+          tile = t0;
+        }
+        if (mine) rank += keys_below(keys, tn, phi_id_key(c.phi, c.id));
+      }
+      if (mine) store_cluster(out, start + rank, c);
+    }
+  }
+};
+
+template<int version>
+__device__ __forceinline__ void
+cluster_item(const ClusterArgs& a, mp::ClusterLds& L, unsigned total, unsigned idx, const mp::DirFetch& f)
+{
+  ClusterItem<version> item(a, L, total, idx);
+  if (!item.seeds(f)) item.seeds_in_tiles(f);
+  item.finish();
 }
 
-// One wave per item (loop = false, the default), or a resident grid (loop = true) whose waves
+// One wave per module pair (loop = false, the default), or a resident grid (loop = true) whose waves
 // take items idx, idx + stride, ... and fetch the next item's bank directory record before
-// working on the current one. Six workgroups per CU (80 VGPRs, no spills for one wave per item:
-// the sort stages its keys and entries in the cluster slices rather than in registers).
+// working on the current one.
 template<int version, bool loop>
-__global__ void __launch_bounds__(mp::waves_per_block* wave_size, 6) k_cluster_mp(
-  const char* raw,
-  const BankEntry* directory,
-  const uint32_t* directory_count,
-  unsigned n_events,
-  const uint32_t* offsets_estimated_input_size,
-  const uint8_t* sp_flags,
-  const Geometry* geometry,
-  const uint8_t* sp_patterns,
-  const float* sp_fx,
-  const float* sp_fy,
-  uint32_t* module_cluster_num,
-  char* sorted_container,
-  char* unsorted_scratch)
+__global__ void __launch_bounds__(mp::waves_per_block* wave_size, 6) k_cluster_mp(ClusterArgs a, unsigned n_events)
 {
-  __shared__ uint32_t s_words[mp::waves_per_block][mp::word_cap];
-  __shared__ uint64_t s_key[mp::waves_per_block][mp::cluster_cap];
-  __shared__ float s_xyz[mp::waves_per_block][3 * mp::cluster_cap];
-  __shared__ uint8_t s_cand[mp::waves_per_block][2 * wave_size];
-  __shared__ mp::Banks s_banks[mp::waves_per_block];
-  __shared__ mp::SortedBanks s_sorted[mp::waves_per_block];
+  __shared__ mp::ClusterLds s_lds[mp::waves_per_block];
   const unsigned wave = threadIdx.x / wave_size;
   const unsigned n_items = n_events * n_module_pairs;
   const unsigned stride = gridDim.x * mp::waves_per_block;
   unsigned idx = blockIdx.x * mp::waves_per_block + wave;
   if (idx >= n_items) return;
-  const unsigned total = offsets_estimated_input_size[n_items];
-  const ClusterSlices sl {s_words[wave], s_key[wave], s_xyz[wave], s_cand[wave]};
+  const unsigned total = a.offsets_estimated_input_size[n_items];
+  mp::DirFetch cur = mp::fetch_dir(a.directory, a.directory_count, idx);
   if constexpr (!loop) {
-    cluster_item<version>(
-      raw, mp::fetch_dir(directory, directory_count, idx), idx, total, offsets_estimated_input_size, sp_flags,
-      *geometry, sp_patterns, sp_fx, sp_fy, module_cluster_num, sorted_container, unsorted_scratch, s_banks[wave], s_sorted[wave], sl);
+    cluster_item<version>(a, s_lds[wave], total, idx, cur);
     return;
   }
-  mp::DirFetch cur = mp::fetch_dir(directory, directory_count, idx);
   for (; idx < n_items; idx += stride) {
     mp::DirFetch next = cur;
-    if (idx + stride < n_items) next = mp::fetch_dir(directory, directory_count, idx + stride);
-    cluster_item<version>(
-      raw, cur, idx, total, offsets_estimated_input_size, sp_flags, *geometry, sp_patterns, sp_fx, sp_fy,
-      module_cluster_num, sorted_container, unsorted_scratch, s_banks[wave], s_sorted[wave], sl);
+    if (idx + stride < n_items) next = mp::fetch_dir(a.directory, a.directory_count, idx + stride);
+    cluster_item<version>(a, s_lds[wave], total, idx, cur);
     cur = next;
   }
 }
@@ -1584,20 +1656,18 @@ hipError_t launch_cluster_mp(const ClusterMpLaunch& a, hipStream_t s)
                      : v == 3 ? reinterpret_cast<const void*>(&k_cluster_mp<3, true>)
                               : reinterpret_cast<const void*>(&k_cluster_mp<4, true>);
   const unsigned grid = mp_grid(kernel, a.n_events * n_module_pairs, a.resident_grid);
+  const ClusterArgs args {a.raw, static_cast<const BankEntry*>(a.directory), a.directory_count,
+                          a.offsets_estimated_input_size, a.sp_flags, reinterpret_cast<const Geometry*>(a.geometry),
+                          a.sp_patterns, a.sp_fx, a.sp_fy, a.module_cluster_num, a.sorted_container, a.unsorted_scratch};
 #define VELO_LAUNCH_CMP(V, L)                                                                                       \
-  hipLaunchKernelGGL(                                                                                               \
-    (k_cluster_mp<V, L>), dim3(grid), dim3(mp::waves_per_block * wave_size), 0, s, a.raw,                            \
-    static_cast<const BankEntry*>(a.directory), a.directory_count, a.n_events, a.offsets_estimated_input_size, a.sp_flags, reinterpret_cast<const Geometry*>(a.geometry),           \
-    a.sp_patterns, a.sp_fx, a.sp_fy, a.module_cluster_num, a.sorted_container, a.unsorted_scratch)
-  switch (a.version * 2 + (a.resident_grid ? 1 : 0)) {
+  hipLaunchKernelGGL((k_cluster_mp<V, L>), dim3(grid), dim3(mp::waves_per_block * wave_size), 0, s, args, a.n_events)
+  switch (v * 2 + (a.resident_grid ? 1 : 0)) {
   case 4: VELO_LAUNCH_CMP(2, false); break;
   case 5: VELO_LAUNCH_CMP(2, true); break;
   case 6: VELO_LAUNCH_CMP(3, false); break;
   case 7: VELO_LAUNCH_CMP(3, true); break;
-  default:
-    if (a.resident_grid) VELO_LAUNCH_CMP(4, true);
-    else VELO_LAUNCH_CMP(4, false);
-    break;
+  case 8: VELO_LAUNCH_CMP(4, false); break;
+  default: VELO_LAUNCH_CMP(4, true); break;
   }
 #undef VELO_LAUNCH_CMP
   return hipGetLastError();

@@ -339,6 +339,21 @@ def test_dense_module_pairs_take_the_tiled_paths(geometry, beamline, constants):
         assert not errs, "\n".join(errs[:20])
 
 
+@pytest.mark.parametrize("fused", [True, False], ids=["fused", "per_algorithm"])
+@pytest.mark.parametrize("version", [2, 4])
+@pytest.mark.parametrize("nu,lowest", [(16.0, 193), (30.0, 440), (45.0, 513)])
+def test_module_pairs_at_the_limits_of_the_clustering_slices(nu, lowest, version, fused, geometry, beamline, constants):
+    """Module pairs on both sides of each limit of the per-wave slices (192 clusters placed there, 256
+    non-isolated words, 512 clusters ranked there) and, per algorithm, banks of more than 64 words:
+    integers and bytes equal the oracle's."""
+    ev = synth.generate(n_events=3, pileup=1, nu=nu, shuffle_sp=1, bank_version=version, seed=41)
+    ref, gpu, status = run_both(f"slices_nu{nu}_v{version}", geometry, beamline, constants, fused, events=ev)
+    assert int(ref["status"][0]) == 0 and status & velo.STATUS_OVERFLOW_MASK == 0
+    assert np.diff(ref["offsets_estimated_input_size"].astype(np.int64)).max() >= lowest
+    errs = parity.compare(gpu, ref, fused)
+    assert not errs, "\n".join(errs[:20])
+
+
 def test_prefix_sum_iota(constants):
     """The reference's own prefix-sum test shape (TestPrefixSum.cu:9-33): iota 1..1000."""
     import torch
