@@ -1049,8 +1049,10 @@ __device__ __forceinline__ void estimate_item(
       *reinterpret_cast<uint4*>(L.table + h) = make_uint4(mp::hash_empty, mp::hash_empty, mp::hash_empty, mp::hash_empty);
   mp::wave_sync_lds();
   if (scan || table) {
-    for (unsigned w = l; w < n_words; w += wave_size) {
-      const unsigned bi = bank_of(w);
+    for (unsigned base = 0; base < n_words; base += wave_size) {
+      const unsigned w = base + l;
+      const unsigned bi = bank_of(w); // by the whole wave: it reads other lanes' registers
+      if (w >= n_words) continue;
       const uint32_t word = raw_words[L.bank[bi].x + w];
       if (w < mp::EstimateLds::word_cap) L.words[w] = word;
       if (scan) continue;

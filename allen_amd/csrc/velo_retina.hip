@@ -7,9 +7,9 @@
 //                           sensor pair (v4) slot, and (first event of the list) the bank of
 //                           each slot
 //   k_retina_decode         one wave per (event, module pair): decodes the module pair's words,
-//                           ranks them by their 64-bit key in LDS and writes every cluster at
-//                           its rank: the reference's sorting-key, permutation and sorted-decode
-//                           kernels in one pass, with no atomics
+//                           ranks them by their 64-bit key in LDS (64 buckets of phi) and writes
+//                           every cluster at its rank: the reference's sorting-key, permutation and
+//                           sorted-decode kernels in one pass
 //
 // Where several words share a key (zero padding words, or identical clusters) they share a rank
 // and the slot keeps the last of them in word order, which is what the reference's CPU target
@@ -21,8 +21,24 @@ namespace velo {
 
 namespace retina {
 constexpr unsigned bank_type = 73; // LHCb::RawBank::VPRetinaCluster (mdf/lhcb/Event/RawBank.h:134)
-constexpr unsigned waves_per_block = 4;
+constexpr unsigned waves_per_block = 2; // a finished wave keeps its LDS until its workgroup ends
 constexpr unsigned key_cap = 512;  // keys of a module pair held in the wave's LDS slice
+constexpr unsigned max_slots_per_mp = 8;
+
+// What one wave holds in LDS: 6 KB.
+struct Slice {
+  int64_t key[key_cap];
+  uint32_t newest[wave_size]; // of each phi bucket's words
+  uint32_t before[wave_size]; // words of the buckets before each
+  uint16_t next[key_cap];     // each word's successor in its bucket
+  const uint32_t* word[max_slots_per_mp]; // the slots' banks
+  uint32_t n_words[max_slots_per_mp], source[max_slots_per_mp];
+};
+constexpr uint32_t none = 0xFFFFu; // ends a bucket's list
+static_assert(key_cap < none, "list ends");
+
+// The bucket of a key: its top six bits, in key order.
+__device__ __forceinline__ unsigned bucket_of(int64_t key) { return static_cast<unsigned>(key >> 58) + 32u; }
 
 template<int version>
 constexpr unsigned slots()
@@ -50,13 +66,13 @@ struct Decoded {
 // the fraction flags, the global position and phi; the key is (phi as u16) << 48 | id, or the
 // largest key for a zero word.
 template<int version>
-__device__ __forceinline__ Decoded decode(const Geometry& g, const RawBank& bank, uint32_t word)
+__device__ __forceinline__ Decoded decode(const Geometry& g, uint32_t source, uint32_t word)
 {
   Decoded d;
   unsigned sensor;
-  if constexpr (version == 2 || version == 3) sensor = bank.sourceID;
-  else sensor = (((bank.sourceID & 0x1FFu) << 1) | ((word >> 22) & 0x1u));
-  d.valid = bank.type == bank_type && sensor < n_sensors;
+  if constexpr (version == 2 || version == 3) sensor = source;
+  else sensor = (((source & 0x1FFu) << 1) | ((word >> 22) & 0x1u));
+  d.valid = sensor < n_sensors;
   if (!d.valid) sensor = 0;
   const float* ltg = g.ltg + 12 * sensor;
   uint32_t cx, cy, or_fx, or_fy;
@@ -151,7 +167,10 @@ __global__ void __launch_bounds__(wave_size) k_retina_sensor_sizes(
   }
 }
 
-// DecodeRetinaClusters.cu:11-395 for one (event, module pair) per wave.
+// DecodeRetinaClusters.cu:11-395 for one (event, module pair) per wave. Bound by the chain of dependent
+// reads (slot, bank, header, word, geometry), so the slots' banks are looked up once, by a lane each,
+// and the first 128 words stay decoded for the second pass; the rank of a word comes from the words
+// of its phi bucket, where it was a comparison with every word. 1000 pile-up events: 33 us (90).
 template<int version>
 __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
   const char* raw,
@@ -175,7 +194,8 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
 {
   constexpr unsigned S = slots<version>();
   constexpr unsigned step = S / n_module_pairs;
-  __shared__ int64_t s_key[waves_per_block][key_cap];
+  __shared__ Slice s_slice[waves_per_block];
+  static_assert(step <= max_slots_per_mp, "slots of a module pair");
   const unsigned wave = threadIdx.x / wave_size, l = lane_id();
   const unsigned item = blockIdx.x * waves_per_block + wave;
   // populate_module_pair_offsets_and_sizes (:11-36), element by element over every event's
@@ -194,80 +214,101 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
   const Geometry& g = *geometry;
   const RawEvent ev(raw, offsets, sizes, types, mep, event_number + event_start);
   const bool in_lds = n <= key_cap;
-  int64_t* keys = s_key[wave];
+  Slice& L = s_slice[wave];
+  L.newest[l] = none;
+  L.before[l] = 0;
 
-  // Decode every word of the module pair (its slots' words, in slot and word order).
+  // The bank of each slot as the first event of the list placed it. A slot whose bank is missing in
+  // this event or of another type has no valid word: such a word has no key in the reference (left
+  // unset there); it ranks last here and is not written.
+  const unsigned first_word = sp_off[mp * step + min(l, step)] - lo; // lane t: words before slot t
+  if (l < step) {
+    const uint32_t bi = retina_bank_index[mp * step + l];
+    L.n_words[l] = 0;
+    if (bi < ev.n_banks) {
+      const RawBank bank = raw_bank<version>(ev, bi);
+      L.word[l] = bank.word;
+      L.source[l] = bank.sourceID;
+      if (bank.type == bank_type) L.n_words[l] = bank_n_sp<version>(bank);
+    }
+  }
+  wave_sync_lds();
+
+  // Decode word k of the module pair (its slots' words, in slot and word order; words past the end
+  // of a bank shorter than in the first event are invalid). The whole wave takes part.
   auto decode_at = [&](unsigned k) {
-    const uint32_t c = lo + k;
-    unsigned s = mp * step;
+    unsigned t = 0, before = 0;
 #pragma unroll
-    for (unsigned t = 1; t < step; ++t)
-      if (sp_off[mp * step + t] <= c) s = mp * step + t;
-    // The slot's bank as the first event of the list placed it; a slot whose bank is missing
-    // or shorter in this event yields an invalid word instead of a read past the bank.
-    const uint32_t bi = retina_bank_index[s];
-    const uint32_t w = c - sp_off[s];
-    if (bi >= ev.n_banks) {
-      Decoded d {};
-      d.valid = false;
-      return d;
+    for (unsigned j = 1; j < step; ++j) {
+      const unsigned start = __builtin_amdgcn_readlane(first_word, j);
+      if (start <= k) {
+        t = j;
+        before = start;
+      }
     }
-    const RawBank bank = raw_bank<version>(ev, bi);
-    if (w >= bank_n_sp<version>(bank)) {
-      Decoded d {};
-      d.valid = false;
-      return d;
-    }
-    return decode<version>(g, bank, bank.word[w]);
+    Decoded d {};
+    if (k < n && k - before < L.n_words[t]) d = decode<version>(g, L.source[t], L.word[t][k - before]);
+    return d;
   };
   uint32_t nonzero = 0;
-  Decoded first {}; // the lane's first word, kept for the ranking pass
-  for (unsigned k = l; k < n; k += wave_size) {
+  Decoded kept[2] {}; // the lane's first two words, for the ranking pass
+  auto first_pass = [&](unsigned k) {
     const Decoded d = decode_at(k);
-    if (k == l) first = d;
-    // A word of another bank type has no key in the reference (left unset there); it ranks
-    // last here and is not written.
+    if (k >= n) return d;
     const int64_t key = d.valid ? d.key : 0x7FFFFFFFFFFFFFFFll;
     hit_sorting_key[lo + k] = key;
-    if (in_lds) keys[k] = key;
+    if (in_lds) {
+      const unsigned bucket = bucket_of(key);
+      L.key[k] = key;
+      atomicAdd(&L.before[bucket], 1u);
+      L.next[k] = static_cast<uint16_t>(atomicExch(&L.newest[bucket], k));
+    }
     if (d.valid) nonzero += d.key != 0x7FFFFFFFFFFFFFFFll;
     else hit_permutations[lo + k] = 0;
-  }
+    return d;
+  };
+  kept[0] = first_pass(l);
+  if (n > wave_size) kept[1] = first_pass(l + wave_size);
+  for (unsigned base = 2 * wave_size; base < n; base += wave_size) first_pass(base + l);
 #pragma unroll
   for (unsigned d = 32; d > 0; d >>= 1) nonzero += __shfl_xor(nonzero, d, wave_size);
   if (l == 0) module_cluster_num[event_number * n_module_pairs + mp] = nonzero;
   if (in_lds) {
+    wave_sync_lds();
+    const uint32_t count = L.before[l], before = wave_inclusive_scan(count) - count;
+    wave_sync_lds();
+    L.before[l] = before;
     wave_sync_lds();
   }
   else {
     __threadfence_block();
     __builtin_amdgcn_wave_barrier();
   }
-  const int64_t* kk = in_lds ? keys : hit_sorting_key + lo;
 
   // Rank by key; the last word of a key's run writes the slot.
   const Clusters out {cluster_container, total};
-  for (unsigned i = l; i < n; i += wave_size) {
-    const Decoded d = i == l ? first : decode_at(i);
-    if (!d.valid) continue;
-    // Every lane reads the same keys (n is wave-uniform), eight reads in flight at a time.
+  auto second_pass = [&](unsigned i, const Decoded& d) {
+    if (!d.valid) return;
     unsigned position = 0;
     bool last = true;
-    unsigned j = 0;
-    for (; j + 8 <= n; j += 8) {
-      int64_t o[8];
-#pragma unroll
-      for (unsigned u = 0; u < 8; ++u) o[u] = kk[j + u];
-#pragma unroll
-      for (unsigned u = 0; u < 8; ++u) {
-        position += d.key > o[u];
-        last = last && !(j + u > i && o[u] == d.key);
+    if (in_lds) {
+      const unsigned bucket = bucket_of(d.key);
+      position = L.before[bucket];
+      for (unsigned j = L.newest[bucket]; j != none;) {
+        const int64_t o = L.key[j];
+        const unsigned next = L.next[j];
+        position += d.key > o;
+        last = last && !(j > i && o == d.key);
+        j = next;
       }
     }
-    for (; j < n; ++j) {
-      const int64_t o = kk[j];
-      position += d.key > o;
-      last = last && !(j > i && o == d.key);
+    else {
+      const int64_t* keys = hit_sorting_key + lo;
+      for (unsigned j = 0; j < n; ++j) {
+        const int64_t o = keys[j];
+        position += d.key > o;
+        last = last && !(j > i && o == d.key);
+      }
     }
     hit_permutations[lo + i] = lo + position;
     if (last) {
@@ -278,7 +319,10 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
       out.xyz()[3 * (size_t) slot + 2] = d.z;
       out.phis()[slot] = d.phi;
     }
-  }
+  };
+  second_pass(l, kept[0]);
+  if (n > wave_size) second_pass(l + wave_size, kept[1]);
+  for (unsigned base = 2 * wave_size; base < n; base += wave_size) second_pass(base + l, decode_at(base + l));
 }
 
 hipError_t launch_retina_sensor_sizes(const RetinaSizesLaunch& a, hipStream_t s)
