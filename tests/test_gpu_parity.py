@@ -354,6 +354,32 @@ def test_module_pairs_at_the_limits_of_the_clustering_slices(nu, lowest, version
     assert not errs, "\n".join(errs[:20])
 
 
+@pytest.mark.parametrize("n_events", [513, 4097])
+def test_search_launch_shapes_by_number_of_events(n_events, geometry, beamline, constants):
+    """The smallest numbers of events that take the second and the third shape of the search's launch,
+    with events of every LDS layout that it has: equal to the oracle."""
+    ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=12.0, high_occupancy_fraction=0.02, high_nu=14.0, seed=43)
+    ref, gpu, status = run_both(f"shape{n_events}", geometry, beamline, constants, True, events=ev)
+    assert int(ref["status"][0]) == 0 and status & velo.STATUS_OVERFLOW_MASK == 0
+    hits = np.diff(ref["offsets_estimated_input_size"].astype(np.int64)[::26])
+    assert hits.min() < 384 and hits.max() > 2048
+    errs = parity.compare(gpu, ref, True)
+    assert not errs, "\n".join(errs[:20])
+
+
+@pytest.mark.parametrize("phi_tolerance", [-0.01, 0.0, 0.2, 0.79, 2.0])
+def test_search_windows_of_other_tolerances(phi_tolerance, geometry, beamline, constants):
+    """Windows that are empty, that end a module pair's phis on both sides, and that are wider than what
+    the phi buckets serve (8192 units, 0.786 rad): the same tracks as the oracle's."""
+    ev = synth.generate(n_events=6, pileup=1, nu=7.6, seed=44)
+    ref = oracle.run(ev, geometry, beamline, phi_tolerance=phi_tolerance)
+    seq = velo.VeloSequence(constants, ev.n_events, max(ev.raw.size, 4096))
+    seq.run(velo.DeviceEvents(ev), phi_tolerance=phi_tolerance)
+    errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+    seq.close()
+    assert not errs, "\n".join(errs[:20])
+
+
 def test_prefix_sum_iota(constants):
     """The reference's own prefix-sum test shape (TestPrefixSum.cu:9-33): iota 1..1000."""
     import torch
