@@ -728,9 +728,20 @@ __device__ __forceinline__ unsigned phi_rank(const PhiT* phi, const IdT* id, uns
   return position;
 }
 
-// K4: one workgroup per (module pair, event). Keys are staged in LDS when they fit.
-constexpr unsigned sort_lds_cap = 2048;
-__global__ void k_sort_by_phi(
+// (phi, id) as one unsigned 64-bit key: phi (signed) in the high word, offset to unsigned. Key
+// order is the sort's (phi, id) order (SortByPhi.cu:90-125), and distinct clusters of a module
+// pair have distinct ids, so the rank of a cluster is the number of keys below its own.
+__device__ __forceinline__ uint64_t phi_id_key(int16_t phi, uint32_t id)
+{
+  return (static_cast<uint64_t>(static_cast<uint16_t>(phi) ^ 0x8000u) << 32) | id;
+}
+
+// K4: one wave per (module pair, event). A cluster's rank is the number of clusters in the phi buckets
+// before its own and of those in its own with a smaller key, which it finds by their list; module pairs
+// of more than sort_lds_cap clusters compare every two. 500 pile-up events: 10 us (35 with 256
+// lanes that compared every two).
+constexpr unsigned sort_lds_cap = 512;
+__global__ void __launch_bounds__(wave_size) k_sort_by_phi(
   const uint32_t* event_list,
   const uint32_t* number_of_events,
   const uint32_t* offsets_estimated_input_size,
@@ -739,30 +750,59 @@ __global__ void k_sort_by_phi(
   char* sorted_container,
   uint32_t* hit_permutation)
 {
-  __shared__ int16_t s_phi[sort_lds_cap];
-  __shared__ uint32_t s_id[sort_lds_cap];
-  const unsigned mp = blockIdx.x;
+  constexpr unsigned none = 0xFFFFu; // ends a bucket's list
+  __shared__ uint64_t s_key[sort_lds_cap];
+  __shared__ uint16_t s_next[sort_lds_cap];
+  __shared__ uint32_t s_newest[wave_size], s_before[wave_size];
+  const unsigned mp = blockIdx.x, l = threadIdx.x;
   const unsigned event_number = event_list ? event_list[blockIdx.y] : blockIdx.y;
   const unsigned total = offsets_estimated_input_size[n_module_pairs * number_of_events[0]];
   const Clusters in {const_cast<char*>(cluster_container), total};
   const Clusters out {sorted_container, total};
   const unsigned start = offsets_estimated_input_size[event_number * n_module_pairs + mp];
   const unsigned n = module_cluster_num[event_number * n_module_pairs + mp];
-  const bool lds = n <= sort_lds_cap;
-  if (lds) {
-    for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
-      s_phi[i] = in.phis()[start + i];
-      s_id[i] = in.ids()[start + i];
+  if (n <= sort_lds_cap) {
+    s_newest[l] = none;
+    s_before[l] = 0;
+    __syncthreads();
+    for (unsigned i = l; i < n; i += wave_size) {
+      const uint64_t key = phi_id_key(in.phis()[start + i], in.ids()[start + i]);
+      const unsigned bucket = static_cast<unsigned>(key >> 42);
+      s_key[i] = key;
+      atomicAdd(&s_before[bucket], 1u);
+      s_next[i] = static_cast<uint16_t>(atomicExch(&s_newest[bucket], i));
     }
     __syncthreads();
+    const uint32_t count = s_before[l], before = wave_inclusive_scan(count) - count;
+    __syncthreads();
+    s_before[l] = before;
+    __syncthreads();
+    for (unsigned i = l; i < n; i += wave_size) {
+      const float* xyz = in.xyz() + 3 * (size_t)(start + i);
+      const float x = xyz[0], y = xyz[1], z = xyz[2];
+      const uint64_t key = s_key[i];
+      const unsigned bucket = static_cast<unsigned>(key >> 42);
+      unsigned rank = s_before[bucket];
+      for (unsigned j = s_newest[bucket]; j != none;) {
+        const uint64_t other = s_key[j];
+        j = s_next[j];
+        rank += other < key;
+      }
+      const size_t slot = start + rank;
+      hit_permutation[slot] = start + i;
+      out.ids()[slot] = static_cast<uint32_t>(key);
+      out.phis()[slot] = static_cast<int16_t>(static_cast<uint16_t>(key >> 32) ^ 0x8000u);
+      out.xyz()[3 * slot] = x;
+      out.xyz()[3 * slot + 1] = y;
+      out.xyz()[3 * slot + 2] = z;
+    }
+    return;
   }
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
-    const unsigned r = lds ? phi_rank(s_phi, s_id, n, i) : phi_rank(in.phis() + start, in.ids() + start, n, i);
-    hit_permutation[start + r] = start + i;
-  }
+  for (unsigned i = l; i < n; i += wave_size)
+    hit_permutation[start + phi_rank(in.phis() + start, in.ids() + start, n, i)] = start + i;
   __threadfence_block();
   __syncthreads();
-  for (unsigned i = threadIdx.x; i < n; i += blockDim.x) {
+  for (unsigned i = l; i < n; i += wave_size) {
     const unsigned src = hit_permutation[start + i];
     out.ids()[start + i] = in.ids()[src];
     out.phis()[start + i] = in.phis()[src];
@@ -845,7 +885,7 @@ hipError_t launch_sort_by_phi(const SortLaunch& a, hipStream_t s)
 {
   if (!a.n_list) return hipSuccess;
   hipLaunchKernelGGL(
-    k_sort_by_phi, dim3(n_module_pairs, a.n_list), dim3(256), 0, s, a.event_list, a.number_of_events,
+    k_sort_by_phi, dim3(n_module_pairs, a.n_list), dim3(wave_size), 0, s, a.event_list, a.number_of_events,
     a.offsets_estimated_input_size, a.module_cluster_num, a.cluster_container, a.sorted_container, a.hit_permutation);
   return hipGetLastError();
 }
@@ -1201,14 +1241,6 @@ static_assert(sizeof(ClusterLds::work) >= rank_bytes(cluster_cap) && cluster_cap
 static_assert(sizeof(Banks) <= 4 * ClusterLds::window_words && non_isolated_cap % 2 == 0, "banks");
 static_assert(offsetof(ClusterLds, xyz) == sizeof(ClusterLds::work), "the ranking reaches into xyz");
 } // namespace mp
-
-// (phi, id) as one unsigned 64-bit key: phi (signed) in the high word, offset to unsigned. Key
-// order is the sort's (phi, id) order (SortByPhi.cu:90-125), and distinct clusters of a module
-// pair have distinct ids, so the rank of a cluster is the number of keys below its own.
-__device__ __forceinline__ uint64_t phi_id_key(int16_t phi, uint32_t id)
-{
-  return (static_cast<uint64_t>(static_cast<uint16_t>(phi) ^ 0x8000u) << 32) | id;
-}
 
 // The number of keys[0 .. n) below `key` (eight reads in flight at a time).
 __device__ __forceinline__ unsigned keys_below(const uint64_t* keys, unsigned n, uint64_t key)
