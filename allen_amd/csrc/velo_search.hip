@@ -1388,8 +1388,11 @@ __device__ __forceinline__ void finish_event(
 // atomic per wave). With event_clock, each workgroup stores at event_clock[10 * event_number]
 // its event's start and end time (wall clock ticks) and, in the counting instantiation, the
 // ticks spent in each Phase.
-template<bool count, int seed_mode, bool persistent>
-__global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, seed_mode == seed_mode_scored ? 3 : 1)
+// waves_per_simd: what the registers leave room for. The scored search takes 155 and runs three; with
+// four (128 registers, 26 values spilled) an event takes 5 % longer, which pays where more events
+// wait than three a CU.
+template<bool count, int seed_mode, bool persistent, unsigned waves_per_simd = seed_mode == seed_mode_scored ? 3 : 1>
+__global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, waves_per_simd)
   k_search_by_triplet(const SearchArgs a)
 {
   extern __shared__ __align__(16) char dyn_all[];
@@ -1632,6 +1635,8 @@ __global__ void k_three_hit_filter(
   if (threadIdx.x == 0) number_of_output[event_number] = base;
 }
 
+constexpr size_t lds_per_cu = 160 * 1024;
+
 // Launch geometry: the seeding scratch, the ring window, the unused-hit list, then the hits.
 size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
 {
@@ -1659,6 +1664,18 @@ static SearchShape search_shape(unsigned n_events)
   return {128, 384, 512, 512, 0};
 }
 
+// The same for the scored search, whose workgroups have 256 lanes (their size is part of the pruning
+// rule): 12 waves of it fit a CU by its registers, so up to 768 events are in flight at once and have
+// the LDS of three workgroups (300 one-vertex events, whole pass: 232 us; 257 with 1760 hits and a
+// window and a list of 1024). More of them take the instantiation of 16 waves a CU and the LDS that
+// four workgroups leave (777 events: 298 us, 371 with three; 1000 pile-up events: 375, 440).
+constexpr unsigned scored_waves_at_three = 3 * 4 * 256; // waves per SIMD, SIMDs, CUs
+static SearchShape scored_shape(unsigned n_events)
+{
+  if (n_events * (256 / wave_size) <= scored_waves_at_three) return {256, 2048, 1024, 512, 0};
+  return {256, 1500, 512, 512, 0};
+}
+
 hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
 {
   if (!a.n_list) return hipSuccess;
@@ -1667,8 +1684,9 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   // wave for the in-wave scorer and decision: workgroups of 64, 128 or 256 lanes. The scorer's
   // weights take LDS from the hits (same residency).
   const bool scored = a.scorer_params != nullptr;
-  const bool shaped = !a.block_dim && !scored && !a.work_counter;
-  const SearchShape shape = shaped ? search_shape(a.n_list) : SearchShape {256, search_default_lds_hits, ring_window, unused_list_cap, 0};
+  const bool shaped = !a.block_dim && !a.work_counter;
+  const SearchShape shape = !shaped ? SearchShape {256, search_default_lds_hits, ring_window, unused_list_cap, 0}
+                            : scored ? scored_shape(a.n_list) : search_shape(a.n_list);
   const unsigned block = a.block_dim ? a.block_dim : shape.block;
   const unsigned hits_per_wave = shape.hits_per_wave;
   // Dynamic LDS stays within the device's per-workgroup limit (less the static part).
@@ -1686,7 +1704,7 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   if ((size_t) max_lds <= fixed) return hipErrorInvalidConfiguration;
   const unsigned max_hits = static_cast<unsigned>(((size_t) max_lds - fixed) / search_bytes_per_hit);
   const unsigned default_hits =
-    scored ? search_default_lds_hits - static_cast<unsigned>((extra + search_bytes_per_hit - 1) / search_bytes_per_hit)
+    scored && !shaped ? search_default_lds_hits - static_cast<unsigned>((extra + search_bytes_per_hit - 1) / search_bytes_per_hit)
            : shape.lds_hits;
   const unsigned lds_hits = min(a.lds_hits ? a.lds_hits : default_hits, max_hits);
   const size_t dyn = search_dynamic_lds(block, lds_hits, window, list_cap) + extra;
@@ -1742,7 +1760,12 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
     if (a.work_counter) VELO_LAUNCH_SEARCH_P(C, L, true);                                                           \
     else VELO_LAUNCH_SEARCH_P(C, L, false);                                                                         \
   } while (0)
+  // Four waves a SIMD where the LDS lets them in and three leave events waiting.
+  const unsigned waves = block / wave_size;
+  const bool four = scored && !a.work_counter && a.n_list > scored_waves_at_three / waves &&
+                    lds_per_cu / (dyn + 1024) * waves >= 16;
   if (a.work_stats) VELO_LAUNCH_SEARCH(true, seed_mode_plain);
+  else if (four) hipLaunchKernelGGL((k_search_by_triplet<false, seed_mode_scored, false, 4>), dim3(grid), dim3(block), dyn, s, k);
   else if (a.scorer_params) VELO_LAUNCH_SEARCH(false, seed_mode_scored);
   else if (a.seed_log.counter) VELO_LAUNCH_SEARCH(false, seed_mode_log);
   else VELO_LAUNCH_SEARCH(false, seed_mode_plain);

@@ -291,3 +291,31 @@ def test_mlp_kernels_at_wave_and_grid_edges(n):
     want = ref.gradient(x, y.astype(np.float64), p)
     np.testing.assert_allclose(g, want, rtol=2e-3, atol=2e-3 * np.abs(want).max())
     np.testing.assert_allclose(loss, ref.loss(x, y, p) / n, rtol=1e-4)
+
+
+@pytest.mark.parametrize("n_events", [768, 769])
+def test_scored_search_on_both_sides_of_its_launch_shapes(n_events, geometry, beamline):
+    """The most events that the scored search holds at three waves a SIMD, and one more, with events of
+    every LDS layout: with a threshold that keeps every seed it is the plain search; at the shipped
+    threshold its tracks are those of the launch whose workgroup size is set by hand."""
+    import oracle
+    from allen_amd import scorer, synth, velo
+    from tests import parity
+    ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=12.0, high_occupancy_fraction=0.02, high_nu=14.0, seed=85)
+    ref = oracle.run(ev, geometry, beamline)
+    params, thr = scorer.trained()
+    seq, constants = _scored_run(geometry, beamline, ev, params, -1e30)
+    assert seq.status() & velo.STATUS_OVERFLOW_MASK == 0
+    errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+    assert not errs, "\n".join(errs[:20])
+    seq.close()
+    constants.close()
+    hits = []
+    for block in (0, 256):
+        seq, constants = _scored_run(geometry, beamline, ev, params, thr, block=block)
+        tracks = int(seq.fetch("offsets_all_velo_tracks", np.uint32, n_events + 1)[-1])
+        offsets = seq.fetch("offsets_velo_track_hit_number", np.uint32, tracks + 1)
+        hits.append((offsets, seq.fetch("velo_track_hits", np.uint8, 16 * int(offsets[-1]))))
+        seq.close()
+        constants.close()
+    assert np.array_equal(hits[0][0], hits[1][0]) and np.array_equal(hits[0][1], hits[1][1])
