@@ -1652,15 +1652,18 @@ struct SearchShape {
 // Few events: every event has its LDS to itself (two workgroups fit a CU), and the launch lasts as
 // long as its largest event: four waves for events from 2100 hits on, all hits in LDS (200 events
 // of up to 1700 hits: 123 us against 142 us with 1500 hits in LDS and coordinates from memory).
-// Up to a few thousand: all of them have to be in flight at once, so the LDS is what four
+// Up to 1024: all of them have to be in flight at once, so the LDS is what four
 // workgroups a CU leave (1000 pile-up events: 210 us; with 1760 hits 220 us, with 128-lane
-// workgroups 310 us, with 512 lanes 213 us). Beyond, the workgroups stream through the chip and the
+// workgroups 310 us, with 512 lanes 213 us). Up to 4096: five workgroups a CU, which their registers
+// allow (whole passes with five and four: 1100 one-vertex events 282 and 346 us, 3000 pile-up events 655
+// and 683 us, 2000 stress events 835 and 844 us). Beyond, the workgroups stream through the chip and the
 // most resident waves win: two waves per event and little LDS (20 000 events: 1.62 ms; 1.93 ms
 // with 256 lanes, 2.46 ms with 1500 hits in LDS, 4.32 ms with 256 lanes and 1760 hits before).
 static SearchShape search_shape(unsigned n_events)
 {
   if (n_events <= 512) return {256, 3072, 1024, 512, 700};
-  if (n_events <= 4096) return {256, 1500, 1024, 512, 700};
+  if (n_events <= 1024) return {256, 1500, 1024, 512, 700};
+  if (n_events <= 4096) return {256, 1180, 512, 512, 700};
   return {128, 384, 512, 512, 0};
 }
 

@@ -354,9 +354,9 @@ def test_module_pairs_at_the_limits_of_the_clustering_slices(nu, lowest, version
     assert not errs, "\n".join(errs[:20])
 
 
-@pytest.mark.parametrize("n_events", [513, 4097])
+@pytest.mark.parametrize("n_events", [513, 1025, 4097])
 def test_search_launch_shapes_by_number_of_events(n_events, geometry, beamline, constants):
-    """The smallest numbers of events that take the second and the third shape of the search's launch,
+    """The smallest numbers of events that take the second, third and fourth shape of the search's launch,
     with events of every LDS layout that it has: equal to the oracle."""
     ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=12.0, high_occupancy_fraction=0.02, high_nu=14.0, seed=43)
     ref, gpu, status = run_both(f"shape{n_events}", geometry, beamline, constants, True, events=ev)
