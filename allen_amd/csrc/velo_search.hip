@@ -514,9 +514,9 @@ constexpr int16_t max_run_tolerance = 8192;
 // it are read four at a time and evaluated without branches, which lets their arithmetic overlap
 // (one dependent operation takes 8 cycles here, an independent one 5; an LDS read 64). Nearly
 // always one pass of four serves the whole wave. Where the walk differs from the run: its
-// |difference| of 16 bits takes a hit exactly opposite for one within any tolerance, which it can
-// reach only as its first hit, with none in the run; those lanes, tolerances
-// beyond max_run_tolerance and module pairs out of order take the walk itself.
+// |difference| of 16 bits takes a hit exactly opposite for one within any tolerance, so it goes on
+// through such hits where they are the next ones after the run (which may be empty); those lanes,
+// tolerances beyond max_run_tolerance and module pairs out of order take the walk itself.
 template<bool count, bool unused_only, typename H>
 __device__ __forceinline__ bool closest_hit(
   WorkCount& wc, const H& hits, const ModulePairData& mp, const Line& l, int16_t phi_tolerance, float& best, uint32_t& best_index)
@@ -540,8 +540,10 @@ __device__ __forceinline__ bool closest_hit(
   const unsigned width = 2u * static_cast<unsigned>(phi_tolerance);
   // Position lo + j of the circle; positions beyond the run only stay in range.
   const auto position = [&](unsigned j) { return mp.hit_start + min(min(lo + j, lo + j - n), n - 1); };
-  const int16_t after = hits.phi(position(length));
-  bool any = false, none_in_run = true;
+  const int16_t after = hits.phi(position(length)); // the end buckets hold no opposite hit
+  const float limit = best;
+  uint32_t visits = 0;
+  bool any = false;
   for (unsigned j0 = 0; j0 < length; j0 += 4) {
     unsigned index[4];
     Hit h[4];
@@ -554,17 +556,19 @@ __device__ __forceinline__ bool closest_hit(
     for (unsigned k = 0; k < 4; ++k) {
       const float scatter = scatter_at(l, h[k]);
       const bool in_run = j0 + k < length && static_cast<uint16_t>(h[k].phi - from) <= width;
-      none_in_run = none_in_run && !in_run;
       const bool visited = in_run && !(unused_only && h[k].used);
-      if constexpr (count) (unused_only ? wc.seed_eval : wc.fwd_eval) += visited;
+      if constexpr (count) visits += visited;
       const bool closer = visited && scatter < best;
       best = closer ? scatter : best;
       best_index = closer ? index[k] : best_index;
       any = any || closer;
     }
   }
-  if (none_in_run && static_cast<uint16_t>(after - l.phi) == 0x8000u)
+  if (static_cast<uint16_t>(after - l.phi) == 0x8000u) {
+    best = limit;
     return closest_hit_walk<count, unused_only>(wc, hits, mp, l, phi_tolerance, best, best_index);
+  }
+  if constexpr (count) (unused_only ? wc.seed_eval : wc.fwd_eval) += visits;
   return any;
 }
 

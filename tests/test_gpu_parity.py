@@ -380,6 +380,27 @@ def test_search_windows_of_other_tolerances(phi_tolerance, geometry, beamline, c
     assert not errs, "\n".join(errs[:20])
 
 
+@pytest.mark.parametrize("seed,phi_tolerance", [(13, 0.25), (42, 0.5), (47, 0.7), (117, 0.25)])
+def test_search_walk_goes_on_through_opposite_hits(seed, phi_tolerance, geometry, beamline, constants):
+    """Sparse noisy events and a scatter limit that any hit meets: the 16-bit |difference| takes a hit
+    exactly opposite for one within the tolerance, so the walk goes on through it where it is the
+    next one after the hits of the window. It decides a seed or an extension in each of these
+    slices (rarely: one event in some ten thousand). The oracle's tracks, in every layout of the hits."""
+    ev = synth.generate(n_events=1000, pileup=0, mean_tracks=3.0, noise_fraction=4.0, seed=seed)
+    ref = oracle.run(ev, geometry, beamline, phi_tolerance=phi_tolerance, max_scatter=1e6)
+    assert int(ref["status"][0]) == 0
+    hits = np.diff(ref["offsets_estimated_input_size"].astype(np.int64)[::26])
+    assert 64 < np.median(hits) < 16 * 64 // 3
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    dev = velo.DeviceEvents(ev)
+    for lds_hits in (0, 64, 1):  # in LDS; mostly phi and flags in LDS; from memory
+        seq.set_tuning("search_lds_hits", lds_hits)
+        seq.run(dev, phi_tolerance=phi_tolerance, max_scatter=1e6)
+        errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+        assert not errs, f"search_lds_hits {lds_hits}:\n" + "\n".join(errs[:20])
+    seq.close()
+
+
 def test_prefix_sum_iota(constants):
     """The reference's own prefix-sum test shape (TestPrefixSum.cu:9-33): iota 1..1000."""
     import torch
