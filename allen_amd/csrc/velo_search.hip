@@ -1346,15 +1346,23 @@ __device__ __forceinline__ float means_square_fit_chi2(const Hit& a, const Hit& 
 // three-hit tracks, with the hits and their flags where the search has them, and the number of
 // hits of the event's tracks (four for each track, one for each extension, three for each kept
 // three-hit track): what the filter, the track-hit count and two scans over the tracks took a
-// launch each for.
+// launch each for. Where the ring of tracks to follow has overflowed, an entry can be read twice and
+// its track extended by two lanes at once, so the stored tracks are counted themselves: the hits
+// are placed by what each track holds.
 template<typename H>
 __device__ __forceinline__ void finish_event(
   const H& hits, const Team& team, SearchShared& sh, Counters& cn, const EventOutputs& o, const SearchArgs& a, unsigned toff)
 {
   if (!a.three_hit_tracks_output) return;
-  if (lane_id() == 0 && cn.extended) atomicAdd(&sh.extended, cn.extended);
-  __threadfence_block(); // other lanes wrote the three-hit tracks
+  const bool overflow = cn.status & status_ttf_ring_overflow;
+  const unsigned n_tracks = min(cn.n_tracks, o.track_capacity);
+  if (lane_id() == 0 && cn.extended && !overflow) atomicAdd(&sh.extended, cn.extended);
+  __threadfence_block(); // other lanes wrote the tracks
   team.sync();
+  if (overflow) {
+    for (unsigned i = threadIdx.x; i < n_tracks; i += team.lanes) atomicAdd(&sh.extended, o.tracks[i].hitsNum - 4u);
+    team.sync();
+  }
   const unsigned n_in = min(cn.three, o.track_capacity);
   TrackletHits* out = a.three_hit_tracks_output + toff;
   unsigned kept = 0;
@@ -1373,7 +1381,7 @@ __device__ __forceinline__ void finish_event(
   }
   if (threadIdx.x == 0) {
     a.number_of_three_hit_tracks_output[o.event_number] = kept;
-    a.event_track_hits[o.event_number] = 4 * min(cn.n_tracks, o.track_capacity) + sh.extended + 3 * kept;
+    a.event_track_hits[o.event_number] = 4 * n_tracks + sh.extended + 3 * kept;
   }
 }
 

@@ -401,6 +401,32 @@ def test_search_walk_goes_on_through_opposite_hits(seed, phi_tolerance, geometry
     seq.close()
 
 
+def test_hit_offsets_of_an_event_that_overflows_the_ring(geometry, beamline, constants):
+    """Events whose tracks to follow overflow the ring raise the status bit and have no specified tracks,
+    but the offsets of the track hits still are the sums of the tracks' hit numbers, and the
+    other events' tracks are the oracle's."""
+    ev = synth.generate(n_events=6, pileup=0, mean_tracks=120.0, high_occupancy_fraction=0.4, high_nu=300.0, seed=47)
+    ref = oracle.run(ev, geometry, beamline, compute_f64=0, max_skipped_modules=2)
+    hits = np.diff(ref["offsets_estimated_input_size"].astype(np.int64)[::26])
+    assert int(ref["status"][0]) == 1 and hits.min() < 3000 and 30000 < hits.max() < 65536
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    seq.run(velo.DeviceEvents(ev), max_skipped_modules=2)
+    assert seq.status() & velo.STATUS_OVERFLOW_MASK == 1
+    off = seq.fetch("offsets_all_velo_tracks", np.uint32, ev.n_events + 1).astype(np.int64)
+    hit_number = seq.fetch("velo_track_hit_number", np.uint32, int(off[-1]))
+    hit_off = seq.fetch("offsets_velo_track_hit_number", np.uint32, int(off[-1]) + 1).astype(np.int64)
+    ids = seq.fetch("velo_track_hits", np.uint32, int(hit_off[-1]))
+    seq.close()
+    np.testing.assert_array_equal(np.diff(hit_off), hit_number)
+    assert np.all((hit_number >= 3) & (hit_number <= 26))
+    ref_off, ref_hit_off = (ref[k].astype(np.int64) for k in ("offsets_all_velo_tracks", "offsets_velo_track_hit_number"))
+    ref_ids = ref["velo_track_hits"][:4 * int(ref_hit_off[-1])].view("<u4")
+    for e in np.nonzero(hits < 20000)[0]:
+        a, b = (slice(o[e], o[e + 1] + 1) for o in (off, ref_off))
+        np.testing.assert_array_equal(np.diff(hit_off[a]), np.diff(ref_hit_off[b]))
+        np.testing.assert_array_equal(ids[hit_off[a][0]:hit_off[a][-1]], ref_ids[ref_hit_off[b][0]:ref_hit_off[b][-1]])
+
+
 def test_prefix_sum_iota(constants):
     """The reference's own prefix-sum test shape (TestPrefixSum.cu:9-33): iota 1..1000."""
     import torch
