@@ -1153,7 +1153,9 @@ __device__ __forceinline__ void track_forwarding(
         // A promoted track beyond the slots of its event is skipped when read back.
         const unsigned p = (cn.ttf + s.r[1]) % max_tracks_to_follow;
         const unsigned last2 = found ? h1_num | (best_h2 << 16) : h0_num | (h1_num << 16);
-        const uint32_t skips = found ? 0u : skipped + (1u << skipped_pos);
+        // The field holds up to seven skipped modules; a limit beyond that is none (counting on would
+        // make a track's entry a seed's).
+        const uint32_t skips = found ? 0u : min(skipped + (1u << skipped_pos), bit_skipped);
         const bool seed = is_seed && !found;
         const uint32_t full = skips | (seed ? bit_seed : 0u) | track_number;
         o.ttf[p] = full;

@@ -316,7 +316,7 @@ typedef struct {
   const velo_constants* constants;
   float phi_tolerance;              /* 0.045 */
   float max_scatter;                /* 0.08 */
-  unsigned max_skipped_modules;     /* 1 */
+  unsigned max_skipped_modules;     /* 1; above 7: no limit */
   unsigned block_dim_x;             /* 0: chosen from the number of events */
 } velo_search_by_triplet_params;
 int velo_search_by_triplet(const velo_search_by_triplet_params* p, hipStream_t stream);

@@ -401,6 +401,38 @@ def test_search_walk_goes_on_through_opposite_hits(seed, phi_tolerance, geometry
     seq.close()
 
 
+@pytest.mark.parametrize("tuning", [{}, {"search_lds_hits": 1}, {"search_ring_window": 64}], ids=["lds", "memory", "ring"])
+@pytest.mark.parametrize("max_skipped_modules", [0, 7, 8, 25])
+def test_search_limits_of_skipped_modules(max_skipped_modules, tuning, geometry, beamline, constants, monkeypatch):
+    """The skipped modules of an entry have three bits. Up to 7 the limit is exact, beyond it there is
+    none: the rules with a field that holds any number (entries that skip 8 modules are common: tracks
+    that end downstream)."""
+    from tests import textbook, textbook_search as ts
+    monkeypatch.setattr(ts, "SKIP_MASK", 0xFF << ts.SKIP_SHIFT)
+    monkeypatch.setattr(ts, "SEED_BIT", 1 << 40)
+    ev = synth.generate(n_events=5, pileup=0, mean_tracks=60.0, seed=48)
+    ref = oracle.run(ev, geometry, beamline, compute_f64=0)
+    zs = textbook.parse_geometry(geometry)["module_zs"]
+    offsets, counts = ref["offsets_estimated_input_size"], ref["module_cluster_num"]
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    for k, v in tuning.items():
+        seq.set_tuning(k, v)
+    seq.run(velo.DeviceEvents(ev), max_skipped_modules=max_skipped_modules)
+    gpu = parity.gpu_buffers(seq, ref)
+    tracks = seq.fetch("tracks", parity.TRACK, ref["tracks"].size)
+    seq.close()
+    for e in range(ev.n_events):
+        want = ts.search(ts.event_from_container(ref["sorted_velo_cluster_container"], offsets, counts, e, zs),
+                         max_skipped_modules=max_skipped_modules if max_skipped_modules <= 7 else 26)
+        toff = int(np.float32(offsets[26 * e]) * np.float32(0.34))
+        n, (n3, ttf) = int(gpu["number_of_velo_tracks"][e]), (int(v) for v in gpu["atomics_velo"][3 * e:3 * e + 2])
+        assert [t["hits"][:t["hitsNum"]].tolist() for t in tracks[toff:toff + n]] == want["tracks"]
+        assert gpu["three_hit_tracks"]["hits"][toff:toff + n3].tolist() == want["three_hit"]
+        assert ttf == want["ttf"]
+        h0, h1 = int(offsets[26 * e]), int(offsets[26 * (e + 1)])
+        np.testing.assert_array_equal(gpu["hit_used"][h0:h1], want["used"])
+
+
 def test_hit_offsets_of_an_event_that_overflows_the_ring(geometry, beamline, constants):
     """Events whose tracks to follow overflow the ring raise the status bit and have no specified tracks,
     but the offsets of the track hits still are the sums of the tracks' hit numbers, and the
