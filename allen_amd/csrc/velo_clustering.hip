@@ -738,8 +738,9 @@ __device__ __forceinline__ uint64_t phi_id_key(int16_t phi, uint32_t id)
 
 // K4: one wave per (module pair, event). A cluster's rank is the number of clusters in the phi buckets
 // before its own and of those in its own with a smaller key, which it finds by their list; module pairs
-// of more than sort_lds_cap clusters compare every two. 500 pile-up events: 10 us (35 with 256
-// lanes that compared every two).
+// of more than sort_lds_cap clusters compare every two. Equal keys (a word twice in a bank) share a
+// rank, and the slot they leave takes the container's first cluster, as the zero that its entry of the
+// permutation holds says. 500 pile-up events: 11 us (37 with 256 lanes that compared every two).
 constexpr unsigned sort_lds_cap = 512;
 __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
   const uint32_t* event_list,
@@ -753,6 +754,7 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
   constexpr unsigned none = 0xFFFFu; // ends a bucket's list
   __shared__ uint64_t s_key[sort_lds_cap];
   __shared__ uint16_t s_next[sort_lds_cap];
+  __shared__ uint8_t s_taken[sort_lds_cap];
   __shared__ uint32_t s_newest[wave_size], s_before[wave_size];
   const unsigned mp = blockIdx.x, l = threadIdx.x;
   const unsigned event_number = event_list ? event_list[blockIdx.y] : blockIdx.y;
@@ -769,6 +771,7 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
       const uint64_t key = phi_id_key(in.phis()[start + i], in.ids()[start + i]);
       const unsigned bucket = static_cast<unsigned>(key >> 42);
       s_key[i] = key;
+      s_taken[i] = 0;
       atomicAdd(&s_before[bucket], 1u);
       s_next[i] = static_cast<uint16_t>(atomicExch(&s_newest[bucket], i));
     }
@@ -777,6 +780,14 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
     __syncthreads();
     s_before[l] = before;
     __syncthreads();
+    const auto write = [&](size_t slot, size_t from, uint64_t key, float x, float y, float z) {
+      hit_permutation[slot] = static_cast<uint32_t>(from);
+      out.ids()[slot] = static_cast<uint32_t>(key);
+      out.phis()[slot] = static_cast<int16_t>(static_cast<uint16_t>(key >> 32) ^ 0x8000u);
+      out.xyz()[3 * slot] = x;
+      out.xyz()[3 * slot + 1] = y;
+      out.xyz()[3 * slot + 2] = z;
+    };
     for (unsigned i = l; i < n; i += wave_size) {
       const float* xyz = in.xyz() + 3 * (size_t)(start + i);
       const float x = xyz[0], y = xyz[1], z = xyz[2];
@@ -788,14 +799,12 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
         j = s_next[j];
         rank += other < key;
       }
-      const size_t slot = start + rank;
-      hit_permutation[slot] = start + i;
-      out.ids()[slot] = static_cast<uint32_t>(key);
-      out.phis()[slot] = static_cast<int16_t>(static_cast<uint16_t>(key >> 32) ^ 0x8000u);
-      out.xyz()[3 * slot] = x;
-      out.xyz()[3 * slot + 1] = y;
-      out.xyz()[3 * slot + 2] = z;
+      s_taken[rank] = 1;
+      write(start + rank, start + i, key, x, y, z);
     }
+    __syncthreads();
+    for (unsigned i = l; i < n; i += wave_size)
+      if (!s_taken[i]) write(start + i, 0, phi_id_key(in.phis()[0], in.ids()[0]), in.xyz()[0], in.xyz()[1], in.xyz()[2]);
     return;
   }
   for (unsigned i = l; i < n; i += wave_size)

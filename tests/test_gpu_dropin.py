@@ -110,6 +110,41 @@ def test_sp_drop_ins_with_event_list(case, geometry, beamline, constants):
     check_views(args, ref, event_list)
 
 
+@pytest.mark.parametrize("nu,lowest,highest", [(2.0, 0, 512), (60.0, 513, 65536)])
+def test_equal_clusters_leave_their_slot_the_first_cluster(nu, lowest, highest, constants):
+    """A super-pixel word twice in a bank makes two clusters with the same phi and id: they share a slot
+    of the sorted container, and the slot they leave takes cluster 0, which its permutation entry
+    names (SortByPhi.cu:49-153), in module pairs that are ranked in LDS and beyond."""
+    ev = synth.generate(n_events=3, pileup=1, nu=nu, seed=69)
+    raw, s16 = ev.raw.copy(), ev.sizes.view("<u2")
+    repeated = 0
+    for e in range(ev.n_events):
+        base = int(ev.offsets[e])
+        nb = int(raw[base:base + 4].view("<u4")[0])
+        boff = raw[base + 4:base + 8 + 4 * nb].view("<u4").astype(np.int64)
+        for b in range(nb):
+            at = base + 8 + 4 * nb + int(boff[b]) + 4
+            words = raw[at:at + int(s16[int(ev.sizes[e]) + b]) // 4 * 4].view("<u4")
+            isolated = np.nonzero(words & 0x80000000)[0]
+            if isolated.size > 1 and b % 3 == 0:
+                words[isolated[1]] = words[isolated[0]]
+                repeated += 1
+    assert repeated > 5
+    dev = velo.DeviceEvents(synth.dataclasses.replace(ev, raw=raw))
+    args = algorithms.velo_sp_sequence(constants, dev, ev.n_events, poison=True)
+    total = args.host["total_number_of_velo_clusters"]
+    offsets = _host(args, "offsets_estimated_input_size", np.uint32, 26 * ev.n_events + 1)
+    counts = _host(args, "module_cluster_num", np.uint32, 26 * ev.n_events)
+    assert lowest <= counts.max() <= highest
+    slots = parity.filled_slots(offsets, counts)
+    permutation = _host(args, "hit_permutation", np.uint32, total)[slots]
+    assert np.count_nonzero(permutation == 0) > 1
+    unsorted = parity.cluster_views(_host(args, "velo_cluster_container", np.uint8, 18 * total), total)
+    in_order = parity.cluster_views(_host(args, "sorted_velo_cluster_container", np.uint8, 18 * total), total)
+    for a, b in zip(in_order, unsorted):
+        np.testing.assert_array_equal(a[slots].view(np.uint8), b[permutation].view(np.uint8))
+
+
 def _view(args, name, dtype, count):
     return args[name].cpu().numpy()[:dtype.itemsize * count].view(dtype)
 
