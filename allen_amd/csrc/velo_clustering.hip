@@ -702,32 +702,6 @@ __global__ void __launch_bounds__(masked_block) k_masked_clustering(
     module_cluster_num[event_number * n_module_pairs + i] = min(count[i], mp_start[i + 1] - mp_start[i]);
 }
 
-// (phi, id) rank of element i among n (SortByPhi.cu:90-125, including its tie rule).
-template<typename PhiT, typename IdT>
-__device__ __forceinline__ unsigned phi_rank(const PhiT* phi, const IdT* id, unsigned n, unsigned i)
-{
-  const int16_t pi = phi[i];
-  const uint32_t ii = id[i];
-  // Eight elements read at a time, so that their loads are in flight together.
-  unsigned position = 0, j = 0;
-  for (; j + 8 <= n; j += 8) {
-    int16_t p[8];
-    uint32_t d[8];
-#pragma unroll
-    for (unsigned u = 0; u < 8; ++u) {
-      p[u] = phi[j + u];
-      d[u] = static_cast<uint32_t>(id[j + u]);
-    }
-#pragma unroll
-    for (unsigned u = 0; u < 8; ++u) position += pi > p[u] || (i != j + u && pi == p[u] && ii > d[u]);
-  }
-  for (; j < n; ++j) {
-    const int16_t pj = phi[j];
-    position += pi > pj || (i != j && pi == pj && ii > (uint32_t) id[j]);
-  }
-  return position;
-}
-
 // (phi, id) as one unsigned 64-bit key: phi (signed) in the high word, offset to unsigned. Key
 // order is the sort's (phi, id) order (SortByPhi.cu:90-125), and distinct clusters of a module
 // pair have distinct ids, so the rank of a cluster is the number of keys below its own.
@@ -738,9 +712,11 @@ __device__ __forceinline__ uint64_t phi_id_key(int16_t phi, uint32_t id)
 
 // K4: one wave per (module pair, event). A cluster's rank is the number of clusters in the phi buckets
 // before its own and of those in its own with a smaller key, which it finds by their list; module pairs
-// of more than sort_lds_cap clusters compare every two. Equal keys (a word twice in a bank) share a
-// rank, and the slot they leave takes the container's first cluster, as the zero that its entry of the
-// permutation holds says. 500 pile-up events: 11 us (37 with 256 lanes that compared every two).
+// of more than sort_lds_cap clusters add up such ranks over tiles of them. Equal keys (a word twice
+// in a bank) share a rank, and the slot they leave takes the container's first cluster, as the zero
+// that its entry of the permutation holds says. 500 pile-up events: 11 us (37 with 256 lanes that
+// compared every two); 600 events of up to 960 clusters a module pair: 117 us (617, and 1190 where one
+// wave compared every two from memory).
 constexpr unsigned sort_lds_cap = 512;
 __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
   const uint32_t* event_list,
@@ -763,12 +739,14 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
   const Clusters out {sorted_container, total};
   const unsigned start = offsets_estimated_input_size[event_number * n_module_pairs + mp];
   const unsigned n = module_cluster_num[event_number * n_module_pairs + mp];
-  if (n <= sort_lds_cap) {
+  const auto key_of = [&](unsigned i) { return phi_id_key(in.phis()[start + i], in.ids()[start + i]); };
+  // Clusters [t0, t0 + tn) to LDS, in lists by the bucket of their phi.
+  const auto enter_tile = [&](unsigned t0, unsigned tn) {
     s_newest[l] = none;
     s_before[l] = 0;
     __syncthreads();
-    for (unsigned i = l; i < n; i += wave_size) {
-      const uint64_t key = phi_id_key(in.phis()[start + i], in.ids()[start + i]);
+    for (unsigned i = l; i < tn; i += wave_size) {
+      const uint64_t key = key_of(t0 + i);
       const unsigned bucket = static_cast<unsigned>(key >> 42);
       s_key[i] = key;
       s_taken[i] = 0;
@@ -780,6 +758,20 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
     __syncthreads();
     s_before[l] = before;
     __syncthreads();
+  };
+  // The tile's clusters below `key`.
+  const auto below = [&](uint64_t key) {
+    const unsigned bucket = static_cast<unsigned>(key >> 42);
+    unsigned rank = s_before[bucket];
+    for (unsigned j = s_newest[bucket]; j != none;) {
+      const uint64_t other = s_key[j];
+      j = s_next[j];
+      rank += other < key;
+    }
+    return rank;
+  };
+  if (n <= sort_lds_cap) {
+    enter_tile(0, n);
     const auto write = [&](size_t slot, size_t from, uint64_t key, float x, float y, float z) {
       hit_permutation[slot] = static_cast<uint32_t>(from);
       out.ids()[slot] = static_cast<uint32_t>(key);
@@ -792,13 +784,7 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
       const float* xyz = in.xyz() + 3 * (size_t)(start + i);
       const float x = xyz[0], y = xyz[1], z = xyz[2];
       const uint64_t key = s_key[i];
-      const unsigned bucket = static_cast<unsigned>(key >> 42);
-      unsigned rank = s_before[bucket];
-      for (unsigned j = s_newest[bucket]; j != none;) {
-        const uint64_t other = s_key[j];
-        j = s_next[j];
-        rank += other < key;
-      }
+      const unsigned rank = below(key);
       s_taken[rank] = 1;
       write(start + rank, start + i, key, x, y, z);
     }
@@ -807,8 +793,17 @@ __global__ void __launch_bounds__(wave_size) k_sort_by_phi(
       if (!s_taken[i]) write(start + i, 0, phi_id_key(in.phis()[0], in.ids()[0]), in.xyz()[0], in.xyz()[1], in.xyz()[2]);
     return;
   }
-  for (unsigned i = l; i < n; i += wave_size)
-    hit_permutation[start + phi_rank(in.phis() + start, in.ids() + start, n, i)] = start + i;
+  // The sum over the tiles is kept where the sorted container will have an id.
+  for (unsigned t0 = 0; t0 < n; t0 += sort_lds_cap) {
+    const bool last = n - t0 <= sort_lds_cap;
+    __syncthreads(); // the tile before has been read
+    enter_tile(t0, min(sort_lds_cap, n - t0));
+    for (unsigned i = l; i < n; i += wave_size) {
+      const unsigned rank = (t0 ? out.ids()[start + i] : 0u) + below(key_of(i));
+      if (last) hit_permutation[start + rank] = start + i;
+      else out.ids()[start + i] = rank;
+    }
+  }
   __threadfence_block();
   __syncthreads();
   for (unsigned i = l; i < n; i += wave_size) {

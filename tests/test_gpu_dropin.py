@@ -24,6 +24,9 @@ CASES = {
     # MEP layout (mep_layout = 1): the same kind of events as fragments grouped by bank.
     "mep_v4_subset": (dict(n_events=30, pileup=1, nu=7.6, seed=67), 24, 5, [20, 3, 11, 7, 0]),
     "mep_v2_subset": (dict(n_events=16, pileup=0, mean_tracks=100.0, bank_version=2, seed=68), 12, 2, [9, 4, 6]),
+    # Events beyond what the launches keep in LDS: more than 4096 track hits and 2047 tracks in an event
+    # (consolidation's binary search), more than 512 clusters in a module pair (the sort's tiles).
+    "v4_crowded": (dict(n_events=7, pileup=1, nu=160.0, seed=70), 6, 1, [4, 1, 2]),
 }
 
 
@@ -104,6 +107,9 @@ def test_sp_drop_ins_with_event_list(case, geometry, beamline, constants):
     assert np.all(gpu["estimated_input_size"].reshape(-1, 26)[unlisted] == 0)
     if len(event_list):
         assert ref["offsets_all_velo_tracks"][-1] > 0
+    if case == "v4_crowded":
+        hits = np.diff(ref["offsets_velo_track_hit_number"].astype(np.int64)[ref["offsets_all_velo_tracks"].astype(np.int64)])
+        assert hits.max() > 4096 and counts.max() > 2047 and ref["module_cluster_num"].max() > 1024
     # The host totals the sequence read back equal the oracle's.
     assert args.host["number_of_reconstructed_velo_tracks"] == int(ref["offsets_all_velo_tracks"][-1])
     assert args.host["total_number_of_velo_clusters"] == int(ref["offsets_estimated_input_size"][-1])
