@@ -170,7 +170,9 @@ __global__ void __launch_bounds__(wave_size) k_retina_sensor_sizes(
 // DecodeRetinaClusters.cu:11-395 for one (event, module pair) per wave. Bound by the chain of dependent
 // reads (slot, bank, header, word, geometry), so the slots' banks are looked up once, by a lane each,
 // and the first 128 words stay decoded for the second pass; the rank of a word comes from the words
-// of its phi bucket, where it was a comparison with every word. 1000 pile-up events: 33 us (90).
+// of its phi bucket, where it was a comparison with every word; beyond key_cap words it is summed over
+// tiles of them. 1000 pile-up events: 33 us (90); 200 events at nu = 60: 88 us (620, and 1340 where a
+// word was compared with every word in memory).
 template<int version>
 __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
   const char* raw,
@@ -250,6 +252,35 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
     if (k < n && k - before < L.n_words[t]) d = decode<version>(g, L.source[t], L.word[t][k - before]);
     return d;
   };
+  // Word k of the slice's tile, in the list of its bucket.
+  auto enter = [&](unsigned k, int64_t key) {
+    const unsigned bucket = bucket_of(key);
+    L.key[k] = key;
+    atomicAdd(&L.before[bucket], 1u);
+    L.next[k] = static_cast<uint16_t>(atomicExch(&L.newest[bucket], k));
+  };
+  // From the number of words in each bucket to those in the buckets before it.
+  auto count_before = [&]() {
+    wave_sync_lds();
+    const uint32_t count = L.before[l], before = wave_inclusive_scan(count) - count;
+    wave_sync_lds();
+    L.before[l] = before;
+    wave_sync_lds();
+  };
+  // The tile's words below a key; last: none of them beyond position i has the key.
+  auto below = [&](int64_t key, int i, bool& last) {
+    const unsigned bucket = bucket_of(key);
+    uint32_t position = L.before[bucket];
+    last = true;
+    for (unsigned j = L.newest[bucket]; j != none;) {
+      const int64_t o = L.key[j];
+      const unsigned next = L.next[j];
+      position += key > o;
+      last = last && !(static_cast<int>(j) > i && o == key);
+      j = next;
+    }
+    return position;
+  };
   uint32_t nonzero = 0;
   Decoded kept[2] {}; // the lane's first two words, for the ranking pass
   auto first_pass = [&](unsigned k) {
@@ -257,12 +288,7 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
     if (k >= n) return d;
     const int64_t key = d.valid ? d.key : 0x7FFFFFFFFFFFFFFFll;
     hit_sorting_key[lo + k] = key;
-    if (in_lds) {
-      const unsigned bucket = bucket_of(key);
-      L.key[k] = key;
-      atomicAdd(&L.before[bucket], 1u);
-      L.next[k] = static_cast<uint16_t>(atomicExch(&L.newest[bucket], k));
-    }
+    if (in_lds) enter(k, key);
     if (d.valid) nonzero += d.key != 0x7FFFFFFFFFFFFFFFll;
     else hit_permutations[lo + k] = 0;
     return d;
@@ -274,45 +300,51 @@ __global__ void __launch_bounds__(waves_per_block* wave_size) k_retina_decode(
   for (unsigned d = 32; d > 0; d >>= 1) nonzero += __shfl_xor(nonzero, d, wave_size);
   if (l == 0) module_cluster_num[event_number * n_module_pairs + mp] = nonzero;
   if (in_lds) {
-    wave_sync_lds();
-    const uint32_t count = L.before[l], before = wave_inclusive_scan(count) - count;
-    wave_sync_lds();
-    L.before[l] = before;
-    wave_sync_lds();
+    count_before();
   }
   else {
+    // More words: the tiles' positions of a word are added up in its entry of the permutation, in the
+    // bits above bit 0, which the word's tile or a later one sets where the word isn't the last of its key.
     __threadfence_block();
     __builtin_amdgcn_wave_barrier();
+    for (unsigned t0 = 0; t0 < n; t0 += key_cap) {
+      if (t0) {
+        wave_sync_lds(); // the tile before has been read
+        L.newest[l] = none;
+        L.before[l] = 0;
+        wave_sync_lds();
+      }
+      for (unsigned k = l; k < min(key_cap, n - t0); k += wave_size) enter(k, hit_sorting_key[lo + t0 + k]);
+      count_before();
+      for (unsigned i = l; i < n; i += wave_size) {
+        const uint32_t sum = t0 ? hit_permutations[lo + i] : 0u;
+        bool last;
+        const uint32_t more = below(hit_sorting_key[lo + i], static_cast<int>(i) - static_cast<int>(t0), last);
+        hit_permutations[lo + i] = (sum + 2 * more) | (last ? 0u : 1u);
+      }
+    }
   }
 
   // Rank by key; the last word of a key's run writes the slot.
   const Clusters out {cluster_container, total};
   auto second_pass = [&](unsigned i, const Decoded& d) {
-    if (!d.valid) return;
-    unsigned position = 0;
-    bool last = true;
+    if (i >= n) return;
+    if (!d.valid) {
+      if (!in_lds) hit_permutations[lo + i] = 0;
+      return;
+    }
+    uint32_t position;
+    bool last;
     if (in_lds) {
-      const unsigned bucket = bucket_of(d.key);
-      position = L.before[bucket];
-      for (unsigned j = L.newest[bucket]; j != none;) {
-        const int64_t o = L.key[j];
-        const unsigned next = L.next[j];
-        position += d.key > o;
-        last = last && !(j > i && o == d.key);
-        j = next;
-      }
+      position = below(d.key, static_cast<int>(i), last);
     }
     else {
-      const int64_t* keys = hit_sorting_key + lo;
-      for (unsigned j = 0; j < n; ++j) {
-        const int64_t o = keys[j];
-        position += d.key > o;
-        last = last && !(j > i && o == d.key);
-      }
+      position = hit_permutations[lo + i] >> 1;
+      last = !(hit_permutations[lo + i] & 1u);
     }
-    hit_permutations[lo + i] = lo + position;
+    const unsigned slot = lo + position;
+    hit_permutations[lo + i] = slot;
     if (last) {
-      const unsigned slot = lo + position;
       out.ids()[slot] = d.id;
       out.xyz()[3 * (size_t) slot] = d.x;
       out.xyz()[3 * (size_t) slot + 1] = d.y;

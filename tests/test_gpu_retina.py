@@ -55,6 +55,42 @@ def test_retina_sequence_matches_oracle(name, geometry, beamline, constants):
         assert ref["offsets_all_velo_tracks"][-1] > 0
 
 
+@pytest.mark.parametrize("version", [3, 4])
+@pytest.mark.parametrize("nu", [60.0, 150.0])
+def test_module_pairs_beyond_the_keys_kept_in_lds(nu, version, geometry, beamline, constants):
+    """Module pairs of more than 512 words, which are ranked tile by tile, with words that are repeated
+    within a tile and in another and with zero words: keys, ranks, counts and the cluster that
+    every written slot holds equal the oracle's."""
+    ev = synth.generate(n_events=3, pileup=1, nu=nu, seed=57, retina=1, bank_version=version)
+    raw, s16 = ev.raw.copy(), ev.sizes.view("<u2")
+    for e in range(ev.n_events):
+        base = int(ev.offsets[e])
+        nb = int(raw[base:base + 4].view("<u4")[0])
+        boff = raw[base + 4:base + 8 + 4 * nb].view("<u4").astype(np.int64)
+        for b in range(0, nb, 5):
+            at = base + 8 + 4 * nb + int(boff[b]) + (8 if version == 3 else 4)
+            words = raw[at:base + 8 + 4 * nb + int(boff[b + 1])].view("<u4") if b + 1 < nb else raw[:0].view("<u4")
+            if words.size > 8:
+                words[1], words[-2], words[-1] = words[0], words[2], 0
+    ev = synth.dataclasses.replace(ev, raw=raw)
+    ref = oracle.run(ev, geometry, beamline, compute_f64=0)
+    est = ref["offsets_estimated_input_size"].astype(np.int64)
+    assert np.diff(est).max() > (1024 if nu > 100 else 512) and np.diff(est).min() < 512
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    seq.run(velo.DeviceEvents(ev))
+    got = {k: seq.fetch(k, ref[k].dtype, ref[k].size) for k in
+           ("offsets_estimated_input_size", "module_cluster_num", "hit_sorting_key", "hit_permutations")}
+    container = seq.fetch("sorted_velo_cluster_container", np.uint8, 18 * int(est[-1]))
+    seq.close()
+    for k, v in got.items():
+        np.testing.assert_array_equal(v, ref[k], err_msg=k)
+    written = np.unique(ref["hit_permutations"])
+    assert written.size < est[-1]  # equal keys share a slot
+    for a, b in zip(parity.cluster_views(container, int(est[-1])),
+                    parity.cluster_views(ref["sorted_velo_cluster_container"], int(est[-1]))):
+        np.testing.assert_array_equal(a[written].view(np.uint8), b[written].view(np.uint8))
+
+
 def test_retina_drop_in_entry_points(geometry, beamline, constants):
     """calculate_number_of_retinaclusters_each_sensor_pair and decode_retinaclusters called
     one by one through the C ABI, with an event list, equal the oracle."""
