@@ -508,6 +508,7 @@ int velo_search_by_triplet(const velo_search_by_triplet_params* p, hipStream_t s
   a.block_dim = p->block_dim_x;
   a.lds_hits = 0;
   a.work_stats = nullptr;
+  a.mean_hits = p->host_total_number_of_velo_clusters / std::max(p->event_list_size, 1u);
   // The reference's memsets (SearchByTriplet.cu:47-49): events left out of dev_event_list keep
   // zero track counts and atomics, and no hit is marked used.
   int rc = hip_status(velo::launch_fill_u32(
@@ -931,6 +932,14 @@ int velo_sequence_set_tuning(velo_sequence* s, const char* knob, unsigned value)
   return VELO_ERR_INVALID_ARGUMENT;
 }
 
+// Hits per event, about, from what the host knows of a slice: a super pixel takes four bytes and makes
+// three quarters of a cluster, a retina word four bytes and makes one; the banks' headers add a tenth.
+static unsigned mean_hits_of(const velo_sequence_input& in)
+{
+  const size_t bytes = in.raw_input_bytes / in.number_of_events;
+  return static_cast<unsigned>(std::min<size_t>(in.retina ? bytes * 5 / 22 : bytes * 2 / 11, 1u << 30));
+}
+
 int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream_t stream)
 {
   if (!s || !in || !in->dev_velo_raw_input || !in->dev_velo_raw_input_offsets || !in->dev_velo_raw_input_sizes ||
@@ -1202,6 +1211,7 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
   k5.number_of_three_hit_tracks_output = s->get<uint32_t>("number_of_three_hit_tracks_output");
   k5.event_track_hits = s->get<uint32_t>("event_track_hits");
   k5.max_chi2 = in->max_chi2;
+  k5.mean_hits = mean_hits_of(*in);
   k5.block_dim = s->search_block;
   k5.lds_hits = s->search_lds_hits;
   k5.ring_window = s->search_ring_window;

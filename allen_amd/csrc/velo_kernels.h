@@ -225,7 +225,7 @@ struct SearchLaunch {
   float phi_tolerance;
   float max_scatter;
   unsigned max_skipped_modules;
-  unsigned block_dim;          // 0: the launcher's choice from the number of events (256 when scored or persistent)
+  unsigned block_dim;          // 0: the launcher's choice from the events (256 when scored or persistent)
   unsigned lds_hits;           // event hits staged in LDS (16 B each); 0: as block_dim
   unsigned long long* work_stats; // optional: seeding evals, forwarding evals, extrapolations, search steps
   unsigned long long* event_clock = nullptr; // optional: per event, event_clock_words u64 of wall clock ticks
@@ -236,6 +236,7 @@ struct SearchLaunch {
   // Scored mode: the scorer's FP32 parameters (mlp::n_params) and the logit threshold.
   const float* scorer_params = nullptr;
   float scorer_threshold = 0.f;
+  unsigned mean_hits = 0; // of an event, about (0: unknown); for the launcher's choices
   // LDS window of the ring of tracks to follow (a power of two, 64..512) and capacity of the
   // seeding's list of unused hits (a multiple of 16, up to 1024); 0: as block_dim.
   unsigned ring_window = 0;
@@ -401,7 +402,8 @@ hipError_t launch_search_split(
   hipEvent_t fork,
   hipEvent_t join);
 constexpr unsigned event_clock_words = 10; // start, end, ticks in 8 phases
-// Event hits staged in LDS by default: four workgroups of 256 lanes fit one CU's 160 KiB.
+// Event hits staged in LDS where the workgroup size is set or the grid persistent: with the window and
+// the list of those launches, three workgroups of 256 lanes fit one CU's 160 KiB.
 constexpr unsigned search_default_lds_hits = 1760;
 size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap);
 // order[0..n) = events by descending hit count (n read on the device).

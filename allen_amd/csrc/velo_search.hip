@@ -1546,7 +1546,15 @@ __global__ void __launch_bounds__(seed_mode == seed_mode_scored ? 256 : 1024, wa
       const GlobalHits hits {gxyz, gph, gused, gids, phi_tables};
       build_phi_tables(hits, sh.mp, phi_tables, hist, hist_waves, team);
       team.sync();
-      search_event<count, seed_mode>(wc, hits, ss, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
+      // The hits leave their LDS to the lists: such events are the ones whose module pairs are long.
+      SeedScratch long_lists = ss;
+      if (4 * a.lds_hits > a.list_cap) {
+        long_lists.list_cap = min(4 * a.lds_hits, unused_list_cap);
+        long_lists.unused = reinterpret_cast<uint16_t*>(dyn);
+        long_lists.before = long_lists.unused + long_lists.list_cap;
+      }
+      search_event<count, seed_mode>(
+        wc, hits, long_lists, sh, cn, o, team, a.phi_tolerance, a.max_scatter, a.max_skipped_modules);
       __threadfence_block(); // the used flags are read back from global memory
       team.sync();
       finish_event(hits, team, sh, cn, o, a, toff);
@@ -1663,33 +1671,48 @@ size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, un
 struct SearchShape {
   unsigned block, lds_hits, window, list_cap, hits_per_wave;
 };
+// Events of more hits than this on average (17 and 36 collisions) are crowded.
+constexpr unsigned crowded_hits = 2600, very_crowded_hits = 5600;
 // Few events: every event has its LDS to itself (two workgroups fit a CU), and the launch lasts as
 // long as its largest event: four waves for events from 2100 hits on, all hits in LDS (200 events
-// of up to 1700 hits: 123 us against 142 us with 1500 hits in LDS and coordinates from memory).
+// of up to 1700 hits: 123 us against 142 us with 1500 hits in LDS and coordinates from memory), lists
+// for module pairs of 1024 hits (200 events at nu = 45: 682 us; 942 with lists of 512). Up to
+// 1024 very crowded ones take it too (600 events at nu = 60: 1065 us; 1373 with the next shape).
+// Crowded ones: what four workgroups a CU leave, with phi and flags of 8800 hits in it and the long
+// lists (1000 events at nu = 30: 592 us, 884 with the next shape; 2000 at nu = 45: 1426, 1982; 5000 at
+// nu = 30: 1942, 2870 with the last).
 // Up to 1024: all of them have to be in flight at once, so the LDS is what four
-// workgroups a CU leave (1000 pile-up events: 210 us; with 1760 hits 220 us, with 128-lane
-// workgroups 310 us, with 512 lanes 213 us). Up to 4096: five workgroups a CU, which their registers
-// allow (whole passes with five and four: 1100 one-vertex events 282 and 346 us, 3000 pile-up events 655
-// and 683 us, 2000 stress events 835 and 844 us). Beyond, the workgroups stream through the chip and the
-// most resident waves win: two waves per event and little LDS (20 000 events: 1.62 ms; 1.93 ms
-// with 256 lanes, 2.46 ms with 1500 hits in LDS, 4.32 ms with 256 lanes and 1760 hits before).
-static SearchShape search_shape(unsigned n_events)
+// workgroups a CU leave (1000 pile-up events: 174 us; with 2240 hits and three a CU 243 us; with
+// 128-lane workgroups 310 us, with 512 lanes 213 us when the pass took 210 us). Up to 4096: five
+// workgroups a CU, which their registers allow (whole passes with five and four: 1100 one-vertex events
+// 282 and 346 us, 3000 pile-up events 655 and 683 us, 2000 stress events 835 and 844 us). Beyond, the
+// workgroups stream through the chip and the most resident waves win: little LDS and two waves per event,
+// up to 6144 events as workgroups of four waves whose last two end at once unless the event is
+// large, since one large event of two waves outlasts these slices (5000 one-vertex events: 457 us, 411
+// with two; with 1 % of them at nu = 60: 909, 1468). 20 000 events: 1.45 ms; 1.73 ms with 256
+// lanes, 2.46 ms with 1500 hits in LDS, 4.32 ms with 256 lanes and 1760 hits before.
+static SearchShape search_shape(unsigned n_events, unsigned mean_hits)
 {
-  if (n_events <= 512) return {256, 3072, 1024, 512, 700};
+  if (n_events <= (mean_hits > very_crowded_hits ? 1024u : 512u)) return {256, 3072, 1024, 1024, 700};
+  if (mean_hits > crowded_hits) return {256, 1650, 512, 1024, 700};
   if (n_events <= 1024) return {256, 1500, 1024, 512, 700};
   if (n_events <= 4096) return {256, 1180, 512, 512, 700};
+  if (n_events <= 6144) return {256, 384, 512, 512, 1100};
   return {128, 384, 512, 512, 0};
 }
 
 // The same for the scored search, whose workgroups have 256 lanes (their size is part of the pruning
 // rule): 12 waves of it fit a CU by its registers, so up to 768 events are in flight at once and have
 // the LDS of three workgroups (300 one-vertex events, whole pass: 232 us; 257 with 1760 hits and a
-// window and a list of 1024). More of them take the instantiation of 16 waves a CU and the LDS that
-// four workgroups leave (777 events: 298 us, 371 with three; 1000 pile-up events: 375, 440).
+// window and a list of 1024; 200 events at nu = 45, search: 968 us; 1064 with a list of 512), as have up to 1024
+// crowded ones (777 events at nu = 30: 608 us; 834 with the next shape). More of them take the
+// instantiation of 16 waves a CU and the LDS that four workgroups leave (777 events: 298 us, 371 with
+// three; 1000 pile-up events: 375, 440).
 constexpr unsigned scored_waves_at_three = 3 * 4 * 256; // waves per SIMD, SIMDs, CUs
-static SearchShape scored_shape(unsigned n_events)
+static SearchShape scored_shape(unsigned n_events, unsigned mean_hits)
 {
-  if (n_events * (256 / wave_size) <= scored_waves_at_three) return {256, 2048, 1024, 512, 0};
+  if (n_events * (256 / wave_size) <= scored_waves_at_three || (n_events <= 1024 && mean_hits > crowded_hits))
+    return {256, 1920, 1024, 1024, 0};
   return {256, 1500, 512, 512, 0};
 }
 
@@ -1703,7 +1726,7 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   const bool scored = a.scorer_params != nullptr;
   const bool shaped = !a.block_dim && !a.work_counter;
   const SearchShape shape = !shaped ? SearchShape {256, search_default_lds_hits, ring_window, unused_list_cap, 0}
-                            : scored ? scored_shape(a.n_list) : search_shape(a.n_list);
+                            : scored ? scored_shape(a.n_list, a.mean_hits) : search_shape(a.n_list, a.mean_hits);
   const unsigned block = a.block_dim ? a.block_dim : shape.block;
   const unsigned hits_per_wave = shape.hits_per_wave;
   // Dynamic LDS stays within the device's per-workgroup limit (less the static part).

@@ -317,7 +317,7 @@ typedef struct {
   float phi_tolerance;              /* 0.045 */
   float max_scatter;                /* 0.08 */
   unsigned max_skipped_modules;     /* 1; above 7: no limit */
-  unsigned block_dim_x;             /* 0: chosen from the number of events */
+  unsigned block_dim_x;             /* 0: chosen from the number of events and their mean size */
 } velo_search_by_triplet_params;
 int velo_search_by_triplet(const velo_search_by_triplet_params* p, hipStream_t stream);
 /* track_container_size of SearchByTriplet.cu:18-28 */
@@ -472,7 +472,7 @@ int velo_sequence_status(velo_sequence* s, hipStream_t stream, unsigned* status)
 /* Knobs applied to subsequent runs:
  *   "search_block"      workgroup size of search_by_triplet (multiple of 64, <= 1024; 0,
  *                       the default: this and the shape's other knobs left at 0 are chosen from
- *                       the number of events; always 256 with the scorer or "search_persistent")
+ *                       the number of events and their mean size; always 256 with the scorer or "search_persistent")
  *   "search_lds_hits"   hits of an event staged in LDS by search_by_triplet (<= 8192, within the
  *                       device's LDS per workgroup; 0: as "search_block", 1760 for a workgroup
  *                       size that is set); up to 16/3 of that many hits keep phi

@@ -354,16 +354,45 @@ def test_module_pairs_at_the_limits_of_the_clustering_slices(nu, lowest, version
     assert not errs, "\n".join(errs[:20])
 
 
-@pytest.mark.parametrize("n_events", [513, 1025, 4097])
-def test_search_launch_shapes_by_number_of_events(n_events, geometry, beamline, constants):
-    """The smallest numbers of events that take the second, third and fourth shape of the search's launch,
-    with events of every LDS layout that it has: equal to the oracle."""
+@pytest.mark.parametrize("n_events,bytes_per_event", [(513, 0), (1025, 0), (4097, 0), (6145, 0), (513, 15000),
+                                                      (513, 32000), (1025, 32000)])
+def test_search_launch_shapes_by_number_of_events(n_events, bytes_per_event, geometry, beamline, constants):
+    """The smallest numbers of events that take the other shapes of the search's launch than the first, and
+    the shapes of crowded slices (the raw bytes are what the host knows of the events' size, and a
+    slice may state more than it fills). With the shape's own hits in LDS, and with 256, where the
+    events take every layout: equal to the oracle."""
     ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=12.0, high_occupancy_fraction=0.02, high_nu=14.0, seed=43)
-    ref, gpu, status = run_both(f"shape{n_events}", geometry, beamline, constants, True, events=ev)
-    assert int(ref["status"][0]) == 0 and status & velo.STATUS_OVERFLOW_MASK == 0
+    ref = oracle.run(ev, geometry, beamline)
+    assert int(ref["status"][0]) == 0
     hits = np.diff(ref["offsets_estimated_input_size"].astype(np.int64)[::26])
-    assert hits.min() < 384 and hits.max() > 2048
-    errs = parity.compare(gpu, ref, True)
+    assert hits.min() < 256 and hits.max() > 2048 and np.any((hits > 256) & (hits < 16 * 256 // 3))
+    stated = max(ev.raw.size, bytes_per_event * n_events)
+    seq = velo.VeloSequence(constants, n_events, stated)
+    dev = velo.DeviceEvents(ev)
+    for lds_hits in (0, 256):
+        seq.set_tuning("search_lds_hits", lds_hits)
+        seq.run(dev, raw_input_bytes=stated)
+        assert seq.status() & velo.STATUS_OVERFLOW_MASK == 0
+        errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+        assert not errs, f"search_lds_hits {lds_hits}:\n" + "\n".join(errs[:20])
+    seq.close()
+
+
+@pytest.mark.parametrize("lds_hits,list_cap", [(256, 64), (64, 64), (16, 64), (64, 512), (0, 0)])
+def test_unused_hit_lists_in_the_lds_of_the_hits(lds_hits, list_cap, geometry, beamline, constants):
+    """Events that are searched in memory keep the lists of unused hits where the hits would be, four
+    entries of both lists a hit and at most 1024, if that is more than list_cap; module pairs beyond
+    take the walk. Module pairs on both sides of 256 and of 512 hits and beyond: equal to the oracle."""
+    ev = synth.generate(n_events=3, pileup=1, nu=70.0, seed=49)
+    ref = oracle.run(ev, geometry, beamline)
+    pairs = np.diff(ref["offsets_estimated_input_size"].astype(np.int64))
+    assert int(ref["status"][0]) == 0 and pairs.max() > 512 and np.any((pairs > 64) & (pairs < 256))
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    seq.set_tuning("search_lds_hits", lds_hits)
+    seq.set_tuning("search_list_cap", list_cap)
+    seq.run(velo.DeviceEvents(ev))
+    errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+    seq.close()
     assert not errs, "\n".join(errs[:20])
 
 

@@ -86,16 +86,18 @@ def test_seed_log_matches_oracle(geometry, beamline):
     constants.close()
 
 
-def _scored_run(geometry, beamline, ev, params, threshold, log_cap=0, block=0):
+def _scored_run(geometry, beamline, ev, params, threshold, log_cap=0, block=0, lds_hits=0, bytes_per_event=0):
     from allen_amd import velo
     constants = velo.VeloConstants(geometry, beamline)
-    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    stated = max(ev.raw.size, bytes_per_event * ev.n_events)
+    seq = velo.VeloSequence(constants, ev.n_events, stated)
     if block:
         seq.set_tuning("search_block", block)
+    seq.set_tuning("search_lds_hits", lds_hits)
     if log_cap:
         seq.set_tuning("seed_log", log_cap)
     seq.set_scorer(params, threshold)
-    seq.run(velo.DeviceEvents(ev))
+    seq.run(velo.DeviceEvents(ev), raw_input_bytes=stated)
     return seq, constants
 
 
@@ -293,29 +295,34 @@ def test_mlp_kernels_at_wave_and_grid_edges(n):
     np.testing.assert_allclose(loss, ref.loss(x, y, p) / n, rtol=1e-4)
 
 
-@pytest.mark.parametrize("n_events", [768, 769])
-def test_scored_search_on_both_sides_of_its_launch_shapes(n_events, geometry, beamline):
-    """The most events that the scored search holds at three waves a SIMD, and one more, with events of
-    every LDS layout: with a threshold that keeps every seed it is the plain search; at the shipped
-    threshold its tracks are those of the launch whose workgroup size is set by hand."""
+@pytest.mark.parametrize("n_events,bytes_per_event", [(768, 0), (769, 0), (769, 15000)])
+def test_scored_search_on_both_sides_of_its_launch_shapes(n_events, bytes_per_event, geometry, beamline):
+    """The most events that the scored search holds at three waves a SIMD, and one more, ordinary and
+    crowded (by the slice's stated bytes). With the shape's own hits in LDS, and with 256, where the
+    events take every layout: with a threshold that keeps every seed it is the plain search; at the
+    shipped threshold its tracks are those of the launch whose workgroup size is set by hand."""
     import oracle
     from allen_amd import scorer, synth, velo
     from tests import parity
     ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=12.0, high_occupancy_fraction=0.02, high_nu=14.0, seed=85)
     ref = oracle.run(ev, geometry, beamline)
+    event_hits = np.diff(ref["offsets_estimated_input_size"].astype(np.int64)[::26])
+    assert event_hits.min() < 256 and event_hits.max() > 2048 and np.any((event_hits > 256) & (event_hits < 16 * 256 // 3))
     params, thr = scorer.trained()
-    seq, constants = _scored_run(geometry, beamline, ev, params, -1e30)
-    assert seq.status() & velo.STATUS_OVERFLOW_MASK == 0
-    errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
-    assert not errs, "\n".join(errs[:20])
-    seq.close()
-    constants.close()
-    hits = []
-    for block in (0, 256):
-        seq, constants = _scored_run(geometry, beamline, ev, params, thr, block=block)
-        tracks = int(seq.fetch("offsets_all_velo_tracks", np.uint32, n_events + 1)[-1])
-        offsets = seq.fetch("offsets_velo_track_hit_number", np.uint32, tracks + 1)
-        hits.append((offsets, seq.fetch("velo_track_hits", np.uint8, 16 * int(offsets[-1]))))
+    for lds_hits in (0, 256):
+        seq, constants = _scored_run(geometry, beamline, ev, params, -1e30, lds_hits=lds_hits, bytes_per_event=bytes_per_event)
+        assert seq.status() & velo.STATUS_OVERFLOW_MASK == 0
+        errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
+        assert not errs, "\n".join(errs[:20])
         seq.close()
         constants.close()
-    assert np.array_equal(hits[0][0], hits[1][0]) and np.array_equal(hits[0][1], hits[1][1])
+        hits = []
+        for block in (0, 256):
+            seq, constants = _scored_run(geometry, beamline, ev, params, thr, block=block, lds_hits=lds_hits,
+                                         bytes_per_event=bytes_per_event)
+            tracks = int(seq.fetch("offsets_all_velo_tracks", np.uint32, n_events + 1)[-1])
+            offsets = seq.fetch("offsets_velo_track_hit_number", np.uint32, tracks + 1)
+            hits.append((offsets, seq.fetch("velo_track_hits", np.uint8, 16 * int(offsets[-1]))))
+            seq.close()
+            constants.close()
+        assert np.array_equal(hits[0][0], hits[1][0]) and np.array_equal(hits[0][1], hits[1][1])
