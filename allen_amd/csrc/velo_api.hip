@@ -438,6 +438,7 @@ int velo_masked_clustering(const velo_masked_clustering_params* p, hipStream_t s
   a.sp_fy = p->constants->dev_sp_fy;
   a.module_cluster_num = p->dev_module_cluster_num;
   a.cluster_container = p->dev_velo_cluster_container;
+  a.mean_hits = p->host_total_number_of_velo_clusters / std::max(p->event_list_size, 1u);
   rc = hip_status(velo::launch_masked_clustering(a, stream));
   if (rc == VELO_OK && p->dev_velo_clusters) {
     // MaskedVeloClustering.cu:519-522: {container, estimated total, 0} per listed event.
@@ -1172,6 +1173,7 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
       k3.sp_fy = s->constants->dev_sp_fy;
       k3.module_cluster_num = mcn;
       k3.cluster_container = s->get<char>("velo_cluster_container");
+      k3.mean_hits = mean_hits_of(*in);
       VELO_TRY(velo::launch_masked_clustering(k3, stream));
       velo::SortLaunch k4;
       k4.event_list = nullptr;

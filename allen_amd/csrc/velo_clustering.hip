@@ -628,10 +628,21 @@ __global__ void __launch_bounds__(estimate_block) k_estimate_input_size(
   if (threadIdx.x == 0) module_candidate_num[event_number] = n_cand;
 }
 
-// K3: one workgroup per event. Phase 1 takes isolated SPs of all banks, phase 2 the candidates.
-constexpr unsigned masked_block = 1024;
+// K3: one workgroup per event. Phase 1 takes isolated SPs of all banks, phase 2 the candidates. Bound by
+// the latency of a wave's banks and candidates one after the other, so up to 512 events, which are all in
+// flight, get 16 waves each (500 pile-up events: 70 us; 78 with 8 waves, 124 with 4, 117 before).
+// With more of them waves that wait for their event's last ones are lost to other events: 8 waves up to
+// 2048 events, or beyond for crowded ones (2000 one-vertex events: 125 us; 183 with 16, 143
+// with 4 and before; 5000 at nu = 30: 1406, 1749, 1625 and 1566), else 4 (10 000 one-vertex events: 532 us;
+// 915 with 16, 586 with 8, 535 before).
+constexpr unsigned max_masked_block = 1024;
+static unsigned masked_block(unsigned n_events, unsigned mean_hits)
+{
+  if (n_events <= 512) return max_masked_block;
+  return n_events <= 2048 || mean_hits > crowded_hits ? 512 : 256;
+}
 template<int version>
-__global__ void __launch_bounds__(masked_block) k_masked_clustering(
+__global__ void __launch_bounds__(max_masked_block) k_masked_clustering(
   const char* raw,
   const uint32_t* offsets,
   const uint32_t* sizes,
@@ -674,11 +685,13 @@ __global__ void __launch_bounds__(masked_block) k_masked_clustering(
       if (!(w & 0x80000000u)) continue;
       ClusterSeed s0, s1;
       const unsigned n = isolated_sp_clusters<version>(sp_patterns, sp_fx, sp_fy, bank.sourceID, w, s0, s1);
+      const ClusterOut c0 = place_cluster(g, seed_sensor<version>(s0), s0);
+      ClusterOut c1;
+      if (n > 1) c1 = place_cluster(g, seed_sensor<version>(s1), s1);
       const unsigned slot = atomicAdd(&count[mp], n);
       const unsigned cap = mp_start[mp + 1] - mp_start[mp];
-      if (slot < cap) store_cluster(clusters, mp_start[mp] + slot, place_cluster(g, seed_sensor<version>(s0), s0));
-      if (n > 1 && slot + 1 < cap)
-        store_cluster(clusters, mp_start[mp] + slot + 1, place_cluster(g, seed_sensor<version>(s1), s1));
+      if (slot < cap) store_cluster(clusters, mp_start[mp] + slot, c0);
+      if (n > 1 && slot + 1 < cap) store_cluster(clusters, mp_start[mp] + slot + 1, c1);
     }
   }
   __syncthreads();
@@ -693,8 +706,8 @@ __global__ void __launch_bounds__(masked_block) k_masked_clustering(
     if (masked_cluster<version>(bank.word, bank_n_sp<version>(bank), cand >> 11, sensor_number, cand & 7u, &c)) {
       const unsigned mp = sensor_number / 8;
       const unsigned slot = atomicAdd(&count[mp], 1u);
-      if (mp < n_module_pairs && slot < mp_start[mp + 1] - mp_start[mp]) 
-        store_cluster(clusters, mp_start[mp] + slot, place_cluster(g, sensor_number, c));
+      const ClusterOut placed = place_cluster(g, sensor_number, c);
+      if (mp < n_module_pairs && slot < mp_start[mp + 1] - mp_start[mp]) store_cluster(clusters, mp_start[mp] + slot, placed);
     }
   }
   __syncthreads();
@@ -872,7 +885,7 @@ hipError_t launch_masked_clustering(const MaskedClusteringLaunch& a, hipStream_t
   if (!a.n_list) return hipSuccess;
 #define VELO_LAUNCH_MC(V)                                                                                           \
   hipLaunchKernelGGL(                                                                                               \
-    k_masked_clustering<V>, dim3(a.n_list), dim3(masked_block), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,      \
+    k_masked_clustering<V>, dim3(a.n_list), dim3(masked_block(a.n_list, a.mean_hits)), 0, s, a.raw, a.offsets, a.sizes, a.types, unsigned(a.mep), a.event_list,      \
     a.event_start, a.number_of_events, a.offsets_estimated_input_size, a.module_candidate_num, a.cluster_candidates, \
     a.candidates_offsets, a.bank_index, reinterpret_cast<const Geometry*>(a.geometry), a.sp_patterns, a.sp_fx,       \
     a.sp_fy, a.module_cluster_num, a.cluster_container)

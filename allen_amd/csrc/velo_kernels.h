@@ -125,6 +125,10 @@ struct EstimateLaunch {
   uint32_t* cluster_candidates;
 };
 
+// Slices whose events hold more hits than this on average (17 collisions) are crowded: launch shapes
+// differ.
+constexpr unsigned crowded_hits = 2600;
+
 struct MaskedClusteringLaunch {
   int version;
   const char* raw;
@@ -147,6 +151,7 @@ struct MaskedClusteringLaunch {
   const float* sp_fy;
   uint32_t* module_cluster_num;
   char* cluster_container;
+  unsigned mean_hits = 0; // of an event, about (0: unknown); for the launcher's choice of the workgroup
 };
 
 struct SortLaunch {

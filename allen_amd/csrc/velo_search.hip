@@ -1671,8 +1671,7 @@ size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, un
 struct SearchShape {
   unsigned block, lds_hits, window, list_cap, hits_per_wave;
 };
-// Events of more hits than this on average (17 and 36 collisions) are crowded.
-constexpr unsigned crowded_hits = 2600, very_crowded_hits = 5600;
+constexpr unsigned very_crowded_hits = 5600; // 36 collisions
 // Few events: every event has its LDS to itself (two workgroups fit a CU), and the launch lasts as
 // long as its largest event: four waves for events from 2100 hits on, all hits in LDS (200 events
 // of up to 1700 hits: 123 us against 142 us with 1500 hits in LDS and coordinates from memory), lists

@@ -378,6 +378,23 @@ def test_search_launch_shapes_by_number_of_events(n_events, bytes_per_event, geo
     seq.close()
 
 
+@pytest.mark.parametrize("n_events,bytes_per_event", [(513, 0), (2049, 0), (2049, 15000)])
+def test_masked_clustering_workgroups_by_number_of_events(n_events, bytes_per_event, geometry, beamline, constants):
+    """The smallest numbers of events that take the masked clustering's smaller workgroups, and the larger
+    of these for crowded slices (by the slice's stated bytes), algorithm by algorithm: the clusters of
+    every module pair are the oracle's."""
+    ev = synth.generate(n_events=n_events, pileup=0, mean_tracks=3.0, high_occupancy_fraction=0.005, high_nu=30.0, seed=50)
+    ref = oracle.run(ev, geometry, beamline, compute_f64=0)
+    stated = max(ev.raw.size, bytes_per_event * n_events)
+    seq = velo.VeloSequence(constants, n_events, stated)
+    seq.set_tuning("fused_clustering", 0)
+    seq.run(velo.DeviceEvents(ev), raw_input_bytes=stated)
+    assert seq.status() & velo.STATUS_OVERFLOW_MASK == int(ref["status"][0]) == 0
+    errs = parity.compare(parity.gpu_buffers(seq, ref), ref, False)
+    seq.close()
+    assert not errs, "\n".join(errs[:20])
+
+
 @pytest.mark.parametrize("lds_hits,list_cap", [(256, 64), (64, 64), (16, 64), (64, 512), (0, 0)])
 def test_unused_hit_lists_in_the_lds_of_the_hits(lds_hits, list_cap, geometry, beamline, constants):
     """Events that are searched in memory keep the lists of unused hits where the hits would be, four
