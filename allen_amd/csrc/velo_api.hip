@@ -972,11 +972,16 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     ev_end = s->ev_pairs[s->n_timed].second;
     ++s->n_timed;
   }
+  // The three-hit filter is part of the search's launch, and the fit of the consolidation's: the launch
+  // that holds a stage is what its time is.
+  const unsigned timed = s->timed_stage == VELO_STAGE_THREE_HIT_FILTER ? unsigned(VELO_STAGE_SEARCH)
+                       : s->timed_stage == VELO_STAGE_KALMAN           ? unsigned(VELO_STAGE_CONSOLIDATE)
+                                                                       : s->timed_stage;
   auto mark_begin = [&](unsigned k) -> int {
-    return s->timed_stage == k ? hip_status(hipEventRecord(ev_begin, stream)) : VELO_OK;
+    return timed == k ? hip_status(hipEventRecord(ev_begin, stream)) : VELO_OK;
   };
   auto mark_end = [&](unsigned k) -> int {
-    return s->timed_stage == k ? hip_status(hipEventRecord(ev_end, stream)) : VELO_OK;
+    return timed == k ? hip_status(hipEventRecord(ev_end, stream)) : VELO_OK;
   };
 #define VELO_MARK(rc_expr)                                                                                          \
   do {                                                                                                              \
@@ -1250,10 +1255,6 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
     VELO_TRY(velo::launch_search_by_triplet(k5, stream));
   }
   VELO_MARK(mark_end(VELO_STAGE_SEARCH));
-  // The three-hit filter ran at the end of each event's search; the consolidation's launch holds
-  // the fit. Their stages' brackets are empty.
-  VELO_MARK(mark_begin(VELO_STAGE_THREE_HIT_FILTER));
-  VELO_MARK(mark_end(VELO_STAGE_THREE_HIT_FILTER));
   velo::TrackOffsetsLaunch k7;
   k7.n_events = E;
   k7.number_of_velo_tracks = k5.number_of_velo_tracks;
@@ -1286,8 +1287,6 @@ int velo_sequence_run(velo_sequence* s, const velo_sequence_input* in, hipStream
   VELO_TRY(velo::launch_track_offsets(k7, stream));
   VELO_TRY(velo::launch_consolidate_and_fit(k8, stream));
   VELO_MARK(mark_end(VELO_STAGE_CONSOLIDATE));
-  VELO_MARK(mark_begin(VELO_STAGE_KALMAN));
-  VELO_MARK(mark_end(VELO_STAGE_KALMAN));
   if (s->pv_finder) {
     velo::PVLaunch pv;
     pv.event_list = nullptr;

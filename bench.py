@@ -320,10 +320,10 @@ def main():
     if status & velo.STATUS_OVERFLOW_MASK:
         log(f"[bench] WARNING status {status:#x}: a fixed-capacity structure overflowed")
 
-    # Per-stage times (diagnostic, outside the timed region) to find the dominant kernel.
+    # Per-stage times (diagnostic, outside the timed region) to find the dominant kernel. The three-hit filter
+    # is part of the search's launch, the fit of the consolidation's.
     stage_ms = {}
-    for stage in ["candidates", "estimate", "clustering", "search", "three_hit_filter", "consolidate", "kalman"] + \
-            (["pv"] if args.pv_finder else []):
+    for stage in ["candidates", "estimate", "clustering", "search", "consolidate"] + (["pv"] if args.pv_finder else []):
         seq.time_stage(stage)
         for _ in range(2):
             seq.run(dev)

@@ -509,10 +509,10 @@ enum {
   VELO_STAGE_CANDIDATES = 2,       /* velo_calculate_number_of_candidates */
   VELO_STAGE_ESTIMATE = 3,         /* velo_estimate_input_size */
   VELO_STAGE_CLUSTERING = 4,       /* masked clustering + sort by phi */
-  VELO_STAGE_SEARCH = 5,           /* velo_search_by_triplet */
-  VELO_STAGE_THREE_HIT_FILTER = 6, /* nothing: the filter is part of the search's launch */
-  VELO_STAGE_CONSOLIDATE = 7,      /* track offsets, consolidation and the Kalman fit, one launch */
-  VELO_STAGE_KALMAN = 8,           /* nothing: see VELO_STAGE_CONSOLIDATE */
+  VELO_STAGE_SEARCH = 5,           /* search_by_triplet with the three-hit filter, one launch */
+  VELO_STAGE_THREE_HIT_FILTER = 6, /* the launch that holds it: as VELO_STAGE_SEARCH */
+  VELO_STAGE_CONSOLIDATE = 7,      /* track offsets, then consolidation with the Kalman fit */
+  VELO_STAGE_KALMAN = 8,           /* the launches that hold it: as VELO_STAGE_CONSOLIDATE */
   VELO_STAGE_PV = 9,               /* the beamline PV finder (knob "pv_finder") */
   VELO_STAGE_COUNT = 9
 };

@@ -269,6 +269,30 @@ def test_captured_sequence_replays(geometry, beamline, constants):
     seq.close()
 
 
+def test_times_of_the_stages_that_share_a_launch(geometry, beamline, constants):
+    """The time of the three-hit filter is that of the search's launch, and the fit's that of the
+    consolidation's, which hold them."""
+    ev = synth.generate(n_events=400, pileup=1, nu=12.0, seed=25)
+    dev = velo.DeviceEvents(ev)
+    seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    seq.run(dev)
+    ms = {}
+    for stage in velo.STAGES:
+        if stage == "pv":
+            continue
+        seq.time_stage(stage)
+        for _ in range(5):
+            seq.run(dev)
+        total, runs = seq.stage_ms()
+        assert runs == 5
+        ms[stage] = total
+    seq.time_stage(None)
+    seq.close()
+    for part, whole in (("three_hit_filter", "search"), ("kalman", "consolidate")):
+        assert 0.5 * ms[whole] < ms[part] < 2.0 * ms[whole]
+    assert all(0.0 < v < 1.2 * ms["all"] for v in ms.values())
+
+
 def test_autotune_keeps_outputs(geometry, beamline, constants):
     """A reduced autotuner sweep: every candidate reproduces the default outputs (the tuner raises
     otherwise) and the chosen knobs are applied to the sequence."""
