@@ -58,7 +58,9 @@ THROUGHPUT_CANDIDATES = tuple({"search_block": b, "search_lds_hits": h}
 
 
 def default_knobs() -> dict:
-    return {"search_block": 256, "search_lds_hits": 0, "search_persistent": 0, "search_largest_first": 1}
+    """The library's own: the launch's shape from the number of events and their size."""
+    return {"search_block": 0, "search_lds_hits": 0, "search_ring_window": 0, "search_list_cap": 0,
+            "search_persistent": 0, "search_largest_first": 1}
 
 
 def apply(seq: velo.VeloSequence, knobs: dict) -> None:
@@ -153,26 +155,29 @@ def tune_throughput(seqs, measure, n_events: int, candidates=THROUGHPUT_CANDIDAT
 
 def tune(seq: velo.VeloSequence, dev: velo.DeviceEvents, reps: int = 3, cache: str | None = None,
          blocks=BLOCKS, lds_hits=LDS_HITS, log=None) -> Result:
-    """Sweeps the knobs on `dev`'s events, applies the fastest result-preserving set to `seq`."""
-    apply(seq, default_knobs())
+    """Sweeps the knobs on `dev`'s events, applies the fastest result-preserving set to `seq`: never
+    one slower here than the library's own choice. Knobs that a candidate leaves out are the defaults."""
+    default = default_knobs()
+    apply(seq, default)
     seq.run(dev)
     reference = _outputs_digest(seq, dev.n_events)
-    key = f"{_device_name()}|{workload_signature(dev, seq)}"
+    # The default is part of the key: what another default was compared with says nothing about this one.
+    key = f"{_device_name()}|{workload_signature(dev, seq)}|block{default['search_block']}"
     if cache and os.path.exists(cache):
         stored = json.load(open(cache)).get(key)
         if stored:
             apply(seq, stored["knobs"])
             return Result(stored["knobs"], stored["search_ms"], stored["default_search_ms"], stored.get("trials", []))
     default_ms = _time_search(seq, dev, reps)
-    best_knobs, best_ms = default_knobs(), default_ms
+    best_knobs, best_ms = default, default_ms
     trials = []
     candidates = []
     for persistent in (0, 1):
         for order in (1, 0):
             for b in blocks:
                 for h in lds_hits:
-                    candidates.append({"search_block": b, "search_lds_hits": h, "search_persistent": persistent,
-                                       "search_largest_first": order})
+                    candidates.append({**default, "search_block": b, "search_lds_hits": h,
+                                       "search_persistent": persistent, "search_largest_first": order})
     for knobs in candidates:
         apply(seq, knobs)
         seq.run(dev)

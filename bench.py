@@ -463,7 +463,7 @@ def main():
 
     # The NN-pruned leg: the same events, streams and search knobs with the learned seed scorer
     # pruning seeds (its groups of seeds must lie in one wave: workgroups of 64, 128 or 256
-    # lanes, else 256), timed the same way.
+    # lanes, else the library's choice), timed the same way.
     nn = None
     if args.nn_pruned:
         from allen_amd import scorer
@@ -474,8 +474,8 @@ def main():
         threshold = shipped_threshold if args.threshold is None else args.threshold
         nn_knobs = {k: v for k, v in knobs.items() if k in ("search_block", "search_lds_hits", "search_ring_window",
                                                              "search_list_cap")}
-        if nn_knobs.get("search_block", 256) not in (64, 128, 256):
-            nn_knobs = {"search_block": 256, "search_lds_hits": 0, "search_ring_window": 0, "search_list_cap": 0}
+        if nn_knobs.get("search_block", 0) not in (0, 64, 128, 256):
+            nn_knobs = {"search_block": 0, "search_lds_hits": 0, "search_ring_window": 0, "search_list_cap": 0}
         for sq in seqs:
             for k, v in nn_knobs.items():
                 sq.set_tuning(k, v)

@@ -295,14 +295,22 @@ def test_times_of_the_stages_that_share_a_launch(geometry, beamline, constants):
 
 def test_autotune_keeps_outputs(geometry, beamline, constants):
     """A reduced autotuner sweep: every candidate reproduces the default outputs (the tuner raises
-    otherwise) and the chosen knobs are applied to the sequence."""
+    otherwise), what they are compared with is the library's default, and the chosen knobs are applied
+    to the sequence."""
     from allen_amd import autotune
     ev = synth.generate(**DATASETS["pileup"])
     dev = velo.DeviceEvents(ev)
     seq = velo.VeloSequence(constants, ev.n_events, ev.raw.size)
+    first = []
+    set_tuning = seq.set_tuning
+    seq.set_tuning = lambda k, v: (first.append((k, v)), set_tuning(k, v))
+    none = autotune.tune(seq, dev, reps=3, blocks=())
+    assert none.trials == [] and none.knobs == autotune.default_knobs()
+    assert all((k, 0) in first for k in ("search_block", "search_lds_hits", "search_ring_window", "search_list_cap"))
+    assert not any(k == "search_block" and v for k, v in first)  # the time compared with is the library's own
     res = autotune.tune(seq, dev, reps=1, blocks=(64, 256), lds_hits=(512, 1760))
     assert len(res.trials) == 16 and res.search_ms <= res.default_search_ms
-    assert res.knobs["search_block"] in (64, 256)
+    assert res.knobs["search_block"] in (0, 64, 256)
     seq.run(dev)
     ref = oracle.run(ev, geometry, beamline)
     errs = parity.compare(parity.gpu_buffers(seq, ref), ref, True)
