@@ -408,8 +408,8 @@ hipError_t launch_search_split(
   hipEvent_t join);
 constexpr unsigned event_clock_words = 10; // start, end, ticks in 8 phases
 // Event hits staged in LDS where the workgroup size is set or the grid persistent: with the window and
-// the list of those launches, three workgroups of 256 lanes fit one CU's 160 KiB.
-constexpr unsigned search_default_lds_hits = 1760;
+// the list of those launches, four workgroups of 64 lanes or three of 128 or more fit a CU's 160 KiB.
+constexpr unsigned search_default_lds_hits = 1740;
 size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap);
 // order[0..n) = events by descending hit count (n read on the device).
 hipError_t launch_order_events_by_hits(

@@ -26,10 +26,10 @@ constexpr unsigned mixed_bytes_per_hit = 3;
 // (a launch parameter, at most 1024); a larger module pair takes the pendulum walk.
 constexpr unsigned unused_list_cap = 1024;
 // Number of tracks to follow kept in LDS, the last positions of the ring (which is written through
-// to HBM and holds all max_tracks_to_follow): a launch parameter, a power of two from 64 to 512,
-// by default 1024. A forwarding step reads the ring and the tracks back from HBM when its entries
-// and those it writes exceed the window: at 512 positions that was the largest events, which set
-// the length of a launch.
+// to HBM and holds all max_tracks_to_follow): a power of two, 64 to 512 where the caller sets it and
+// 512 or 1024 where the launch chooses. A forwarding step reads the ring and the tracks back from HBM when
+// its entries and those it writes exceed the window: at 512 positions that was the largest events,
+// which set the length of a launch.
 constexpr unsigned ring_window = 1024;
 constexpr unsigned max_ring_window_knob = 512;
 static_assert(max_tracks_to_follow % ring_window == 0, "window positions follow ring positions");
@@ -1734,18 +1734,25 @@ hipError_t launch_search_by_triplet(const SearchLaunch& a, hipStream_t s)
   if (scored && block != 64 && block != 128 && block != 256) return hipErrorInvalidConfiguration;
   // The LDS window of the ring: a power of two from 64 to 512 (it divides the ring); the list
   // of unused hits: a multiple of 16 up to 1024 (relative positions fit 16 bits either way).
-  const unsigned window = a.ring_window ? a.ring_window : shape.window;
+  unsigned window = a.ring_window ? a.ring_window : shape.window;
   const unsigned list_cap = a.list_cap ? a.list_cap : shape.list_cap;
   if (window < 64 || a.ring_window > max_ring_window_knob || (window & (window - 1)) || list_cap % 16 || list_cap > unused_list_cap)
     return hipErrorInvalidValue;
   const size_t extra = scored ? scorer_lds_bytes + 16 : 0;
-  const size_t fixed = search_dynamic_lds(block, 0, window, list_cap) + extra + 1024;
-  if ((size_t) max_lds <= fixed) return hipErrorInvalidConfiguration;
-  const unsigned max_hits = static_cast<unsigned>(((size_t) max_lds - fixed) / search_bytes_per_hit);
   const unsigned default_hits =
     scored && !shaped ? search_default_lds_hits - static_cast<unsigned>((extra + search_bytes_per_hit - 1) / search_bytes_per_hit)
            : shape.lds_hits;
-  const unsigned lds_hits = min(a.lds_hits ? a.lds_hits : default_hits, max_hits);
+  const unsigned wanted_hits = a.lds_hits ? a.lds_hits : default_hits;
+  // Where the caller sets the workgroup or its hits, the long window must not cost a CU a workgroup
+  // (256 lanes and 4096 hits, 1000 pile-up events: 437 us with one workgroup a CU, 245 with two).
+  if (!a.ring_window && (!shaped || a.lds_hits)) {
+    const auto per_cu = [&](unsigned w) { return lds_per_cu / (search_dynamic_lds(block, wanted_hits, w, list_cap) + extra + 1024); };
+    if (per_cu(max_ring_window_knob) > per_cu(window)) window = max_ring_window_knob;
+  }
+  const size_t fixed = search_dynamic_lds(block, 0, window, list_cap) + extra + 1024;
+  if ((size_t) max_lds <= fixed) return hipErrorInvalidConfiguration;
+  const unsigned max_hits = static_cast<unsigned>(((size_t) max_lds - fixed) / search_bytes_per_hit);
+  const unsigned lds_hits = min(wanted_hits, max_hits);
   const size_t dyn = search_dynamic_lds(block, lds_hits, window, list_cap) + extra;
   // Persistent mode: as many workgroups as stay resident (they take events from the counter).
   unsigned grid = a.n_list;

@@ -472,9 +472,10 @@ int velo_sequence_status(velo_sequence* s, hipStream_t stream, unsigned* status)
 /* Knobs applied to subsequent runs:
  *   "search_block"      workgroup size of search_by_triplet (multiple of 64, <= 1024; 0,
  *                       the default: this and the shape's other knobs left at 0 are chosen from
- *                       the number of events and their mean size; always 256 with the scorer or "search_persistent")
+ *                       the number of events and their mean size; always 256 with the scorer or
+ *                       "search_persistent")
  *   "search_lds_hits"   hits of an event staged in LDS by search_by_triplet (<= 8192, within the
- *                       device's LDS per workgroup; 0: as "search_block", 1760 for a workgroup
+ *                       device's LDS per workgroup; 0: as "search_block", 1740 for a workgroup
  *                       size that is set); up to 16/3 of that many hits keep phi
  *                       and flags in LDS and coordinates in global memory, larger events run on
  *                       global memory

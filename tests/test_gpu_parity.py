@@ -148,6 +148,7 @@ def test_batched_mix_graph_replays(geometry, beamline, constants):
 TUNINGS = {
     "block64": {"search_block": 64},
     "block1024": {"search_block": 1024, "search_lds_hits": 2048},
+    "many_lds_hits": {"search_block": 256, "search_lds_hits": 4096},  # the ring's window gives way to them
     "mixed_lds": {"search_block": 256, "search_lds_hits": 600},   # phi + used in LDS, xyz global
     "global_hits": {"search_block": 128, "search_lds_hits": 64},  # everything in global memory
     "event_order": {"search_largest_first": 0},                   # events in their own order
