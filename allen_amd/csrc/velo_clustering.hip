@@ -4,10 +4,10 @@
 //   k_bank_index             VeloCalculateNumberOfCandidates.cu:35-43   last-writer-wins in CPU order
 //   k_estimate_input_size    EstimateInputSize.cu:10-239                one workgroup per event
 //   k_masked_clustering      MaskedVeloClustering.cu:131-576            one workgroup per event
-//   k_sort_by_phi            SortByPhi.cu:49-153                        one workgroup per module pair
-//   k_cluster_sorted         K2+K3+K4 fused: one workgroup per (event, module pair); the
-//                            module pair's SP words are staged in LDS, clusters are built and
-//                            rank-sorted by (phi, id) in LDS and written once, already sorted.
+//   k_sort_by_phi            SortByPhi.cu:49-153                        one wave per module pair
+//   k_bank_directory, k_estimate_mp, k_cluster_mp
+//                            the same for the whole sequence: the banks of every module pair,
+//                            then one wave per module pair for K2, and for K3 and K4 together
 //
 // The cluster arithmetic (pattern lookup, 64-bit mask growth, centroid, local->global
 // transform, hit_phi_16) is evaluated exactly as in the reference with fp contraction off.
@@ -1228,7 +1228,7 @@ __global__ void __launch_bounds__(mp::waves_per_block* wave_size) k_estimate_mp(
   }
 }
 
-// What one wave of k_cluster_mp holds in LDS: 5.8 KB, so that seven workgroups fit a CU.
+// What one wave of k_cluster_mp holds in LDS: 5.6 KB, so that 28 waves fit a CU.
 namespace mp {
 constexpr unsigned non_isolated_cap = 256; // non-isolated SP words of a module pair
 constexpr unsigned cluster_cap = 192;      // its clusters; more of them go through global memory

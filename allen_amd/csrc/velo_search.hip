@@ -214,8 +214,8 @@ struct WorkCount {
 };
 
 // forwarding; h1 compaction; seeding step 1 split into the h0 search (h1 and phi reads, then
-// the search in the previous module pair), the choice of the h0 candidates, and the wait at the
-// fence that ends the step; seeding steps 2 and 3; the rest.
+// the search in the previous module pair) and the choice of the h0 candidates; a place for a wait
+// that there is no more (always zero); the scoring of the pairs; the append; the rest.
 enum Phase {
   phase_forwarding,
   phase_compaction,
