@@ -38,7 +38,7 @@ HBM_PEAK_GBS = 8000.0                    # MI355X HBM3E
 VALU_PEAK_TOPS = 256 * 64 * 2.4e9 / 1e12  # 256 CUs x 64 lanes x 2.4 GHz, non-packed lane ops/s
 VALU_ISSUE_PEAK_G = 1024 * 2.4e9 / 4 / 1e9  # 1024 SIMDs, one wave64 VALU instruction per 4 cycles each
 LDS_PEAK_GBS = 256 * 256 * 2.4e9 / 1e9    # 256 CUs x 256 B/clk (CDNA4, 128-bit reads) x 2.4 GHz
-CPU_SHARE = 16                            # host cores that belong to one GPU of the box
+CPU_SHARE = 16                            # host cores that belong to one GPU
 
 
 def cpu_model() -> str:
@@ -124,7 +124,7 @@ def main():
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--cpu-threads", type=int, default=0,
                     help="threads of the CPU baseline; 0: the host cores this process may use, at most the 16 "
-                         "that are one GPU's share of the box (both figures are reported)")
+                         "that are one GPU's share of the host (both figures are reported)")
     ap.add_argument("--cpu-seconds", type=float, default=10.0,
                     help="CPU work of the all-core baseline sample (the single-thread sample takes half)")
     ap.add_argument("--search-block", type=int, default=0)
@@ -521,7 +521,7 @@ def main():
                         "platform level), default contraction",
                "cpu_model": cpu_model(), "host_cores_usable": usable,
                "cores_note": f"{threads} threads: the host cores usable here, at most the {CPU_SHARE} that are one "
-                             f"GPU's share of the box" if not args.cpu_threads else "set by --cpu-threads",
+                             f"GPU's share of the host" if not args.cpu_threads else "set by --cpu-threads",
                "sample": f"{sample.n_events} events of the same workload x {reps} repetitions, one event per task "
                          f"on {threads} std::threads ({secs:.1f} s); single thread: {sample.n_events} events x "
                          f"{reps1} repetitions ({secs1:.1f} s) -> {eps1:.1f} events/s",
