@@ -1660,11 +1660,22 @@ __global__ void k_three_hit_filter(
 constexpr size_t lds_per_cu = 160 * 1024;
 
 // Launch geometry: the seeding scratch, the ring window, the unused-hit list, then the hits.
-size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
+static constexpr size_t launch_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
 {
   return seed_scratch_bytes_per_lane * (size_t) block + window_bytes(window) + 2 * 2 * (size_t) list_cap +
          phi_tables_bytes + (size_t) lds_hits * search_bytes_per_hit;
 }
+size_t search_dynamic_lds(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
+{
+  return launch_lds(block, lds_hits, window, list_cap);
+}
+// The workgroups of a launch that the LDS of a CU holds.
+static constexpr unsigned workgroups_a_cu(unsigned block, unsigned lds_hits, unsigned window, unsigned list_cap)
+{
+  return static_cast<unsigned>(lds_per_cu / (launch_lds(block, lds_hits, window, list_cap) + sizeof(SearchShared) + 16));
+}
+static_assert(workgroups_a_cu(64, search_default_lds_hits, max_ring_window_knob, unused_list_cap) == 4, "default hits");
+static_assert(workgroups_a_cu(256, search_default_lds_hits, ring_window, unused_list_cap) == 3, "default hits");
 
 // Shape of a launch whose workgroup size is left to it: lanes, hits in LDS, ring window,
 // unused-hit list, and the hits of an event per working wave.
@@ -1699,6 +1710,8 @@ static SearchShape search_shape(unsigned n_events, unsigned mean_hits)
   if (n_events <= 6144) return {256, 384, 512, 512, 1100};
   return {128, 384, 512, 512, 0};
 }
+static_assert(workgroups_a_cu(256, 3072, 1024, 1024) == 2 && workgroups_a_cu(256, 1650, 512, 1024) == 4 &&
+              workgroups_a_cu(256, 1500, 1024, 512) == 4 && workgroups_a_cu(256, 1180, 512, 512) == 5, "the shapes' residency");
 
 // The same for the scored search, whose workgroups have 256 lanes (their size is part of the pruning
 // rule): 12 waves of it fit a CU by its registers, so up to 768 events are in flight at once and have
